@@ -56,6 +56,7 @@ enum WsSlot {
     WS_SOLVE1,     // solver reductions
     WS_SOLVE2,     // solver metadata
     WS_NET,        // preconditioner-network activations
+    WS_ERR,        // error flags raised by kernels (pinned, one word per device)
     WS_NSLOTS
 };
 void *workspace(int slot, size_t bytes, hipStream_t stream);

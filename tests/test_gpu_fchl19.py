@@ -101,3 +101,23 @@ def test_c_abi_device_resident(config0):
     Xo, dXo = oracle.fchl19_batch(C[:64], Q[:64], N[:64], grad=True)
     assert row_rel_err(X.numpy(), Xo, lead=2) < 1e-12
     assert row_rel_err(dX.numpy(), dXo, lead=2) < 1e-12
+
+
+# (atoms of the largest molecule, molecules, parameters): one atom to the most whose pair
+# records fit in LDS, batches that share a centre among 8, 2 and 1 work-groups, feature
+# blocks that do not fill a tile and ones that take several
+@pytest.mark.parametrize("ma,nm,kw", [
+    (1, 3, {}), (2, 1, {}), (3, 5, dict(nFourier=3)), (9, 40, dict(nRs2=41, nRs3=37)),
+    (13, 70, dict(nRs2=3, nRs3=1, nFourier=8)), (32, 2, dict(elements=[8])), (44, 1, {})])
+def test_jacobian_kernel_edges(fr, ma, nm, kw):
+    from kernelforge_amd import synthetic
+
+    rng = np.random.default_rng(100 * ma + nm)
+    el = np.array(kw.get("elements", [1, 6, 7, 8, 16]))
+    Ns = np.concatenate([[ma], rng.integers(1, ma + 1, nm - 1)]).astype(int)
+    C, Q, N = synthetic.pad_batch([synthetic._place_atoms(rng, n) for n in Ns],
+                                  [rng.choice(el, n).astype(np.int32) for n in Ns])
+    X, dX = fr.generate_fchl_acsf_batch(C, Q, N, with_gradients=True, **kw)
+    Xo, dXo = oracle.fchl19_batch(C, Q, N, grad=True, **kw)
+    assert row_rel_err(X, Xo, lead=2) < 1e-12
+    assert row_rel_err(dX, dXo, lead=2) < 1e-12
