@@ -11,18 +11,32 @@
 // (src/local_kernels.cpp:2895-3425).  Collecting terms per label, with
 //   beta_ij = (e/s^4) inner_ij + c_ij alpha_E[b(j)]
 //   G = C * ALPHA_DESC + B * X2 - diag(B 1) * X1
-// so each label is two FP64 MFMA GEMMs over packed rows:
-//   T = X1 [X2; ALPHA_DESC]^T            (query block x 2 R2, K = rep)
-//   elementwise: T -> [B | C] plus the per-row E and B 1 (one wave per query row)
-//   G = T [X2; ALPHA_DESC]               (query block x rep, K = 2 R2)
+// so each label is two FP64 MFMA products over packed rows:
+//   [S | P] = X1 [X2; ALPHA_DESC]^T, turned into T = [B | C] in registers
+//   G = T [X2; ALPHA_DESC]
 // then one pass over dX1 forms J_ai^T (G_ai - w_ai x_ai) per query atom, and per-
 // molecule sums in a fixed order (deterministic, no atomics).
+//
+// The products run over the descriptor columns that are non-zero in the training side
+// (X2 or ALPHA_DESC): the others add exact zeros to S, P and G whatever the query holds
+// (C9H8O4 conformers use 312 of 720).  All labels share each launch: the packed rows of a
+// label start at a multiple of 16 and are padded with zero rows to one, and a list of
+// segments (label, query rows) tells a wave which tile it has.  Operands go from global
+// memory straight into registers: the 16 values of a row that four MFMA steps need are
+// 32 contiguous bytes per lane when the summation index of a step is permuted the same way
+// in both operands (lane group g holds k = 4 g + u at step u), so no LDS tile and no
+// barrier is needed, and a product with a handful of query rows runs at the speed its
+// training rows can be read.
+//
+// Measured (whole calls on 21-atom C/H/O conformers, with the descriptors): one molecule
+// against 200 in a plan 84 us (2,110 before: one wave per atom for the back-projection,
+// 64-row tiles without splits for the products); 100 against 1,000, float32 in and out,
+// 2.6 ms (8.6), of which the two products 0.56 ms each at 36 TFLOP/s.
 #include <algorithm>
 #include <new>
 #include <cmath>
 #include <vector>
 
-#include "gemm_f64.hpp"
 #include "kf_common.hpp"
 #include "local_plan.hpp"
 
@@ -30,6 +44,8 @@ namespace kf {
 namespace {
 
 constexpr int NT = 256;
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
 
 __device__ inline double wave_sum(double v) {
 #pragma unroll
@@ -71,28 +87,86 @@ __global__ __launch_bounds__(NT) void alpha_desc_kernel(const double *__restrict
     }
 }
 
-// Gather packed rows: dst[r, :] = src[idx[r], :] for r < rows, with the squared
-// norm (n2) and optionally the dot with a second gathered matrix (dot).
-__global__ __launch_bounds__(NT) void gather_rows(const double *__restrict__ src,
-                                                  const double *__restrict__ src2,
-                                                  const int *__restrict__ idx, int rows, int rep,
-                                                  double *__restrict__ dst,
-                                                  double *__restrict__ dst2,
-                                                  double *__restrict__ n2,
-                                                  double *__restrict__ dot) {
+// One segment: a run of packed query rows of one label against the label's training rows.
+struct MvSeg {
+    int q0, R1;           // first packed query row, rows (q0 a multiple of 16)
+    int r2, R2, R2p;      // first packed training row, rows, rows padded to 16
+    int nsplit;           // splits of the summation over the training rows in G = T [X2; AD]
+    int it1, it2;         // first item of the segment in the two products' launches
+    size_t toff, goff, eoff;  // offsets into T, the partial G and the partial row sums
+};
+
+// Segment of item / row `x`: the last one whose start (by `at`) is not beyond it.
+template <class At>
+__device__ inline int find_seg(const MvSeg *segs, int nseg, int x, At at) {
+    int s = 0;
+    while (s + 1 < nseg && at(segs[s + 1]) <= x) ++s;
+    return s;
+}
+
+// flag[f] = 1 when column f is non-zero in X2 or AD for an atom of the training set.  A
+// work-group takes `per` molecules and its threads a column each, leaving a column at its
+// first non-zero value.
+__global__ __launch_bounds__(NT) void train_cols_kernel(const double *__restrict__ X2,
+                                                        const double *__restrict__ AD,
+                                                        const int *__restrict__ N, int nm, int ma,
+                                                        int rep, int per, int *__restrict__ flag) {
+    const int b0 = blockIdx.x * per, b1 = min(b0 + per, nm);
+    for (int f = threadIdx.x; f < rep; f += NT) {
+        bool nz = false;
+        for (int b = b0; b < b1 && !nz; ++b) {
+            const int nb = min(max(N[b], 0), ma);
+            const size_t base = (size_t)b * ma * rep + f;
+            for (int i = 0; i < nb && !nz; i += 4) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const size_t at = base + (size_t)min(i + u, nb - 1) * rep;
+                    nz |= (X2[at] != 0.0) | (AD[at] != 0.0);
+                }
+            }
+        }
+        if (nz) flag[f] = 1;
+    }
+}
+
+// Packed row r < rows takes source row src[r] (-1: a zero row) on the columns with
+// inv[f] >= 0 (its place in the packed row of nfp columns, the rest zero).  For a training
+// set (src2) row r goes to the stacked block of its segment, X2 rows first, then AD rows,
+// with |x|^2, x . ad and the molecule's alpha_E; for a query set to row r with |x|^2.
+__global__ __launch_bounds__(NT) void pack_rows_kernel(const double *__restrict__ src,
+                                                       const double *__restrict__ src2,
+                                                       const int *__restrict__ idx, int rows,
+                                                       int ma, int rep,
+                                                       const int *__restrict__ inv, int nf, int nfp,
+                                                       const MvSeg *__restrict__ segs, int nseg,
+                                                       const double *__restrict__ aE,
+                                                       double *__restrict__ dst,
+                                                       double *__restrict__ n2,
+                                                       double *__restrict__ dot,
+                                                       double *__restrict__ aEr) {
     const int lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= rows) return;
-    const double *s = src + (size_t)idx[r] * rep;
-    const double *s2 = src2 ? src2 + (size_t)idx[r] * rep : nullptr;
+    const int at = idx[r];
+    double *d = dst + (size_t)r * nfp, *da = nullptr;
+    if (src2) {
+        const MvSeg &S = segs[find_seg(segs, nseg, r, [](const MvSeg &t) { return t.r2; })];
+        d = dst + (size_t)(S.r2 + r) * nfp;
+        da = d + (size_t)S.R2p * nfp;
+    }
+    for (int f = nf + lane; f < nfp; f += 64) {
+        d[f] = 0.0;
+        if (da) da[f] = 0.0;
+    }
     double nn = 0.0, dd = 0.0;
     for (int f = lane; f < rep; f += 64) {
-        const double v = s[f];
-        dst[(size_t)r * rep + f] = v;
+        const int c = inv[f];
+        const double v = at >= 0 ? src[(size_t)at * rep + f] : 0.0;
+        if (c >= 0) d[c] = v;
         nn = fma(v, v, nn);
-        if (s2) {
-            const double w = s2[f];
-            dst2[(size_t)r * rep + f] = w;
+        if (src2) {
+            const double w = at >= 0 ? src2[(size_t)at * rep + f] : 0.0;
+            if (c >= 0) da[c] = w;
             dd = fma(v, w, dd);
         }
     }
@@ -101,162 +175,621 @@ __global__ __launch_bounds__(NT) void gather_rows(const double *__restrict__ src
     if (lane == 0) {
         n2[r] = nn;
         if (dot) dot[r] = dd;
+        if (aEr) aEr[r] = (aE && at >= 0) ? aE[at / ma] : 0.0;
     }
 }
 
-// T (rows x 2 R2) = [S | P] -> [B | C] in place, one wave per query row:
+// Work-group -> tile index, consecutive tiles on one XCD (work-groups are dealt round-robin
+// over eight of them) so that the waves that share an operand share an L2.
+__device__ inline int xcd_tile() {
+    const int g = blockIdx.x, G = gridDim.x;
+    return (G % 8 == 0) ? (g % 8) * (G / 8) + g / 8 : g;
+}
+
+// The four summation steps of 16 columns: k = 4 g + u at step u for lane group g.
+__device__ inline void load4(const double *p, double (&v)[4]) {
+    const v2d a = *reinterpret_cast<const v2d *>(p), b = *reinterpret_cast<const v2d *>(p + 2);
+    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+}
+
+// T = [B | C] of a tile of 16 MF query rows x 16 NFT training rows per wave (KW = 1) or per
+// work-group with its four waves each taking a quarter of the columns (KW = 4, for launches
+// with too few tiles to fill the GPU: one molecule against 200 conformers is 263 tiles).
 //   d2 = n1 + n2 - 2 S, e = exp(cexp d2), c = e / s^2, inner = P - rdot
 //   B = (e / s^4) inner + c aE,  C = c
-// Row outputs: erow = sum(e aE + c inner) (when wanted), wsum = sum(B).
-__global__ __launch_bounds__(NT) void coef_kernel(double *__restrict__ T, int rows, int R2,
-                                                  const double *__restrict__ n1,
-                                                  const double *__restrict__ n2,
-                                                  const double *__restrict__ rdot,
-                                                  const double *__restrict__ aE, double cexp,
-                                                  double inv_s2, const int *__restrict__ qsrc,
-                                                  double *__restrict__ erow,
-                                                  double *__restrict__ wsum) {
-    const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= rows) return;
-    double *S = T + (size_t)r * 2 * R2, *P = S + R2;
-    const double nq = n1[r];
-    double es = 0.0, ws = 0.0;
-    for (int t = lane; t < R2; t += 64) {
-        const double d2 = fmax(nq + n2[t] - 2.0 * S[t], 0.0);
-        const double e = exp(cexp * d2), c = e * inv_s2;
-        const double inner = P[t] - rdot[t];
-        const double ae = aE ? aE[t] : 0.0;
-        const double bco = c * inv_s2 * inner + c * ae;
-        es += e * ae + c * inner;
-        ws += bco;
-        S[t] = bco;
-        P[t] = c;
+// and per 16 training rows the row sums of e aE + c inner (ep) and of B (wp).
+template <int MF, int NFT, int KW>
+__global__ __launch_bounds__(NT, 2) void coef_kernel(
+    const MvSeg *__restrict__ segs, int nseg, int items, const double *__restrict__ Xq, int qrows,
+    const double *__restrict__ nq, const double *__restrict__ P2, const double *__restrict__ n2,
+    const double *__restrict__ rdot, const double *__restrict__ aE, int nfp, double cexp,
+    double inv_s2, double *__restrict__ T, double *__restrict__ ep, double *__restrict__ wp) {
+    __shared__ double red[KW > 1 ? KW : 1][KW > 1 ? MF * NFT * 8 : 1][64];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int item = KW == 1 ? xcd_tile() * 4 + wv : xcd_tile();
+    if (item >= items) return;
+    const MvSeg S = segs[find_seg(segs, nseg, item, [](const MvSeg &t) { return t.it1; })];
+    const int mt = (S.R1 + 16 * MF - 1) / (16 * MF);
+    const int loc = item - S.it1, m0 = (loc % mt) * 16 * MF, n0 = (loc / mt) * 16 * NFT;
+    const double *pa[MF], *pb[NFT], *pd[NFT];
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+        pa[m] = Xq + (size_t)min(S.q0 + m0 + 16 * m + r, qrows - 1) * nfp + 4 * g;
+#pragma unroll
+    for (int n = 0; n < NFT; ++n) {
+        pb[n] = P2 + (size_t)(2 * S.r2 + min(n0 + 16 * n + r, S.R2p - 1)) * nfp + 4 * g;
+        pd[n] = pb[n] + (size_t)S.R2p * nfp;
+    }
+    v4d s[MF][NFT], p[MF][NFT];
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+#pragma unroll
+        for (int n = 0; n < NFT; ++n) s[m][n] = p[m][n] = (v4d){0.0, 0.0, 0.0, 0.0};
+    double a[2][MF][4], b[2][NFT][4], d[2][NFT][4];
+    auto load = [&](int buf, int k) {
+#pragma unroll
+        for (int m = 0; m < MF; ++m) load4(pa[m] + k, a[buf][m]);
+#pragma unroll
+        for (int n = 0; n < NFT; ++n) {
+            load4(pb[n] + k, b[buf][n]);
+            load4(pd[n] + k, d[buf][n]);
+        }
+    };
+    auto mul = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int m = 0; m < MF; ++m)
+#pragma unroll
+                for (int n = 0; n < NFT; ++n) {
+                    s[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[buf][m][u], b[buf][n][u],
+                                                                   s[m][n], 0, 0, 0);
+                    p[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[buf][m][u], d[buf][n][u],
+                                                                   p[m][n], 0, 0, 0);
+                }
+    };
+    constexpr int step = 16 * KW;
+    const int kb = KW == 1 ? 0 : 16 * wv;
+    if (kb < nfp) load(0, kb);
+    for (int k = kb; k < nfp; k += 2 * step) {
+        if (k + step < nfp) load(1, k + step);
+        mul(0);
+        if (k + step >= nfp) break;
+        if (k + 2 * step < nfp) load(0, k + 2 * step);
+        mul(1);
+    }
+    if (KW > 1) {
+#pragma unroll
+        for (int m = 0; m < MF; ++m)
+#pragma unroll
+            for (int n = 0; n < NFT; ++n)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    red[wv][(m * NFT + n) * 8 + v][lane] = s[m][n][v];
+                    red[wv][(m * NFT + n) * 8 + 4 + v][lane] = p[m][n][v];
+                }
+        __syncthreads();
+    }
+    const int nfr = S.R2p >> 4;
+    const size_t ldt = 2 * (size_t)S.R2p;
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+#pragma unroll
+        for (int n = 0; n < NFT; ++n) {
+            if (KW > 1 && ((m * NFT + n) & 3) != wv) continue;
+            const int t = n0 + 16 * n + r;
+            if (n0 + 16 * n >= S.R2p) continue;
+            const bool live = t < S.R2;
+            const double nt = n2[S.r2 + t], rd = rdot[S.r2 + t], ae = aE[S.r2 + t];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = m0 + 16 * m + mfma16_row_f64(lane, v);
+                double sv = s[m][n][v], pv = p[m][n][v];
+                if (KW > 1) {
+                    sv = pv = 0.0;
+#pragma unroll
+                    for (int w = 0; w < KW; ++w) {
+                        sv += red[w][(m * NFT + n) * 8 + v][lane];
+                        pv += red[w][(m * NFT + n) * 8 + 4 + v][lane];
+                    }
+                }
+                const double q = nq[min(S.q0 + row, qrows - 1)];
+                const double d2 = fmax(q + nt - 2.0 * sv, 0.0);
+                const double e = live ? exp(cexp * d2) : 0.0, c = e * inv_s2;
+                // 0 * q: a query row with an infinity or a NaN in a column that the
+                // training side lacks still gives NaN
+                const double inner = pv - rd + 0.0 * q;
+                double bco = c * inv_s2 * inner + c * ae;
+                double es = e * ae + c * inner;
+                if (!live) bco = es = 0.0;
+                if (row < S.R1 && T) {
+                    T[S.toff + row * ldt + t] = bco;
+                    T[S.toff + row * ldt + S.R2p + t] = c;
+                }
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1) {
+                    es += __shfl_xor(es, o, 64);
+                    bco += __shfl_xor(bco, o, 64);
+                }
+                if (r == 0 && row < S.R1) {
+                    ep[S.eoff + (size_t)row * nfr + (n0 >> 4) + n] = es;
+                    wp[S.eoff + (size_t)row * nfr + (n0 >> 4) + n] = bco;
+                }
+            }
+        }
+}
+
+// Partial G = T [X2; AD] over `ks` of the 2 R2p summed rows: a wave has 16 MF query rows x
+// 64 columns of one split.  Without splits the product of a few query rows has as many
+// tiles as columns / 64: 12 work-groups for one 21-atom molecule.
+template <int MF>
+__global__ __launch_bounds__(NT, 2) void weighted_rows_kernel(const MvSeg *__restrict__ segs, int nseg,
+                                                           int items, int ks,
+                                                           const double *__restrict__ T,
+                                                           const double *__restrict__ P2, int nfp,
+                                                           double *__restrict__ G) {
+    constexpr int NF = 4;
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int item = xcd_tile() * 4 + wv;
+    if (item >= items) return;
+    const MvSeg S = segs[find_seg(segs, nseg, item, [](const MvSeg &t) { return t.it2; })];
+    const int mt = (S.R1 + 16 * MF - 1) / (16 * MF), nt = (nfp + 63) / 64;
+    const int loc = item - S.it2, n0 = (loc % nt) * 64, m0 = (loc / nt % mt) * 16 * MF,
+              split = loc / (nt * mt);
+    const int kb = split * ks, ke = min(kb + ks, 2 * S.R2p);
+    const double *pa[MF], *pb[NF];
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+        pa[m] = T + S.toff + (size_t)min(m0 + 16 * m + r, S.R1 - 1) * (2 * S.R2p) + 4 * g;
+#pragma unroll
+    for (int n = 0; n < NF; ++n)
+        pb[n] = P2 + (size_t)(2 * S.r2 + 4 * g) * nfp + min(n0 + 16 * n + r, nfp - 1);
+    v4d c[MF][NF];
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+#pragma unroll
+        for (int n = 0; n < NF; ++n) c[m][n] = (v4d){0.0, 0.0, 0.0, 0.0};
+    double a[2][MF][4], b[2][NF][4];
+    auto load = [&](int buf, int k) {
+#pragma unroll
+        for (int m = 0; m < MF; ++m) load4(pa[m] + k, a[buf][m]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int n = 0; n < NF; ++n) b[buf][n][u] = pb[n][(size_t)(k + u) * nfp];
+    };
+    auto mul = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int m = 0; m < MF; ++m)
+#pragma unroll
+                for (int n = 0; n < NF; ++n)
+                    c[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[buf][m][u], b[buf][n][u],
+                                                                   c[m][n], 0, 0, 0);
+    };
+    load(0, kb);
+    for (int k = kb; k < ke; k += 32) {
+        if (k + 16 < ke) load(1, k + 16);
+        mul(0);
+        if (k + 16 >= ke) break;
+        if (k + 32 < ke) load(0, k + 32);
+        mul(1);
+    }
+    double *out = G + S.goff + (size_t)split * S.R1 * nfp;
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+#pragma unroll
+        for (int n = 0; n < NF; ++n)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = m0 + 16 * m + mfma16_row_f64(lane, v), col = n0 + 16 * n + r;
+                if (row < S.R1 && col < nfp) out[(size_t)row * nfp + col] = c[m][n][v];
+            }
+}
+
+// One packed query row and one run of features per work-group:
+//   Fat[part][src, c] = sum over the run of dX1[src, f, c] (G[f] - w X1[src, f])
+// with G summed over its splits and w, E over the partial row sums, in a fixed order.
+// The rows of dX1 are contiguous, so the threads take nrow rows of nc columns at a time.
+// Bound by the read of dX1; the runs (`parts`, at most 16) give a batch of a few molecules
+// enough work-groups to draw on the whole memory system.
+__global__ __launch_bounds__(NT) void backproj_kernel(const MvSeg *__restrict__ segs, int nseg,
+                                                      int row0, const double *__restrict__ G,
+                                                      const double *__restrict__ ep,
+                                                      const double *__restrict__ wp,
+                                                      const double *__restrict__ X1,
+                                                      const double *__restrict__ dX1,
+                                                      const int *__restrict__ idx,
+                                                      const int *__restrict__ inv,
+                                                      const int *__restrict__ offs, int ma,
+                                                      int rep, int nfp, int natoms,
+                                                      double *__restrict__ erow,
+                                                      double *__restrict__ Fat) {
+    extern __shared__ double lds[];  // the run's features, then a partial sum per thread
+    __shared__ double part_e[4], part_w[4];
+    const int row = row0 + blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int src = idx[row];
+    if (src < 0) return;
+    const MvSeg S = segs[find_seg(segs, nseg, row, [](const MvSeg &t) { return t.q0; })];
+    const int loc = row - S.q0, nfr = S.R2p >> 4;
+    double es = 0.0, w = 0.0;
+    for (int t = tid; t < nfr; t += NT) {
+        es += ep[S.eoff + (size_t)loc * nfr + t];
+        w += wp[S.eoff + (size_t)loc * nfr + t];
     }
     es = wave_sum(es);
-    ws = wave_sum(ws);
+    w = wave_sum(w);
     if (lane == 0) {
-        if (erow) erow[qsrc[r]] = es;
-        wsum[r] = ws;
+        part_e[wv] = es;
+        part_w[wv] = w;
     }
-}
-
-// Fat[qsrc[r], c] = sum_f dX1[qsrc[r], f, c] (G[r, f] - wsum[r] X1p[r, f]).
-__global__ __launch_bounds__(NT) void backproj_kernel(const double *__restrict__ G,
-                                                      const double *__restrict__ X1p,
-                                                      const double *__restrict__ wsum,
-                                                      const double *__restrict__ dX1,
-                                                      const int *__restrict__ qsrc,
-                                                      const int *__restrict__ N1, int rows,
-                                                      int ma, int rep,
-                                                      double *__restrict__ Fat) {
-    const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= rows) return;
-    const int src = qsrc[r], a = src / ma;
-    const int nc = 3 * min(max(N1[a], 0), ma), ld = 3 * ma;
-    const double *J = dX1 + (size_t)src * rep * ld;
-    const double *g = G + (size_t)r * rep, *x = X1p + (size_t)r * rep;
-    const double w = wsum[r];
-    double *o = Fat + (size_t)src * ld;
-    // Jacobian columns in groups of 128 (two per lane); one group for up to 42 atoms
-    for (int c0 = 0; c0 < nc; c0 += 128) {
-        const int ca = c0 + lane, cb = c0 + lane + 64;
-        double s0 = 0.0, s1 = 0.0;
-        for (int f = 0; f < rep; ++f) {
-            const double gv = g[f] - w * x[f];
-            const double *row = J + (size_t)f * ld;
-            if (ca < nc) s0 = fma(row[ca], gv, s0);
-            if (cb < nc) s1 = fma(row[cb], gv, s1);
+    __syncthreads();
+    w = part_w[0] + part_w[1] + part_w[2] + part_w[3];
+    if (erow && blockIdx.y == 0 && tid == 0)
+        erow[src] = part_e[0] + part_e[1] + part_e[2] + part_e[3];
+    if (!Fat) return;
+    const int run = (rep + gridDim.y - 1) / gridDim.y;
+    const int f0 = blockIdx.y * run, fn = min(run, rep - f0);
+    for (int t = tid; t < fn; t += NT) {
+        const int c = inv[f0 + t];
+        double gv = 0.0;
+        if (c >= 0) {
+            const double *gp = G + S.goff + (size_t)loc * nfp + c;
+            const size_t st = (size_t)S.R1 * nfp;
+            int k = 0;
+            for (; k + 4 <= S.nsplit; k += 4) {
+                const double g0 = gp[k * st], g1 = gp[(k + 1) * st], g2 = gp[(k + 2) * st],
+                             g3 = gp[(k + 3) * st];
+                gv = (((gv + g0) + g1) + g2) + g3;
+            }
+            for (; k < S.nsplit; ++k) gv += gp[k * st];
         }
-        if (ca < nc) o[ca] = s0;
-        if (cb < nc) o[cb] = s1;
+        lds[t] = gv - w * X1[(size_t)src * rep + f0 + t];
     }
-}
-
-// E[a] = sum_i erow[a*ma+i]; F[offs[a] + c] = sum_i Fat[a*ma+i, c] (fixed order).
-__global__ __launch_bounds__(NT) void reduce_mol_kernel(const double *__restrict__ erow,
-                                                        const double *__restrict__ Fat,
-                                                        const int *__restrict__ N,
-                                                        const int *__restrict__ offs, int nm,
-                                                        int ma, double *__restrict__ E,
-                                                        double *__restrict__ F) {
-    const int a = blockIdx.x;
-    if (a >= nm) return;
-    const int na = min(max(N[a], 0), ma), ld = 3 * ma;
-    if (E && threadIdx.x == 0) {
+    __syncthreads();
+    double *red = lds + run;
+    const int a = src / ma, ld = 3 * ma, nc = offs[a + 1] - offs[a];
+    const double *J = dX1 + ((size_t)src * rep + f0) * ld;
+    double *o = Fat + ((size_t)blockIdx.y * natoms + src) * ld;
+    // columns in groups of NT (one for up to 85 atoms)
+    for (int c0 = 0; c0 < nc; c0 += NT) {
+        const int cn = min(nc - c0, NT), nrow = NT / cn, rr = tid / cn, c = c0 + tid - rr * cn;
         double s = 0.0;
-        for (int i = 0; i < na; ++i) s += erow[(size_t)a * ma + i];
-        E[a] = s;
-    }
-    if (F)
-        for (int c = threadIdx.x; c < 3 * na; c += blockDim.x) {
-            double s = 0.0;
-            for (int i = 0; i < na; ++i) s += Fat[((size_t)a * ma + i) * ld + c];
-            F[offs[a] + c] = s;
+        if (rr < nrow) {
+            int f = rr;
+            for (; f + 7 * nrow < fn; f += 8 * nrow) {
+                double j[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) j[u] = J[(size_t)(f + u * nrow) * ld + c];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) s = fma(j[u], lds[f + u * nrow], s);
+            }
+            for (; f < fn; f += nrow) s = fma(J[(size_t)f * ld + c], lds[f], s);
         }
-}
-
-// backproj_kernel with the molecule's atom count taken from the force offsets
-// (3 N[a] = offs[a + 1] - offs[a]), so a plan needs no N array at execution.
-__global__ __launch_bounds__(NT) void backproj_plan_kernel(const double *__restrict__ G,
-                                                           const double *__restrict__ X1p,
-                                                           const double *__restrict__ wsum,
-                                                           const double *__restrict__ dX1,
-                                                           const int *__restrict__ qsrc,
-                                                           const int *__restrict__ offs, int rows,
-                                                           int ma, int rep,
-                                                           double *__restrict__ Fat) {
-    const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= rows) return;
-    const int src = qsrc[r], a = src / ma;
-    const int nc = offs[a + 1] - offs[a], ld = 3 * ma;
-    const double *J = dX1 + (size_t)src * rep * ld;
-    const double *g = G + (size_t)r * rep, *x = X1p + (size_t)r * rep;
-    const double w = wsum[r];
-    double *o = Fat + (size_t)src * ld;
-    // Jacobian columns in groups of 128 (two per lane); one group for up to 42 atoms
-    for (int c0 = 0; c0 < nc; c0 += 128) {
-        const int ca = c0 + lane, cb = c0 + lane + 64;
-        double s0 = 0.0, s1 = 0.0;
-        for (int f = 0; f < rep; ++f) {
-            const double gv = g[f] - w * x[f];
-            const double *row = J + (size_t)f * ld;
-            if (ca < nc) s0 = fma(row[ca], gv, s0);
-            if (cb < nc) s1 = fma(row[cb], gv, s1);
+        red[tid] = s;
+        __syncthreads();
+        if (tid < cn) {
+            for (int x = 1; x < nrow; ++x) s += red[x * cn + tid];
+            o[c0 + tid] = s;
         }
-        if (ca < nc) o[ca] = s0;
-        if (cb < nc) o[cb] = s1;
+        __syncthreads();
     }
 }
 
-// reduce_mol_kernel with atom counts from the force offsets.
-__global__ __launch_bounds__(NT) void reduce_plan_kernel(const double *__restrict__ erow,
-                                                         const double *__restrict__ Fat,
-                                                         const int *__restrict__ offs, int nm,
-                                                         int ma, double *__restrict__ E,
-                                                         double *__restrict__ F) {
-    const int a = blockIdx.x;
-    if (a >= nm) return;
+// E[a] = sum_i erow[a*ma+i]; F[offs[a] + c] = sum over the parts and the atoms of
+// Fat[part][a*ma+i, c] (fixed order).  Atom counts come from the force offsets.  The
+// (part, atom) rows are dealt over the groups of nc threads: one molecule of 21 atoms in 16
+// parts is 336 rows, a 30 us chain for one thread per column.
+constexpr int kReduceThreads = 512;
+__global__ __launch_bounds__(kReduceThreads) void reduce_mol_kernel(
+    const double *__restrict__ erow, const double *__restrict__ Fat, int parts,
+    const int *__restrict__ offs, int natoms, int ma, double *__restrict__ E,
+    double *__restrict__ F) {
+    __shared__ double red[kReduceThreads];
+    const int a = blockIdx.x, tid = threadIdx.x;
     const int nc = offs[a + 1] - offs[a], na = nc / 3, ld = 3 * ma;
-    if (threadIdx.x == 0) {
+    if (E && tid < 64) {
         double s = 0.0;
-        for (int i = 0; i < na; ++i) s += erow[(size_t)a * ma + i];
-        E[a] = s;
+        for (int i = tid; i < na; i += 64) s += erow[(size_t)a * ma + i];
+        s = wave_sum(s);
+        if (tid == 0) E[a] = s;
     }
-    for (int c = threadIdx.x; c < nc; c += blockDim.x) {
+    if (!F) return;
+    for (int c0 = 0; c0 < nc; c0 += kReduceThreads) {
+        const int cn = min(nc - c0, kReduceThreads), nrow = kReduceThreads / cn, rr = tid / cn;
+        const double *q = Fat + (size_t)a * ma * ld + c0 + tid - rr * cn;
         double s = 0.0;
-        for (int i = 0; i < na; ++i) s += Fat[((size_t)a * ma + i) * ld + c];
-        F[offs[a] + c] = s;
+        if (rr < nrow) {
+#pragma unroll 4
+            for (int t = rr; t < parts * na; t += nrow)
+                s += q[((size_t)(t / na) * natoms + t % na) * ld];
+        }
+        red[tid] = s;
+        __syncthreads();
+        if (tid < cn) {
+            for (int x = 1; x < nrow; ++x) s += red[x * cn + tid];
+            F[offs[a] + c0 + tid] = s;
+        }
+        __syncthreads();
     }
 }
 
-// Expand alpha_E (per molecule) to the packed train rows.
-__global__ void expand_mol(const double *__restrict__ aE, const int *__restrict__ src, int rows,
-                           int ma, double *__restrict__ out) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < rows) out[r] = aE[src[r] / ma];
+// ---------------------------------------------------------------------------
+// Host side: the layout of one matvec (packed rows, segments, rounds) and its launches.
+// ---------------------------------------------------------------------------
+struct MvRound {
+    int seg0, nseg;    // segments of the round
+    int row0, rows;    // packed query rows they cover
+    int items1, items2, ks;
+    bool wide, split_k;  // 32-row tiles; KW = 4
+};
+
+struct MvLayout {
+    int nm1 = 0, ma1 = 0, rep = 0, nf = 0, nfp = 0, parts = 1;
+    int q_rows = 0, t_rows = 0;             // packed rows, padding included
+    std::vector<int> offs, src1, src2, inv;  // force offsets, packed rows' sources, columns
+    std::vector<MvSeg> segs;
+    std::vector<MvRound> rounds;
+    size_t T_len = 0, G_len = 0, e_len = 0;  // per round, the largest
+    // one device block of ints: segments first (8-byte aligned), then the vectors
+    size_t meta_bytes() const {
+        return sizeof(MvSeg) * segs.size() +
+               sizeof(int) * (offs.size() + src1.size() + src2.size() + inv.size());
+    }
+    void write_meta(char *p) const {
+        auto put = [&](const void *v, size_t n) { std::copy((const char *)v, (const char *)v + n, p); p += n; };
+        put(segs.data(), sizeof(MvSeg) * segs.size());
+        put(offs.data(), sizeof(int) * offs.size());
+        put(src1.data(), sizeof(int) * src1.size());
+        put(src2.data(), sizeof(int) * src2.size());
+        put(inv.data(), sizeof(int) * inv.size());
+    }
+    size_t train_doubles() const { return (size_t)2 * t_rows * nfp + 3 * (size_t)t_rows; }
+    size_t query_doubles() const {
+        return (size_t)q_rows * nfp + q_rows + (q_rows & 1) + T_len + G_len + 2 * e_len;
+    }
+    size_t acc_doubles(bool forces) const {
+        const size_t natom = (size_t)nm1 * ma1;
+        return natom + (forces ? (size_t)parts * natom * 3 * ma1 : 0);
+    }
+};
+// device addresses of a layout's pieces
+struct MvDev {
+    const MvSeg *segs;
+    const int *offs, *src1, *src2, *inv;
+    double *P2, *n2, *rdot, *aE;
+    double *Xq, *nq, *T, *G, *ep, *wp;
+    double *erow, *Fat;
+};
+
+int round_up16(int n) { return (n + 15) & ~15; }
+
+// T of one round stays within this many doubles (1 GiB), whatever the query set's size.
+constexpr size_t kTBudget = (size_t(1) << 30) / sizeof(double);
+
+void mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, int ma1,
+               const std::vector<int> &q2, const std::vector<int> &n2, int nm2, int ma2, int rep,
+               const int *flag, bool forces, MvLayout &L) {
+    L.nm1 = nm1;
+    L.ma1 = ma1;
+    L.rep = rep;
+    const std::vector<int> labels = distinct_labels(q1.data(), n1.data(), nm1, ma1);
+    LocalPlan p1, p2;
+    build_plan(q1.data(), n1.data(), nm1, ma1, labels, p1);
+    if (nm2 > 0) build_plan(q2.data(), n2.data(), nm2, ma2, labels, p2);
+    L.offs.assign(nm1 + 1, 0);
+    for (int a = 0; a < nm1; ++a) L.offs[a + 1] = L.offs[a] + 3 * clamp_atoms(n1[a], ma1);
+    L.inv.assign(rep, -1);
+    for (int f = 0; f < rep; ++f)
+        if (flag[f]) L.inv[f] = L.nf++;
+    L.nfp = std::max(16, round_up16(L.nf));
+    const int nt2 = (L.nfp + 63) / 64;
+    int q0 = 0, r2 = 0;
+    MvRound R{};
+    size_t T = 0, G = 0, E = 0;
+    auto close = [&]() {  // choose the round's variants and lay its segments out
+        if (R.nseg == 0) return;
+        int maxR1 = 0;
+        for (int s = R.seg0; s < R.seg0 + R.nseg; ++s) maxR1 = std::max(maxR1, L.segs[s].R1);
+        // 32-row tiles read the training rows once for two row fragments; up to 16 query
+        // rows of a label (one molecule) would leave half of such a tile empty
+        R.wide = maxR1 > 16;
+        const int mf = R.wide ? 32 : 16;
+        long tiles = 0, work = 0;
+        for (int s = R.seg0; s < R.seg0 + R.nseg; ++s) {
+            const MvSeg &g = L.segs[s];
+            const long mt = (g.R1 + mf - 1) / mf;
+            tiles += mt * ((g.R2p + 31) / 32);
+            work += mt * nt2 * 2 * g.R2p;
+        }
+        R.split_k = !R.wide || tiles < 2048;
+        // rows summed per split: about 2,048 waves (two per SIMD) over all tiles, in whole
+        // groups of 16, at least 64 so that a wave's start-up does not dominate
+        R.ks = (int)std::max<long>(64, (work / 2048 + 15) & ~15L);
+        const int nft = R.wide && !R.split_k ? 32 : 16;
+        for (int s = R.seg0; s < R.seg0 + R.nseg; ++s) {
+            MvSeg &g = L.segs[s];
+            const int mt = (g.R1 + mf - 1) / mf;
+            g.nsplit = (2 * g.R2p + R.ks - 1) / R.ks;
+            g.it1 = R.items1;
+            g.it2 = R.items2;
+            R.items1 += mt * ((g.R2p + nft - 1) / nft);
+            R.items2 += mt * nt2 * g.nsplit;
+            g.toff = T;
+            g.goff = G;
+            g.eoff = E;
+            T += (size_t)g.R1 * 2 * g.R2p;
+            G += (size_t)g.nsplit * g.R1 * L.nfp;
+            E += (size_t)g.R1 * (g.R2p / 16);
+        }
+        L.T_len = std::max(L.T_len, forces ? T + (T & 1) : 0);
+        L.G_len = std::max(L.G_len, forces ? G : 0);
+        L.e_len = std::max(L.e_len, E);
+        L.rounds.push_back(R);
+        T = G = E = 0;
+        R = MvRound{};
+    };
+    size_t held = 0;
+    for (int l = 0; l < p1.nlabels; ++l) {
+        const int *m1 = &p1.mol_row[(size_t)l * (nm1 + 1)];
+        const int R1 = m1[nm1] - m1[0];
+        int R2 = 0, b2 = 0;
+        if (nm2 > 0) {
+            const int *m2 = &p2.mol_row[(size_t)l * (nm2 + 1)];
+            b2 = m2[0];
+            R2 = m2[nm2] - b2;
+        }
+        if (R1 == 0) continue;
+        const int R2p = round_up16(R2);
+        L.src2.insert(L.src2.end(), p2.src.begin() + b2, p2.src.begin() + b2 + R2);
+        L.src2.insert(L.src2.end(), R2p - R2, -1);
+        const int qb = std::max<int>(64, (int)std::min<size_t>(
+                                             (size_t)round_up16(R1),
+                                             kTBudget / std::max(1, 2 * R2p) / 64 * 64));
+        for (int x = 0; x < R1; x += qb) {
+            const int n = std::min(qb, R1 - x), np = round_up16(n);
+            const size_t need = (size_t)n * 2 * R2p;
+            if (R.nseg > 0 && held + need > kTBudget) {
+                close();
+                held = 0;
+            }
+            if (R.nseg == 0) {
+                R.seg0 = (int)L.segs.size();
+                R.row0 = q0;
+            }
+            held += need;
+            L.segs.push_back({q0, n, r2, R2, R2p, 0, 0, 0, 0, 0, 0});
+            ++R.nseg;
+            R.rows += np;
+            L.src1.insert(L.src1.end(), p1.src.begin() + m1[0] + x, p1.src.begin() + m1[0] + x + n);
+            L.src1.insert(L.src1.end(), np - n, -1);
+            q0 += np;
+        }
+        r2 += R2p;
+    }
+    close();
+    L.q_rows = q0;
+    L.t_rows = r2;
+    // runs of features per query row in the back-projection: 2,048 work-groups, at most 16
+    L.parts = std::max(1, std::min({16, 2048 / std::max(1, q0), (rep + 31) / 32}));
+}
+
+MvDev mv_place(const MvLayout &L, char *meta, double *train, double *query, double *acc) {
+    MvDev D{};
+    D.segs = reinterpret_cast<const MvSeg *>(meta);
+    D.offs = reinterpret_cast<const int *>(meta + sizeof(MvSeg) * L.segs.size());
+    D.src1 = D.offs + L.offs.size();
+    D.src2 = D.src1 + L.src1.size();
+    D.inv = D.src2 + L.src2.size();
+    D.P2 = train;
+    D.n2 = D.P2 + (size_t)2 * L.t_rows * L.nfp;
+    D.rdot = D.n2 + L.t_rows;
+    D.aE = D.rdot + L.t_rows;
+    D.Xq = query;
+    D.nq = D.Xq + (size_t)L.q_rows * L.nfp;
+    D.T = D.nq + L.q_rows + (L.q_rows & 1);
+    D.G = D.T + L.T_len;
+    D.ep = D.G + L.G_len;
+    D.wp = D.ep + L.e_len;
+    D.erow = acc;
+    D.Fat = acc + (size_t)L.nm1 * L.ma1;
+    return D;
+}
+
+int mv_pack_train(const MvLayout &L, const MvDev &D, const double *X2, const double *ad,
+                  const double *aE, int ma2, hipStream_t stream) {
+    if (L.t_rows == 0) return KF_OK;
+    hipLaunchKernelGGL(pack_rows_kernel, dim3((L.t_rows + 3) / 4), dim3(NT), 0, stream, X2, ad,
+                       D.src2, L.t_rows, ma2, L.rep, D.inv, L.nf, L.nfp, D.segs,
+                       (int)L.segs.size(), aE, D.P2, D.n2, D.rdot, D.aE);
+    KF_HIP_TRY(hipGetLastError());
+    return KF_OK;
+}
+
+// mode bits: 1 E, 2 F
+int mv_run(const MvLayout &L, const MvDev &D, const double *X1, const double *dX1, double sigma,
+           double *E, double *F, int mode, hipStream_t stream) {
+    const double cexp = -1.0 / (2.0 * sigma * sigma), inv_s2 = 1.0 / (sigma * sigma);
+    const int natoms = L.nm1 * L.ma1;
+    if (L.q_rows > 0) {
+        hipLaunchKernelGGL(pack_rows_kernel, dim3((L.q_rows + 3) / 4), dim3(NT), 0, stream, X1,
+                           (const double *)nullptr, D.src1, L.q_rows, L.ma1, L.rep, D.inv, L.nf,
+                           L.nfp, D.segs, (int)L.segs.size(), (const double *)nullptr, D.Xq, D.nq,
+                           (double *)nullptr, (double *)nullptr);
+        KF_HIP_TRY(hipGetLastError());
+    }
+    const bool forces = mode & 2;
+    for (const MvRound &R : L.rounds) {
+        const MvSeg *segs = D.segs + R.seg0;
+        if (R.items1 > 0) {
+            auto coef = [&](auto kern, int per) {
+                hipLaunchKernelGGL(kern, dim3((R.items1 + per - 1) / per), dim3(NT), 0, stream,
+                                   segs, R.nseg, R.items1, D.Xq, L.q_rows, D.nq, D.P2, D.n2,
+                                   D.rdot, D.aE, L.nfp, cexp, inv_s2,
+                                   forces ? D.T : (double *)nullptr, D.ep, D.wp);
+            };
+            if (!R.wide) coef(coef_kernel<1, 1, 4>, 1);
+            else if (R.split_k) coef(coef_kernel<2, 1, 4>, 1);
+            else coef(coef_kernel<2, 2, 1>, 4);
+            KF_HIP_TRY(hipGetLastError());
+        }
+        if (forces && R.items2 > 0) {
+            hipLaunchKernelGGL(R.wide ? weighted_rows_kernel<2> : weighted_rows_kernel<1>,
+                               dim3((R.items2 + 3) / 4), dim3(NT), 0, stream, segs, R.nseg,
+                               R.items2, R.ks, D.T, D.P2, L.nfp, D.G);
+            KF_HIP_TRY(hipGetLastError());
+        }
+        const size_t lds = sizeof(double) * ((L.rep + L.parts - 1) / L.parts + NT);
+        hipLaunchKernelGGL(backproj_kernel, dim3(R.rows, forces ? L.parts : 1), dim3(NT), lds,
+                           stream, segs, R.nseg, R.row0, D.G, D.ep, D.wp, X1, dX1, D.src1, D.inv,
+                           D.offs, L.ma1, L.rep, L.nfp, natoms,
+                           (mode & 1) ? D.erow : (double *)nullptr,
+                           forces ? D.Fat : (double *)nullptr);
+        KF_HIP_TRY(hipGetLastError());
+    }
+    hipLaunchKernelGGL(reduce_mol_kernel, dim3(L.nm1), dim3(kReduceThreads), 0, stream, D.erow, D.Fat,
+                       L.parts, D.offs, natoms, L.ma1, (mode & 1) ? E : (double *)nullptr,
+                       forces ? F : (double *)nullptr);
+    KF_HIP_TRY(hipGetLastError());
+    return KF_OK;
+}
+
+// Labels and counts of both sets and the training side's used columns on the host, with one
+// synchronisation.
+int mv_read(const int *Q1, const int *N1, int nm1, int ma1, const double *X2, const double *ad,
+            const int *Q2, const int *N2, int nm2, int ma2, int rep, std::vector<int> &q1,
+            std::vector<int> &n1, std::vector<int> &q2, std::vector<int> &n2,
+            std::vector<int> &flag, hipStream_t stream) {
+    flag.assign(rep, 0);
+    int *dflag = nullptr, *hflag = nullptr;
+    if (nm2 > 0 && ma2 > 0) {
+        dflag = static_cast<int *>(workspace(WS_AUX1, sizeof(int) * rep, stream));
+        hflag = static_cast<int *>(host_staging(WS_AUX3, sizeof(int) * rep));
+        KF_REQUIRE(dflag && hflag, KF_ERR_NOMEM, "workspace allocation failed");
+        KF_HIP_TRY(hipMemsetAsync(dflag, 0, sizeof(int) * rep, stream));
+        const int per = std::max(1, (nm2 + 1023) / 1024);
+        hipLaunchKernelGGL(train_cols_kernel, dim3((nm2 + per - 1) / per), dim3(NT), 0, stream, X2,
+                           ad, N2, nm2, ma2, rep, per, dflag);
+        KF_HIP_TRY(hipGetLastError());
+        KF_HIP_TRY(hipMemcpyAsync(hflag, dflag, sizeof(int) * rep, hipMemcpyDeviceToHost, stream));
+    }
+    int rc;
+    if (nm2 > 0) {
+        const size_t nq = (size_t)nm2 * ma2;
+        int *stage = static_cast<int *>(host_staging(WS_AUX1, sizeof(int) * (nq + nm2)));
+        KF_REQUIRE(stage, KF_ERR_NOMEM, "pinned staging allocation failed");
+        if (nq)
+            KF_HIP_TRY(hipMemcpyAsync(stage, Q2, sizeof(int) * nq, hipMemcpyDeviceToHost, stream));
+        KF_HIP_TRY(hipMemcpyAsync(stage + nq, N2, sizeof(int) * nm2, hipMemcpyDeviceToHost, stream));
+        if ((rc = read_metadata(Q1, N1, nm1, ma1, q1, n1, stream, WS_AUX0))) return rc;
+        q2.assign(stage, stage + nq);
+        n2.assign(stage + nq, stage + nq + nm2);
+    } else if ((rc = read_metadata(Q1, N1, nm1, ma1, q1, n1, stream, WS_AUX0))) {
+        return rc;
+    }
+    if (hflag) std::copy(hflag, hflag + rep, flag.begin());
+    return KF_OK;
 }
 
 // modes: bit 1 E, bit 2 F, bit 4 alpha_E terms
@@ -273,130 +806,46 @@ int matvec_impl(const double *X1, const double *dX1, const double *X2, const dou
     KF_REQUIRE(!(mode & 2) || dX1, KF_ERR_ARG, "null dX1");  // F may be null when naq1 == 0
     KF_REQUIRE(!(mode & 1) || E, KF_ERR_ARG, "null E");
     KF_REQUIRE(!(mode & 4) || nm2 == 0 || aE, KF_ERR_ARG, "null alpha_E");
-    std::vector<int> q1, n1, q2, n2;
+    std::vector<int> q1, n1, q2, n2, flag;
     int rc;
-    if ((rc = read_metadata(Q1, N1, nm1, ma1, q1, n1, stream, WS_AUX0))) return rc;
-    if (nm2 > 0 && (rc = read_metadata(Q2, N2, nm2, ma2, q2, n2, stream, WS_AUX1))) return rc;
-    std::vector<int> labels = distinct_labels(q1.data(), n1.data(), nm1, ma1);
-    LocalPlan p1, p2;
-    build_plan(q1.data(), n1.data(), nm1, ma1, labels, p1);
-    if (nm2 > 0) build_plan(q2.data(), n2.data(), nm2, ma2, labels, p2);
-    std::vector<int> offs(nm1 + 1, 0);
-    for (int a = 0; a < nm1; ++a) offs[a + 1] = offs[a] + 3 * clamp_atoms(n1[a], ma1);
-
-    // device metadata: offs | src1 | src2
-    const size_t n_meta = offs.size() + p1.src.size() + (nm2 > 0 ? p2.src.size() : 0);
-    int *meta = static_cast<int *>(workspace(WS_PLAN, sizeof(int) * n_meta, stream));
-    int *stage = static_cast<int *>(host_staging(WS_PLAN, sizeof(int) * n_meta));
-    KF_REQUIRE(meta && stage, KF_ERR_NOMEM, "workspace allocation failed");
-    std::copy(offs.begin(), offs.end(), stage);
-    std::copy(p1.src.begin(), p1.src.end(), stage + offs.size());
-    if (nm2 > 0) std::copy(p2.src.begin(), p2.src.end(), stage + offs.size() + p1.src.size());
-    KF_HIP_TRY(hipMemcpyAsync(meta, stage, sizeof(int) * n_meta, hipMemcpyHostToDevice, stream));
-    const int *d_offs = meta, *d_src1 = meta + offs.size(),
-              *d_src2 = d_src1 + p1.src.size();
-
-    // per-atom outputs (zero for atoms without matches)
-    const size_t natom1 = (size_t)nm1 * ma1;
-    double *erow = nullptr, *Fat = nullptr;
-    {
-        const size_t bytes = sizeof(double) * (natom1 + ((mode & 2) ? natom1 * 3 * ma1 : 0));
-        double *w = static_cast<double *>(workspace(WS_AUX3, bytes, stream));
-        KF_REQUIRE(w, KF_ERR_NOMEM, "workspace allocation failed (%zu B)", bytes);
-        KF_HIP_TRY(hipMemsetAsync(w, 0, bytes, stream));
-        erow = w;
-        if (mode & 2) Fat = w + natom1;
-    }
+    if ((rc = mv_read(Q1, N1, nm1, ma1, X2, ad, Q2, N2, nm2, ma2, rep, q1, n1, q2, n2, flag,
+                      stream)))
+        return rc;
+    MvLayout L;
+    mv_layout(q1, n1, nm1, ma1, q2, n2, nm2, ma2, rep, flag.data(), mode & 2, L);
+    char *meta = static_cast<char *>(workspace(WS_PLAN, L.meta_bytes(), stream));
+    char *stage = static_cast<char *>(host_staging(WS_PLAN, L.meta_bytes()));
+    const size_t qb = sizeof(double) * L.query_doubles();
+    // (not in WS_PACK or WS_PACK2: the matrix-free solver keeps its operands there)
+    const size_t tpad = (L.train_doubles() + 31) & ~size_t(31);
+    double *train = static_cast<double *>(workspace(WS_AUX2, sizeof(double) * tpad + qb, stream));
+    double *query = train + tpad;
+    double *acc = static_cast<double *>(
+        workspace(WS_AUX3, sizeof(double) * L.acc_doubles(mode & 2), stream));
+    KF_REQUIRE(meta && stage && train && acc, KF_ERR_NOMEM,
+               "workspace allocation failed (%zu B)", sizeof(double) * tpad + qb);
+    L.write_meta(stage);
+    KF_HIP_TRY(hipMemcpyAsync(meta, stage, L.meta_bytes(), hipMemcpyHostToDevice, stream));
+    const MvDev D = mv_place(L, meta, train, query, acc);
     ScopedTimer timer(TM_MATVEC, stream);
-    const double cexp = -1.0 / (2.0 * sigma * sigma), inv_s2 = 1.0 / (sigma * sigma);
-    for (int l = 0; l < p1.nlabels && nm2 > 0; ++l) {
-        const int r1b = p1.mol_row[(size_t)l * (nm1 + 1)], R1 = p1.mol_row[(size_t)l * (nm1 + 1) + nm1] - r1b;
-        const int r2b = p2.mol_row[(size_t)l * (nm2 + 1)], R2 = p2.mol_row[(size_t)l * (nm2 + 1) + nm2] - r2b;
-        if (R1 == 0 || R2 == 0) continue;
-        // packed train block: [X2 (R2 x rep); AD (R2 x rep)], n2, rdot, aE per row
-        const size_t train_bytes = sizeof(double) * ((size_t)2 * R2 * rep + 3 * (size_t)R2);
-        // query block size: T = QB x 2 R2 and G = QB x rep within ~1 GiB
-        const size_t budget = size_t(1) << 30;
-        int QB = (int)std::min<size_t>(R1, std::max<size_t>(64, budget / (sizeof(double) *
-                                                                             ((size_t)2 * R2 + 2 * rep + 2))));
-        const size_t q_bytes = sizeof(double) * ((size_t)QB * (2 * R2 + 2 * rep) + 2 * (size_t)QB);
-        char *ws = static_cast<char *>(workspace(WS_AUX2, train_bytes + q_bytes, stream));
-        KF_REQUIRE(ws, KF_ERR_NOMEM, "workspace allocation failed (%zu B)", train_bytes + q_bytes);
-        double *P2 = reinterpret_cast<double *>(ws);
-        double *AD2 = P2 + (size_t)R2 * rep;
-        double *nrm2 = AD2 + (size_t)R2 * rep, *rdot = nrm2 + R2, *aEr = rdot + R2;
-        double *T = aEr + R2;
-        double *Xq = T + (size_t)QB * 2 * R2, *G = Xq + (size_t)QB * rep;
-        double *nq = G + (size_t)QB * rep, *wsum = nq + QB;
-        hipLaunchKernelGGL(gather_rows, dim3((R2 + 3) / 4), dim3(NT), 0, stream, X2, ad,
-                           d_src2 + r2b, R2, rep, P2, AD2, nrm2, rdot);
-        KF_HIP_TRY(hipGetLastError());
-        if (mode & 4) {
-            hipLaunchKernelGGL(expand_mol, dim3((R2 + 255) / 256), dim3(256), 0, stream, aE,
-                               d_src2 + r2b, R2, ma2, aEr);
-            KF_HIP_TRY(hipGetLastError());
-        }
-        for (int q0 = 0; q0 < R1; q0 += QB) {
-            const int qb = std::min(QB, R1 - q0);
-            const int *qsrc = d_src1 + r1b + q0;
-            hipLaunchKernelGGL(gather_rows, dim3((qb + 3) / 4), dim3(NT), 0, stream, X1,
-                               (const double *)nullptr, qsrc, qb, rep, Xq, (double *)nullptr, nq,
-                               (double *)nullptr);
-            KF_HIP_TRY(hipGetLastError());
-            // T = Xq [X2; AD]^T
-            if ((rc = gemm::gemm_f64<true>(qb, 2 * R2, rep, 1.0, Xq, rep, P2, rep, 0.0, T,
-                                           (size_t)2 * R2, stream)))
-                return rc;
-            hipLaunchKernelGGL(coef_kernel, dim3((qb + 3) / 4), dim3(NT), 0, stream, T, qb, R2,
-                               nq, nrm2, rdot, (mode & 4) ? aEr : (const double *)nullptr, cexp,
-                               inv_s2, qsrc, (mode & 1) ? erow : (double *)nullptr, wsum);
-            KF_HIP_TRY(hipGetLastError());
-            if (mode & 2) {
-                // G = [B | C] [X2; AD]
-                if ((rc = gemm::gemm_f64<false>(qb, rep, 2 * R2, 1.0, T, (size_t)2 * R2, P2, rep,
-                                                0.0, G, rep, stream)))
-                    return rc;
-                hipLaunchKernelGGL(backproj_kernel, dim3((qb + 3) / 4), dim3(NT), 0, stream, G, Xq,
-                                   wsum, dX1, qsrc, N1, qb, ma1, rep, Fat);
-                KF_HIP_TRY(hipGetLastError());
-            }
-        }
-    }
-    hipLaunchKernelGGL(reduce_mol_kernel, dim3(nm1), dim3(128), 0, stream, erow, Fat, N1, d_offs,
-                       nm1, ma1, (mode & 1) ? E : (double *)nullptr,
-                       (mode & 2) ? F : (double *)nullptr);
-    KF_HIP_TRY(hipGetLastError());
-    return KF_OK;
-}
-
-// Fill a buffer with zeros by a kernel (stream-ordered, and safe inside a captured graph).
-__global__ void zero_fill(double *__restrict__ p, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x)
-        p[i] = 0.0;
+    if ((rc = mv_pack_train(L, D, X2, ad, (mode & 4) ? aE : nullptr, ma2, stream))) return rc;
+    return mv_run(L, D, X1, dX1, sigma, E, F, mode, stream);
 }
 
 }  // namespace
 }  // namespace kf
 
 // A full matvec planned once for fixed labels of the query set and a fixed training side
-// (descriptors, alpha_desc, alpha_E): the label plans, the packed training rows of every
-// label with their norms and dot products, and the query workspace all live in device
-// memory owned by the plan, so an execution neither reads anything back nor allocates.
+// (descriptors, alpha_desc, alpha_E): the layout, the packed training rows of every label
+// with their norms and dot products, and the query workspace all live in device memory
+// owned by the plan, so an execution neither reads anything back nor allocates.
 struct kf_matvec_plan {
     int device = 0;
-    int nm1 = 0, ma1 = 0, nm2 = 0, ma2 = 0, rep = 0;
     double sigma = 1.0;
-    struct Label {
-        int r1b, R1, R2, QB;
-        size_t train_off;  // doubles into `train`
-    };
-    std::vector<Label> labels;
-    int QBmax = 0;
-    size_t q_doubles = 0;  // per-execution query workspace
-    int *meta = nullptr;   // offs (nm1 + 1) | src1
-    double *train = nullptr, *query = nullptr, *acc = nullptr;  // acc: erow | Fat
-    size_t acc_doubles = 0;
+    kf::MvLayout layout;
+    kf::MvDev dev{};
+    char *meta = nullptr;
+    double *train = nullptr, *query = nullptr, *acc = nullptr;
     ~kf_matvec_plan() {
         (void)hipFree(meta);
         (void)hipFree(train);
@@ -427,61 +876,24 @@ int plan_create(const int *Q1, const int *N1, int nm1, int ma1, const double *X2
     KF_REQUIRE(Q1 && N1 && (nm2 == 0 || (X2 && ad && aE && Q2 && N2)), KF_ERR_ARG,
                "null pointer");
     KF_HIP_TRY(hipGetDevice(&P->device));
-    P->nm1 = nm1; P->ma1 = ma1; P->nm2 = nm2; P->ma2 = ma2; P->rep = rep; P->sigma = sigma;
-    std::vector<int> q1, n1, q2, n2;
+    P->sigma = sigma;
+    std::vector<int> q1, n1, q2, n2, flag;
     int rc;
-    if ((rc = read_metadata(Q1, N1, nm1, ma1, q1, n1, stream, WS_AUX0))) return rc;
-    if (nm2 > 0 && (rc = read_metadata(Q2, N2, nm2, ma2, q2, n2, stream, WS_AUX1))) return rc;
-    std::vector<int> labels = distinct_labels(q1.data(), n1.data(), nm1, ma1);
-    LocalPlan p1, p2;
-    build_plan(q1.data(), n1.data(), nm1, ma1, labels, p1);
-    if (nm2 > 0) build_plan(q2.data(), n2.data(), nm2, ma2, labels, p2);
-    std::vector<int> meta(nm1 + 1 + p1.src.size(), 0);
-    for (int a = 0; a < nm1; ++a) meta[a + 1] = meta[a] + 3 * clamp_atoms(n1[a], ma1);
-    std::copy(p1.src.begin(), p1.src.end(), meta.begin() + nm1 + 1);
-    std::vector<int> src2_all;
-    size_t train_doubles = 0;
-    for (int l = 0; l < p1.nlabels && nm2 > 0; ++l) {
-        const int r1b = p1.mol_row[(size_t)l * (nm1 + 1)];
-        const int R1 = p1.mol_row[(size_t)l * (nm1 + 1) + nm1] - r1b;
-        const int r2b = p2.mol_row[(size_t)l * (nm2 + 1)];
-        const int R2 = p2.mol_row[(size_t)l * (nm2 + 1) + nm2] - r2b;
-        if (R1 == 0 || R2 == 0) continue;
-        const size_t budget = size_t(1) << 30;
-        const int QB = (int)std::min<size_t>(
-            R1, std::max<size_t>(64, budget / (sizeof(double) * ((size_t)2 * R2 + 2 * rep + 2))));
-        P->labels.push_back({r1b, R1, R2, QB, train_doubles});
-        train_doubles += (size_t)2 * R2 * rep + 3 * (size_t)R2;
-        P->q_doubles = std::max(P->q_doubles,
-                                (size_t)QB * (2 * (size_t)R2 + 2 * (size_t)rep) + 2 * (size_t)QB);
-        P->QBmax = std::max(P->QBmax, QB);
-        src2_all.insert(src2_all.end(), p2.src.begin() + r2b, p2.src.begin() + r2b + R2);
-    }
-    const size_t natom1 = (size_t)nm1 * ma1;
-    P->acc_doubles = natom1 + natom1 * 3 * ma1;
-    if ((rc = plan_alloc((void **)&P->meta, sizeof(int) * (meta.size() + src2_all.size()))))
+    if ((rc = mv_read(Q1, N1, nm1, ma1, X2, ad, Q2, N2, nm2, ma2, rep, q1, n1, q2, n2, flag,
+                      stream)))
         return rc;
-    if ((rc = plan_alloc((void **)&P->train, sizeof(double) * train_doubles))) return rc;
-    if ((rc = plan_alloc((void **)&P->query, sizeof(double) * P->q_doubles))) return rc;
-    if ((rc = plan_alloc((void **)&P->acc, sizeof(double) * P->acc_doubles))) return rc;
-    meta.insert(meta.end(), src2_all.begin(), src2_all.end());
-    KF_HIP_TRY(hipMemcpyAsync(P->meta, meta.data(), sizeof(int) * meta.size(),
-                              hipMemcpyHostToDevice, stream));
-    // pack the training side of every label once
-    const int *d_src2 = P->meta + nm1 + 1 + p1.src.size();
-    size_t s2 = 0;
-    for (const auto &L : P->labels) {
-        double *P2 = P->train + L.train_off;
-        double *AD2 = P2 + (size_t)L.R2 * rep;
-        double *nrm2 = AD2 + (size_t)L.R2 * rep, *rdot = nrm2 + L.R2, *aEr = rdot + L.R2;
-        hipLaunchKernelGGL(gather_rows, dim3((L.R2 + 3) / 4), dim3(NT), 0, stream, X2, ad,
-                           d_src2 + s2, L.R2, rep, P2, AD2, nrm2, rdot);
-        hipLaunchKernelGGL(expand_mol, dim3((L.R2 + 255) / 256), dim3(256), 0, stream, aE,
-                           d_src2 + s2, L.R2, ma2, aEr);
-        KF_HIP_TRY(hipGetLastError());
-        s2 += L.R2;
-    }
-    // the host vectors above are released on return: wait for the copy that reads them
+    MvLayout &L = P->layout;
+    mv_layout(q1, n1, nm1, ma1, q2, n2, nm2, ma2, rep, flag.data(), true, L);
+    if ((rc = plan_alloc((void **)&P->meta, L.meta_bytes()))) return rc;
+    if ((rc = plan_alloc((void **)&P->train, sizeof(double) * L.train_doubles()))) return rc;
+    if ((rc = plan_alloc((void **)&P->query, sizeof(double) * L.query_doubles()))) return rc;
+    if ((rc = plan_alloc((void **)&P->acc, sizeof(double) * L.acc_doubles(true)))) return rc;
+    std::vector<char> meta(L.meta_bytes());
+    L.write_meta(meta.data());
+    KF_HIP_TRY(hipMemcpyAsync(P->meta, meta.data(), meta.size(), hipMemcpyHostToDevice, stream));
+    P->dev = mv_place(L, P->meta, P->train, P->query, P->acc);
+    if ((rc = mv_pack_train(L, P->dev, X2, ad, aE, ma2, stream))) return rc;
+    // the host vector above is released on return: wait for the copy that reads it
     KF_HIP_TRY(hipStreamSynchronize(stream));
     return KF_OK;
 }
@@ -493,43 +905,7 @@ int plan_execute(const kf_matvec_plan *P, const double *X1, const double *dX1, d
     KF_HIP_TRY(hipGetDevice(&dev));
     KF_REQUIRE(dev == P->device, KF_ERR_ARG, "plan was created on device %d, current is %d",
                P->device, dev);
-    const int nm1 = P->nm1, ma1 = P->ma1, rep = P->rep;
-    const int *d_offs = P->meta, *d_src1 = P->meta + nm1 + 1;
-    const int *N1 = nullptr;  // atom counts are baked into the plan (offs, row lists)
-    double *erow = P->acc, *Fat = P->acc + (size_t)nm1 * ma1;
-    hipLaunchKernelGGL(zero_fill, dim3(256), dim3(256), 0, stream, P->acc, P->acc_doubles);
-    const double cexp = -1.0 / (2.0 * P->sigma * P->sigma), inv_s2 = 1.0 / (P->sigma * P->sigma);
-    int rc;
-    for (const auto &L : P->labels) {
-        const double *P2 = P->train + L.train_off;
-        const double *nrm2 = P2 + (size_t)2 * L.R2 * rep, *rdot = nrm2 + L.R2, *aEr = rdot + L.R2;
-        double *T = P->query;
-        double *Xq = T + (size_t)L.QB * 2 * L.R2, *G = Xq + (size_t)L.QB * rep;
-        double *nq = G + (size_t)L.QB * rep, *wsum = nq + L.QB;
-        for (int q0 = 0; q0 < L.R1; q0 += L.QB) {
-            const int qb = std::min(L.QB, L.R1 - q0);
-            const int *qsrc = d_src1 + L.r1b + q0;
-            hipLaunchKernelGGL(gather_rows, dim3((qb + 3) / 4), dim3(NT), 0, stream, X1,
-                               (const double *)nullptr, qsrc, qb, rep, Xq, (double *)nullptr, nq,
-                               (double *)nullptr);
-            if ((rc = gemm::gemm_f64<true>(qb, 2 * L.R2, rep, 1.0, Xq, rep, P2, rep, 0.0, T,
-                                           (size_t)2 * L.R2, stream)))
-                return rc;
-            hipLaunchKernelGGL(coef_kernel, dim3((qb + 3) / 4), dim3(NT), 0, stream, T, qb, L.R2,
-                               nq, nrm2, rdot, aEr, cexp, inv_s2, qsrc, erow, wsum);
-            if ((rc = gemm::gemm_f64<false>(qb, rep, 2 * L.R2, 1.0, T, (size_t)2 * L.R2, P2, rep,
-                                            0.0, G, rep, stream)))
-                return rc;
-            hipLaunchKernelGGL(backproj_plan_kernel, dim3((qb + 3) / 4), dim3(NT), 0, stream, G,
-                               Xq, wsum, dX1, qsrc, d_offs, qb, ma1, rep, Fat);
-            KF_HIP_TRY(hipGetLastError());
-        }
-    }
-    (void)N1;
-    hipLaunchKernelGGL(reduce_plan_kernel, dim3(nm1), dim3(128), 0, stream, erow, Fat, d_offs,
-                       nm1, ma1, E, F);
-    KF_HIP_TRY(hipGetLastError());
-    return KF_OK;
+    return mv_run(P->layout, P->dev, X1, dX1, P->sigma, E, F, 1 | 2, stream);
 }
 
 }  // namespace

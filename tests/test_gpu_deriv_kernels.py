@@ -189,6 +189,36 @@ def test_alpha_desc_and_matvecs(lk, case):
     assert rel_err(np.concatenate([E, F]), y) < 1e-9
 
 
+# (nm1, ma1, nm2, ma2, rep, labels, zero columns of the training side): 16-row tiles with the
+# summation shared by four waves, 32-row tiles with and without that, a training side
+# without a query label, atoms without a match, columns that only the query has, more
+# rows than one pass holds (two rounds of the 1 GiB coefficient block), and more columns
+# than threads in the back-projection's work-group
+@pytest.mark.parametrize("case", [
+    (1, 16, 9, 5, 37, 1, 20), (1, 17, 5, 16, 16, 1, 0), (1, 90, 2, 3, 6, 2, 1),
+    (7, 12, 11, 9, 33, 4, 33), (60, 25, 62, 25, 17, 1, 1), (830, 10, 830, 10, 3, 1, 1)])
+def test_matvec_variants(lk, case):
+    nm1, ma1, nm2, ma2, rep, nlab, nzero = case
+    full = nm1 > 100  # every atom present, so that the coefficient block is over its limit
+    X1, dX1, Q1, N1 = rand_set(nm1, ma1, rep, nlab, 31 + ma1, ma1 if full or nm1 == 1 else 0)
+    X2, _, Q2, N2 = rand_set(nm2, ma2, rep, max(1, nlab - 1), 131 + ma2, ma2 if full else 0)
+    rng = np.random.default_rng(6)
+    ad = rng.standard_normal((nm2, ma2, rep))
+    live = np.arange(ma2)[None] < N2[:, None]
+    ad[~live] = 0.0
+    X2[..., rep - nzero:] = 0.0
+    ad[..., rep - nzero:] = 0.0
+    aE = rng.standard_normal(nm2)
+    s = 1.6
+    E, F = lk.kernel_gaussian_local_full_matvec(X1, dX1, X2, ad, aE, Q1, Q2, N1, N2, s)
+    Eo, Fo = oracle.full_matvec(X1, dX1, X2, ad, aE, Q1, Q2, N1, N2, s)
+    assert rel_err(E, Eo) < TOL and rel_err(F, Fo) < TOL
+    Fh = lk.kernel_gaussian_local_hessian_matvec(X1, dX1, X2, ad, Q1, Q2, N1, N2, s)
+    assert rel_err(Fh, oracle.hessian_matvec(X1, dX1, X2, ad, Q1, Q2, N1, N2, s)) < TOL
+    Ej = lk.kernel_gaussian_local_jacobian_t_matvec(X1, X2, ad, Q1, Q2, N1, N2, s)
+    assert rel_err(Ej, oracle.jacobian_t_matvec(X1, X2, ad, Q1, Q2, N1, N2, s)) < TOL
+
+
 def test_matvec_conformers_symmetric(lk):
     """Training-set operator on C9H8O4 conformers equals the RFP E+F kernel times alpha."""
     from kernelforge_amd import synthetic
