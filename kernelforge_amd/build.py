@@ -28,7 +28,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["kf_runtime.hip", "fchl19.hip", "local_scalar.hip", "local_mixed.hip", "rfp_chol.hip",
+HIP_SOURCES = ["kf_runtime.hip", "fchl19.hip", "local_scalar.hip", "local_direct.hip", "local_mixed.hip", "rfp_chol.hip",
                "rfp_convert.hip", "rfp_solve.hip", "local_deriv.hip",
                "local_matvec.hip", "ef_pcg.hip", "mlp.hip", "feature_compact.hip",
                "fchl19v2.hip"]

@@ -1,0 +1,445 @@
+// local_direct.hip -- the scalar local kernels (local_scalar.hip) for small calls.
+//
+// The blocked kernel of local_scalar.hip packs and orders the molecules by the descriptor
+// windows they use and gives each work-group a block of molecule pairs, whose labels and
+// tiles it walks one after another.  For a few hundred thousand molecule pairs that leaves
+// most of the GPU waiting on the longest chain, and the packing and ordering cost as much
+// as the products.  This form has no packing: rows are read where they are, in 32 x 32
+// tiles of one label's Gram matrix (a work-group's four waves share the descriptor columns
+// of a tile while there are few tiles, a wave has a tile of its own beyond that), straight
+// from global memory into registers (32-byte loads with the summation index of a step
+// permuted the same way in both operands, as in local_matvec.hip).  The tile's rows pass
+// through the registers whole, so their squared norms come from the same loads.  The
+// exponentials go to memory (8 bytes per matched atom pair), and a second kernel sums
+// those of each molecule pair in a fixed order.
+// Measured for the symmetric kernel (whole call): 50 molecules 84 us against 1,001 of the
+// blocked form with its 64 x 64 blocks (268 with the smallest blocks), 400 molecules 301
+// against 2,499 (446), 800 molecules 826 against 3,129 (873); one molecule against 1,000
+// 129 against 474 us.
+#include <algorithm>
+#include <cmath>
+
+#include "local_direct.hpp"
+#include "reg_pipeline.hpp"
+
+namespace kf {
+namespace {
+
+constexpr int NT = 256;
+constexpr int TE = 32;  // tile edge (rows of one label)
+// Row tiles of a band: its rows (2.9 MB of 720 columns in 32-row tiles) stay in an XCD's L2
+// while the column tiles pass, so the columns are fetched once per band instead of once per
+// row tile.
+constexpr int BT = 16;
+constexpr int kLdsTiles = 384;
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+// One label: its packed rows of both sets and where its exponentials go.
+struct DirectSeg {
+    int r1, R1, r2, R2;
+    int it, pad;      // first tile
+    size_t eoff, ld;  // exponentials: R1 rows of ld (R2)
+};
+
+// Consecutive tiles (which share operands) on one XCD: work-groups are dealt round-robin
+// over eight of them.
+__device__ inline int xcd_tile() {
+    const int g = blockIdx.x, G = gridDim.x;
+    return (G % 8 == 0) ? (g % 8) * (G / 8) + g / 8 : g;
+}
+
+template <class At>
+__device__ inline int seg_of(const DirectSeg *segs, int nseg, int x, At at) {
+    int s = 0;
+    while (s + 1 < nseg && at(segs[s + 1]) <= x) ++s;
+    return s;
+}
+
+// Columns k + 2 g, + 1, + 8 and + 9 of a row for lane group g: two loads that together take
+// 128 contiguous bytes of 16 rows, 64 at a time, or four where rows are not 16-byte aligned
+// (VEC = false).
+template <bool VEC>
+__device__ inline void load4(const double *p, double (&v)[4]) {
+    if (VEC) {
+        const v2d a = *reinterpret_cast<const v2d *>(p), b = *reinterpret_cast<const v2d *>(p + 8);
+        v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = p[u < 2 ? u : u + 6];
+    }
+}
+
+// Row and column tile of tile `loc` of a label: bands of BT row tiles, each walked column
+// tile by column tile.  False below the diagonal (first columns of a symmetric band).
+template <bool SYMM>
+__device__ inline bool tile_at(const DirectSeg &S, int te, int loc, int &rt, int &ct) {
+    const int nrt = (S.R1 + te - 1) / te, nct = (S.R2 + te - 1) / te;
+    int r0 = 0;
+    for (;; r0 += BT) {
+        const int n = min(BT, nrt - r0) * (SYMM ? nct - r0 : nct);
+        if (loc < n) break;
+        loc -= n;
+    }
+    const int h = min(BT, nrt - r0);
+    rt = r0 + loc % h;
+    ct = (SYMM ? r0 : 0) + loc / h;
+    return !SYMM || ct >= rt;
+}
+
+// Exponentials of a 16 x 16 fragment: s its Gram entries, rows from row0 with squared norms
+// in `nr` (lane r holds row r's), this lane's column with squared norm nc.
+__device__ inline void put_exps(const DirectSeg &S, const double (&s)[4], int row0, int col,
+                                double nr, double nc, double cy, const double *etab, int lane,
+                                double *Ex) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int rr = mfma16_row_f64(lane, v);
+        const double e = exp_scaled(fma(s[v], -2.0 * cy, cy * __shfl(nr, rr, 64) + cy * nc), etab);
+        if (row0 + rr < S.R1 && col < S.R2) Ex[S.eoff + (row0 + rr) * S.ld + col] = e;
+    }
+}
+
+// 32 x 32 tiles, one per work-group, its waves each taking every fourth 16 columns of the
+// descriptors straight into registers: no barrier until the end, the shortest chain.
+template <bool SYMM, bool VEC>
+__global__ __launch_bounds__(NT, 3) void exp_tiles_kernel(const DirectSeg *__restrict__ segs,
+                                                          int nseg, int tiles,
+                                                          const double *__restrict__ X1,
+                                                          const int *__restrict__ src1,
+                                                          const double *__restrict__ X2,
+                                                          const int *__restrict__ src2, int rep,
+                                                          double cy, double *__restrict__ Ex) {
+    constexpr int F = TE / 16, KW = 4;
+    __shared__ double red[KW][F * F * 4][64];
+    __shared__ double nrm[KW][2 * F * 16];
+    __shared__ double etab[64];
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    if (tid < 64) etab[tid] = kExp2Tab64[tid];
+    const int tile = xcd_tile();
+    const DirectSeg S = segs[seg_of(segs, nseg, tile, [](const DirectSeg &t) { return t.it; })];
+    int rt, ct;
+    if (!tile_at<SYMM>(S, TE, tile - S.it, rt, ct)) return;
+    const double *pa[F], *pb[F];
+#pragma unroll
+    for (int m = 0; m < F; ++m) {  // rows past the label's end repeat its last one
+        pa[m] = X1 + (size_t)src1[S.r1 + min(rt * TE + 16 * m + r, S.R1 - 1)] * rep + 2 * g;
+        pb[m] = X2 + (size_t)src2[S.r2 + min(ct * TE + 16 * m + r, S.R2 - 1)] * rep + 2 * g;
+    }
+    v4d c[F][F];
+    double na[F], nb[F];
+#pragma unroll
+    for (int m = 0; m < F; ++m) {
+        na[m] = nb[m] = 0.0;
+#pragma unroll
+        for (int n = 0; n < F; ++n) c[m][n] = (v4d){0.0, 0.0, 0.0, 0.0};
+    }
+    double a[2][F][4], b[2][F][4];
+    auto load = [&](int buf, int k) {
+#pragma unroll
+        for (int m = 0; m < F; ++m) {
+            load4<VEC>(pa[m] + k, a[buf][m]);
+            load4<VEC>(pb[m] + k, b[buf][m]);
+        }
+    };
+    auto mul = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+            for (int m = 0; m < F; ++m)
+#pragma unroll
+                for (int n = 0; n < F; ++n)
+                    c[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[buf][m][u], b[buf][n][u],
+                                                                   c[m][n], 0, 0, 0);
+#pragma unroll
+            for (int m = 0; m < F; ++m) {
+                na[m] = fma(a[buf][m][u], a[buf][m][u], na[m]);
+                nb[m] = fma(b[buf][m][u], b[buf][m][u], nb[m]);
+            }
+        }
+    };
+    const int whole = rep & ~15, kb = 16 * wv;
+    reg_pipeline((whole - kb + 16 * KW - 1) / (16 * KW),
+                 [&](int buf, int i) { load(buf, kb + i * 16 * KW); }, mul);
+    if (whole < rep && wv == KW - 1) {  // the last, partial 16 columns
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = whole + (u < 2 ? u : u + 6);
+            const bool in = k + 2 * g < rep;
+            const int at = in ? k : rep - 1 - 2 * g;
+#pragma unroll
+            for (int m = 0; m < F; ++m) {
+                const double x = pa[m][at], y = pb[m][at];
+                a[0][m][u] = in ? x : 0.0;
+                b[0][m][u] = in ? y : 0.0;
+            }
+        }
+        mul(0);
+    }
+#pragma unroll
+    for (int m = 0; m < F; ++m) {
+        na[m] += __shfl_xor(na[m], 16, 64);
+        na[m] += __shfl_xor(na[m], 32, 64);
+        nb[m] += __shfl_xor(nb[m], 16, 64);
+        nb[m] += __shfl_xor(nb[m], 32, 64);
+        if (g == 0) {
+            nrm[wv][16 * m + r] = na[m];
+            nrm[wv][16 * (F + m) + r] = nb[m];
+        }
+#pragma unroll
+        for (int n = 0; n < F; ++n)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) red[wv][(m * F + n) * 4 + v][lane] = c[m][n][v];
+    }
+    __syncthreads();
+    const int m = wv / F, n = wv % F;  // a fragment per wave
+    double nr = 0.0, nc = 0.0, s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int w = 0; w < KW; ++w) {
+        nr += nrm[w][16 * m + r];
+        nc += nrm[w][16 * (F + n) + r];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) s[v] += red[w][(m * F + n) * 4 + v][lane];
+    }
+    put_exps(S, s, rt * TE + 16 * m, ct * TE + 16 * n + r, nr, nc, cy, etab, lane, Ex);
+}
+
+// 64 x 64 tiles, 16 columns of both operands at a time through LDS (double-buffered, one
+// barrier a step), each wave a 32 x 32 quarter.  A row's 16 columns are four threads' loads
+// of 64 contiguous bytes: with a lane per row instead (operands straight into registers)
+// every lane is a cache access of its own, and the accesses, one a cycle, bound the kernel
+// (92% of its cycles; 920 us at 800 molecules against 675 here).  LDS holds fragments in lane order, 16-byte units with
+// the row XORed by 4 (column pair) so that neither the stores nor the reads conflict.
+constexpr int TL = 64;
+template <bool SYMM, bool VEC>
+__global__ __launch_bounds__(NT, 4) void exp_tiles_lds_kernel(
+    const DirectSeg *__restrict__ segs, int nseg, int tiles, const double *__restrict__ X1,
+    const int *__restrict__ src1, const double *__restrict__ X2, const int *__restrict__ src2,
+    int rep, double cy, double *__restrict__ Ex) {
+    // [buffer][operand][row group][8-column half][lane]
+    __shared__ v2d sh[2][2][4][2][64];
+    __shared__ double nrm[2][TL], etab[64];
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    if (tid < 64) etab[tid] = kExp2Tab64[tid];
+    const int tile = xcd_tile();
+    const DirectSeg S = segs[seg_of(segs, nseg, tile, [](const DirectSeg &t) { return t.it; })];
+    int rt, ct;
+    if (!tile_at<SYMM>(S, TL, tile - S.it, rt, ct)) return;
+    const int row = tid >> 2, part = tid & 3;
+    const double *pa = X1 + (size_t)src1[S.r1 + min(rt * TL + row, S.R1 - 1)] * rep + 2 * part;
+    const double *pb = X2 + (size_t)src2[S.r2 + min(ct * TL + row, S.R2 - 1)] * rep + 2 * part;
+    const int unit = 16 * part + ((row & 15) ^ (4 * part)), grp = row >> 4;
+    const int rdu = 16 * g + (r ^ (4 * g)), wr = wv >> 1, wc = wv & 1;
+    double a[4], b[4], na = 0.0, nb = 0.0;
+    auto load = [&](int k) {
+        load4<VEC>(pa + k, a);
+        load4<VEC>(pb + k, b);
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            na = fma(a[u], a[u], na);
+            nb = fma(b[u], b[u], nb);
+        }
+        sh[buf][0][grp][0][unit] = (v2d){a[0], a[1]};
+        sh[buf][0][grp][1][unit] = (v2d){a[2], a[3]};
+        sh[buf][1][grp][0][unit] = (v2d){b[0], b[1]};
+        sh[buf][1][grp][1][unit] = (v2d){b[2], b[3]};
+    };
+    v4d c[2][2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) c[m][n] = (v4d){0.0, 0.0, 0.0, 0.0};
+    auto mul = [&](int buf) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            v2d x[2], y[2];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                x[m] = sh[buf][0][2 * wr + m][h][rdu];
+                y[m] = sh[buf][1][2 * wc + m][h][rdu];
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+#pragma unroll
+                    for (int n = 0; n < 2; ++n)
+                        c[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[m][u], y[n][u], c[m][n],
+                                                                       0, 0, 0);
+        }
+    };
+    const int whole = rep >> 4, steps = (rep + 15) >> 4;
+    auto load_tail = [&]() {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = 16 * whole + (u < 2 ? u : u + 6);
+            const bool in = k + 2 * part < rep;
+            const int at = in ? k : rep - 1 - 2 * part;
+            const double x = pa[at], y = pb[at];
+            a[u] = in ? x : 0.0;
+            b[u] = in ? y : 0.0;
+        }
+    };
+    if (whole > 0) load(0);
+    else load_tail();
+    store(0);
+    __syncthreads();
+    for (int i = 0; i < steps; ++i) {
+        const bool more = i + 1 < steps;  // uniform
+        if (more) {
+            if (i + 1 < whole) load(16 * (i + 1));
+            else load_tail();
+        }
+        mul(i & 1);
+        if (more) store((i + 1) & 1);
+        __syncthreads();
+    }
+    na += __shfl_xor(na, 1, 64);
+    na += __shfl_xor(na, 2, 64);
+    nb += __shfl_xor(nb, 1, 64);
+    nb += __shfl_xor(nb, 2, 64);
+    if (part == 0) {
+        nrm[0][row] = na;
+        nrm[1][row] = nb;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int rl = 32 * wr + 16 * m, cl = 32 * wc + 16 * n;
+            const double s[4] = {c[m][n][0], c[m][n][1], c[m][n][2], c[m][n][3]};
+            put_exps(S, s, rt * TL + rl, ct * TL + cl + r, nrm[0][rl + r], nrm[1][cl + r], cy, etab,
+                     lane, Ex);
+        }
+}
+
+// K[a, b] = sum over the labels and the label's rows of a and b of the exponentials.  Eight
+// lanes share a molecule pair, each taking every eighth row of a.
+template <int MODE>
+__global__ __launch_bounds__(NT) void pair_sums_kernel(const DirectSeg *__restrict__ segs,
+                                                       const double *__restrict__ Ex,
+                                                       const int *__restrict__ mol1,
+                                                       const int *__restrict__ mol2, int nseg,
+                                                       int nm1, int nm2,
+                                                       double *__restrict__ out) {
+    constexpr bool SYMM = MODE != DIRECT_RECT;
+    const int nbk = (nm2 + 31) / 32, sub = threadIdx.x & 7;
+    const int a = blockIdx.x / nbk, b = (blockIdx.x % nbk) * 32 + (threadIdx.x >> 3);
+    if (b >= nm2 || (SYMM && b < a)) return;
+    double s = 0.0;
+    for (int l = 0; l < nseg; ++l) {
+        const DirectSeg &S = segs[l];
+        const int *ma = mol1 + (size_t)l * (nm1 + 1) + a, *mb = mol2 + (size_t)l * (nm2 + 1) + b;
+        const int i0 = ma[0] - S.r1, i1 = ma[1] - S.r1, j0 = mb[0] - S.r2, j1 = mb[1] - S.r2;
+        for (int i = i0 + sub; i < i1; i += 8) {
+            const double *e = Ex + S.eoff;
+            if (SYMM && a == b) {  // only tiles of the upper triangle were formed
+                for (int j = j0; j < j1; ++j) s += e[(size_t)min(i, j) * S.ld + max(i, j)];
+            } else {
+                int j = j0;
+                for (; j + 4 <= j1; j += 4) {
+                    const double *p = e + (size_t)i * S.ld + j;
+                    s += (p[0] + p[1]) + (p[2] + p[3]);
+                }
+                for (; j < j1; ++j) s += e[(size_t)i * S.ld + j];
+            }
+        }
+    }
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    s += __shfl_xor(s, 4, 64);
+    if (sub) return;
+    if (MODE == DIRECT_SYMM_RFP) {
+        out[rfp_upper((size_t)nm1, a, b)] = s;
+    } else {
+        out[(size_t)a * nm2 + b] = s;
+        if (SYMM) out[(size_t)b * nm2 + a] = s;
+    }
+}
+
+}  // namespace
+
+int local_direct(int mode, const LocalPlan &p1, const double *X1, const LocalPlan &p2,
+                 const double *X2, int rep, double cy, double *out, int timer_id,
+                 hipStream_t stream) {
+    const bool symm = mode != DIRECT_RECT;
+    const int L = p1.nlabels, nm1 = p1.nm, nm2 = p2.nm;
+    std::vector<DirectSeg> segs(L);
+    // 64 x 64 tiles once there are enough to fill the GPU and they are not mostly padding: one
+    // costs about 2.8 of the 32 x 32 ones (800 molecules 675 us against 950; one molecule
+    // against 10,000, whose 14 atoms fill neither, 257 against 185)
+    auto count = [&](int te) {
+        int n = 0;
+        for (int l = 0; l < L; ++l) {
+            const int *a = &p1.mol_row[(size_t)l * (nm1 + 1)], *b = &p2.mol_row[(size_t)l * (nm2 + 1)];
+            const int t1 = ceil_div(a[nm1] - a[0], te), t2 = ceil_div(b[nm2] - b[0], te);
+            segs[l].it = n;
+            if (t1 > 0 && t2 > 0)
+                for (int r0 = 0; r0 < t1; r0 += BT) n += std::min(BT, t1 - r0) * (symm ? t2 - r0 : t2);
+        }
+        return n;
+    };
+    int tiles = count(TL);
+    const int small = count(TE);
+    const bool lds = tiles >= kLdsTiles && 2.8 * tiles < small;
+    tiles = lds ? count(TL) : small;
+    size_t elen = 0;
+    for (int l = 0; l < L; ++l) {
+        const int *a = &p1.mol_row[(size_t)l * (nm1 + 1)], *b = &p2.mol_row[(size_t)l * (nm2 + 1)];
+        const int R1 = a[nm1] - a[0], R2 = b[nm2] - b[0];
+        segs[l] = {a[0], R1, b[0], R2, segs[l].it, 0, elen, (size_t)R2};
+        elen += (size_t)R1 * R2;
+    }
+    // one upload: segments, then the rows' sources and the molecules' row ranges
+    const size_t n1 = p1.src.size(), m1 = p1.mol_row.size();
+    const size_t n2 = symm ? 0 : p2.src.size(), m2 = symm ? 0 : p2.mol_row.size();
+    const size_t bytes = sizeof(DirectSeg) * L + sizeof(int) * (n1 + m1 + n2 + m2);
+    char *dev = static_cast<char *>(workspace(WS_PLAN, bytes, stream));
+    char *stage = static_cast<char *>(host_staging(WS_PLAN, bytes));
+    double *Ex = static_cast<double *>(workspace(WS_PACK, sizeof(double) * elen, stream));
+    KF_REQUIRE(dev && stage && Ex, KF_ERR_NOMEM, "workspace allocation failed (%zu B)",
+               sizeof(double) * elen);
+    std::copy(segs.begin(), segs.end(), reinterpret_cast<DirectSeg *>(stage));
+    int *h = reinterpret_cast<int *>(stage + sizeof(DirectSeg) * L);
+    h = std::copy(p1.src.begin(), p1.src.end(), h);
+    h = std::copy(p1.mol_row.begin(), p1.mol_row.end(), h);
+    if (!symm) {
+        h = std::copy(p2.src.begin(), p2.src.end(), h);
+        std::copy(p2.mol_row.begin(), p2.mol_row.end(), h);
+    }
+    KF_HIP_TRY(hipMemcpyAsync(dev, stage, bytes, hipMemcpyHostToDevice, stream));
+    const DirectSeg *dseg = reinterpret_cast<const DirectSeg *>(dev);
+    const int *src1 = reinterpret_cast<const int *>(dev + sizeof(DirectSeg) * L);
+    const int *mol1 = src1 + n1, *src2 = symm ? src1 : mol1 + m1, *mol2 = symm ? mol1 : src2 + n2;
+    ScopedTimer timer(timer_id, stream);
+    const bool vec = rep % 2 == 0 && ((reinterpret_cast<size_t>(X1) | reinterpret_cast<size_t>(X2)) & 15) == 0;
+    if (tiles > 0) {
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(tiles), dim3(NT), 0, stream, dseg, L, tiles, X1, src1, X2,
+                               src2, rep, cy, Ex);
+        };
+        if (symm) {
+            if (lds) vec ? launch(exp_tiles_lds_kernel<true, true>) : launch(exp_tiles_lds_kernel<true, false>);
+            else vec ? launch(exp_tiles_kernel<true, true>) : launch(exp_tiles_kernel<true, false>);
+        } else {
+            if (lds) vec ? launch(exp_tiles_lds_kernel<false, true>) : launch(exp_tiles_lds_kernel<false, false>);
+            else vec ? launch(exp_tiles_kernel<false, true>) : launch(exp_tiles_kernel<false, false>);
+        }
+        KF_HIP_TRY(hipGetLastError());
+    }
+    const unsigned grid = (unsigned)nm1 * (unsigned)ceil_div(nm2, 32);
+    auto sums = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, stream, dseg, Ex, mol1, mol2, L, nm1, nm2,
+                           out);
+    };
+    if (mode == DIRECT_SYMM_RFP) sums(pair_sums_kernel<DIRECT_SYMM_RFP>);
+    else if (mode == DIRECT_SYMM_DENSE) sums(pair_sums_kernel<DIRECT_SYMM_DENSE>);
+    else sums(pair_sums_kernel<DIRECT_RECT>);
+    KF_HIP_TRY(hipGetLastError());
+    return KF_OK;
+}
+
+}  // namespace kf

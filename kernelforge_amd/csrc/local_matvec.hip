@@ -22,9 +22,9 @@
 // (C9H8O4 conformers use 312 of 720).  All labels share each launch: the packed rows of a
 // label start at a multiple of 16 and are padded with zero rows to one, and a list of
 // segments (label, query rows) tells a wave which tile it has.  Operands go from global
-// memory straight into registers: the 16 values of a row that four MFMA steps need are
-// 32 contiguous bytes per lane when the summation index of a step is permuted the same way
-// in both operands (lane group g holds k = 4 g + u at step u), so no LDS tile and no
+// memory straight into registers: the 16 values of a row that four MFMA steps need are two
+// 16-byte loads per lane when the summation index of a step is permuted the same way in
+// both operands (lane group g holds k = 2 g, 2 g + 1, 2 g + 8, 2 g + 9), so no LDS tile and no
 // barrier is needed, and a product with a handful of query rows runs at the speed its
 // training rows can be read.
 //
@@ -39,6 +39,7 @@
 
 #include "kf_common.hpp"
 #include "local_plan.hpp"
+#include "reg_pipeline.hpp"
 
 namespace kf {
 namespace {
@@ -186,9 +187,10 @@ __device__ inline int xcd_tile() {
     return (G % 8 == 0) ? (g % 8) * (G / 8) + g / 8 : g;
 }
 
-// The four summation steps of 16 columns: k = 4 g + u at step u for lane group g.
+// The four summation steps of 16 columns: k = 2 g, 2 g + 1, 2 g + 8, 2 g + 9 for lane group
+// g, so that a load takes 64 contiguous bytes of 16 rows.
 __device__ inline void load4(const double *p, double (&v)[4]) {
-    const v2d a = *reinterpret_cast<const v2d *>(p), b = *reinterpret_cast<const v2d *>(p + 2);
+    const v2d a = *reinterpret_cast<const v2d *>(p), b = *reinterpret_cast<const v2d *>(p + 8);
     v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
 }
 
@@ -214,10 +216,10 @@ __global__ __launch_bounds__(NT, 2) void coef_kernel(
     const double *pa[MF], *pb[NFT], *pd[NFT];
 #pragma unroll
     for (int m = 0; m < MF; ++m)
-        pa[m] = Xq + (size_t)min(S.q0 + m0 + 16 * m + r, qrows - 1) * nfp + 4 * g;
+        pa[m] = Xq + (size_t)min(S.q0 + m0 + 16 * m + r, qrows - 1) * nfp + 2 * g;
 #pragma unroll
     for (int n = 0; n < NFT; ++n) {
-        pb[n] = P2 + (size_t)(2 * S.r2 + min(n0 + 16 * n + r, S.R2p - 1)) * nfp + 4 * g;
+        pb[n] = P2 + (size_t)(2 * S.r2 + min(n0 + 16 * n + r, S.R2p - 1)) * nfp + 2 * g;
         pd[n] = pb[n] + (size_t)S.R2p * nfp;
     }
     v4d s[MF][NFT], p[MF][NFT];
@@ -248,16 +250,9 @@ __global__ __launch_bounds__(NT, 2) void coef_kernel(
                                                                    p[m][n], 0, 0, 0);
                 }
     };
-    constexpr int step = 16 * KW;
     const int kb = KW == 1 ? 0 : 16 * wv;
-    if (kb < nfp) load(0, kb);
-    for (int k = kb; k < nfp; k += 2 * step) {
-        if (k + step < nfp) load(1, k + step);
-        mul(0);
-        if (k + step >= nfp) break;
-        if (k + 2 * step < nfp) load(0, k + 2 * step);
-        mul(1);
-    }
+    reg_pipeline((nfp - kb + 16 * KW - 1) / (16 * KW),
+                 [&](int buf, int i) { load(buf, kb + i * 16 * KW); }, mul);
     if (KW > 1) {
 #pragma unroll
         for (int m = 0; m < MF; ++m)
@@ -340,10 +335,10 @@ __global__ __launch_bounds__(NT, 2) void weighted_rows_kernel(const MvSeg *__res
     const double *pa[MF], *pb[NF];
 #pragma unroll
     for (int m = 0; m < MF; ++m)
-        pa[m] = T + S.toff + (size_t)min(m0 + 16 * m + r, S.R1 - 1) * (2 * S.R2p) + 4 * g;
+        pa[m] = T + S.toff + (size_t)min(m0 + 16 * m + r, S.R1 - 1) * (2 * S.R2p) + 2 * g;
 #pragma unroll
     for (int n = 0; n < NF; ++n)
-        pb[n] = P2 + (size_t)(2 * S.r2 + 4 * g) * nfp + min(n0 + 16 * n + r, nfp - 1);
+        pb[n] = P2 + (size_t)(2 * S.r2 + 2 * g) * nfp + min(n0 + 16 * n + r, nfp - 1);
     v4d c[MF][NF];
 #pragma unroll
     for (int m = 0; m < MF; ++m)
@@ -356,7 +351,7 @@ __global__ __launch_bounds__(NT, 2) void weighted_rows_kernel(const MvSeg *__res
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int n = 0; n < NF; ++n) b[buf][n][u] = pb[n][(size_t)(k + u) * nfp];
+            for (int n = 0; n < NF; ++n) b[buf][n][u] = pb[n][(size_t)(k + (u < 2 ? u : u + 6)) * nfp];
     };
     auto mul = [&](int buf) {
 #pragma unroll
@@ -368,14 +363,7 @@ __global__ __launch_bounds__(NT, 2) void weighted_rows_kernel(const MvSeg *__res
                     c[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[buf][m][u], b[buf][n][u],
                                                                    c[m][n], 0, 0, 0);
     };
-    load(0, kb);
-    for (int k = kb; k < ke; k += 32) {
-        if (k + 16 < ke) load(1, k + 16);
-        mul(0);
-        if (k + 16 >= ke) break;
-        if (k + 32 < ke) load(0, k + 32);
-        mul(1);
-    }
+    reg_pipeline((ke - kb) / 16, [&](int buf, int i) { load(buf, kb + i * 16); }, mul);
     double *out = G + S.goff + (size_t)split * S.R1 * nfp;
 #pragma unroll
     for (int m = 0; m < MF; ++m)

@@ -77,6 +77,38 @@ inline void build_plan(const int *Q, const int *N, int nm, int ma, const std::ve
     }
 }
 
+// Atoms (i < N[a]) of each of the given (sorted) labels.
+inline std::vector<long long> label_counts(const int *Q, const int *N, int nm, int ma,
+                                           const std::vector<int> &labels) {
+    constexpr int kDirect = 256;
+    long long direct[kDirect] = {};
+    std::vector<long long> out(labels.size(), 0);
+    for (int a = 0; a < nm; ++a) {
+        const int na = clamp_atoms(N[a], ma);
+        const int *q = Q + (size_t)a * ma;
+        for (int i = 0; i < na; ++i) {
+            if (q[i] >= 0 && q[i] < kDirect) {
+                ++direct[q[i]];
+            } else {
+                const auto it = std::lower_bound(labels.begin(), labels.end(), q[i]);
+                if (it != labels.end() && *it == q[i]) ++out[it - labels.begin()];
+            }
+        }
+    }
+    for (size_t l = 0; l < labels.size(); ++l)
+        if (labels[l] >= 0 && labels[l] < kDirect) out[l] = direct[labels[l]];
+    return out;
+}
+
+// Label-matched atom pairs of two sets; half of them (rounded up per label) for the
+// symmetric kernels, where both are one set.
+inline long long matched_pairs(const std::vector<long long> &c1, const std::vector<long long> &c2,
+                               bool symm) {
+    long long n = 0;
+    for (size_t l = 0; l < c1.size(); ++l) n += symm ? (c1[l] * c2[l] + 1) / 2 : c1[l] * c2[l];
+    return n;
+}
+
 // Sorted distinct labels of the atoms (i < N[a]).  Labels in [0, 256) (atomic numbers)
 // are collected in a presence table; any others are sorted and merged in.
 inline std::vector<int> distinct_labels(const int *Q, const int *N, int nm, int ma) {

@@ -34,6 +34,7 @@
 #include <cmath>
 #include <vector>
 
+#include "local_direct.hpp"
 #include "local_mixed.hpp"
 
 namespace kf {
@@ -41,7 +42,7 @@ namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-constexpr int MB = 64;       // molecules per output block
+constexpr int MB = 64;       // most molecules per output block (block_size)
 constexpr int TS = 64;       // sub-tile edge (packed rows)
 constexpr int KA = 32;       // row-operand chunk staged in LDS (descriptor columns)
 constexpr int KS = 16;       // column-operand sub-chunk held in registers
@@ -99,30 +100,39 @@ __device__ __forceinline__ unsigned long long slice_windows(unsigned long long b
 }
 
 // mask[a] = windows in which some atom of molecule a is non-zero (two words per molecule).
-// One wave per molecule.
+// One work-group per molecule, the 64-column slices dealt over its waves (one wave for all
+// slices: 78 us for 800 molecules, a chain of 168 loads).
 __global__ __launch_bounds__(256) void mol_winmask_kernel(const double *__restrict__ X,
-                                                          const int *__restrict__ N, int nm,
-                                                          int ma, int rep,
+                                                          const int *__restrict__ N, int ma,
+                                                          int rep,
                                                           unsigned long long *__restrict__ mask) {
-    const int a = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (a >= nm) return;
+    __shared__ unsigned long long part[4][2];
+    const int a = blockIdx.x;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int na = min(max(N[a], 0), ma);
     const double *x = X + (size_t)a * ma * rep;
     unsigned long long w0 = 0, w1 = 0;
-    for (int j = 0; j * 64 < rep && 4 * j < kMaxWin; ++j) {
+    for (int j = wave; j * 64 < rep && 4 * j < kMaxWin; j += 4) {
         const int k = j * 64 + lane;
         bool nz = false;
         if (k < rep)
-            for (int i = 0; i < na; ++i) nz |= x[(size_t)i * rep + k] != 0.0;
+            for (int i = 0; i < na; i += 4) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    nz |= x[(size_t)min(i + u, na - 1) * rep + k] != 0.0;
+            }
         const unsigned long long w = slice_windows(__ballot(nz));
         if (j < 16) w0 |= w << (4 * j);
         else w1 |= w << (4 * j - 64);
     }
     if (lane == 0) {
-        mask[2 * (size_t)a] = w0;
-        mask[2 * (size_t)a + 1] = w1;
+        part[wave][0] = w0;
+        part[wave][1] = w1;
     }
+    __syncthreads();
+    if (threadIdx.x < 2)
+        mask[2 * (size_t)a + threadIdx.x] = part[0][threadIdx.x] | part[1][threadIdx.x] |
+                                            part[2][threadIdx.x] | part[3][threadIdx.x];
 }
 
 // pack: Xp[row, k] = X[xrow, k] (k < rep), 0 for rep <= k < rep_pad, where the plan's
@@ -251,12 +261,13 @@ __device__ __forceinline__ unsigned long long wave_or64(unsigned long long m) {
 // work-group per (label, block), a wave per tile.
 __global__ __launch_bounds__(256) void tile_mask_kernel(const unsigned long long *__restrict__ rowmask,
                                                         const int *__restrict__ mol_row, int nm,
-                                                        int nblk, const int *__restrict__ tbase,
+                                                        int mb, int nblk,
+                                                        const int *__restrict__ tbase,
                                                         ulonglong2 *__restrict__ tmask) {
     const int la = blockIdx.x, l = la / nblk, A = la - l * nblk;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int *mr = mol_row + (size_t)l * (nm + 1);
-    const int r0 = mr[A * MB], r1 = mr[min(A * MB + MB, nm)];
+    const int r0 = mr[A * mb], r1 = mr[min(A * mb + mb, nm)];
     const int nt = (r1 - r0 + TS - 1) / TS;
     for (int t = wave; t < nt; t += 4) {
         const int r = r0 + t * TS + lane;
@@ -661,6 +672,7 @@ struct WinArgs {
     const int *perm1, *perm2;     // output index of each molecule (null: identity)
     const double *mu1, *mu2;      // int8-split form: the rows' scales (null: FP64 form)
     int nblk1, nblk2, nwin;       // blocks per set, windows of the padded descriptor
+    int mb1, mb2;                 // molecules per block of each set (<= MB)
 };
 
 // NS = 0: FP64 operands (rows of rep_pad doubles), two column tiles per row tile;
@@ -706,8 +718,8 @@ __global__ __launch_bounds__(NT, NS ? 2 : 3) void local_scalar_f64_kernel(
     __syncthreads();
     double *const accL = g_acc_slots + (size_t)s_slot * (MB * AP);
     const int A = ab.x, B = ab.y;
-    const int a0 = A * MB, na = min(MB, nm1 - a0);
-    const int b0 = B * MB, nb = min(MB, nm2 - b0);
+    const int a0 = A * wa.mb1, na = min(wa.mb1, nm1 - a0);
+    const int b0 = B * wa.mb2, nb = min(wa.mb2, nm2 - b0);
     const bool diag = (MODE != RECT) && (A == B);
     const int ob = tid & (MB - 1), oa0 = (tid / MB) * (MB / 4);
     const int lrow = tid >> 2, bcol = wave * 16 + (lane & 15);
@@ -718,7 +730,7 @@ __global__ __launch_bounds__(NT, NS ? 2 : 3) void local_scalar_f64_kernel(
     GramI8Args g8;
     g8.stk = (lane & 3) ^ ((lane >> 3) & 3);
     g8.rdo = (lane & 15) * 64 + 16 * ((lane >> 4) ^ (((lane & 15) >> 1) & 3));
-    for (int k = tid; k < MB * AP; k += NT) accL[k] = 0.0;
+    for (int k = tid; k < na * AP; k += NT) accL[k] = 0.0;
     if (tid < 64) etab[tid] = kExp2Tab64[tid];  // ordered by the label loop's first barrier
 
     for (int l = 0; l < L; ++l) {
@@ -977,7 +989,7 @@ struct DevicePacked {
     int *mol_row = nullptr, *src = nullptr, *perm = nullptr, *tbase = nullptr;
     unsigned long long *rowmask = nullptr;
     ulonglong2 *tmask = nullptr;  // null: windows not masked
-    int rows = 0, rep_pad = 0, nblk = 0, nwin = 0;
+    int rows = 0, rep_pad = 0, mb = 0, nblk = 0, nwin = 0;
 };
 
 inline int padded_rep(int rep) { return (rep + KA - 1) / KA * KA; }
@@ -996,8 +1008,7 @@ int molecule_windows(const double *X, const int *N, int nm, int ma, int rep, int
     auto *dm = static_cast<unsigned long long *>(workspace(ws, bytes, stream));
     auto *hm = static_cast<unsigned long long *>(host_staging(ws, bytes));
     KF_REQUIRE(dm && hm, KF_ERR_NOMEM, "workspace allocation failed (%zu B)", bytes);
-    hipLaunchKernelGGL(mol_winmask_kernel, dim3((nm + 3) / 4), dim3(256), 0, stream, X, N, nm, ma,
-                       rep, dm);
+    hipLaunchKernelGGL(mol_winmask_kernel, dim3(nm), dim3(256), 0, stream, X, N, ma, rep, dm);
     KF_HIP_TRY(hipGetLastError());
     KF_HIP_TRY(hipMemcpyAsync(hm, dm, bytes, hipMemcpyDeviceToHost, stream));
     KF_HIP_TRY(hipStreamSynchronize(stream));
@@ -1104,11 +1115,12 @@ void permute_metadata(const std::vector<int> &Q, const std::vector<int> &N, int 
 // Upload the plan (plus the molecule order, if any), pack the rows and, when the windows
 // are masked, build the masks of the kernel's row tiles.
 int upload_and_pack(const LocalPlan &p, const std::vector<int> &perm, const double *X, int rep,
-                    int ns, int ws_pack, int ws_plan, hipStream_t stream, DevicePacked &d) {
+                    int ns, int mb, int ws_pack, int ws_plan, hipStream_t stream, DevicePacked &d) {
     d.rows = p.rows;
     d.nwin = ns ? i8_windows(rep) : padded_rep(rep) / KS;
     d.rep_pad = ns ? d.nwin * kI8WinBytes : padded_rep(rep);
-    d.nblk = (p.nm + MB - 1) / MB;
+    d.mb = mb;
+    d.nblk = (p.nm + mb - 1) / mb;
     const bool masked = windows_masked(rep, ns);
     const size_t mr_n = p.mol_row.size(), src_n = p.src.size(), perm_n = perm.size();
     const size_t nla = (size_t)p.nlabels * d.nblk;
@@ -1117,7 +1129,7 @@ int upload_and_pack(const LocalPlan &p, const std::vector<int> &perm, const doub
     for (int l = 0; l < p.nlabels; ++l)
         for (int A = 0; A < d.nblk; ++A) {
             const int *mr = p.mol_row.data() + (size_t)l * (p.nm + 1);
-            const int rows = mr[std::min(A * MB + MB, p.nm)] - mr[A * MB];
+            const int rows = mr[std::min(A * mb + mb, p.nm)] - mr[A * mb];
             tbase[(size_t)l * d.nblk + A + 1] = tbase[(size_t)l * d.nblk + A] + (rows + TS - 1) / TS;
         }
     const size_t ntile_masks = masked ? (size_t)tbase[nla] : 0;
@@ -1161,7 +1173,7 @@ int upload_and_pack(const LocalPlan &p, const std::vector<int> &perm, const doub
         KF_HIP_TRY(hipGetLastError());
         if (masked && nla > 0) {
             hipLaunchKernelGGL(tile_mask_kernel, dim3((unsigned)nla), dim3(256), 0, stream,
-                               d.rowmask, d.mol_row, p.nm, d.nblk, d.tbase, d.tmask);
+                               d.rowmask, d.mol_row, p.nm, mb, d.nblk, d.tbase, d.tmask);
             KF_HIP_TRY(hipGetLastError());
         }
     }
@@ -1181,6 +1193,8 @@ WinArgs win_args(const DevicePacked &d1, const DevicePacked &d2) {
     w.nblk1 = d1.nblk;
     w.nblk2 = d2.nblk;
     w.nwin = d1.nwin;
+    w.mb1 = d1.mb;
+    w.mb2 = d2.mb;
     return w;
 }
 
@@ -1223,6 +1237,26 @@ int upload_block_order(int nb1, int nb2, bool symm, hipStream_t stream, const in
     *dev = d;
     *grid = (unsigned)order.size();
     return KF_OK;
+}
+
+// Up to this many label-matched atom pairs the packing-free form (local_direct.hip) is
+// faster: 800 molecules (2.2e7 pairs) 826 us a call against 873, 333 against 2,000 (4.5e7)
+// 1,496 against 1,835; beyond, skipping the zero windows pays: 1,200 molecules (4.9e7) 1,618
+// against 1,500, 1,500 against 1,500 (1.5e8) 6.3 ms against 3.9.
+constexpr long long kDirectPairs = 40000000;
+
+// Molecules per block of the symmetric kernel for `pairs` matched atom pairs.  Small blocks
+// give more work-groups and a shorter longest one, large ones fuller tiles (1,600 molecules,
+// 8.7e7 pairs: blocks of 24 2.0 ms, 32 2.0, 64 3.6; 3,200, 3.5e8: 6.9, 6.4 and 7.6; 6,400,
+// 1.4e9: 25.8, 24.4 and 22.3).
+int symm_block(long long pairs) { return pairs < 140000000 ? 24 : pairs < 1100000000 ? 32 : MB; }
+
+// The rectangular kernel's, by the same measure (333 against 10,000 molecules: 16 x 32
+// 5.0 ms, 32 x 64 5.7, 64 x 64 7.1; 1,500 against 12,000: 22.1, 19.8 and 21.3 ms).
+void rect_blocks(long long pairs, int &mb1, int &mb2) {
+    const bool small = pairs < 460000000;
+    mb1 = small ? 16 : 32;
+    mb2 = small ? 32 : 64;
 }
 
 // Launch of the scalar kernel in its FP64 form (ns = 0) or int8-split form (ns slices).
@@ -1280,6 +1314,19 @@ int symm_impl(int precision, const double *X, const int *Q, const int *N, int nm
         build_plan(hQ.data(), hN.data(), nm, ma, labels, p);
         return local_mixed_symm(MODE == SYMM_DENSE, X, nm, ma, rep, sigma, p, out, stream);
     }
+    const double cy = -kExpScale / (2.0 * sigma * sigma);  // squared distance -> exp_scaled's y
+    if (labels.empty()) {  // no atoms at all: zero output
+        const size_t n = MODE == SYMM_RFP ? (size_t)nm * (nm + 1) / 2 : (size_t)nm * nm;
+        KF_HIP_TRY(hipMemsetAsync(out, 0, n * sizeof(double), stream));
+        return KF_OK;
+    }
+    const std::vector<long long> cnt = label_counts(hQ.data(), hN.data(), nm, ma, labels);
+    const long long pairs = matched_pairs(cnt, cnt, true);
+    if (ns == 0 && pairs <= kDirectPairs) {
+        build_plan(hQ.data(), hN.data(), nm, ma, labels, p);
+        return local_direct(MODE == SYMM_RFP ? DIRECT_SYMM_RFP : DIRECT_SYMM_DENSE, p, X, p, X,
+                            rep, cy, static_cast<double *>(out), TM_LOCAL_SYMM, stream);
+    }
     std::vector<int> perm, Qp, Np;
     if (windows_masked(rep, ns)) {
         std::vector<unsigned long long> mm;
@@ -1291,14 +1338,9 @@ int symm_impl(int precision, const double *X, const int *Q, const int *N, int nm
         build_plan(hQ.data(), hN.data(), nm, ma, labels, p);
     }
     DevicePacked d;
-    if ((rc = upload_and_pack(p, perm, X, rep, ns, WS_PACK, WS_PLAN, stream, d))) return rc;
-    const int nblk = (nm + MB - 1) / MB;
-    const double cy = -kExpScale / (2.0 * sigma * sigma);  // squared distance -> exp_scaled's y
-    if (p.nlabels == 0) {  // no atoms at all: zero output
-        const size_t n = MODE == SYMM_RFP ? (size_t)nm * (nm + 1) / 2 : (size_t)nm * nm;
-        KF_HIP_TRY(hipMemsetAsync(out, 0, n * sizeof(double), stream));
-        return KF_OK;
-    }
+    const int mb = ns ? MB : symm_block(pairs);
+    if ((rc = upload_and_pack(p, perm, X, rep, ns, mb, WS_PACK, WS_PLAN, stream, d))) return rc;
+    const int nblk = d.nblk;
     const int2 *order = nullptr;
     unsigned grid = 0;
     if ((rc = upload_block_order(nblk, nblk, true, stream, &order, &grid))) return rc;
@@ -1360,6 +1402,16 @@ extern "C" int kf_local_kernel(int precision, const double *X1, const double *X2
         return local_mixed_rect(X1, X2, nm1, nm2, max_atoms1, max_atoms2, rep, sigma, p1, p2,
                                 static_cast<float *>(K), stream);
     }
+    const double cy = -kExpScale / (2.0 * sigma * sigma);  // squared distance -> exp_scaled's y
+    const long long pairs =
+        matched_pairs(label_counts(q1.data(), n1.data(), nm1, max_atoms1, labels),
+                      label_counts(q2.data(), n2.data(), nm2, max_atoms2, labels), false);
+    if (ns == 0 && pairs <= kDirectPairs) {
+        build_plan(q1.data(), n1.data(), nm1, max_atoms1, labels, p1);
+        build_plan(q2.data(), n2.data(), nm2, max_atoms2, labels, p2);
+        return local_direct(DIRECT_RECT, p1, X1, p2, X2, rep, cy, static_cast<double *>(K),
+                            TM_LOCAL_RECT, stream);
+    }
     std::vector<int> perm1, perm2;
     if (windows_masked(rep, ns)) {
         std::vector<unsigned long long> m1, m2;
@@ -1378,10 +1430,11 @@ extern "C" int kf_local_kernel(int precision, const double *X1, const double *X2
         build_plan(q2.data(), n2.data(), nm2, max_atoms2, labels, p2);
     }
     DevicePacked d1, d2;
-    if ((rc = upload_and_pack(p1, perm1, X1, rep, ns, WS_PACK, WS_PLAN, stream, d1))) return rc;
-    if ((rc = upload_and_pack(p2, perm2, X2, rep, ns, WS_PACK2, WS_PLAN2, stream, d2))) return rc;
-    const int nblk1 = (nm1 + MB - 1) / MB, nblk2 = (nm2 + MB - 1) / MB;
-    const double cy = -kExpScale / (2.0 * sigma * sigma);  // squared distance -> exp_scaled's y
+    int mb1 = MB, mb2 = MB;
+    if (ns == 0) rect_blocks(pairs, mb1, mb2);
+    if ((rc = upload_and_pack(p1, perm1, X1, rep, ns, mb1, WS_PACK, WS_PLAN, stream, d1))) return rc;
+    if ((rc = upload_and_pack(p2, perm2, X2, rep, ns, mb2, WS_PACK2, WS_PLAN2, stream, d2))) return rc;
+    const int nblk1 = d1.nblk, nblk2 = d2.nblk;
     const int2 *order = nullptr;
     unsigned grid = 0;
     if ((rc = upload_block_order(nblk1, nblk2, false, stream, &order, &grid))) return rc;

@@ -43,6 +43,57 @@ def test_rect_random(lk, nm1, nm2):
     assert rel_err(K, oracle.kernel_rect(x1, x2, q1, q2, n1, n2, 0.9)) < 1e-12
 
 
+# the packing-free form: rows of one label about a tile's edge and over it, descriptors of
+# one column, whole and partial groups of 16, odd ones (rows that are not 16-byte aligned)
+@pytest.mark.parametrize("nm,ma,rep", [(16, 2, 1), (33, 1, 31), (64, 2, 16), (230, 9, 1),
+                                       (230, 9, 15), (230, 9, 16), (231, 9, 50)])
+def test_direct_tiles(lk, nm, ma, rep):
+    x, q, n = random_set(nm, ma, rep, 1, 7 * nm + rep, nmin=ma)
+    s = 1.1 * np.sqrt(rep)
+    assert rel_err(lk.kernel_gaussian_symm(x, q, n, s), oracle.kernel_symm(x, q, n, s)) < 1e-12
+    assert rel_err(lk.kernel_gaussian_symm_rfp(x, q, n, s),
+                   oracle.kernel_symm_rfp(x, q, n, s)) < 1e-12
+    m = nm // 2 + 1
+    assert rel_err(lk.kernel_gaussian(x[:m], x, q[:m], q, n[:m], n, s),
+                   oracle.kernel_rect(x[:m], x, q[:m], q, n[:m], n, s)) < 1e-12
+
+
+@pytest.mark.parametrize("nm,ma", [(40, 3), (230, 9)])
+def test_direct_unaligned_rows(nm, ma):
+    """Descriptors that start 8 bytes off a 16-byte boundary (a view into a larger array)."""
+    from kernelforge_amd import capi
+
+    x, q, n = random_set(nm, ma, 48, 1, 3, nmin=ma)
+    DA = capi.DeviceArray
+    d = DA.from_numpy(np.concatenate([[0.0], x.reshape(-1)]))
+    dq, dn, K = DA.from_numpy(q), DA.from_numpy(n), DA(nm * (nm + 1) // 2)
+    capi.local_kernel_symm_rfp(capi.KF_PREC_F64, d.ptr + 8, dq.ptr, dn.ptr, nm, ma, 48, 5.0, K.ptr)
+    capi.synchronize()
+    assert rel_err(K.numpy(), oracle.kernel_symm_rfp(x, q, n, 5.0)) < 1e-12
+
+
+# the blocked form's block sizes (molecules of a block not a divisor of the set's), over the
+# matched atom pairs up to which the packing-free form runs
+@pytest.mark.parametrize("nm,rep", [(235, 24), (437, 9)])
+def test_symm_block_sizes(lk, nm, rep):
+    x, q, n = windowed_set(nm, 40, 16 * rep, 1, nm)
+    n[:] = 40
+    s = 0.35 * np.sqrt(16 * rep)
+    assert rel_err(lk.kernel_gaussian_symm(x, q, n, s), oracle.kernel_symm(x, q, n, s)) < 1e-12
+    assert rel_err(lk.kernel_gaussian_symm_rfp(x, q, n, s),
+                   oracle.kernel_symm_rfp(x, q, n, s)) < 1e-12
+
+
+@pytest.mark.parametrize("nm1,nm2,rep", [(101, 260, 40), (431, 707, 17)])
+def test_rect_block_sizes(lk, nm1, nm2, rep):
+    x1, q1, n1 = windowed_set(nm1, 40, rep, 1, 21)
+    x2, q2, n2 = windowed_set(nm2, 40, rep, 1, 22)
+    n1[:] = n2[:] = 40
+    s = 0.35 * np.sqrt(rep)
+    assert rel_err(lk.kernel_gaussian(x1, x2, q1, q2, n1, n2, s),
+                   oracle.kernel_rect(x1, x2, q1, q2, n1, n2, s)) < 1e-12
+
+
 def windowed_set(nm, ma, rep, nlab, seed, ngroups=7):
     """Random rows whose columns fall into groups (spans not aligned to the kernel's
     16-column windows) that each molecule uses or leaves at zero, single atoms dropping
