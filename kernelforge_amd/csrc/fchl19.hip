@@ -7,12 +7,11 @@
 // transcribed; it agrees with the reference to FP64 rounding.
 //
 // Work decomposition
-//  * representation: one workgroup (4 waves) per molecule.  Two-body: one
-//    thread per (atom, 8-wide radial chunk), pair quantities recomputed per
-//    chunk, every output written once (no atomics).  Three-body: one wave per
-//    centre; lanes first evaluate up to 64 triplets' geometry into LDS records,
-//    then lanes switch to owning output slots (l, t) and stream the records, so
-//    each rep entry has exactly one writer and a fixed summation order.
+//  * representation: a work-group per molecule, a batch of centres at a time.
+//    Neighbour pairs are numbered by element-pair channel; threads evaluate one
+//    (centre, pair) each into LDS, then own (channel, centre, radial term) and
+//    sum the pairs in registers, so each rep entry has exactly one writer and a
+//    fixed summation order.
 //  * Jacobian: one or more workgroups per (molecule, centre).  Six scalars per
 //    ordered neighbour pair in LDS; threads own (neighbour, radial term) and sum
 //    over the partners in registers; an element-pair channel's rows are put
@@ -54,11 +53,11 @@ __device__ inline int pair_channel(int nelem, int p, int q) {
 
 __device__ inline double cut_fn(double r, double cut) {
     const double inv = cut > 0.0 ? 1.0 / cut : 0.0;
-    return 0.5 * (cos(M_PI * r * inv) + 1.0);
+    return 0.5 * (cospi(r * inv) + 1.0);
 }
 __device__ inline double cut_dfn(double r, double cut) {
     const double inv = cut > 0.0 ? 1.0 / cut : 0.0;
-    return -0.5 * M_PI * inv * sin(M_PI * r * inv);
+    return -0.5 * M_PI * inv * sinpi(r * inv);
 }
 
 __device__ inline double dist(const double *R, int i, int j) {
@@ -98,165 +97,261 @@ __device__ inline void wave_sync() {
 }
 
 // ---------------------------------------------------------------------------
-// Representation kernel: one workgroup per molecule.
-// dynamic LDS: coords (max_atoms*3) | elem (max_atoms ints) |
-//              per wave: records (64 * (3 + na)) + acc (nchan*nb3*na)
+// Representation kernel: one work-group per molecule (several when the batch is small, each
+// with a run of its rows), a batch of centres at a time.
+//
+// Atoms are sorted by element once.  Leaving out the centre then leaves every element's
+// neighbours an index range, and the neighbour pairs of an element-pair channel too (a
+// np x nq grid, or a triangle); which ranges depends only on the centre's element.  Per
+// batch -- as many centres as have `pairs` neighbour pairs between them (13 of a 14-atom
+// molecule) -- the threads evaluate one (centre, neighbour) each (unit vector, cutoff,
+// two-body scalars), then one (centre, pair) each (rbar and the amplitude of every angular
+// term), and then own one channel, centre and two radial terms each and sum its pairs in
+// registers.  The lanes of a wave are of one channel and consecutive centres, whose pair
+// counts differ by little, so they run the same number of steps.  Every output has one
+// writing lane and a fixed summation order.  Bound by the FP64 VALU: the exponentials (one
+// per pair and radial term) and the pair geometry.  20,000 molecules of 5-23 atoms take
+// 2.30 ms (5.40 with a read-modify-write of an LDS accumulator per record and slot, 3.33 with
+// a wave per centre, 2.65 with one radial term per thread); without the exponential sums 1.5,
+// without the pair geometry 1.7, without both 1.0, of which the stores 0.4.
 // ---------------------------------------------------------------------------
 constexpr int kRepThreads = 256;
-constexpr int kRepWaves = kRepThreads / 64;
-constexpr int kK2Chunk = 8;
+constexpr int kLB = 2;  // radial terms per thread
+constexpr int kNbrFields = 8;  // unit vector, distance, cutoff, three two-body scalars
 
-__global__ __launch_bounds__(kRepThreads) void fchl19_rep_kernel(
+// LDS, in doubles: exp table | coordinates | neighbours (kNbrFields x nbrs) | pairs
+// ((1 + na) x pairs) | ints: element, atoms by element, place of an atom in that order,
+// first atom of an element, elements of a channel, first pair of a channel by the centre's
+// element
+struct RepLds {
+    int R, nbr, pair, ints, nbrs, pairs, total_ints;
+};
+__host__ __device__ inline RepLds rep_lds(int ma, int nelem, int nchan, int na) {
+    RepLds g;
+    g.nbrs = ma > 192 ? ma : 192;
+    g.pairs = 3072 / (1 + na) < 64 ? 64 : 3072 / (1 + na);
+    g.R = 64;
+    g.nbr = g.R + 3 * ma + (ma & 1);
+    g.pair = g.nbr + kNbrFields * g.nbrs;
+    g.ints = g.pair + (1 + na) * g.pairs;
+    g.total_ints = 3 * ma + nelem + 1 + nchan + nelem * (nchan + 1);
+    return g;
+}
+__host__ inline size_t rep_lds_bytes(int ma, int nelem, int nchan, int na) {
+    const RepLds g = rep_lds(ma, nelem, nchan, na);
+    return sizeof(double) * (size_t)g.ints + sizeof(int) * (size_t)g.total_ints;
+}
+
+__global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
     const double *__restrict__ coords, const int *__restrict__ Q, const int *__restrict__ N,
     FchlParams P, double *__restrict__ X, int *__restrict__ err) {
-    extern __shared__ double smem[];
-    const int m = blockIdx.x;
-    const int ma = P.max_atoms;
+    extern __shared__ __align__(16) double smem[];
+    __shared__ int next;
+    const int m = blockIdx.x, tid = threadIdx.x;
+    const int ma = P.max_atoms, nelem = P.nelem, nchan = P.nchan;
     int n = N[m];
     n = n < 0 ? 0 : (n > ma ? ma : n);
-    double *R = smem;
-    int *el = reinterpret_cast<int *>(R + 3 * ma);
-    double *wave_base = reinterpret_cast<double *>(el + ((ma + 1) & ~1));
-    const int rec_w = 3 + P.na;
-    const int acc_n = P.nchan * P.nb3 * P.na;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    double *recs = wave_base + (size_t)wave * (64 * rec_w + acc_n);
-    double *acc = recs + 64 * rec_w;
+    const RepLds g = rep_lds(ma, nelem, nchan, P.na);
+    double *tab = smem, *R = smem + g.R, *nbr = smem + g.nbr, *rbar = smem + g.pair,
+           *amp = rbar + g.pairs;
+    const double *ex = nbr, *ey = ex + g.nbrs, *ez = ey + g.nbrs, *rr = ez + g.nbrs,
+                 *fc = rr + g.nbrs, *t_mu = fc + g.nbrs, *t_sc = t_mu + g.nbrs,
+                 *t_f = t_sc + g.nbrs;
+    int *el = reinterpret_cast<int *>(smem + g.ints), *ord = el + ma, *place = ord + ma,
+        *est = place + ma, *chan = est + nelem + 1, *cst = chan + nchan;
 
     const double *Cm = coords + (size_t)m * ma * 3;
-    for (int t = threadIdx.x; t < 3 * n; t += blockDim.x) R[t] = Cm[t];
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-        const int e = elem_index(P, Q[(size_t)m * ma + t]);
-        el[t] = e;
-        if (e < 0) *err = 1;
+    bool bad = false;
+    for (int t = tid; t < 3 * n; t += kRepThreads) R[t] = Cm[t];
+    for (int t = tid; t < n; t += kRepThreads) {
+        el[t] = elem_index(P, Q[(size_t)m * ma + t]);
+        bad |= el[t] < 0;
+    }
+    if (tid < 64) tab[tid] = kExp2Tab64[tid];
+    for (int c = tid; c < nchan; c += kRepThreads) {
+        int p = 0, q = c;
+        while (q >= nelem - p) q -= nelem - p, ++p;
+        chan[c] = p << 16 | (p + q);
+    }
+    double *Xm = X + (size_t)m * ma * P.rs;
+    // a molecule with an unknown element is reported through *err; its rows are zeroed
+    if (__syncthreads_or(bad)) {
+        if (tid == 0) *err = 1;
+        n = 0;
+    }
+    const int per = (ma + gridDim.y - 1) / gridDim.y, row0 = blockIdx.y * per,
+              row1 = min(row0 + per, ma), cen1 = min(row1, n);
+    const int pad0 = max(row0, n);  // padding rows
+    if (pad0 < row1) {
+        double *d = Xm + (size_t)pad0 * P.rs;
+        const int cnt = (row1 - pad0) * P.rs;
+        for (int t = tid; t < cnt; t += kRepThreads) d[t] = 0.0;
+    }
+    if (row0 >= cen1) return;
+    for (int t = tid; t < n; t += kRepThreads) {
+        int rank = 0;
+        for (int s = 0; s < n; ++s) rank += (int)((el[s] < el[t]) | ((el[s] == el[t]) & (s < t)));
+        ord[rank] = t;
+        place[t] = rank;
+    }
+    for (int e = tid; e <= nelem; e += kRepThreads) {
+        int c = 0;
+        for (int s = 0; s < n; ++s) c += (int)(el[s] < e);
+        est[e] = c;
     }
     __syncthreads();
-    // a molecule with an unknown element is reported through *err; its rows are zeroed
-    bool bad = false;
-    for (int t = 0; t < n; ++t) bad |= el[t] < 0;
-
-    double *Xm = X + (size_t)m * ma * P.rs;
-    // zero the padding rows
-    for (size_t t = (size_t)n * P.rs + threadIdx.x; t < (size_t)ma * P.rs; t += blockDim.x)
-        Xm[t] = 0.0;
-    if (bad) {
-        for (size_t t = threadIdx.x; t < (size_t)n * P.rs; t += blockDim.x) Xm[t] = 0.0;
-        return;
+    for (int t = tid; t < nelem * (nchan + 1); t += kRepThreads) {
+        const int e = t / (nchan + 1), c1 = t - e * (nchan + 1);
+        int off = 0;
+        for (int c = 0; c < c1; ++c) {
+            const int p = chan[c] >> 16, q = chan[c] & 0xffff;
+            const int np = est[p + 1] - est[p] - (p == e), nq = est[q + 1] - est[q] - (q == e);
+            off += p == q ? np * (np - 1) / 2 : np * nq;
+        }
+        cst[t] = off;
     }
+    __syncthreads();
 
-    // ---- two-body: thread per (atom i, radial chunk) ----
-    const int nchunk = (P.nb2 + kK2Chunk - 1) / kK2Chunk;
-    for (int item = threadIdx.x; item < n * nchunk; item += blockDim.x) {
-        const int i = item / nchunk, k0 = (item % nchunk) * kK2Chunk;
-        const int kn = (P.nb2 - k0) < kK2Chunk ? (P.nb2 - k0) : kK2Chunk;
-        for (int e = 0; e < P.nelem; ++e) {
-            double v[kK2Chunk];
+    const int npair = (n - 1) * (n - 2) / 2;
+    const int batch = max(1, min(g.nbrs / n, npair > 0 ? g.pairs / npair : n));
+    const double ysc = -P.eta3 * kExpScale;
+    for (int i0 = row0; i0 < cen1; i0 += batch) {
+        const int B = min(batch, cen1 - i0);
+        __syncthreads();  // the previous batch's reads are done
+        // ---- (centre, neighbour) ----
+        for (int t = tid; t < B * n; t += kRepThreads) {
+            const int b = t / n, j = t - b * n, i = i0 + b;
+            double *f = nbr + t;
+            const double r = dist(R, i, j), ir = 1.0 / (r > kEps ? r : kEps);
+            for (int c = 0; c < 3; ++c) f[c * g.nbrs] = (R[3 * j + c] - R[3 * i + c]) * ir;
+            f[3 * g.nbrs] = r;
+            f[4 * g.nbrs] = cut_fn(r, P.acut);
+            TwoBody tb;
+            double mu = 0.0, sc = 0.0, fac = 0.0;
+            if (j != i && !(r > P.rcut) && two_body(P, r, tb, false)) {
+                mu = tb.mu;
+                sc = -0.5 * kExpScale / tb.s2;
+                fac = tb.f * tb.pref0;
+            }
+            f[5 * g.nbrs] = mu;
+            f[6 * g.nbrs] = sc;
+            f[7 * g.nbrs] = fac;
+        }
+        __syncthreads();
+        // ---- two-body: (element, centre, k) ----
+        for (int t = tid; t < nelem * B * P.nb2; t += kRepThreads) {
+            const int eb = t / P.nb2, k = t - eb * P.nb2, e = eb / B, b = eb - e * B, i = i0 + b;
+            double v = 0.0;
+            for (int s = est[e]; s < est[e + 1]; ++s) {
+                const int x = b * n + ord[s];
+                if (t_f[x] != 0.0) {
+                    const double L = P.logRs2[k] - t_mu[x];
+                    v += t_f[x] * exp_scaled(L * L * t_sc[x], tab);
+                }
+            }
+            Xm[(size_t)i * P.rs + e * P.nb2 + k] = v / P.Rs2[k];
+        }
+        // ---- three-body, in one chunk unless a single centre has more than g.pairs ----
+        for (int q0 = 0; q0 == 0 || q0 < npair; q0 += g.pairs) {
+            const int qn = B > 1 ? npair : min(g.pairs, npair - q0);  // pairs of a centre here
+            if (q0 > 0) __syncthreads();
+            if (tid == 0) next = 0;
+            // the neighbours' pairs (ja < ka in the order by element) as a triangle; a pair's
+            // place is its channel's first one plus its index in the channel
+            const float inv_np = 1.0f / (float)max(npair, 1);
+            const int n1 = n - 1;
+            for (int t = tid; t < B * npair; t += kRepThreads) {
+                const int b = (int)(((float)t + 0.5f) * inv_np), x = t - b * npair, i = i0 + b;
+                int ja = (int)((2 * n1 - 1 - sqrtf((float)((2 * n1 - 1) * (2 * n1 - 1) - 8 * x))) * 0.5f);
+                while (ja > 0 && x < ja * (2 * n1 - ja - 1) / 2) --ja;
+                while (x >= (ja + 1) * (2 * n1 - ja - 2) / 2) ++ja;
+                const int ka = ja + 1 + x - ja * (2 * n1 - ja - 1) / 2;
+                const int pi = place[i], ei = el[i];
+                const int j = ord[ja + (ja >= pi)], k = ord[ka + (ka >= pi)];
+                const int p = el[j], q = el[k];
+                const int jl = ja - est[p] + (p > ei), kl = ka - est[q] + (q > ei);
+                const int np = est[p + 1] - est[p] - (p == ei), nq = est[q + 1] - est[q] - (q == ei);
+                const int at = cst[ei * (nchan + 1) + pair_channel(nelem, p, q)] +
+                               (p == q ? jl * (2 * np - jl - 1) / 2 + kl - jl - 1 : jl * nq + kl) - q0;
+                if (B == 1 && (at < 0 || at >= qn)) continue;  // another chunk's
+                const int xj = b * n + j, xk = b * n + k;
+                const double rij = rr[xj], rik = rr[xk];
+                double fa = 0.0, ci = 0.0, rb = 0.0;
+                if (!(rij > P.acut) && !(rik > P.acut)) {
+                    const double rjk = dist(R, j, k), ijk = 1.0 / (rjk > kEps ? rjk : kEps);
+                    const double wx = (R[3 * k] - R[3 * j]) * ijk,
+                                 wy = (R[3 * k + 1] - R[3 * j + 1]) * ijk,
+                                 wz = (R[3 * k + 2] - R[3 * j + 2]) * ijk;
+                    ci = ex[xj] * ex[xk] + ey[xj] * ey[xk] + ez[xj] * ez[xk];
+                    ci = ci > 1.0 ? 1.0 : (ci < -1.0 ? -1.0 : ci);
+                    const double cj = -(ex[xj] * wx + ey[xj] * wy + ez[xj] * wz);
+                    const double ck = ex[xk] * wx + ey[xk] * wy + ez[xk] * wz;
+                    const double prod = rik * rij * rjk;
+                    fa = fc[xj] * fc[xk] * (1.0 + 3.0 * ci * cj * ck) * P.w3 /
+                         pow(prod > kEps ? prod : kEps, P.d3);
+                    rb = 0.5 * (rij + rik);
+                }
+                const int rec = b * qn + at;
+                rbar[rec] = rb;
+                const double si = sqrt(fmax(0.0, 1.0 - ci * ci));
+                double cp = 1.0, sp = 0.0, cc = ci, sc = si;
+                int o = 1;
+                for (int h = 0; 2 * h < P.na; ++h) {
+                    while (h < P.nharm && o < 2 * h + 1) {
+                        const double cn = 2.0 * ci * cc - cp, sn = 2.0 * ci * sc - sp;
+                        cp = cc; sp = sc; cc = cn; sc = sn; ++o;
+                    }
+                    const double w = h < P.nharm ? P.angw[h] * fa : 0.0;
+                    amp[(2 * h) * g.pairs + rec] = w * cc;
+                    amp[(2 * h + 1) * g.pairs + rec] = w * sc;
+                }
+            }
+            __syncthreads();
+            // (channel, centre, kLB radial terms)
+            const int nlb = (P.nb3 + kLB - 1) / kLB;
+            for (;;) {
+                // the waves draw 64 items at a time: channels differ in length
+                int t0 = 0;
+                if ((tid & 63) == 0) t0 = atomicAdd(&next, 64);
+                const int t = __shfl(t0, 0, 64) + (tid & 63);
+                if (t - (tid & 63) >= nchan * B * nlb) break;
+                if (t >= nchan * B * nlb) continue;
+                const int cb = t / nlb, l0 = (t - cb * nlb) * kLB, c = cb / B, b = cb - c * B,
+                          i = i0 + b;
+                const int *cs = cst + el[i] * (nchan + 1);
+                const int lo = max(cs[c], q0) - q0, hi = min(cs[c + 1], q0 + qn) - q0;
+                const bool first = q0 == 0 || q0 <= cs[c];  // nothing of it before this chunk
+                if (hi <= lo && q0 > 0) continue;
+                double *dst = Xm + (size_t)i * P.rs + P.three_off + (c * P.nb3 + l0) * P.na;
+                const int ln = min(kLB, P.nb3 - l0);
+                double rs3[kLB];
 #pragma unroll
-            for (int kk = 0; kk < kK2Chunk; ++kk) v[kk] = 0.0;
-            for (int j = 0; j < n; ++j) {
-                if (j == i || el[j] != e) continue;
-                const double r = dist(R, i, j);
-                if (r > P.rcut) continue;
-                TwoBody tb;
-                if (!two_body(P, r, tb, false)) continue;
+                for (int u = 0; u < kLB; ++u) rs3[u] = P.Rs3[min(l0 + u, P.nb3 - 1)];
+                for (int ta = 0; ta < P.na; ta += 2) {
+                    double v0[kLB], v1[kLB];
 #pragma unroll
-                for (int kk = 0; kk < kK2Chunk; ++kk) {
-                    if (kk < kn) {
-                        const double L = P.logRs2[k0 + kk] - tb.mu;
-                        v[kk] += tb.f * tb.pref0 * exp(-0.5 * L * L / tb.s2) / P.Rs2[k0 + kk];
+                    for (int u = 0; u < kLB; ++u) v0[u] = v1[u] = 0.0;
+                    const double *a0 = amp + ta * g.pairs, *a1 = a0 + g.pairs;
+                    for (int x = b * qn + lo; x < b * qn + hi; ++x) {
+                        const double rb = rbar[x], c0 = a0[x], c1 = a1[x];
+#pragma unroll
+                        for (int u = 0; u < kLB; ++u) {
+                            const double dr = rb - rs3[u];
+                            const double e = exp_scaled(ysc * (dr * dr), tab);
+                            v0[u] = fma(e, c0, v0[u]);
+                            v1[u] = fma(e, c1, v1[u]);
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < kLB; ++u) {
+                        if (u >= ln) break;
+                        double *d = dst + u * P.na + ta;
+                        d[0] = first ? v0[u] : d[0] + v0[u];
+                        d[1] = first ? v1[u] : d[1] + v1[u];
                     }
                 }
             }
-            double *dst = Xm + (size_t)i * P.rs + e * P.nb2 + k0;
-            for (int kk = 0; kk < kn; ++kk) dst[kk] = v[kk];
         }
-    }
-
-    // ---- three-body: one wave per centre ----
-    const int nslot = P.nb3 * P.na;
-    for (int i = wave; i < n; i += kRepWaves) {
-        for (int t = lane; t < acc_n; t += 64) acc[t] = 0.0;
-        const double *Ri = R + 3 * i;
-        const int npairs = n * (n - 1) / 2;
-        for (int p0 = 0; p0 < npairs; p0 += 64) {
-            // phase A: lane -> pair index p0 + lane -> (j, k), j < k
-            int valid = 0;
-            double rec_chan = 0, rec_rbar = 0, rec_fa = 0;
-            double ang[2 * kMaxHarm];
-            const int p = p0 + lane;
-            if (p < npairs) {
-                // invert p = j*n - j(j+1)/2 + (k - j - 1)
-                int j = 0, rem = p;
-                while (rem >= n - 1 - j) { rem -= n - 1 - j; ++j; }
-                const int k = j + 1 + rem;
-                if (j != i && k != i) {
-                    const double rij = dist(R, i, j), rik = dist(R, i, k);
-                    if (rij <= P.acut && rik <= P.acut) {
-                        const double rjk = dist(R, j, k);
-                        const double *Rj = R + 3 * j, *Rk = R + 3 * k;
-                        const double iij = 1.0 / (rij > kEps ? rij : kEps);
-                        const double iik = 1.0 / (rik > kEps ? rik : kEps);
-                        const double ijk = 1.0 / (rjk > kEps ? rjk : kEps);
-                        double eij[3], eik[3], ejk[3];
-                        for (int c = 0; c < 3; ++c) {
-                            eij[c] = (Rj[c] - Ri[c]) * iij;
-                            eik[c] = (Rk[c] - Ri[c]) * iik;
-                            ejk[c] = (Rk[c] - Rj[c]) * ijk;
-                        }
-                        double ci = eij[0] * eik[0] + eij[1] * eik[1] + eij[2] * eik[2];
-                        ci = ci > 1.0 ? 1.0 : (ci < -1.0 ? -1.0 : ci);
-                        const double cj = -(eij[0] * ejk[0] + eij[1] * ejk[1] + eij[2] * ejk[2]);
-                        const double ck = eik[0] * ejk[0] + eik[1] * ejk[1] + eik[2] * ejk[2];
-                        const double prod = rik * rij * rjk;
-                        const double ksi3 = (1.0 + 3.0 * ci * cj * ck) * P.w3 /
-                                            pow(prod > kEps ? prod : kEps, P.d3);
-                        const double si = sqrt(fmax(0.0, 1.0 - ci * ci));
-                        double cp = 1.0, sp = 0.0, cc = ci, sc = si;
-                        int o = 1;
-                        for (int h = 0; h < P.nharm; ++h) {
-                            while (o < 2 * h + 1) {
-                                const double cn = 2.0 * ci * cc - cp, sn = 2.0 * ci * sc - sp;
-                                cp = cc; sp = sc; cc = cn; sc = sn; ++o;
-                            }
-                            ang[2 * h] = P.angw[h] * cc;
-                            ang[2 * h + 1] = P.angw[h] * sc;
-                        }
-                        for (int t = 2 * P.nharm; t < P.na; ++t) ang[t] = 0.0;
-                        rec_chan = pair_channel(P.nelem, el[j], el[k]);
-                        rec_rbar = 0.5 * (rij + rik);
-                        rec_fa = cut_fn(rij, P.acut) * cut_fn(rik, P.acut) * ksi3;
-                        valid = 1;
-                    }
-                }
-            }
-            // compact valid records (wave ballot prefix)
-            const unsigned long long mask = __ballot(valid);
-            const int cnt = __popcll(mask);
-            if (valid) {
-                const int slot = __popcll(mask & ((1ull << lane) - 1ull));
-                double *rr = recs + slot * rec_w;
-                rr[0] = rec_chan;
-                rr[1] = rec_rbar;
-                rr[2] = rec_fa;
-                for (int t = 0; t < P.na; ++t) rr[3 + t] = ang[t];
-            }
-            wave_sync();
-            // phase B: lane owns slots s = (l, t)
-            for (int s = lane; s < nslot; s += 64) {
-                const int l = s / P.na, t = s % P.na;
-                const double rs3 = P.Rs3[l];
-                for (int q = 0; q < cnt; ++q) {
-                    const double *rr = recs + q * rec_w;
-                    const double dr = rr[1] - rs3;
-                    const double v = rr[3 + t] * exp(-P.eta3 * dr * dr) * rr[2];
-                    acc[(int)rr[0] * nslot + s] += v;
-                }
-            }
-            wave_sync();
-        }
-        double *dst = Xm + (size_t)i * P.rs + P.three_off;
-        for (int t = lane; t < acc_n; t += 64) dst[t] = acc[t];
-        wave_sync();
     }
 }
 
@@ -675,8 +770,7 @@ extern "C" int kf_fchl19_f64(const double *coords, const int *Q, const int *N, i
     if (rc) return rc;
     // LDS of the kernels below (whole molecules staged per workgroup)
     const int ma = max_atoms;
-    const size_t lds_rep = sizeof(double) * (3 * ma) + sizeof(int) * ((ma + 1) & ~1) +
-                           sizeof(double) * kRepWaves * (64 * (3 + P.na) + P.nchan * P.nb3 * P.na);
+    const size_t lds_rep = rep_lds_bytes(ma, P.nelem, P.nchan, P.na);
     const size_t lds_grad = grad_lds_bytes(ma, P.nb2, P.nb3, P.na);
     const size_t lds = dX ? lds_grad : lds_rep;
     if (ma > kMaxAtoms || lds > 160 * 1024) {
@@ -697,8 +791,11 @@ extern "C" int kf_fchl19_f64(const double *coords, const int *Q, const int *N, i
     *err = 0;
     ScopedTimer timer(TM_FCHL19, stream);
     if (!dX) {
-        hipLaunchKernelGGL(fchl19_rep_kernel, dim3(nm), dim3(kRepThreads), lds, stream, coords, Q,
-                           N, P, X, err);
+        // up to a work-group per two rows while there are fewer molecules than the GPU takes
+        // work-groups
+        const int splits = std::max(1, std::min((ma + 1) / 2, 1024 / nm));
+        hipLaunchKernelGGL(fchl19_rep_kernel, dim3(nm, splits), dim3(kRepThreads), lds, stream,
+                           coords, Q, N, P, X, err);
     } else {
         KF_REQUIRE(P.nelem * P.nb2 > 0, KF_ERR_BASIS, "empty two-body basis");
         // Several work-groups per centre while the batch has fewer centres than the GPU takes

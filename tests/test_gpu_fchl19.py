@@ -121,3 +121,22 @@ def test_jacobian_kernel_edges(fr, ma, nm, kw):
     Xo, dXo = oracle.fchl19_batch(C, Q, N, grad=True, **kw)
     assert row_rel_err(X, Xo, lead=2) < 1e-12
     assert row_rel_err(dX, dXo, lead=2) < 1e-12
+
+
+# one atom to more than the pair storage holds in one go (47 atoms: 1,035 pairs a centre),
+# batches of a few centres, one radial term left over per thread, many angular terms (a
+# smaller pair storage: several chunks from 21 atoms on), one element, work-groups sharing
+# a molecule
+@pytest.mark.parametrize("ma,nm,kw", [
+    (1, 2, {}), (2, 1, {}), (3, 1500, dict(nRs3=1)), (8, 130, dict(nRs2=41, nRs3=37)),
+    (23, 1, dict(nFourier=8, nRs3=7)), (47, 3, {}), (60, 2, dict(elements=[8], nRs3=3))])
+def test_representation_kernel_edges(fr, ma, nm, kw):
+    from kernelforge_amd import synthetic
+
+    rng = np.random.default_rng(10 * ma + nm)
+    el = np.array(kw.get("elements", [1, 6, 7, 8, 16]))
+    Ns = np.concatenate([[ma], rng.integers(1, ma + 1, nm - 1)]).astype(int)
+    C, Q, N = synthetic.pad_batch([synthetic._place_atoms(rng, n) for n in Ns],
+                                  [rng.choice(el, n).astype(np.int32) for n in Ns])
+    X = fr.generate_fchl_acsf_batch(C, Q, N, **kw)
+    assert row_rel_err(X, oracle.fchl19_batch(C, Q, N, **kw), lead=2) < 1e-12
