@@ -234,3 +234,27 @@ def test_matvec_conformers_symmetric(lk):
     E, F = lk.kernel_gaussian_local_full_matvec(X, dX, X, ad, a[:8], Q, Q, N, N, 2.0)
     K = oracle.full_symm(X, dX, Q, N, 2.0)
     assert rel_err(np.concatenate([E, F]), K @ a) < 1e-9
+
+
+@pytest.mark.parametrize("nm,ma,rep", [(1, 2, 5), (70, 2, 300), (3, 30, 97), (40, 5, 17)])
+def test_unused_columns_found_anywhere(lk, nm, ma, rep):
+    """A column used by a single entry -- of the last live atom, in the Jacobian only, or of a
+    padded atom, which does not count -- in sets of fewer and of more atoms than the first
+    look samples."""
+    X, dX, Q, N = rand_set(nm, ma, rep, 2, 17 * nm + rep, 1)
+    live = np.arange(ma)[None] < N[:, None]
+    X[live] *= rng_mask(X[live].shape, 3)
+    dX[:, :, rep // 2:] = 0.0
+    X[:, :, rep // 2:] = 0.0
+    a, i = nm - 1, N[-1] - 1
+    dX[a, i, rep - 1, 3 * N[-1] - 1] = 0.7
+    X[a, i, rep - 2] = -0.4
+    dX[~live] = 0.0
+    X[~live, rep - 3] = 9.0
+    X[~live, : rep // 2] = 0.0
+    got = lk.kernel_gaussian_hessian_symm(X, dX, Q, N, 1.3)
+    assert rel_err(got, oracle.hessian_symm(X, dX, Q, N, 1.3)) < TOL
+
+
+def rng_mask(shape, seed):
+    return (np.random.default_rng(seed).random(shape) < 0.5).astype(np.float64)
