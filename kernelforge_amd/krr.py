@@ -10,8 +10,8 @@ other.  Every kernel, solve and descriptor here runs through this package's HIP 
   instead of one call per molecule (models/representations.py:102-150);
 * training kernels: ``kernel_gaussian_symm_rfp`` / ``_hessian_symm_rfp`` /
   ``_full_symm_rfp`` straight into RFP, solved by ``cho_solve_rfp``;
-* prediction: the rectangular and Jacobian kernels (energy mode) or the matrix-free
-  descriptor-space matvecs with the precomputed alpha_desc (force and E+F modes).
+* prediction: the matrix-free descriptor-space matvecs, with the weights of the training
+  molecules (energy mode) or the precomputed alpha_desc (force and E+F modes).
 
 The model is host-side orchestration; it holds NumPy arrays, as the reference's does.
 """
@@ -120,6 +120,14 @@ def compute_fchl19(coords_list, z_list, elements, with_gradients=True, repr_para
     reference's models/representations.py:102-150 lays them out.  With gradients the
     three-body term keeps the first angular harmonic only, like the reference's gradient
     path (src/fchl19_repr.cpp:449,523-528)."""
+    X, dX, _, _, Q, N = _device_fchl19(coords_list, z_list, elements, with_gradients, repr_params)
+    capi.synchronize()
+    return X.numpy(), (dX.numpy() if dX is not None else None), Q, N
+
+
+def _device_fchl19(coords_list, z_list, elements, with_gradients=True, repr_params=None):
+    """compute_fchl19 with the descriptors left on the GPU: (X, dX or None, labels, counts as
+    device arrays, Q, N)."""
     params = dict(repr_params or {})
     unknown = sorted(set(params) - set(REPR_KEYS))
     if unknown:
@@ -145,8 +153,7 @@ def compute_fchl19(coords_list, z_list, elements, with_gradients=True, repr_para
     dX = DA((nm, ma, rep, 3 * ma)) if with_gradients else None
     capi.fchl19(dC.ptr, dQ.ptr, dN.ptr, nm, ma, X.ptr, dX.ptr if dX is not None else 0,
                 elements=tuple(int(e) for e in elements), **params)
-    capi.synchronize()
-    return X.numpy(), (dX.numpy() if dX is not None else None), Q, N
+    return X, dX, dQ, dN, Q, N
 
 
 class LocalKRRModel:
@@ -271,29 +278,67 @@ class LocalKRRModel:
                 dX, Q, N, alpha_F)
 
     def _predict(self, coords_list, z_list):
+        """(energies, forces) without the energy baseline.
+
+        One descriptor-space product per call, on descriptors that stay on the GPU: with
+        weights per training molecule (energy mode: alpha_desc = 0) or per training atom and
+        descriptor (alpha_desc).  No kernel matrix is formed, and of the query set only the
+        results are copied back (the Jacobians of 8 molecules are 73 MB)."""
+        mode, nm = self.training_mode_, len(z_list)
+        if nm == 0 or (mode != ENERGY_ONLY and self._alpha_desc is None):
+            return self._predict_kernels(coords_list, z_list)
+        DA, L, s = capi.DeviceArray, capi.lib(), self.sigma
+        X, dX, dQ, dN, Q, N = _device_fchl19(coords_list, z_list, self.elements, True,
+                                             self.repr_params)
+        _, ma, rep = X.shape
+        Xt = np.ascontiguousarray(self._X_tr, dtype=np.float64)
+        Qt = np.ascontiguousarray(self._Q_tr, dtype=np.int32)
+        Nt = np.ascontiguousarray(self._N_tr, dtype=np.int32)
+        if Xt.ndim != 3 or Xt.shape[2] != rep:
+            raise ValueError("X1 and X2 must have the same representation size")
+        nt, mt = Xt.shape[:2]
+        if Qt.shape != (nt, mt) or Nt.shape != (nt,):
+            raise ValueError("Q and N of the training set do not match its descriptors")
+        dXt, dQt, dNt = DA.from_numpy(Xt), DA.from_numpy(Qt), DA.from_numpy(Nt)
+        if mode == ENERGY_ONLY:
+            ad = DA(Xt.shape)
+            ad.zero()
+        else:
+            if np.size(self._alpha_desc) != Xt.size:
+                raise ValueError("alpha_desc does not match the training descriptors")
+            ad = DA.from_numpy(np.asarray(self._alpha_desc, dtype=np.float64))
+        E, F = DA(nm), DA(3 * int(N.sum()))
+        dims = (nm, nt, ma, mt, rep, s)
+        if mode == FORCE_ONLY:
+            capi.check(L.kf_local_hessian_matvec(X.ptr, dX.ptr, dXt.ptr, ad.ptr, dQ.ptr, dQt.ptr,
+                                                 dN.ptr, dNt.ptr, *dims, F.ptr, None),
+                       "kf_local_hessian_matvec")
+            capi.check(L.kf_local_jacobian_t_matvec(X.ptr, dXt.ptr, ad.ptr, dQ.ptr, dQt.ptr, dN.ptr,
+                                                    dNt.ptr, *dims, E.ptr, None),
+                       "kf_local_jacobian_t_matvec")
+            return -E.numpy(), F.numpy()
+        a = np.asarray(self._alpha, dtype=np.float64)[: self._n_train]
+        if a.shape != (nt,):
+            raise ValueError("alpha does not match the training set")
+        aE = DA.from_numpy(a)
+        capi.check(L.kf_local_full_matvec(X.ptr, dX.ptr, dXt.ptr, ad.ptr, aE.ptr, dQ.ptr, dQt.ptr,
+                                          dN.ptr, dNt.ptr, *dims, E.ptr, F.ptr or None, None),
+                   "kf_local_full_matvec")
+        return E.numpy(), -F.numpy()
+
+    def _predict_kernels(self, coords_list, z_list):
+        """_predict through explicit kernels: a force model whose file holds no alpha_desc."""
         Xt, dXt, Qt, Nt = self._descriptors(coords_list, z_list)
         X, dX, Q, N, a, s = self._X_tr, self._dX_tr, self._Q_tr, self._N_tr, self._alpha, self.sigma
-        mode = self.training_mode_
-        if mode == ENERGY_ONLY:
+        if self.training_mode_ == ENERGY_ONLY:
             E = local_kernels.kernel_gaussian(Xt, X, Qt, Q, Nt, N, s) @ a
             F = local_kernels.kernel_gaussian_jacobian_t(Xt, dXt, X, Qt, Q, Nt, N, s) @ a
-        elif mode == FORCE_ONLY:
-            if self._alpha_desc is not None:
-                F = local_kernels.kernel_gaussian_local_hessian_matvec(
-                    Xt, dXt, X, self._alpha_desc, Qt, Q, Nt, N, s)
-                E = -local_kernels.kernel_gaussian_local_jacobian_t_matvec(
-                    Xt, X, self._alpha_desc, Qt, Q, Nt, N, s)
-            else:  # a model file without alpha_desc: explicit kernels
-                F = local_kernels.kernel_gaussian_hessian(Xt, dXt, X, dX, Qt, Q, Nt, N, s) @ a
-                E = -(local_kernels.kernel_gaussian_jacobian(Xt, X, dX, Qt, Q, Nt, N, s) @ a)
+        elif self.training_mode_ == FORCE_ONLY:
+            F = local_kernels.kernel_gaussian_hessian(Xt, dXt, X, dX, Qt, Q, Nt, N, s) @ a
+            E = -(local_kernels.kernel_gaussian_jacobian(Xt, X, dX, Qt, Q, Nt, N, s) @ a)
         else:
-            if self._alpha_desc is not None:
-                E, Fneg = local_kernels.kernel_gaussian_local_full_matvec(
-                    Xt, dXt, X, self._alpha_desc, a[: self._n_train], Qt, Q, Nt, N, s)
-                F = -Fneg
-            else:
-                y = local_kernels.kernel_gaussian_full(Xt, dXt, X, dX, Qt, Q, Nt, N, s) @ a
-                E, F = y[: len(z_list)], -y[len(z_list):]
+            y = local_kernels.kernel_gaussian_full(Xt, dXt, X, dX, Qt, Q, Nt, N, s) @ a
+            E, F = y[: len(z_list)], -y[len(z_list):]
         return np.asarray(E, dtype=np.float64), np.asarray(F, dtype=np.float64)
 
     def _training_fit(self):
