@@ -404,9 +404,12 @@ __global__ __launch_bounds__(NT) void deriv_prep_kernel(DerivArgs A, int pair0) 
 //   V_i (3 n_x x ncol) = J_xi^T (3 n_x x rep) * D (rep x ncol),  D[f][c] = x_xi[f] - x_yj[f]
 // which streams each J_xi row once for the whole group (the one-pair form streamed it
 // once per pair).  The columns depend only on the label of atom i, so they are listed
-// once per label of x, and the (atom, pair of 16-column fragments) items of a label are
-// dealt over the four waves; A operands (J rows, shared by the two fragments) and B
+// once per label of x, and the (atom, pair of 16-column fragments) items are dealt over the
+// waves of the group's work-groups; A operands (J rows, shared by the two fragments) and B
 // operands (differences, formed in registers) come straight from HBM, 16 features ahead.
+// Held to 256 registers: at the 347 it takes otherwise one wave fits a SIMD, and 200
+// conformers of 21 atoms take 10.3 ms instead of 8.8 (16-byte loads of the descriptor rows
+// with the summation index permuted spill more than they save: 13.8).
 // ---------------------------------------------------------------------------
 constexpr int PG = 8;  // partners per group
 
@@ -417,7 +420,7 @@ struct ProjGroup {
 };
 
 template <int NPF>
-__global__ __launch_bounds__(NT) void deriv_vproj_kernel(DerivArgs A, const ProjGroup *groups) {
+__global__ __launch_bounds__(NT, 2) void deriv_vproj_kernel(DerivArgs A, const ProjGroup *groups) {
     __shared__ int qx[MAXA], qy[PG][MAXA], ny[PG], ist[PG][MAXA], rnk[PG][MAXA], rx[MAXA];
     __shared__ int cols[PG * MAXA], wbase[5], gy[PG], gslot[PG], xl[MAXA], s_nl;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, col = lane & 15, kr = lane >> 4;
@@ -478,7 +481,10 @@ __global__ __launch_bounds__(NT) void deriv_vproj_kernel(DerivArgs A, const Proj
 
     // one pass per label of x (taken at its first atom, rx == 0): the columns are every
     // label-matched (k, j) of the group, the same for all atoms of x with that label, and
-    // the (atom, column fragment) items of the label are dealt over the four waves
+    // the (atom, column fragment) items of all labels are dealt over the waves of the
+    // group's gridDim.y work-groups
+    const int nw = 4 * gridDim.y;
+    int turn = 4 * blockIdx.y + wv;  // items until this wave's next
     __syncthreads();  // tables ready (rx decides the passes below, uniformly)
     for (int i0 = 0; i0 < nx; ++i0) {
         if (rx[i0] != 0) continue;  // not the first atom of its label (uniform)
@@ -514,7 +520,8 @@ __global__ __launch_bounds__(NT) void deriv_vproj_kernel(DerivArgs A, const Proj
         // and not stored.
         const int npf2 = (ncf + 1) >> 1;
         const int nitems = s_nl * npf2;
-        for (int it = wv; it < nitems; it += 4) {
+        int it = turn;
+        for (; it < nitems; it += nw) {
             const int i = xl[it / npf2], zp = it % npf2;
             const double *xi = xx0 + (size_t)i * rep;
             const double *Ji = Jx0 + (size_t)i * rep * lda;
@@ -601,6 +608,7 @@ __global__ __launch_bounds__(NT) void deriv_vproj_kernel(DerivArgs A, const Proj
                 }
             }
         }
+        turn = it - nitems;
     }
 }
 
@@ -623,7 +631,8 @@ __global__ __launch_bounds__(NT) void deriv_vproj_kernel(DerivArgs A, const Proj
 template <int MODE, int NK, int NP>
 __device__ __forceinline__ void ff_pair(const DerivArgs &A, int a, int b, int na, int nb,
                                         const double *Cm, double *Jbuf, int np,
-                                        const double *mc, const double *slot) {
+                                        const double *mc, const double *slot, int f0, int fe,
+                                        double *part) {
     constexpr int NX = (NK + 3) / 4;         // 16-row fragments of C / T (atoms of a)
     constexpr int FFR = 4 * NK, FFP = 16 * NP;  // staged J_a feature: rows x columns
     constexpr int NEL = FFR * FFP, NST = (NEL + NT - 1) / NT;  // elements, per thread
@@ -690,32 +699,32 @@ __device__ __forceinline__ void ff_pair(const DerivArgs &A, int a, int b, int na
     } while (0)
     // prologue: J_a(0) in buffer 0, J_a(1) in registers, T(0), J_b(1)
     double *const J0 = Jbuf, *const J1 = Jbuf + NEL;
-    KF_FF_STAGE_LOAD(0);
+    KF_FF_STAGE_LOAD(f0);
     KF_FF_STAGE_STORE(J0);
-    KF_FF_STAGE_LOAD(min(1, rep - 1));
-    KF_FF_LOAD_B(0, 0);
+    KF_FF_STAGE_LOAD(min(f0 + 1, fe - 1));
+    KF_FF_LOAD_B(0, f0);
     KF_FF_T(0);
-    KF_FF_LOAD_B(1, min(1, rep - 1));
+    KF_FF_LOAD_B(1, min(f0 + 1, fe - 1));
     __syncthreads();
-    for (int f = 0; f < rep; f += 2) {
+    for (int f = f0; f < fe; f += 2) {
         // feature f: buffer J0, T slot 0; prepare f+1 (J1, T slot 1) and loads for f+2
         KF_FF_STAGE_STORE(J1);
-        KF_FF_STAGE_LOAD(min(f + 2, rep - 1));
+        KF_FF_STAGE_LOAD(min(f + 2, fe - 1));
         if (busy) {
             KF_FF_T(1);
             KF_FF_MAIN(0, J0);
         }
-        KF_FF_LOAD_B(0, min(f + 2, rep - 1));
+        KF_FF_LOAD_B(0, min(f + 2, fe - 1));
         __syncthreads();
-        if (f + 1 >= rep) break;
+        if (f + 1 >= fe) break;
         // feature f+1: buffer J1, T slot 1; prepare f+2 (J0, T slot 0) and loads for f+3
         KF_FF_STAGE_STORE(J0);
-        KF_FF_STAGE_LOAD(min(f + 3, rep - 1));
+        KF_FF_STAGE_LOAD(min(f + 3, fe - 1));
         if (busy) {
             KF_FF_T(0);
             KF_FF_MAIN(1, J1);
         }
-        KF_FF_LOAD_B(1, min(f + 3, rep - 1));
+        KF_FF_LOAD_B(1, min(f + 3, fe - 1));
         __syncthreads();
     }
 #undef KF_FF_STAGE_LOAD
@@ -724,8 +733,8 @@ __device__ __forceinline__ void ff_pair(const DerivArgs &A, int a, int b, int na
 #undef KF_FF_T
 #undef KF_FF_MAIN
     if (!busy) continue;
-    // rank-1 part: acc -= sum_m (w_m v_m) u_m^T, K = matched pairs
-    {
+    // rank-1 part (of the first run of features): acc -= sum_m (w_m v_m) u_m^T, K = matched pairs
+    if (f0 == 0) {
         const double *V = slot + A.maxm, *U = V + (size_t)A.maxm * A.ldv;
         // loads of clamped (valid) entries, unconditional, masked by selects on '&'
         // conditions ('&&' turns into a branch around each load, which is then waited
@@ -755,7 +764,10 @@ __device__ __forceinline__ void ff_pair(const DerivArgs &A, int a, int b, int na
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int r = 16 * y + mfma16_row_f64(lane, v);
-            if (r < nca && tc < ncb) out.ff(r, tc, acc[y][v]);
+            if (r < nca && tc < ncb) {
+                if (part) part[(size_t)r * A.ldu + tc] = acc[y][v];
+                else out.ff(r, tc, acc[y][v]);
+            }
         }
     }
 }
@@ -778,7 +790,8 @@ inline size_t ff_lds_bytes(int ma1, int ma2) {
 // Shape buckets by m = max(atoms of a, atoms of b): NK k-steps of 4 atoms, NP 16-column
 // force blocks (3 m columns).
 template <int MODE>
-__global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0) {
+__global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0,
+                                                         double *__restrict__ parts) {
     __shared__ double Cm[32 * 33];
     extern __shared__ double Jbuf[];  // two staged J_a features of the largest bucket
     __shared__ int qa[MAXA], qb_[MAXA], ist[MAXA + 1], mi[MAXM], mj[MAXM];
@@ -812,7 +825,7 @@ __global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0)
         Cm[mi[m] * 33 + mj[m]] = c;
     }
     __syncthreads();
-    {
+    if (blockIdx.y == 0) {
         // EE = sum_m e_m, FE = -sum_m c_m v_m, EF = sum_m c_m u_m from the slot
         Out<MODE> out{A.out, A.ld, a, b, A.offs1[a], A.offs2[b], A.ebase1, A.ebase2};
         const double *V = slot + A.maxm, *U = V + (size_t)A.maxm * A.ldv;
@@ -833,13 +846,37 @@ __global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0)
         }
     }
     if (na == 0 || nb == 0) return;
+    // this work-group's run of features, and where its part of FF goes if there are several
+    const int run = (A.rep + gridDim.y - 1) / gridDim.y, f0 = blockIdx.y * run,
+              fe = min(f0 + run, A.rep);
+    double *part = gridDim.y > 1 ? parts + ((size_t)(t - pair0) * gridDim.y + blockIdx.y) *
+                                               A.ldv * A.ldu
+                                 : nullptr;
     const int mx = na > nb ? na : nb;
-    if (mx <= 5) ff_pair<MODE, 2, 1>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot);
-    else if (mx <= 10) ff_pair<MODE, 3, 2>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot);
-    else if (mx <= 16) ff_pair<MODE, 4, 3>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot);
-    else if (mx <= 21) ff_pair<MODE, 6, 4>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot);
-    else if (mx <= 24) ff_pair<MODE, 6, 5>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot);
-    else ff_pair<MODE, 8, 6>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot);
+    if (mx <= 5) ff_pair<MODE, 2, 1>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
+    else if (mx <= 10) ff_pair<MODE, 3, 2>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
+    else if (mx <= 16) ff_pair<MODE, 4, 3>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
+    else if (mx <= 21) ff_pair<MODE, 6, 4>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
+    else if (mx <= 24) ff_pair<MODE, 6, 5>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
+    else ff_pair<MODE, 8, 6>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
+}
+
+// FF of a pair from the parts of its runs of features, in order.
+template <int MODE>
+__global__ __launch_bounds__(NT) void ff_sum_kernel(DerivArgs A, int pair0, int runs,
+                                                    const double *__restrict__ parts) {
+    const int t = pair0 + blockIdx.x;
+    const int a = A.pairs[t].x, b = A.pairs[t].y;
+    const int nca = 3 * clampi(A.n1[a], 0, A.ma1), ncb = 3 * clampi(A.n2[b], 0, A.ma2);
+    Out<MODE> out{A.out, A.ld, a, b, A.offs1[a], A.offs2[b], A.ebase1, A.ebase2};
+    const size_t len = (size_t)A.ldv * A.ldu;
+    const double *p = parts + (size_t)blockIdx.x * runs * len;
+    for (int e = threadIdx.x; e < nca * ncb; e += NT) {
+        const int r = e / ncb, c = e - r * ncb;
+        double s = 0.0;
+        for (int k = 0; k < runs; ++k) s += p[k * len + (size_t)r * A.ldu + c];
+        out.ff(r, c, s);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -974,18 +1011,37 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
         if (has_ff(MODE)) {
             const unsigned ng = (unsigned)(gstart[bi + 1] - gstart[bi]);
             const ProjGroup *gp = dgroups + gstart[bi];
+            // Few groups: up to eight work-groups share the items of one, whose longest chain
+            // (a 23-atom molecule's some 50 items over four waves) else bounds the launch: 370
+            // groups of mixed molecules 0.76 ms, 1.29 with one each
+            const dim3 vg(ng, std::max(1u, std::min(8u, 2048u / ng)));
             switch (npf) {
-                case 1: hipLaunchKernelGGL(deriv_vproj_kernel<1>, dim3(ng), dim3(NT), 0, stream, A, gp); break;
-                case 2: hipLaunchKernelGGL(deriv_vproj_kernel<2>, dim3(ng), dim3(NT), 0, stream, A, gp); break;
-                case 3: hipLaunchKernelGGL(deriv_vproj_kernel<3>, dim3(ng), dim3(NT), 0, stream, A, gp); break;
-                case 4: hipLaunchKernelGGL(deriv_vproj_kernel<4>, dim3(ng), dim3(NT), 0, stream, A, gp); break;
-                case 5: hipLaunchKernelGGL(deriv_vproj_kernel<5>, dim3(ng), dim3(NT), 0, stream, A, gp); break;
-                default: hipLaunchKernelGGL(deriv_vproj_kernel<6>, dim3(ng), dim3(NT), 0, stream, A, gp); break;
+                case 1: hipLaunchKernelGGL(deriv_vproj_kernel<1>, vg, dim3(NT), 0, stream, A, gp); break;
+                case 2: hipLaunchKernelGGL(deriv_vproj_kernel<2>, vg, dim3(NT), 0, stream, A, gp); break;
+                case 3: hipLaunchKernelGGL(deriv_vproj_kernel<3>, vg, dim3(NT), 0, stream, A, gp); break;
+                case 4: hipLaunchKernelGGL(deriv_vproj_kernel<4>, vg, dim3(NT), 0, stream, A, gp); break;
+                case 5: hipLaunchKernelGGL(deriv_vproj_kernel<5>, vg, dim3(NT), 0, stream, A, gp); break;
+                default: hipLaunchKernelGGL(deriv_vproj_kernel<6>, vg, dim3(NT), 0, stream, A, gp); break;
             }
             KF_HIP_TRY(hipGetLastError());
-            hipLaunchKernelGGL(deriv_ff_kernel<MODE>, dim3(nb), dim3(NT), ff_lds_bytes(A.ma1, A.ma2),
-                               stream, A, (int)p0);
+            // Few pairs: each pair's features in several runs (of 32 and more), so that there
+            // are about 2,048 work-groups, four per slot of the GPU (512): 703 pairs of mixed
+            // molecules of 5-23 atoms 3.5 ms, 4.5 with one run each
+            const int runs = std::max(1, std::min((int)(2048 / nb), A.rep / 32));
+            double *parts = nullptr;
+            if (runs > 1) {
+                const size_t bytes = sizeof(double) * nb * runs * (size_t)A.ldv * A.ldu;
+                parts = static_cast<double *>(workspace(WS_AUX0, bytes, stream));
+                KF_REQUIRE(parts, KF_ERR_NOMEM, "workspace allocation failed (%zu B)", bytes);
+            }
+            hipLaunchKernelGGL(deriv_ff_kernel<MODE>, dim3(nb, runs), dim3(NT),
+                               ff_lds_bytes(A.ma1, A.ma2), stream, A, (int)p0, parts);
             KF_HIP_TRY(hipGetLastError());
+            if (runs > 1) {
+                hipLaunchKernelGGL(ff_sum_kernel<MODE>, dim3(nb), dim3(NT), 0, stream, A, (int)p0,
+                                   runs, parts);
+                KF_HIP_TRY(hipGetLastError());
+            }
         }
     }
     return KF_OK;

@@ -236,6 +236,21 @@ def test_matvec_conformers_symmetric(lk):
     assert rel_err(np.concatenate([E, F]), K @ a) < 1e-9
 
 
+# pairs whose features are dealt over several work-groups: 22 runs, runs of unequal length
+# (the last shorter), two runs, one run from 2,048 pairs on; groups of one molecule shared
+# by eight work-groups and by one
+@pytest.mark.parametrize("nm,ma,rep", [(2, 23, 720), (5, 7, 101), (44, 4, 67), (65, 3, 64)])
+def test_feature_runs(lk, nm, ma, rep):
+    X, dX, Q, N = rand_set(nm, ma, rep, 2, nm + rep)
+    got = lk.kernel_gaussian_full_symm(X, dX, Q, N, 2.1)
+    assert rel_err(got, oracle.full_symm(X, dX, Q, N, 2.1)) < TOL
+    got = lk.kernel_gaussian_full_symm_rfp(X, dX, Q, N, 2.1)
+    assert rel_err(got, oracle.full_symm_rfp(X, dX, Q, N, 2.1)) < TOL
+    m = max(1, nm // 3)
+    got = lk.kernel_gaussian_hessian(X[:m], dX[:m], X, dX, Q[:m], Q, N[:m], N, 2.1)
+    assert rel_err(got, oracle.hessian(X[:m], dX[:m], X, dX, Q[:m], Q, N[:m], N, 2.1)) < TOL
+
+
 @pytest.mark.parametrize("nm,ma,rep", [(1, 2, 5), (70, 2, 300), (3, 30, 97), (40, 5, 17)])
 def test_unused_columns_found_anywhere(lk, nm, ma, rep):
     """A column used by a single entry -- of the last live atom, in the Jacobian only, or of a
