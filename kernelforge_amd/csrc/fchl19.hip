@@ -785,8 +785,8 @@ extern "C" int kf_fchl19_f64(const double *coords, const int *Q, const int *N, i
     // no launch to clear it and no copy to read it
     int dev = 0;
     KF_HIP_TRY(hipGetDevice(&dev));
-    int *err = static_cast<int *>(host_staging(WS_ERR, sizeof(int) * 64));
-    KF_REQUIRE(err && dev >= 0 && dev < 64, KF_ERR_NOMEM, "pinned staging allocation failed");
+    int *err = static_cast<int *>(host_staging(WS_ERR, sizeof(int) * kErrWords));
+    KF_REQUIRE(err && dev >= 0 && dev < kErrWords / 2, KF_ERR_NOMEM, "pinned staging allocation failed");
     err += dev;
     *err = 0;
     ScopedTimer timer(TM_FCHL19, stream);

@@ -56,7 +56,7 @@ enum WsSlot {
     WS_SOLVE1,     // solver reductions
     WS_SOLVE2,     // solver metadata
     WS_NET,        // preconditioner-network activations
-    WS_ERR,        // error flags raised by kernels (pinned, one word per device)
+    WS_ERR,        // pinned words, one per device and use: error flags, factorization info
     WS_NSLOTS
 };
 void *workspace(int slot, size_t bytes, hipStream_t stream);
@@ -66,6 +66,8 @@ void *workspace(int slot, size_t bytes, hipStream_t stream);
 constexpr int kAuxEvents = 4;
 hipStream_t aux_stream();
 hipEvent_t aux_event(int i);
+
+constexpr int kErrWords = 128;  // of WS_ERR: 64 devices' error flags, then their infos
 
 // Pinned host staging for small metadata round trips.
 void *host_staging(int slot, size_t bytes);

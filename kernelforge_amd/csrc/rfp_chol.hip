@@ -106,52 +106,12 @@ __device__ inline void store_tile(T *__restrict__ a, const Tile &t, int rn, int 
     }
 }
 
+// a + l2 I, and the factorization's info word cleared.
 template <typename T>
-__global__ void add_diag(T *a, int n, double l2) {
+__global__ void add_diag(T *a, int n, double l2, int *info) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < n) a[rfp_lower((size_t)n, j, j)] += T(l2);
-}
-
-// Li = L^-1 for a lower-triangular w x w LDS tile (pitch TP), right-looking
-// substitution on the identity, one barrier per row: phase q scales row q into the
-// unused upper triangle of Li (and dgi[q]) and subtracts L[r][q] * row q / L[q][q] from
-// every row r > q; the lower triangle is restored at the end.  Li is w x w, fully
-// written (zeros above the diagonal).
-template <typename T, typename U>
-__device__ inline void tri_inverse(const T *L, U *Li, U *dgi, int w) {
-    const int ti = threadIdx.x >> 4, tc = threadIdx.x & 15;
-    for (int idx = threadIdx.x; idx < w * w; idx += blockDim.x) {
-        const int i = idx / w, c = idx - i * w;
-        Li[i * TP + c] = (i == c) ? U(1) : U(0);
-    }
-    __syncthreads();
-    for (int q = 0; q < w; ++q) {
-        const U rq = U(1) / (U)L[q * TP + q];
-        if (ti == 0)
-            for (int c = tc; c <= q; c += 16) {
-                const U v = Li[q * TP + c] * rq;
-                if (c < q) Li[c * TP + q] = v; else dgi[q] = v;
-            }
-        for (int r = q + 1 + ti; r < w; r += 16) {
-            const U lr = (U)L[r * TP + q] * rq;
-            for (int c = tc; c <= q; c += 16) Li[r * TP + c] -= lr * Li[q * TP + c];
-        }
-        __syncthreads();
-    }
-    for (int idx = threadIdx.x; idx < w * w; idx += blockDim.x) {
-        const int i = idx / w, c = idx - i * w;
-        if (i > c) {
-            Li[i * TP + c] = Li[c * TP + i];
-        } else if (i == c) {
-            Li[i * TP + i] = dgi[i];
-        }
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < w * w; idx += blockDim.x) {
-        const int i = idx / w, c = idx - i * w;
-        if (i < c) Li[i * TP + c] = U(0);
-    }
-    __syncthreads();
+    if (j == 0) *info = 0;
+    if (j < n && l2 != 0.0) a[rfp_lower((size_t)n, j, j)] += T(l2);
 }
 
 // POTRF of diagonal tile J plus its inverse (lower) into inv[NB*NB], four waves.
@@ -183,6 +143,77 @@ __device__ __forceinline__ float recip_sqrt(float v) { return rsqrtf(v); }
 constexpr int HB = NB / 2;   // half block of the blocked inverse
 constexpr int HP = HB + 1;   // LDS pitch of its pieces
 
+// inv (row-major, NB x NB) = the inverse of the lower-triangular tile S (LDS, pitch TP, its
+// rows and columns past w the identity's), with `dinv` the reciprocals of its diagonal and
+// Wk LDS for (NB + HB) * HP values; four waves.  Blocked on the two 32-row halves: lane i of
+// wave 0 runs forward substitution for column i % 32 of the inverse of diagonal block i / 32
+// (both blocks at once, 32 steps) while the other waves run `meanwhile`, and the
+// off-diagonal block -L1^-1 B L0^-1 is two 32x32x32 MFMA products, one 16x16 fragment per
+// wave.  Entries past w are zero.
+template <typename T, class Meanwhile>
+__device__ __forceinline__ void tile_inverse(const T *S, const T *dinv, T *Wk, int w, T *inv,
+                                             Meanwhile meanwhile) {
+    T *const Di = Wk;            // row 32h + q, column c: (L_h^-1)[q][c]
+    T *const Zs = Wk + NB * HP;  // B L0^-1
+    const int i = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int h = i >> 5, cc = i & (HB - 1);
+    if (q == 0) {
+        // column cc of L_h^-1 (h = i / 32): x[p] = (delta_p,cc - sum_{k<p} L_h[p][k] x[k]) / L_h[p][p],
+        // with the reciprocals of the diagonal kept from the factorization
+        T x[HB];
+#pragma unroll
+        for (int p = 0; p < HB; ++p) {
+            const int g = h * HB + p;
+            T lq[HB];
+#pragma unroll
+            for (int k = 0; k < p; ++k) lq[k] = S[g * TP + h * HB + k];
+            const T dq = dinv[g];
+            __builtin_amdgcn_sched_barrier(0);
+            T acc[4] = {p == cc ? T(1) : T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int k = 0; k < p; ++k) acc[k & 3] -= lq[k] * x[k];
+            x[p] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) * dq;
+        }
+#pragma unroll
+        for (int p = 0; p < HB; ++p) Di[(h * HB + p) * HP + cc] = x[p];
+    } else {
+        meanwhile();
+    }
+    __syncthreads();
+    // Z = B L0^-1, then W = -L1^-1 Z, as 16x16x4 MFMA fragments (A[m][k] from lane
+    // m + 16k, B[k][n] from lane n + 16k), fragment q on wave q
+    typedef typename Vec4<T>::type V4;
+    const int l16 = i & 15, kq = i >> 4, u = q >> 1, v = q & 1;
+    {
+        V4 z = V4{0, 0, 0, 0};
+#pragma unroll
+        for (int k0 = 0; k0 < HB; k0 += 4)
+            z = mfma4(S[(HB + u * 16 + l16) * TP + k0 + kq], Di[(k0 + kq) * HP + v * 16 + l16], z);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Zs[(u * 16 + mfma16_row<T>(i, e)) * HP + v * 16 + l16] = z[e];
+    }
+    __syncthreads();
+    {
+        V4 z = V4{0, 0, 0, 0};
+#pragma unroll
+        for (int k0 = 0; k0 < HB; k0 += 4)
+            z = mfma4(-Di[(HB + u * 16 + l16) * HP + k0 + kq], Zs[(k0 + kq) * HP + v * 16 + l16], z);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int rr = HB + u * 16 + mfma16_row<T>(i, e), c = v * 16 + l16;
+            inv[rr * NB + c] = (rr < w && c < w) ? z[e] : T(0);
+        }
+    }
+    // inv (row-major, NB x NB): the diagonal blocks from Di, zeros above them; rows 16q ..
+    // 16q+15 on wave q
+#pragma unroll
+    for (int p = 16 * q; p < 16 * q + 16; ++p) {
+        const int hq = p / HB;
+        if (hq == h) inv[p * NB + i] = (p < w && i < w) ? Di[p * HP + cc] : T(0);
+        else if (hq == 0) inv[p * NB + i] = T(0);  // above the diagonal blocks
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void potrf_diag(T *a, Part P, int J, T *inv, int *info) {
     constexpr int PQ = 18;  // pitch of a published quarter panel (16-byte aligned rows)
@@ -191,8 +222,6 @@ __global__ __launch_bounds__(256) void potrf_diag(T *a, Part P, int J, T *inv, i
     __shared__ T Wk[WK];  // the quarter panels while factoring, then Di and Zs
     __shared__ T dinv[NB];
     __shared__ int fail_s[2];
-    T *const Di = Wk;            // row 32h + q, column c: (L_h^-1)[q][c]
-    T *const Zs = Wk + NB * HP;  // B L0^-1
     if (*info) return;
     // these waves are the whole critical path of the factorization: let them issue ahead of
     // the trailing-update waves that share their CU
@@ -263,66 +292,14 @@ __global__ __launch_bounds__(256) void potrf_diag(T *a, Part P, int J, T *inv, i
 #pragma unroll
     for (int c = 0; c < 16; ++c) S[i * TP + 16 * q + c] = 16 * q + c <= i ? r[c] : T(0);
     __syncthreads();
-    const int h = i >> 5, cc = i & (HB - 1);
-    if (q == 0) {
-        // column cc of L_h^-1 (h = i / 32): x[p] = (delta_p,cc - sum_{k<p} L_h[p][k] x[k]) / L_h[p][p],
-        // with the reciprocals of the diagonal kept from the factorization
-        T x[HB];
-#pragma unroll
-        for (int p = 0; p < HB; ++p) {
-            const int g = h * HB + p;
-            T lq[HB];
-#pragma unroll
-            for (int k = 0; k < p; ++k) lq[k] = S[g * TP + h * HB + k];
-            const T dq = dinv[g];
-            __builtin_amdgcn_sched_barrier(0);
-            T acc[4] = {p == cc ? T(1) : T(0), T(0), T(0), T(0)};
-#pragma unroll
-            for (int k = 0; k < p; ++k) acc[k & 3] -= lq[k] * x[k];
-            x[p] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) * dq;
-        }
-#pragma unroll
-        for (int p = 0; p < HB; ++p) Di[(h * HB + p) * HP + cc] = x[p];
-    } else {  // waves 1..3 store the factor meanwhile (coalesced along the contiguous axis)
+    tile_inverse<T>(S, dinv, Wk, w, inv, [&]() {
+        // waves 1..3 store the factor meanwhile (coalesced along the contiguous axis)
         for (int idx = tid - 64; idx < NB * NB; idx += 192) {
             int rr, c;
             if (t.rs == 1) { rr = idx % NB; c = idx / NB; } else { c = idx % NB; rr = idx / NB; }
             if (rr < w && c < w && rr >= c) a[t.base + rr * t.rs + c * t.cs] = S[rr * TP + c];
         }
-    }
-    __syncthreads();
-    // Z = B L0^-1, then W = -L1^-1 Z, as 16x16x4 MFMA fragments (A[m][k] from lane
-    // m + 16k, B[k][n] from lane n + 16k), fragment q on wave q
-    typedef typename Vec4<T>::type V4;
-    const int l16 = i & 15, kq = i >> 4, u = q >> 1, v = q & 1;
-    {
-        V4 z = V4{0, 0, 0, 0};
-#pragma unroll
-        for (int k0 = 0; k0 < HB; k0 += 4)
-            z = mfma4(S[(HB + u * 16 + l16) * TP + k0 + kq], Di[(k0 + kq) * HP + v * 16 + l16], z);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) Zs[(u * 16 + mfma16_row<T>(i, e)) * HP + v * 16 + l16] = z[e];
-    }
-    __syncthreads();
-    {
-        V4 z = V4{0, 0, 0, 0};
-#pragma unroll
-        for (int k0 = 0; k0 < HB; k0 += 4)
-            z = mfma4(-Di[(HB + u * 16 + l16) * HP + k0 + kq], Zs[(k0 + kq) * HP + v * 16 + l16], z);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int rr = HB + u * 16 + mfma16_row<T>(i, e), c = v * 16 + l16;
-            inv[rr * NB + c] = (rr < w && c < w) ? z[e] : T(0);
-        }
-    }
-    // inv (row-major, NB x NB): the diagonal blocks from Di, zeros above them; rows 16q ..
-    // 16q+15 on wave q
-#pragma unroll
-    for (int p = 16 * q; p < 16 * q + 16; ++p) {
-        const int hq = p / HB;
-        if (hq == h) inv[p * NB + i] = (p < w && i < w) ? Di[p * HP + cc] : T(0);
-        else if (hq == 0) inv[p * NB + i] = T(0);  // above the diagonal blocks
-    }
+    });
 }
 
 // Panel: A_IJ <- A_IJ * inv^T for every block row I > J (one WG per I).
@@ -744,11 +721,13 @@ __device__ inline const double *xtile(const double *X, int g, int i, int j) {
     return X + ((size_t)g * kGrpTiles + gtile(i, j)) * kTileElems;
 }
 
-// Diagonal tiles of every group's X: the inverses of the 64 x 64 diagonal blocks.
+// Diagonal tiles of every group's X: the inverses of the 64 x 64 diagonal blocks, as the
+// factorization forms its own (11 us; 65 with one barrier and one division per row).
 template <typename T>
 __global__ __launch_bounds__(256) void inv_diag_all(const T *a, Part P, double *X) {
     __shared__ double L[NB * TP];
-    __shared__ double Li[NB * TP];
+    __shared__ double Wk[(NB + HB) * HP];
+    __shared__ double dinv[NB];
     const int J = blockIdx.x;
     const int s0 = P.start(J), w = P.width(J);
     const Tile t = tile_at(P, s0, s0);
@@ -758,35 +737,47 @@ __global__ __launch_bounds__(256) void inv_diag_all(const T *a, Part P, double *
         int r, c;
         if (t.rs == 1) { r = idx % NB; c = idx / NB; } else { c = idx % NB; r = idx / NB; }
         const T v = a[t.base + (size_t)min(r, w - 1) * t.rs + (size_t)min(c, w - 1) * t.cs];
-        L[r * TP + c] = ((r < w) & (c < w) & (r >= c)) ? (double)v : 0.0;
-        Li[r * TP + c] = 0.0;
+        const double pad = r == c ? 1.0 : 0.0;
+        L[r * TP + c] = ((r < w) & (c < w)) ? (r >= c ? (double)v : 0.0) : pad;
     }
-    __shared__ double dgi[NB];
     __syncthreads();
-    tri_inverse<double, double>(L, Li, dgi, w);
-    double *dst = xtile(X, J / kGrp, J % kGrp, J % kGrp);
-    for (int idx = threadIdx.x; idx < kTileElems; idx += blockDim.x) {
-        const int r = idx / NB, c = idx % NB;
-        dst[idx] = (r < w && c < w) ? Li[r * TP + c] : 0.0;
+    if (threadIdx.x < NB) dinv[threadIdx.x] = 1.0 / L[threadIdx.x * TP + threadIdx.x];
+    __syncthreads();
+    tile_inverse<double>(L, dinv, Wk, w, xtile(X, J / kGrp, J % kGrp, J % kGrp), []() {});
+}
+
+// acc += A B for two 64 x 64 LDS tiles (pitch TP), on MFMA: wave w has the 32 x 32 quarter
+// (w / 2, w % 2) as 2 x 2 fragments.
+__device__ __forceinline__ void tile_mm(const double *A, const double *B, v4d (&acc)[2][2]) {
+    const int lane = threadIdx.x & 63, wr = threadIdx.x >> 7, wc = (threadIdx.x >> 6) & 1;
+#pragma unroll 4
+    for (int k0 = 0; k0 < NB; k0 += 4) {
+        const int kk = k0 + (lane >> 4);
+        double av[2], bv[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            av[u] = A[(32 * wr + 16 * u + (lane & 15)) * TP + kk];
+            bv[u] = B[kk * TP + 32 * wc + 16 * u + (lane & 15)];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int v = 0; v < 2; ++v) acc[u][v] = mfma4(av[u], bv[v], acc[u][v]);
     }
 }
 
-// 64 x 64 FP64 product of two LDS tiles (pitch TP), 4 x 4 outputs per thread:
-// acc[u][v] += sum_k A[(4 ty + u) * TP + k] * B[k * TP + 4 tx + v].
-__device__ __forceinline__ void tile_mm(const double *A, const double *B, double (&acc)[4][4]) {
-    const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-#pragma unroll 4
-    for (int k = 0; k < NB; ++k) {
-        double av[4], bv[4];
+// f(row, column, value) for the entries of a tile_mm result this lane holds.
+template <class F>
+__device__ __forceinline__ void tile_each(const v4d (&acc)[2][2], F f) {
+    const int lane = threadIdx.x & 63, wr = threadIdx.x >> 7, wc = (threadIdx.x >> 6) & 1;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) av[u] = A[(4 * ty + u) * TP + k];
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) bv[v] = B[k * TP + 4 * tx + v];
+        for (int v = 0; v < 2; ++v)
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[u][v] += av[u] * bv[v];
-    }
+            for (int e = 0; e < 4; ++e)
+                f(32 * wr + 16 * u + mfma16_row_f64(lane, e), 32 * wc + 16 * v + (lane & 15),
+                  acc[u][v][e]);
 }
 
 // A row-major 64 x 64 FP64 tile from global memory into LDS (pitch TP).
@@ -807,9 +798,8 @@ __global__ __launch_bounds__(256) void inv_group_offdiag(const T *a, Part P, dou
     const int g = blockIdx.x / (kGrp - 1), j = blockIdx.x % (kGrp - 1);
     const int J0 = g * kGrp, m = min(kGrp, P.nblk - J0);
     if (j + 1 >= m) return;
-    const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
     for (int i = j + 1; i < m; ++i) {
-        double acc[4][4] = {};
+        v4d acc[2][2] = {};
         const int ri = P.start(J0 + i), wi = P.width(J0 + i);
         for (int k = j; k < i; ++k) {
             __syncthreads();  // the previous product is done with As and Bs
@@ -831,18 +821,12 @@ __global__ __launch_bounds__(256) void inv_group_offdiag(const T *a, Part P, dou
         }
         __syncthreads();
         xtile_to_lds(xtile(X, g, i, i), As);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Bs[(4 * ty + u) * TP + 4 * tx + v] = acc[u][v];
+        tile_each(acc, [&](int r, int c, double v) { Bs[r * TP + c] = v; });
         __syncthreads();
-        double out[4][4] = {};
+        v4d out[2][2] = {};
         tile_mm(As, Bs, out);
         double *dst = xtile(X, g, i, j);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) dst[(4 * ty + u) * NB + 4 * tx + v] = -out[u][v];
+        tile_each(out, [&](int r, int c, double v) { dst[r * NB + c] = -v; });
         __syncthreads();  // the stores of X(i, j) before the next row reads them
     }
 }
@@ -1065,19 +1049,15 @@ __global__ __launch_bounds__(256) void bwd_group_upd(const T *a, Part P, int g, 
 // start are slower (246.8 ms at 32,000).
 constexpr int kWideFrom = 200;
 
+// Up to this many blocks the factorization is right-looking with one update launch per
+// block step on the caller's stream: the chain of small launches is the whole time, and a
+// rank-64 update of everything (7-10 us) is shorter than a deep update of the next block
+// column (14 us: one work-group a tile walks its whole depth) and needs no second stream.
+// Order 1,501: 0.98 ms against 1.25 with the look-ahead; 2,800: 2.15, 2.40; 4,000: 3.83, 3.63.
+constexpr int kPlainTo = 48;
+
 template <typename T>
-int potrf_impl(T *a, int n, double l2, hipStream_t stream) {
-    KF_REQUIRE(a && n > 0, KF_ERR_ARG, "n must be > 0");
-    const Part P = make_part(n);
-    char *ws = static_cast<char *>(workspace(WS_AUX2, sizeof(T) * NB * NB + 256, stream));
-    KF_REQUIRE(ws, KF_ERR_NOMEM, "workspace allocation failed");
-    int *info = reinterpret_cast<int *>(ws);
-    T *inv = reinterpret_cast<T *>(ws + 256);
-    KF_HIP_TRY(hipMemsetAsync(info, 0, sizeof(int), stream));
-    ScopedTimer timer(TM_POTRF, stream);
-    if (l2 != 0.0) {
-        hipLaunchKernelGGL(add_diag<T>, dim3((n + 255) / 256), dim3(256), 0, stream, a, n, l2);
-    }
+int potrf_lookahead(T *a, const Part &P, T *inv, int *info, hipStream_t stream) {
     // Look-ahead over outer panels (widths from next()).  factor(p) = diagonal POTRF + inverse,
     // panel TRSM and the in-panel updates of panel p; it runs on the aux stream while
     // the caller's stream applies panel p-1 to everything right of panel p.  Per p:
@@ -1131,12 +1111,42 @@ int potrf_impl(T *a, int n, double l2, hipStream_t stream) {
                                J0, J1, info);
         }
     }
+    return KF_OK;
+}
+
+template <typename T>
+int potrf_impl(T *a, int n, double l2, hipStream_t stream) {
+    KF_REQUIRE(a && n > 0, KF_ERR_ARG, "n must be > 0");
+    const Part P = make_part(n);
+    char *ws = static_cast<char *>(workspace(WS_AUX2, sizeof(T) * NB * NB + 256, stream));
+    KF_REQUIRE(ws, KF_ERR_NOMEM, "workspace allocation failed");
+    int *info = reinterpret_cast<int *>(ws);
+    T *inv = reinterpret_cast<T *>(ws + 256);
+    int dev = 0;
+    KF_HIP_TRY(hipGetDevice(&dev));
+    int *h = static_cast<int *>(host_staging(WS_ERR, sizeof(int) * kErrWords));
+    KF_REQUIRE(h && dev >= 0 && dev < kErrWords / 2, KF_ERR_NOMEM, "pinned staging allocation failed");
+    h += kErrWords / 2 + dev;
+    ScopedTimer timer(TM_POTRF, stream);
+    hipLaunchKernelGGL(add_diag<T>, dim3((n + 255) / 256), dim3(256), 0, stream, a, n, l2, info);
+    int rc = 0;
+    if (P.nblk <= kPlainTo) {
+        for (int J = 0; J < P.nblk; ++J) {
+            hipLaunchKernelGGL(potrf_diag<T>, dim3(1), dim3(256), 0, stream, a, P, J, inv, info);
+            const int m = P.nblk - J - 1;
+            if (m == 0) break;
+            hipLaunchKernelGGL(trsm_panel<T>, dim3(m), dim3(256), 0, stream, a, P, J, inv, info);
+            hipLaunchKernelGGL(syrk_range<T>, dim3((unsigned)range_tiles(P, J + 1, P.nblk)),
+                               dim3(256), 0, stream, a, P, J, J + 1, J + 1, P.nblk, info);
+        }
+    } else if ((rc = potrf_lookahead(a, P, inv, info, stream))) {
+        return rc;
+    }
     KF_HIP_TRY(hipGetLastError());
     timer.stop();
-    int h = 0;
-    KF_HIP_TRY(hipMemcpyAsync(&h, info, sizeof(int), hipMemcpyDeviceToHost, stream));
+    KF_HIP_TRY(hipMemcpyAsync(h, info, sizeof(int), hipMemcpyDeviceToHost, stream));
     KF_HIP_TRY(hipStreamSynchronize(stream));
-    return h;
+    return *h;
 }
 
 // Scratch of a solve: the group inverses X, then the intermediate y = L^-1 b.  Every byte

@@ -34,6 +34,24 @@ def to_rfp(K):
     return arf
 
 
+# the last order of the plain factorization (48 blocks of 64) and the first of the look-ahead
+# one, regions that end inside a block, several right-hand sides
+@pytest.mark.parametrize("n,nrhs", [(3009, 1), (3072, 2), (3073, 3), (3100, 1)])
+def test_factor_and_solve_at_the_change_of_form(n, nrhs):
+    from kernelforge_amd import capi
+
+    K = spd(n, n)
+    b = np.random.default_rng(2).standard_normal((nrhs, n))
+    d, x = capi.DeviceArray.from_numpy(to_rfp(K)), capi.DeviceArray.from_numpy(b)
+    capi.rfp_potrf(capi.KF_PREC_F64, d.ptr, n, 0.0)
+    capi.rfp_potrs(capi.KF_PREC_F64, d.ptr, n, x.ptr, nrhs)
+    capi.synchronize()
+    fac, info = sl.get_lapack_funcs("pftrf", (K,))(n, to_rfp(K), transr="N", uplo="U")
+    assert info == 0
+    assert rel_err(d.numpy(), fac) < 1e-11
+    assert rel_err(x.numpy(), np.linalg.solve(K, b.T).T) < 1e-10
+
+
 def test_golden(km):
     g = np.load(os.path.join(ROOT, "tests", "golden", "rfp_ref.npz"))
     a = km.cho_solve_rfp(g["arf"].copy(), g["y"], l2=float(g["l2"]))
