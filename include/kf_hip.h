@@ -102,6 +102,17 @@ int kf_fchl19_f64(const double *coords, const int *Q, const int *N, int nm, int 
                   double acut, double two_body_decay, double three_body_decay, double w3,
                   double *X, double *dX, void *stream);
 
+/* kf_fchl19_f64 with its results rounded to float32 as they are written (coordinates and
+ * arithmetic in FP64), for callers that keep float32 descriptors: half the bytes, and no
+ * FP64 copy of the Jacobians.  For the sizes that kf_fchl19_f32_fits names (returns 1; with
+ * Jacobians when grad is not 0); KF_ERR_ARG for others, where values are added up in X. */
+int kf_fchl19_f32_fits(int max_atoms, int nelem, int nRs2, int nRs3, int nabasis, int grad);
+int kf_fchl19_f32(const double *coords, const int *Q, const int *N, int nm, int max_atoms,
+                  const int *elements, int nelem, const double *Rs2, int nRs2, const double *Rs3,
+                  int nRs3, int nabasis, double eta2, double eta3, double zeta, double rcut,
+                  double acut, double two_body_decay, double three_body_decay, double w3,
+                  float *X, float *dX, void *stream);
+
 /* FCHL19v2 representation (and optionally its Jacobian) of a padded batch, with
  * selectable bases.  Replaces kf::fchl19v2::generate (src/fchl19v2_repr.cpp:2874) and
  * generate_and_gradients (:2919).  two_body_type / three_body_type index the reference's
@@ -222,6 +233,13 @@ int kf_local_full_matvec(const double *X1, const double *dX1, const double *X2,
                          const int *Q2, const int *N1, const int *N2, int nm1, int nm2,
                          int max_atoms1, int max_atoms2, int rep, double sigma, double *E,
                          double *F, void *stream);
+
+/* kf_local_full_matvec on float32 arrays (arithmetic and results in FP64). */
+int kf_local_full_matvec_f32(const float *X1, const float *dX1, const float *X2,
+                             const float *alpha_desc, const float *alpha_E, const int *Q1,
+                             const int *Q2, const int *N1, const int *N2, int nm1, int nm2,
+                             int max_atoms1, int max_atoms2, int rep, double sigma, double *E,
+                             double *F, void *stream);
 
 /* F (naq1,) = Hessian kernel @ alpha_F.  Replaces kernel_gaussian_local_hessian_matvec
  * (src/local_kernels.hpp:171-191, src/local_kernels.cpp:2895-3145). */

@@ -71,6 +71,14 @@ def f64(t: torch.Tensor, name: str) -> torch.Tensor:
     return t.to(torch.float64).contiguous()
 
 
+def f32(t: torch.Tensor, name: str) -> torch.Tensor:
+    """FP32 contiguous view or copy, for the entry points that read float32."""
+    device_tensor(t, name)
+    if not (t.is_floating_point()):
+        raise TypeError(f"{name} must be a floating-point tensor")
+    return t.to(torch.float32).contiguous()
+
+
 def i32(t: torch.Tensor, name: str) -> torch.Tensor:
     device_tensor(t, name)
     if t.is_floating_point() or t.is_complex():

@@ -43,6 +43,10 @@ SIGNATURES = {
     "kf_fchl19_f64": [_vp, _vp, _vp, _c_int, _c_int, _vp, _c_int, _vp, _c_int, _vp, _c_int,
                       _c_int, _c_double, _c_double, _c_double, _c_double, _c_double, _c_double,
                       _c_double, _c_double, _vp, _vp, _vp],
+    "kf_fchl19_f32_fits": [_c_int] * 6,
+    "kf_fchl19_f32": [_vp, _vp, _vp, _c_int, _c_int, _vp, _c_int, _vp, _c_int, _vp, _c_int,
+                      _c_int, _c_double, _c_double, _c_double, _c_double, _c_double, _c_double,
+                      _c_double, _c_double, _vp, _vp, _vp],
     "kf_fchl19v2_f64": [_vp, _vp, _vp, _c_int, _c_int, _vp, _c_int, _vp, _c_int, _vp, _c_int,
                         _vp, _c_int, _c_int, _c_int, _c_int] + [_c_double] * 11 + [_vp, _vp, _vp],
     "kf_local_kernel_symm_rfp": [_c_int, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_double, _vp,
@@ -69,6 +73,7 @@ SIGNATURES = {
     "kf_local_kernel_full_symm_rfp": [_vp] * 4 + [_c_int] * 3 + [_c_double, _vp, _vp],
     "kf_local_alpha_desc": [_vp, _vp, _vp, _c_int, _c_int, _c_int, _vp, _vp, _vp],
     "kf_local_full_matvec": [_vp] * 9 + [_c_int] * 5 + [_c_double, _vp, _vp, _vp],
+    "kf_local_full_matvec_f32": [_vp] * 9 + [_c_int] * 5 + [_c_double, _vp, _vp, _vp],
     "kf_local_hessian_matvec": [_vp] * 8 + [_c_int] * 5 + [_c_double, _vp, _vp],
     "kf_local_jacobian_t_matvec": [_vp] * 7 + [_c_int] * 5 + [_c_double, _vp, _vp],
     "kf_matvec_plan_create": [_vp, _vp, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int,
@@ -204,18 +209,19 @@ def fchl_basis(elements=(1, 6, 7, 8, 16), nRs2=24, nRs3=20, nFourier=1, rcut=8.0
 
 def fchl19(coords, Q, N, nm, max_atoms, X, dX=0, stream=0, elements=(1, 6, 7, 8, 16), nRs2=24,
            nRs3=20, nFourier=1, eta2=0.32, eta3=2.7, zeta=math.pi, rcut=8.0, acut=8.0,
-           two_body_decay=1.8, three_body_decay=0.57, three_body_weight=13.4):
-    """kf_fchl19_f64 on device pointers (dX=0 for the representation only)."""
+           two_body_decay=1.8, three_body_decay=0.57, three_body_weight=13.4, f32=False):
+    """kf_fchl19_f64 (f32: kf_fchl19_f32, results in float32) on device pointers (dX=0 for the
+    representation only)."""
     el, Rs2, Rs3, nab, w3 = fchl_basis(elements, nRs2, nRs3, nFourier, rcut, acut, eta3,
                                        three_body_weight, grad=bool(dX))
     el_a = (ctypes.c_int * len(el))(*el)
     r2 = (ctypes.c_double * len(Rs2))(*Rs2)
     r3 = (ctypes.c_double * len(Rs3))(*Rs3)
-    rc = lib().kf_fchl19_f64(coords, Q, N, nm, max_atoms, ctypes.cast(el_a, _vp), len(el),
-                             ctypes.cast(r2, _vp), len(Rs2), ctypes.cast(r3, _vp), len(Rs3), nab,
-                             eta2, eta3, zeta, rcut, acut, two_body_decay, three_body_decay, w3,
-                             X, dX or None, stream or None)
-    return check(rc, "kf_fchl19_f64")
+    fn = lib().kf_fchl19_f32 if f32 else lib().kf_fchl19_f64
+    rc = fn(coords, Q, N, nm, max_atoms, ctypes.cast(el_a, _vp), len(el), ctypes.cast(r2, _vp),
+            len(Rs2), ctypes.cast(r3, _vp), len(Rs3), nab, eta2, eta3, zeta, rcut, acut,
+            two_body_decay, three_body_decay, w3, X, dX or None, stream or None)
+    return check(rc, "kf_fchl19_f32" if f32 else "kf_fchl19_f64")
 
 
 def rep_size(nelem=5, nRs2=24, nRs3=20, nabasis=2):

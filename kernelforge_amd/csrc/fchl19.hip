@@ -142,9 +142,10 @@ __host__ inline size_t rep_lds_bytes(int ma, int nelem, int nchan, int na) {
     return sizeof(double) * (size_t)g.ints + sizeof(int) * (size_t)g.total_ints;
 }
 
+template <typename O>
 __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
     const double *__restrict__ coords, const int *__restrict__ Q, const int *__restrict__ N,
-    FchlParams P, double *__restrict__ X, int *__restrict__ err) {
+    FchlParams P, O *__restrict__ X, int *__restrict__ err) {
     extern __shared__ __align__(16) double smem[];
     __shared__ int next;
     const int m = blockIdx.x, tid = threadIdx.x;
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
         while (q >= nelem - p) q -= nelem - p, ++p;
         chan[c] = p << 16 | (p + q);
     }
-    double *Xm = X + (size_t)m * ma * P.rs;
+    O *Xm = X + (size_t)m * ma * P.rs;
     // a molecule with an unknown element is reported through *err; its rows are zeroed
     if (__syncthreads_or(bad)) {
         if (tid == 0) *err = 1;
@@ -183,9 +184,9 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
               row1 = min(row0 + per, ma), cen1 = min(row1, n);
     const int pad0 = max(row0, n);  // padding rows
     if (pad0 < row1) {
-        double *d = Xm + (size_t)pad0 * P.rs;
+        O *d = Xm + (size_t)pad0 * P.rs;
         const int cnt = (row1 - pad0) * P.rs;
-        for (int t = tid; t < cnt; t += kRepThreads) d[t] = 0.0;
+        for (int t = tid; t < cnt; t += kRepThreads) d[t] = O(0);
     }
     if (row0 >= cen1) return;
     for (int t = tid; t < n; t += kRepThreads) {
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
                     v += t_f[x] * exp_scaled(L * L * t_sc[x], tab);
                 }
             }
-            Xm[(size_t)i * P.rs + e * P.nb2 + k] = v / P.Rs2[k];
+            Xm[(size_t)i * P.rs + e * P.nb2 + k] = O(v / P.Rs2[k]);
         }
         // ---- three-body, in one chunk unless a single centre has more than g.pairs ----
         for (int q0 = 0; q0 == 0 || q0 < npair; q0 += g.pairs) {
@@ -322,7 +323,7 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
                 const int lo = max(cs[c], q0) - q0, hi = min(cs[c + 1], q0 + qn) - q0;
                 const bool first = q0 == 0 || q0 <= cs[c];  // nothing of it before this chunk
                 if (hi <= lo && q0 > 0) continue;
-                double *dst = Xm + (size_t)i * P.rs + P.three_off + (c * P.nb3 + l0) * P.na;
+                O *dst = Xm + (size_t)i * P.rs + P.three_off + (c * P.nb3 + l0) * P.na;
                 const int ln = min(kLB, P.nb3 - l0);
                 double rs3[kLB];
 #pragma unroll
@@ -345,9 +346,9 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
 #pragma unroll
                     for (int u = 0; u < kLB; ++u) {
                         if (u >= ln) break;
-                        double *d = dst + u * P.na + ta;
-                        d[0] = first ? v0[u] : d[0] + v0[u];
-                        d[1] = first ? v1[u] : d[1] + v1[u];
+                        O *d = dst + u * P.na + ta;
+                        d[0] = O(first ? v0[u] : d[0] + v0[u]);
+                        d[1] = O(first ? v1[u] : d[1] + v1[u]);
                     }
                 }
             }
@@ -411,23 +412,26 @@ __host__ inline size_t grad_lds_bytes(int ma, int nb2, int nb3, int na) {
 }
 
 // n doubles of `src` (LDS; zeros when null) to dst, 16 bytes a lane where dst allows it.
-__device__ inline void stream_out(double *dst, const double *src, int n) {
-    typedef double d2 __attribute__((ext_vector_type(2)));
-    if (((reinterpret_cast<size_t>(dst) & 15) | (n & 1)) == 0) {
-        for (int t = threadIdx.x; t < n / 2; t += kGradThreads) {
-            d2 v = {0.0, 0.0};
-            if (src) v = reinterpret_cast<const d2 *>(src)[t];
-            reinterpret_cast<d2 *>(dst)[t] = v;
+template <typename O>
+__device__ inline void stream_out(O *dst, const double *src, int n) {
+    constexpr int V = 16 / sizeof(O);
+    typedef O vec __attribute__((ext_vector_type(V)));
+    if (((reinterpret_cast<size_t>(dst) & 15) | (n % V)) == 0) {
+        for (int t = threadIdx.x; t < n / V; t += kGradThreads) {
+            vec v;
+#pragma unroll
+            for (int u = 0; u < V; ++u) v[u] = src ? O(src[t * V + u]) : O(0);
+            reinterpret_cast<vec *>(dst)[t] = v;
         }
     } else {
-        for (int t = threadIdx.x; t < n; t += kGradThreads)
-            dst[t] = src ? src[t] : 0.0;
+        for (int t = threadIdx.x; t < n; t += kGradThreads) dst[t] = src ? O(src[t]) : O(0);
     }
 }
 
+template <typename O>
 __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
     const double *__restrict__ coords, const int *__restrict__ Q, const int *__restrict__ N,
-    FchlParams P, int splits, double *__restrict__ X, double *__restrict__ dX,
+    FchlParams P, int splits, O *__restrict__ X, O *__restrict__ dX,
     int *__restrict__ err) {
     extern __shared__ __align__(16) double smem[];
     const int m = blockIdx.y, i = blockIdx.x / splits, split = blockIdx.x % splits;
@@ -436,8 +440,8 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
     const int ld = 3 * ma;
     int n = N[m];
     n = n < 0 ? 0 : (n > ma ? ma : n);
-    double *Xi = X + ((size_t)m * ma + i) * P.rs;
-    double *dXi = dX + ((size_t)m * ma + i) * P.rs * ld;
+    O *Xi = X + ((size_t)m * ma + i) * P.rs;
+    O *dXi = dX + ((size_t)m * ma + i) * P.rs * ld;
     const GradLds g = grad_lds(ma, P.nb2, P.nb3, P.na);
     double *tab = smem + g.tab, *R = smem + g.R, *u4 = smem + g.u4, *fc = smem + g.f,
            *dfc = smem + g.df, *two = smem + g.two, *rec = smem + g.rec, *tile = smem + g.tile,
@@ -466,8 +470,8 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
     auto zero_unit = [&](int unit) {
         int f0, nr;
         unit_rows(unit, f0, nr);
-        for (int t = tid; t < nr; t += kGradThreads) Xi[f0 + t] = 0.0;
-        stream_out(dXi + (size_t)f0 * ld, nullptr, nr * ld);
+        for (int t = tid; t < nr; t += kGradThreads) Xi[f0 + t] = O(0);
+        stream_out<O>(dXi + (size_t)f0 * ld, nullptr, nr * ld);
     };
 
     bool bad = false;
@@ -696,11 +700,11 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
                 tile[row * ld + 3 * i + d] = s;
             } else {
                 for (int a = 0; a < np; ++a) s += vals[row * ma + a];
-                Xi[f0 + row] = (!is2 && p == q) ? 0.5 * s : s;
+                Xi[f0 + row] = O((!is2 && p == q) ? 0.5 * s : s);
             }
         }
         __syncthreads();
-        stream_out(dXi + (size_t)f0 * ld, tile, nr * ld);
+        stream_out<O>(dXi + (size_t)f0 * ld, tile, nr * ld);
         __syncthreads();
     }
 }
@@ -748,17 +752,23 @@ int build_params(FchlParams &P, int max_atoms, const int *elements, int nelem, c
     return KF_OK;
 }
 
-}  // namespace
-}  // namespace kf
+// Whether the kernels above take this batch (else kf_fchl19_f64 takes the FCHL19v2 kernel), and
+// whether they write each value once: a representation whose centres have more pairs than one
+// chunk holds is added up in X itself.
+bool fchl19_fits(int ma, int nelem, int nchan, int nb2, int nb3, int na, bool grad) {
+    return ma <= kMaxAtoms && (grad ? grad_lds_bytes(ma, nb2, nb3, na)
+                                    : rep_lds_bytes(ma, nelem, nchan, na)) <= 160 * 1024;
+}
+bool fchl19_one_chunk(int ma, int nelem, int nchan, int na) {
+    return (long)(ma - 1) * (ma - 2) / 2 <= rep_lds(ma, nelem, nchan, na).pairs;
+}
 
-extern "C" int kf_fchl19_f64(const double *coords, const int *Q, const int *N, int nm,
-                             int max_atoms, const int *elements, int nelem, const double *Rs2,
-                             int nRs2, const double *Rs3, int nRs3, int nabasis, double eta2,
-                             double eta3, double zeta, double rcut, double acut,
-                             double two_body_decay, double three_body_decay, double w3,
-                             double *X, double *dX, void *stream_) {
-    kf::EntryGuard kf_entry_guard_(kf::as_stream(stream_));
-    using namespace kf;
+template <typename O>
+int fchl19_impl(const double *coords, const int *Q, const int *N, int nm, int max_atoms,
+                const int *elements, int nelem, const double *Rs2, int nRs2, const double *Rs3,
+                int nRs3, int nabasis, double eta2, double eta3, double zeta, double rcut,
+                double acut, double two_body_decay, double three_body_decay, double w3, O *X,
+                O *dX, void *stream_) {
     hipStream_t stream = as_stream(stream_);
     KF_REQUIRE(nm >= 0, KF_ERR_ARG, "nm must be >= 0");
     if (nm == 0) return KF_OK;
@@ -773,7 +783,11 @@ extern "C" int kf_fchl19_f64(const double *coords, const int *Q, const int *N, i
     const size_t lds_rep = rep_lds_bytes(ma, P.nelem, P.nchan, P.na);
     const size_t lds_grad = grad_lds_bytes(ma, P.nb2, P.nb3, P.na);
     const size_t lds = dX ? lds_grad : lds_rep;
-    if (ma > kMaxAtoms || lds > 160 * 1024) {
+    const bool fits = fchl19_fits(ma, P.nelem, P.nchan, P.nb2, P.nb3, P.na, dX != nullptr);
+    if constexpr (sizeof(O) == sizeof(float)) {
+        KF_REQUIRE(fits && (dX || fchl19_one_chunk(ma, P.nelem, P.nchan, P.na)), KF_ERR_ARG,
+                   "max_atoms %d is too large for float32 results (kf_fchl19_f32_fits)", ma);
+    } else if (!fits) {
         // Large molecules: the FCHL19v2 kernel with the log-normal two-body and odd-Fourier
         // r_bar three-body bases is this representation (same values and Jacobian, the
         // gradient path's first-harmonic convention included) and stages no molecule in LDS.
@@ -794,20 +808,55 @@ extern "C" int kf_fchl19_f64(const double *coords, const int *Q, const int *N, i
         // up to a work-group per two rows while there are fewer molecules than the GPU takes
         // work-groups
         const int splits = std::max(1, std::min((ma + 1) / 2, 1024 / nm));
-        hipLaunchKernelGGL(fchl19_rep_kernel, dim3(nm, splits), dim3(kRepThreads), lds, stream,
+        hipLaunchKernelGGL(fchl19_rep_kernel<O>, dim3(nm, splits), dim3(kRepThreads), lds, stream,
                            coords, Q, N, P, X, err);
     } else {
         KF_REQUIRE(P.nelem * P.nb2 > 0, KF_ERR_BASIS, "empty two-body basis");
         // Several work-groups per centre while the batch has fewer centres than the GPU takes
-        // work-groups (256 CUs, three each): one
-        // molecule of 21 atoms takes 20 us with 8 per centre (181 us before, one per centre)
+        // work-groups (256 CUs, three each): one molecule of 21 atoms takes 20 us with 8 per centre (181 us before, one per centre)
         const long centres = (long)nm * ma;
         const int splits = centres >= 768 ? 1 : (int)std::min<long>(8, 768 / centres);
-        hipLaunchKernelGGL(fchl19_grad_kernel, dim3(ma * splits, nm), dim3(kGradThreads), lds,
+        hipLaunchKernelGGL(fchl19_grad_kernel<O>, dim3(ma * splits, nm), dim3(kGradThreads), lds,
                            stream, coords, Q, N, P, splits, X, dX, err);
     }
     KF_HIP_TRY(hipGetLastError());
     KF_HIP_TRY(hipStreamSynchronize(stream));
     KF_REQUIRE(*static_cast<volatile int *>(err) == 0, KF_ERR_ELEMENT, "nuclear_z contains an element not present in elements");
     return KF_OK;
+}
+
+}  // namespace
+}  // namespace kf
+
+extern "C" int kf_fchl19_f64(const double *coords, const int *Q, const int *N, int nm,
+                             int max_atoms, const int *elements, int nelem, const double *Rs2,
+                             int nRs2, const double *Rs3, int nRs3, int nabasis, double eta2,
+                             double eta3, double zeta, double rcut, double acut,
+                             double two_body_decay, double three_body_decay, double w3,
+                             double *X, double *dX, void *stream) {
+    kf::EntryGuard kf_entry_guard_(kf::as_stream(stream));
+    return kf::fchl19_impl<double>(coords, Q, N, nm, max_atoms, elements, nelem, Rs2, nRs2, Rs3,
+                                   nRs3, nabasis, eta2, eta3, zeta, rcut, acut, two_body_decay,
+                                   three_body_decay, w3, X, dX, stream);
+}
+
+extern "C" int kf_fchl19_f32_fits(int max_atoms, int nelem, int nRs2, int nRs3, int nabasis,
+                                  int grad) {
+    using namespace kf;
+    if (max_atoms < 1 || nelem < 1 || nRs2 < 1 || nRs3 < 1 || nabasis < 1) return 0;
+    const int nchan = nelem * (nelem + 1) / 2;
+    return fchl19_fits(max_atoms, nelem, nchan, nRs2, nRs3, nabasis, grad != 0) &&
+           (grad || fchl19_one_chunk(max_atoms, nelem, nchan, nabasis));
+}
+
+extern "C" int kf_fchl19_f32(const double *coords, const int *Q, const int *N, int nm,
+                             int max_atoms, const int *elements, int nelem, const double *Rs2,
+                             int nRs2, const double *Rs3, int nRs3, int nabasis, double eta2,
+                             double eta3, double zeta, double rcut, double acut,
+                             double two_body_decay, double three_body_decay, double w3, float *X,
+                             float *dX, void *stream) {
+    kf::EntryGuard kf_entry_guard_(kf::as_stream(stream));
+    return kf::fchl19_impl<float>(coords, Q, N, nm, max_atoms, elements, nelem, Rs2, nRs2, Rs3,
+                                  nRs3, nabasis, eta2, eta3, zeta, rcut, acut, two_body_decay,
+                                  three_body_decay, w3, X, dX, stream);
 }

@@ -1,6 +1,7 @@
 """Torch-tensor interface of the FCHL19 representation, with the function names and
 arguments of the reference's GPU module (python/kernelforge/cuda_fchl19_repr.pyi:5-81),
-on the FP64 HIP kernel of libkf_hip.so (kf_fchl19_f64).
+on the FP64 HIP kernels of libkf_hip.so (kf_fchl19_f64; kf_fchl19_f32 rounds the results to
+float32 as it writes them).
 
 Q holds element indices in [0, nelements) as in the reference's GPU module (the host
 module fchl19_repr takes nuclear charges and an element list instead).  The results
@@ -43,15 +44,20 @@ def _run(coords, Q, N, nelements, grad, nRs2, nRs3, nFourier, eta2, eta3, zeta, 
         raise ValueError("nelements must be >= 1")
     nab = max(2 * int(nFourier), 2) if grad else 2 * int(nFourier)
     rep = capi.rep_size(nelements, nRs2, nRs3, nab)
-    X = torch.empty((nm, ma, rep), dtype=torch.float64, device=C.device)
-    dX = torch.empty((nm, ma, rep, ma, 3), dtype=torch.float64, device=C.device) if grad else None
-    tb.lib()  # binds the library to torch's runtime (checked once)
+    lib = tb.lib()  # binds the library to torch's runtime (checked once)
+    # float32 results are written by the kernels themselves for all but large molecules
+    f32 = dtype == torch.float32 and lib.kf_fchl19_f32_fits(ma, nelements, nRs2, nRs3, nab,
+                                                            int(grad)) == 1
+    made = dtype if f32 else torch.float64
+    X = torch.empty((nm, ma, rep), dtype=made, device=C.device)
+    dX = torch.empty((nm, ma, rep, ma, 3), dtype=made, device=C.device) if grad else None
     capi.fchl19(C.data_ptr(), Qi.data_ptr(), Ni.data_ptr(), nm, ma, X.data_ptr(),
                 dX.data_ptr() if grad else 0, tb.stream_of(C), elements=tuple(range(nelements)),
                 nRs2=nRs2, nRs3=nRs3, nFourier=nFourier, eta2=eta2, eta3=eta3, zeta=zeta,
                 rcut=rcut, acut=acut, two_body_decay=two_body_decay,
-                three_body_decay=three_body_decay, three_body_weight=three_body_weight)
-    if dtype != torch.float64:
+                three_body_decay=three_body_decay, three_body_weight=three_body_weight,
+                f32=f32)
+    if made != dtype:
         X = X.to(dtype)
         dX = dX.to(dtype) if grad else None
     return (X, dX) if grad else X

@@ -30,8 +30,8 @@ __all__ = [
 ]
 
 
-def _xqn(X, Q, N, tag=""):
-    X = tb.f64(X, "X" + tag)
+def _xqn(X, Q, N, tag="", to=tb.f64):
+    X = to(X, "X" + tag)
     if X.dim() != 3:
         raise ValueError(f"X{tag} must have shape (nm, max_atoms, rep)")
     nm, ma, rep = X.shape
@@ -41,8 +41,8 @@ def _xqn(X, Q, N, tag=""):
     return X, Q, N, nm, ma, rep
 
 
-def _dx(dX, nm, ma, rep, tag=""):
-    dX = tb.f64(dX, "dX" + tag)
+def _dx(dX, nm, ma, rep, tag="", to=tb.f64):
+    dX = to(dX, "dX" + tag)
     if dX.numel() != nm * ma * rep * 3 * ma:
         raise ValueError(f"dX{tag} must have shape (nm, max_atoms, rep, 3*max_atoms)")
     return dX.reshape(nm, ma, rep, 3 * ma)
@@ -163,21 +163,24 @@ def kernel_gaussian_full_matvec(X_q, dX_q, Q_q, N_q, X_t, Q_t, N_t, alpha_E, alp
     """(E_pred (nm_q,), F_pred (naq_q,)) = K_full(query, train) @ [alpha_E; alpha_F] with
     alpha_desc_F from compute_alpha_desc (the full kernel is never formed)."""
     tb.same_device(X_q, dX_q, Q_q, N_q, X_t, Q_t, N_t, alpha_E, alpha_desc_F)
-    dtype = tb.out_dtype(X_q, dX_q, X_t, alpha_E, alpha_desc_F)
-    X1, Q1, N1, nm1, ma1, rep = _xqn(X_q, Q_q, N_q, "_q")
-    X2, Q2, N2, nm2, ma2, _ = _xqn(X_t, Q_t, N_t, "_t")
-    dX1 = _dx(dX_q, nm1, ma1, rep, "_q")
-    ad = tb.f64(alpha_desc_F, "alpha_desc_F")
-    aE = tb.f64(alpha_E, "alpha_E").reshape(-1)
+    floats = (X_q, dX_q, X_t, alpha_E, alpha_desc_F)
+    dtype = tb.out_dtype(*floats)
+    # float32 operands go to the kernels as they are (they are widened as they are read)
+    f32 = all(t.dtype == torch.float32 for t in floats)
+    to = tb.f32 if f32 else tb.f64
+    X1, Q1, N1, nm1, ma1, rep = _xqn(X_q, Q_q, N_q, "_q", to)
+    X2, Q2, N2, nm2, ma2, _ = _xqn(X_t, Q_t, N_t, "_t", to)
+    dX1 = _dx(dX_q, nm1, ma1, rep, "_q", to)
+    ad = to(alpha_desc_F, "alpha_desc_F")
+    aE = to(alpha_E, "alpha_E").reshape(-1)
     _check_train(ad, aE, nm2, ma2, rep)
     E = torch.empty(nm1, dtype=torch.float64, device=X1.device)
     F = torch.empty(tb.naq(N1, ma1), dtype=torch.float64, device=X1.device)
-    tb.check(tb.lib().kf_local_full_matvec(X1.data_ptr(), dX1.data_ptr(), X2.data_ptr(),
-                                           ad.data_ptr(), aE.data_ptr(), Q1.data_ptr(),
-                                           Q2.data_ptr(), N1.data_ptr(), N2.data_ptr(), nm1, nm2,
-                                           ma1, ma2, rep, _sigma(sigma), E.data_ptr(),
-                                           F.data_ptr() if F.numel() else None, tb.stream_of(E)),
-             "kernel_gaussian_full_matvec")
+    fn = tb.lib().kf_local_full_matvec_f32 if f32 else tb.lib().kf_local_full_matvec
+    tb.check(fn(X1.data_ptr(), dX1.data_ptr(), X2.data_ptr(), ad.data_ptr(), aE.data_ptr(),
+                Q1.data_ptr(), Q2.data_ptr(), N1.data_ptr(), N2.data_ptr(), nm1, nm2, ma1, ma2,
+                rep, _sigma(sigma), E.data_ptr(), F.data_ptr() if F.numel() else None,
+                tb.stream_of(E)), "kernel_gaussian_full_matvec")
     return (E, F) if dtype == torch.float64 else (E.to(dtype), F.to(dtype))
 
 

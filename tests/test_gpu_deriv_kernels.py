@@ -219,6 +219,30 @@ def test_matvec_variants(lk, case):
     assert rel_err(Ej, oracle.jacobian_t_matvec(X1, X2, ad, Q1, Q2, N1, N2, s)) < TOL
 
 
+def test_matvec_float32_operands(lk):
+    """float32 operands give what the same numbers held in FP64 give."""
+    from kernelforge_amd import capi
+
+    X1, dX1, Q1, N1 = rand_set(6, 11, 41, 3, 5)
+    X2, _, Q2, N2 = rand_set(9, 8, 41, 3, 6)
+    rng = np.random.default_rng(8)
+    ad, aE = rng.standard_normal((9, 8, 41)), rng.standard_normal(9)
+    X2[..., 30:] = 0.0
+    ad[..., 30:] = 0.0
+    naq = 3 * int(N1.sum())
+    ints = [capi.DeviceArray.from_numpy(a.astype(np.int32)) for a in (Q1, Q2, N1, N2)]
+    out = []
+    for dtype, fn in ((np.float32, "kf_local_full_matvec_f32"), (np.float64, "kf_local_full_matvec")):
+        ops = [capi.DeviceArray.from_numpy(a.astype(np.float32).astype(dtype)) for a in (X1, dX1, X2, ad, aE)]
+        E, F = capi.DeviceArray(6), capi.DeviceArray(naq)
+        capi.check(getattr(capi.lib(), fn)(*(o.ptr for o in ops), *(i.ptr for i in ints), 6, 9, 11,
+                                           8, 41, 1.6, E.ptr, F.ptr, None), fn)
+        capi.synchronize()
+        out.append((E.numpy(), F.numpy()))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
 def test_matvec_conformers_symmetric(lk):
     """Training-set operator on C9H8O4 conformers equals the RFP E+F kernel times alpha."""
     from kernelforge_amd import synthetic

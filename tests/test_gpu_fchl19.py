@@ -123,6 +123,36 @@ def test_jacobian_kernel_edges(fr, ma, nm, kw):
     assert row_rel_err(dX, dXo, lead=2) < 1e-12
 
 
+# float32 results are the FP64 ones rounded: rows whose blocks are and are not whole 16-byte
+# words, and sizes that the float32 entry point leaves to the FP64 one
+@pytest.mark.parametrize("ma,nm,grad,kw", [
+    (1, 2, True, {}), (9, 30, True, dict(nRs2=41, nRs3=37)), (12, 3, True, dict(nRs3=3)),
+    (45, 1, True, {}), (3, 700, False, dict(nRs3=1)), (23, 20, False, {}), (47, 3, False, {})])
+def test_float32_results(fr, ma, nm, grad, kw):
+    from kernelforge_amd import capi, synthetic
+
+    rng = np.random.default_rng(7 * ma + nm)
+    Ns = np.concatenate([[ma], rng.integers(1, ma + 1, nm - 1)]).astype(int)
+    C, Q, N = synthetic.pad_batch([synthetic._place_atoms(rng, n) for n in Ns],
+                                  [rng.choice([1, 6, 7, 8, 16], n).astype(np.int32) for n in Ns])
+    p = dict(nRs2=24, nRs3=20) | kw
+    rep = capi.rep_size(5, p["nRs2"], p["nRs3"], 2)
+    Cd, Qd, Nd = (capi.DeviceArray.from_numpy(a) for a in (C, Q.astype(np.int32), N.astype(np.int32)))
+    out = []
+    for f32 in (False, True):
+        X = capi.DeviceArray((nm, ma, rep), np.float32 if f32 else np.float64)
+        J = capi.DeviceArray((nm, ma, rep, 3 * ma), X.dtype) if grad else None
+        if f32 and not capi.lib().kf_fchl19_f32_fits(ma, 5, p["nRs2"], p["nRs3"], 2, int(grad)):
+            with pytest.raises(ValueError):
+                capi.fchl19(Cd.ptr, Qd.ptr, Nd.ptr, nm, ma, X.ptr, J.ptr if grad else 0, f32=True, **p)
+            return
+        capi.fchl19(Cd.ptr, Qd.ptr, Nd.ptr, nm, ma, X.ptr, J.ptr if grad else 0, f32=f32, **p)
+        capi.synchronize()
+        out.append([X.numpy()] + ([J.numpy()] if grad else []))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a.astype(np.float32), b)
+
+
 # one atom to more than the pair storage holds in one go (47 atoms: 1,035 pairs a centre),
 # batches of a few centres, one radial term left over per thread, many angular terms (a
 # smaller pair storage: several chunks from 21 atoms on), one element, work-groups sharing
