@@ -1027,7 +1027,9 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
             // Few pairs: each pair's features in several runs (of 32 and more), so that there
             // are about 2,048 work-groups, four per slot of the GPU (512): 703 pairs of mixed
             // molecules of 5-23 atoms 3.5 ms, 4.5 with one run each
-            const int runs = std::max(1, std::min((int)(2048 / nb), A.rep / 32));
+            int runs = std::max(1, std::min((int)(2048 / nb), A.rep / 32));
+            const int run = (A.rep + runs - 1) / runs;
+            runs = (A.rep + run - 1) / run;  // none of them empty
             double *parts = nullptr;
             if (runs > 1) {
                 const size_t bytes = sizeof(double) * nb * runs * (size_t)A.ldv * A.ldu;
