@@ -25,7 +25,9 @@
 // Every output entry belongs to exactly one molecule pair, so no atomics are used
 // and results are deterministic.
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "feature_compact.hpp"
@@ -65,6 +67,12 @@ __host__ __device__ constexpr bool is_rfp(int m) {
     return m == M_HESS_SYMM_RFP || m == M_FULL_SYMM_RFP;
 }
 
+// The order in which a molecule's atoms are taken by deriv_ff_kernel.
+struct FfOrder {
+    signed char row[MAXA];  // atom in row r, -1 for none
+    signed char col[MAXA];  // atom of force columns 3r .. 3r+2, -1 past the last
+};
+
 struct DerivArgs {
     const double *x1, *dx1, *x2, *dx2;
     const int *q1, *q2, *n1, *n2;
@@ -79,10 +87,11 @@ struct DerivArgs {
     double *slot;  // per-pair scratch: e[maxm] | V[maxm][ldv] | U[maxm][ldu]
     size_t slot_len;
     int maxm, ldv, ldu;
+    const FfOrder *order1, *order2;               // a row per molecule (Hessian forms)
+    const uint2 *blocks1, *blocks2;               // ff_blocks_kernel: a word per (molecule, feature)
 };
 
 __device__ inline int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
-
 
 __device__ inline double wave_sum(double v) {
 #pragma unroll
@@ -623,21 +632,130 @@ __global__ __launch_bounds__(NT, 2) void deriv_vproj_kernel(DerivArgs A, const P
 // column l%16), so T_f's accumulators feed the second product without a shuffle.
 // Wave w owns q-block w (16 force columns of b) and all p-blocks of a.  J_a[:,f,:] is
 // shared by the four waves: it is staged through two LDS buffers (one barrier per
-// feature); T for f+1 is formed while the product of f runs and the operands of f+2
-// are loaded during f.  Atoms are padded to 4*NK (rows of C past na / columns past nb
-// are zero, the matching Jacobian rows are clamped reads), force columns to 16*NP
-// (clamped reads, never stored).  Every global load is unconditional.
+// feature); T for f+1 is formed after the product of f, whose loads have then come in,
+// and the operands of f+2 are loaded during f.  Every global load is unconditional.
+//
+// The matrix cores bound it, and most of what they would multiply is zero: C joins atoms of
+// one label, and a feature that belongs to some labels (an FCHL19 channel) changes only with
+// the positions of atoms of those labels and of its own centre.  So a molecule's atoms are
+// taken in an order that puts atoms of one label next to each other (rows: 4*NK places,
+// labels starting at multiples of 4 where they fit; force columns: the same order without
+// gaps, 16*NP), ff_blocks_kernel notes per feature which 4-row by 16-column blocks of the
+// Jacobian hold anything, and a wave leaves out the MFMAs of empty blocks: for 21 atoms of 3
+// labels 20 of 36 remain (the busiest wave's q-block 23), and 20,100 pairs of such molecules
+// take 26.5 ms instead of 34.6, 703 pairs of 5-23 mixed atoms 2.0 instead of 3.4; what is
+// lost against the count is the waves' wait for one another at each feature's barrier.  Exact
+// zeros alone are left out, so the sums are the same.  Where
+// 0 * x would not be 0 (a feature or a coefficient that is not finite) all blocks are taken.
+// Rows past the atoms of a molecule are rows of C that are zero.
+// Pairs of up to kFfDense atoms take every block, atoms in their own order: they have one or
+// two of the four q-blocks, each step is then a chain of loads and waits rather than of MFMAs,
+// and the words add to it (45,150 pairs of 5 atoms 9.9 ms with them, 7.4 without; 20,100 of 10
+// atoms 8.3 and 7.3; of 12 atoms 9.5 and 11.3).
 // ---------------------------------------------------------------------------
+// blocks[m][f]: bit 8 y + s set when rows 4s .. 4s+3, columns 16y .. 16y+15 of feature f hold
+// a value that is not zero; bit 63 when one is not finite.  A wave takes a feature at a
+// time, its lanes the force columns.  Bound by the read of the Jacobians.
+constexpr int kBlkRun = 32;   // features per work-group
+constexpr int kFfDense = 10;  // atoms up to which every block is taken
+__global__ __launch_bounds__(NT) void ff_blocks_kernel(const double *__restrict__ dx,
+                                                       const int *__restrict__ N,
+                                                       const FfOrder *__restrict__ order, int ma,
+                                                       int rep, uint2 *__restrict__ blocks) {
+    __shared__ int row[MAXA], blk[3 * MAXA];
+    const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, n = clampi(N[m], 0, ma);
+    const int ld = 3 * ma, nc = 3 * n;
+    if (tid < MAXA) {
+        const int r = order[m].row[tid], c = order[m].col[tid];
+        if (r >= 0) row[r] = tid >> 2;
+        if (c >= 0)
+            for (int d = 0; d < 3; ++d) blk[3 * c + d] = (3 * tid + d) >> 4;
+    }
+    __syncthreads();
+    const int c0 = min(lane, max(nc - 1, 0)), c1 = min(lane + 64, max(nc - 1, 0));
+    // 32-bit words and shifts: a 64-bit shift by a VGPR has been seen to use another register's
+    // value where the amount is in the last VGPR that the kernel allocates
+    const int y0 = n ? blk[c0] : 0, y1 = n ? blk[c1] : 0;
+    const int f1 = min(rep, (int)(blockIdx.y + 1) * kBlkRun);
+    for (int f = blockIdx.y * kBlkRun + (tid >> 6); f < f1; f += NT / 64) {
+        unsigned w0 = 0, w1 = 0, bad = 0;  // of the lane's columns; any value not finite
+        const double *p = dx + ((size_t)m * ma * rep + f) * ld;
+        for (int i0 = 0; i0 < n; i0 += 4) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const double *pi = p + (size_t)min(i0 + u, n - 1) * rep * ld;
+                v[u] = pi[c0];
+                v[u + 4] = pi[c1];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned bit = 1u << row[min(i0 + u, n - 1)];
+                w0 |= v[u] != 0.0 ? bit : 0u;
+                w1 |= v[u + 4] != 0.0 ? bit : 0u;
+                bad |= (!(fabs(v[u]) <= DBL_MAX) | !(fabs(v[u + 4]) <= DBL_MAX)) ? 1u : 0u;
+            }
+        }
+        w0 <<= 8 * (y0 & 3);
+        w1 <<= 8 * (y1 & 3);
+        unsigned lo = (y0 < 4 ? w0 : 0u) | (y1 < 4 ? w1 : 0u);
+        unsigned hi = (y0 < 4 ? 0u : w0) | (y1 < 4 ? 0u : w1) | bad << 31;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            lo |= (unsigned)__shfl_xor((int)lo, o, 64);
+            hi |= (unsigned)__shfl_xor((int)hi, o, 64);
+        }
+        if (lane == 0) blocks[(size_t)m * rep + f] = make_uint2(lo, hi);
+    }
+}
+
+// What a pair's work-group keeps in LDS.
+struct FfPair {
+    double Cm[32 * 33];                  // C by rows of a and b
+    int ra[MAXA], rb[MAXA];              // atom in a row (a valid one where there is none)
+    int pa[3 * MAXA], pb[3 * MAXA];      // force column of the molecule at place c
+    int cg[8];                           // bit s: row groups (this, s) of a and b share a label
+    int full;                            // C holds values that are not finite
+};
+
+__device__ inline unsigned long long ff_uniform(uint2 v) {
+    return (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)v.y) << 32 |
+           (unsigned)__builtin_amdgcn_readfirstlane((int)v.x);
+}
+
+// fn(0) ... fn(N - 1), each with its index as a constant: the operands below then stay in
+// registers of their own (left to loop unrolling, conditional MFMAs move them about).
+template <int N, int I = 0, typename Fn>
+__device__ __forceinline__ void static_for(Fn &&fn) {
+    if constexpr (I < N) {
+        fn(std::integral_constant<int, I>{});
+        static_for<N, I + 1>(fn);
+    }
+}
+
+// One feature's operands: J_b (column operands), T, the row groups of T that hold anything
+// and the block word of J_a.
+template <int NK, int NX>
+struct FfOperand {
+    double jb[NK];
+    v4d t[NX];
+    int rows;
+    unsigned long long blocks;
+};
+
 template <int MODE, int NK, int NP>
 __device__ __forceinline__ void ff_pair(const DerivArgs &A, int a, int b, int na, int nb,
-                                        const double *Cm, double *Jbuf, int np,
+                                        const FfPair &L, double *Jbuf, int np,
                                         const double *mc, const double *slot, int f0, int fe,
                                         double *part) {
+    typedef unsigned long long u64;
     constexpr int NX = (NK + 3) / 4;         // 16-row fragments of C / T (atoms of a)
     constexpr int FFR = 4 * NK, FFP = 16 * NP;  // staged J_a feature: rows x columns
     constexpr int NEL = FFR * FFP, NST = (NEL + NT - 1) / NT;  // elements, per thread
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, col = lane & 15,
-              kr = lane >> 4;
+    constexpr int ALL = (1 << NK) - 1;
+    constexpr bool SPARSE = NP >= 3;  // more than kFfDense atoms
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kr = lane >> 4,
+              wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rep = A.rep, nca = 3 * na, ncb = 3 * nb;
     const int nqb = (ncb + 15) >> 4;
     const int lda = 3 * A.ma1, ldb = 3 * A.ma2;
@@ -648,90 +766,116 @@ __device__ __forceinline__ void ff_pair(const DerivArgs &A, int a, int b, int na
 #pragma unroll
     for (int u = 0; u < NST; ++u) {
         const int e = min(tid + NT * u, NEL - 1), r = e / FFP, c = e % FFP;
-        soff[u] = min(r, na - 1) * rep * lda + min(c, nca - 1);
+        soff[u] = L.ra[r] * rep * lda + L.pa[min(c, nca - 1)];
     }
-    // column-operand rows 4s + kr of b: affine in s except the last k-step (clamped)
-    const int sb = 4 * rep * ldb, rb0 = kr * rep * ldb;
-    const int rbL = min(4 * (NK - 1) + kr, nb - 1) * rep * ldb;
+    int rb[NK], cg[NK], cx[NX], full = __builtin_amdgcn_readfirstlane(L.full);
+#pragma unroll
+    for (int s = 0; s < NK; ++s) rb[s] = L.rb[4 * s + kr] * rep * ldb;
+#pragma unroll
+    for (int x = 0; x < NX; ++x) cx[x] = 0;
+#pragma unroll
+    for (int s = 0; s < NK; ++s) {
+        cg[s] = __builtin_amdgcn_readfirstlane(L.cg[s]);
+        cx[s / 4] |= cg[s];
+    }
+    double c[NX * NK];  // A operands of T
+    static_for<NX * NK>([&](auto e) { c[e] = L.Cm[(16 * (e / NK) + col) * 33 + 4 * (e % NK) + kr]; });
+    const uint2 *wa = A.blocks1 + (size_t)a * rep, *wb = A.blocks2 + (size_t)b * rep;
     Out<MODE> out{A.out, A.ld, a, b, A.offs1[a], A.offs2[b], A.ebase1, A.ebase2};
     // rounds of four q-blocks (more than one only past 21 atoms of b)
     for (int qr = 0; 4 * qr < nqb; ++qr) {
     const int qb = 4 * qr + wv;
     const bool busy = qb < nqb;
-    const int q = min(16 * qb + col, ncb - 1);
+    const int q = L.pb[min(16 * qb + col, ncb - 1)];
 
     v4d acc[NP];
 #pragma unroll
     for (int y = 0; y < NP; ++y) acc[y] = (v4d){0.0, 0.0, 0.0, 0.0};
-    double st[NST], jb[2][NK];
-    v4d tt[2][NX];
-#define KF_FF_STAGE_LOAD(F)                                                                   \
-    do {                                                                                      \
-        const double *pa_ = dxa + (size_t)(F) * lda;                                          \
-        _Pragma("unroll") for (int u = 0; u < NST; ++u) st[u] = pa_[soff[u]];                 \
-    } while (0)
-#define KF_FF_STAGE_STORE(BUF)                                                                \
-    do {                                                                                      \
-        _Pragma("unroll") for (int u = 0; u < NST; ++u)                                       \
-            if (NEL % NT == 0 || tid + NT * u < NEL) (BUF)[tid + NT * u] = st[u];             \
-    } while (0)
-#define KF_FF_LOAD_B(S, F)                                                                    \
-    do {                                                                                      \
-        const double *pb_ = dxb + (size_t)(F) * ldb + q;                                      \
-        _Pragma("unroll") for (int s = 0; s < NK; ++s)                                        \
-            jb[S][s] = pb_[s < NK - 1 ? rb0 + s * sb : rbL];                                  \
-    } while (0)
-#define KF_FF_T(S)                                                                            \
-    do {                                                                                      \
-        _Pragma("unroll") for (int x = 0; x < NX; ++x) tt[S][x] = (v4d){0.0, 0.0, 0.0, 0.0};  \
-        _Pragma("unroll") for (int s = 0; s < NK; ++s)                                        \
-            _Pragma("unroll") for (int x = 0; x < NX; ++x)                                    \
-                tt[S][x] = __builtin_amdgcn_mfma_f64_16x16x4f64(                              \
-                    Cm[(16 * x + col) * 33 + 4 * s + kr], jb[S][s], tt[S][x], 0, 0, 0);       \
-    } while (0)
-#define KF_FF_MAIN(S, BUF)                                                                    \
-    do {                                                                                      \
-        _Pragma("unroll") for (int s = 0; s < NK; ++s)                                        \
-            _Pragma("unroll") for (int y = 0; y < NP; ++y)                                    \
-                acc[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(                                \
-                    (BUF)[(4 * s + kr) * FFP + 16 * y + col], tt[S][s >> 2][s & 3], acc[y],   \
-                    0, 0, 0);                                                                 \
-    } while (0)
+    double st[NST];
+    FfOperand<NK, NX> o0, o1;
+    uint2 la, lb;  // the words of the next feature
+    auto stage_load = [&](int f) {
+        const double *p = dxa + (size_t)f * lda;
+        static_for<NST>([&](auto u) { st[u] = p[soff[u]]; });
+    };
+    auto stage_store = [&](double *buf) {
+        static_for<NST>([&](auto u) {
+            if (NEL % NT == 0 || tid + NT * u < NEL) buf[tid + NT * u] = st[u];
+        });
+    };
+    // the words of a feature and its column operands
+    auto load_b = [&](FfOperand<NK, NX> &o, int f) {
+        if (SPARSE) la = wa[f], lb = wb[f];
+        const double *p = dxb + (size_t)f * ldb + q;
+        static_for<NK>([&](auto s) { o.jb[s] = p[rb[s]]; });
+    };
+    // T of the feature whose words were loaded last
+    auto form_t = [&](FfOperand<NK, NX> &o) {
+        const u64 a_ = SPARSE ? ff_uniform(la) : 0, b_ = SPARSE ? ff_uniform(lb) : 0;
+        const bool all = !SPARSE || (full | (((a_ | b_) >> 63) != 0));
+        const int m = all ? ALL : int(b_ >> (8 * qb)) & ALL;
+        o.blocks = all ? ~0ull : a_;
+        int act = all ? ALL : 0;
+        static_for<NK>([&](auto s) { act |= (cg[s] & m) ? 1 << s : 0; });
+        o.rows = act;
+        static_for<NX>([&](auto x) {
+            const int mx = all ? ALL : cx[x] & m;
+            v4d t = {0.0, 0.0, 0.0, 0.0};
+            static_for<NK>([&](auto s) {
+                if (!SPARSE || (mx >> s & 1))
+                    t = __builtin_amdgcn_mfma_f64_16x16x4f64(c[x * NK + s], o.jb[s], t, 0, 0, 0);
+            });
+            o.t[x] = t;
+        });
+    };
+    // J_a's rows of a group are read from LDS while the group before is multiplied
+    double av[2][NP];
+    auto load_a = [&](const double *buf, auto s) {
+        static_for<NP>([&](auto y) { av[s % 2][y] = buf[(4 * s + kr) * FFP + 16 * y + col]; });
+    };
+    auto add_product = [&](const FfOperand<NK, NX> &o, const double *buf) {
+        static_for<NK>([&](auto s) {
+            if constexpr (s + 1 < NK) load_a(buf, std::integral_constant<int, s + 1>{});
+            if (!SPARSE || __builtin_expect(o.rows >> s & 1, 1))
+                static_for<NP>([&](auto y) {
+                    if (!SPARSE || (o.blocks >> (8 * y + s) & 1))
+                        acc[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            av[s % 2][y], o.t[s / 4][s % 4], acc[y], 0, 0, 0);
+                });
+        });
+    };
     // prologue: J_a(0) in buffer 0, J_a(1) in registers, T(0), J_b(1)
     double *const J0 = Jbuf, *const J1 = Jbuf + NEL;
-    KF_FF_STAGE_LOAD(f0);
-    KF_FF_STAGE_STORE(J0);
-    KF_FF_STAGE_LOAD(min(f0 + 1, fe - 1));
-    KF_FF_LOAD_B(0, f0);
-    KF_FF_T(0);
-    KF_FF_LOAD_B(1, min(f0 + 1, fe - 1));
+    stage_load(f0);
+    stage_store(J0);
+    stage_load(min(f0 + 1, fe - 1));
+    load_b(o0, f0);
+    form_t(o0);
+    load_b(o1, min(f0 + 1, fe - 1));
     __syncthreads();
     for (int f = f0; f < fe; f += 2) {
-        // feature f: buffer J0, T slot 0; prepare f+1 (J1, T slot 1) and loads for f+2
-        KF_FF_STAGE_STORE(J1);
-        KF_FF_STAGE_LOAD(min(f + 2, fe - 1));
+        // feature f: buffer J0, T in o0; prepare f+1 (J1, T in o1) and loads for f+2
+        stage_store(J1);
+        stage_load(min(f + 2, fe - 1));
         if (busy) {
-            KF_FF_T(1);
-            KF_FF_MAIN(0, J0);
+            load_a(J0, std::integral_constant<int, 0>{});
+            add_product(o0, J0);
+            form_t(o1);
         }
-        KF_FF_LOAD_B(0, min(f + 2, fe - 1));
+        load_b(o0, min(f + 2, fe - 1));
         __syncthreads();
         if (f + 1 >= fe) break;
-        // feature f+1: buffer J1, T slot 1; prepare f+2 (J0, T slot 0) and loads for f+3
-        KF_FF_STAGE_STORE(J0);
-        KF_FF_STAGE_LOAD(min(f + 3, fe - 1));
+        // feature f+1: buffer J1, T in o1; prepare f+2 (J0, T in o0) and loads for f+3
+        stage_store(J0);
+        stage_load(min(f + 3, fe - 1));
         if (busy) {
-            KF_FF_T(0);
-            KF_FF_MAIN(1, J1);
+            load_a(J1, std::integral_constant<int, 0>{});
+            add_product(o1, J1);
+            form_t(o0);
         }
-        KF_FF_LOAD_B(1, min(f + 3, fe - 1));
+        load_b(o1, min(f + 3, fe - 1));
         __syncthreads();
     }
-#undef KF_FF_STAGE_LOAD
-#undef KF_FF_STAGE_STORE
-#undef KF_FF_LOAD_B
-#undef KF_FF_T
-#undef KF_FF_MAIN
     if (!busy) continue;
     // rank-1 part (of the first run of features): acc -= sum_m (w_m v_m) u_m^T, K = matched pairs
     if (f0 == 0) {
@@ -744,12 +888,12 @@ __device__ __forceinline__ void ff_pair(const DerivArgs &A, int a, int b, int na
             const bool ok = m < np;
             const int mm = min(m, np - 1);
             const double w = ok ? -mc[mm] * A.inv_s2 : 0.0;  // -e/s^4
-            const int qq = 16 * qb + col;
-            const double u = U[(size_t)mm * A.ldu + min(qq, ncb - 1)];
-            const double bv = (ok & (qq < ncb)) ? u : 0.0;
+            const double u = U[(size_t)mm * A.ldu + q];
+            const double bv = (ok & (16 * qb + col < ncb)) ? u : 0.0;
             double vv[NP];
 #pragma unroll
-            for (int y = 0; y < NP; ++y) vv[y] = V[(size_t)mm * A.ldv + min(16 * y + col, nca - 1)];
+            for (int y = 0; y < NP; ++y)
+                vv[y] = V[(size_t)mm * A.ldv + L.pa[min(16 * y + col, nca - 1)]];
 #pragma unroll
             for (int y = 0; y < NP; ++y) {
                 const int p = 16 * y + col;
@@ -765,8 +909,8 @@ __device__ __forceinline__ void ff_pair(const DerivArgs &A, int a, int b, int na
         for (int v = 0; v < 4; ++v) {
             const int r = 16 * y + mfma16_row_f64(lane, v);
             if (r < nca && tc < ncb) {
-                if (part) part[(size_t)r * A.ldu + tc] = acc[y][v];
-                else out.ff(r, tc, acc[y][v]);
+                if (part) part[(size_t)L.pa[r] * A.ldu + q] = acc[y][v];
+                else out.ff(L.pa[r], q, acc[y][v]);
             }
         }
     }
@@ -792,20 +936,35 @@ inline size_t ff_lds_bytes(int ma1, int ma2) {
 template <int MODE>
 __global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0,
                                                          double *__restrict__ parts) {
-    __shared__ double Cm[32 * 33];
+    __shared__ FfPair L;
     extern __shared__ double Jbuf[];  // two staged J_a features of the largest bucket
-    __shared__ int qa[MAXA], qb_[MAXA], ist[MAXA + 1], mi[MAXM], mj[MAXM];
+    __shared__ int qa[MAXA], qb_[MAXA], ia[MAXA], ib[MAXA], ist[MAXA + 1], mi[MAXM], mj[MAXM];
     __shared__ double mc[MAXM];
     __shared__ int s_np;
     const int tid = threadIdx.x;
     const int t = pair0 + pair_slot();
     const int a = A.pairs[t].x, b = A.pairs[t].y;
     const int na = clampi(A.n1[a], 0, A.ma1), nb = clampi(A.n2[b], 0, A.ma2);
+    const int mx = na > nb ? na : nb;
+    const bool sparse = mx > kFfDense;
     // a molecule without atoms still gets its zero EE / FE / EF entries written
     const double *slot = A.slot + (size_t)(t - pair0) * A.slot_len;
     if (tid < na) qa[tid] = A.q1[(size_t)a * A.ma1 + tid];
     if (tid < nb) qb_[tid] = A.q2[(size_t)b * A.ma2 + tid];
-    for (int e = tid; e < 32 * 33; e += NT) Cm[e] = 0.0;
+    for (int e = tid; e < 32 * 33; e += NT) L.Cm[e] = 0.0;
+    if (tid < 8) L.cg[tid] = 0;
+    if (tid == 0) L.full = 0;
+    if (tid >= 64 && tid < 64 + 2 * MAXA) {  // the orders of both molecules
+        const int r = (tid - 64) % MAXA, second = (tid - 64) / MAXA;
+        int at = r < (second ? nb : na) ? r : -1, c = at;
+        if (sparse) {
+            const FfOrder &o = second ? A.order2[b] : A.order1[a];
+            at = o.row[r], c = o.col[r];
+        }
+        (second ? L.rb : L.ra)[r] = max(at, 0);
+        if (at >= 0) (second ? ib : ia)[at] = r;
+        for (int d = 0; d < 3; ++d) (second ? L.pb : L.pa)[3 * r + d] = 3 * max(c, 0) + d;
+    }
     __syncthreads();
     if (tid == 0) {  // matched list, i-major: the order of the slot entries
         int cnt = 0;
@@ -822,7 +981,12 @@ __global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0,
     for (int m = tid; m < np; m += NT) {
         const double c = slot[m] * A.inv_s2;
         mc[m] = c;
-        Cm[mi[m] * 33 + mj[m]] = c;
+        const int r = ia[mi[m]], k = ib[mj[m]];
+        L.Cm[r * 33 + k] = c;
+        if (sparse) {
+            atomicOr(&L.cg[r >> 2], 1 << (k >> 2));
+            if (!(fabs(c) <= DBL_MAX)) L.full = 1;
+        }
     }
     __syncthreads();
     if (blockIdx.y == 0) {
@@ -852,13 +1016,12 @@ __global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0,
     double *part = gridDim.y > 1 ? parts + ((size_t)(t - pair0) * gridDim.y + blockIdx.y) *
                                                A.ldv * A.ldu
                                  : nullptr;
-    const int mx = na > nb ? na : nb;
-    if (mx <= 5) ff_pair<MODE, 2, 1>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
-    else if (mx <= 10) ff_pair<MODE, 3, 2>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
-    else if (mx <= 16) ff_pair<MODE, 4, 3>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
-    else if (mx <= 21) ff_pair<MODE, 6, 4>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
-    else if (mx <= 24) ff_pair<MODE, 6, 5>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
-    else ff_pair<MODE, 8, 6>(A, a, b, na, nb, Cm, Jbuf, np, mc, slot, f0, fe, part);
+    if (mx <= 5) ff_pair<MODE, 2, 1>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+    else if (mx <= 10) ff_pair<MODE, 3, 2>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+    else if (mx <= 16) ff_pair<MODE, 4, 3>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+    else if (mx <= 21) ff_pair<MODE, 6, 4>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+    else if (mx <= 24) ff_pair<MODE, 6, 5>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+    else ff_pair<MODE, 8, 6>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
 }
 
 // FF of a pair from the parts of its runs of features, in order.
@@ -910,6 +1073,42 @@ void side_meta(const std::vector<int> &hQ, const std::vector<int> &hN, int nm, i
     s.naq = acc;
 }
 
+// Atoms by label: labels start at multiples of 4 rows where the 4 * nk rows of the molecule's
+// bucket allow it, and 16 rows are filled with labels that fit whole as far as possible.
+FfOrder ff_order(const int *q, int n) {
+    FfOrder o;
+    std::fill(o.row, o.row + MAXA, (signed char)-1);
+    std::fill(o.col, o.col + MAXA, (signed char)-1);
+    int nk, np;
+    ff_bucket(n, nk, np);
+    std::vector<std::vector<int>> sets;  // atoms of each label, the largest set first
+    for (int i = 0; i < n; ++i) {
+        size_t k = 0;
+        while (k < sets.size() && q[sets[k][0]] != q[i]) ++k;
+        if (k == sets.size()) sets.emplace_back();
+        sets[k].push_back(i);
+    }
+    std::stable_sort(sets.begin(), sets.end(), [](const std::vector<int> &u, const std::vector<int> &v) {
+        return u.size() > v.size();
+    });
+    int groups = 0, r = 0, c = 0;
+    for (const auto &s : sets) groups += ((int)s.size() + 3) / 4;
+    const bool aligned = groups <= nk;
+    while (!sets.empty()) {
+        size_t k = 0;
+        if (aligned)
+            while (k < sets.size() && (int)(sets[k].size() + 3) / 4 > 4 - r / 4 % 4) ++k;
+        if (k == sets.size()) k = 0;
+        for (int at : sets[k]) {
+            o.row[r++] = (signed char)at;
+            o.col[c++] = (signed char)at;
+        }
+        if (aligned) r = (r + 3) / 4 * 4;
+        sets.erase(sets.begin() + k);
+    }
+    return o;
+}
+
 template <int MODE>
 int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1,
                  const SideMeta &s2, int nlab, hipStream_t stream) {
@@ -918,10 +1117,20 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
     // offsets + pair list to the device (one staging copy)
     const size_t n_off = s1.offs.size() + s2.offs.size();
     const size_t pair_off = (sizeof(int) * n_off + 15) / 16 * 16;
-    const size_t bytes = pair_off + sizeof(int2) * npairs;
+    const bool one_set = is_symm(MODE) || MODE == M_DIAG_BLOCKS;
+    const size_t order_off = pair_off + sizeof(int2) * npairs, nm1 = s1.n.size(),
+                 nm2 = one_set ? 0 : s2.n.size();
+    const size_t bytes = order_off + (has_ff(MODE) ? sizeof(FfOrder) * (nm1 + nm2) : 0);
     char *dev = static_cast<char *>(workspace(WS_PLAN, bytes, stream));
     char *stage = static_cast<char *>(host_staging(WS_PLAN, bytes));
     KF_REQUIRE(dev && stage, KF_ERR_NOMEM, "workspace allocation failed (%zu B)", bytes);
+    if (has_ff(MODE)) {
+        FfOrder *o = reinterpret_cast<FfOrder *>(stage + order_off);
+        for (size_t m = 0; m < nm1; ++m)
+            o[m] = ff_order(s1.q.data() + m * A.ma1, (s1.offs[m + 1] - s1.offs[m]) / 3);
+        for (size_t m = 0; m < nm2; ++m)
+            o[nm1 + m] = ff_order(s2.q.data() + m * A.ma2, (s2.offs[m + 1] - s2.offs[m]) / 3);
+    }
     std::copy(s1.offs.begin(), s1.offs.end(), reinterpret_cast<int *>(stage));
     std::copy(s2.offs.begin(), s2.offs.end(), reinterpret_cast<int *>(stage) + s1.offs.size());
     std::copy(pairs.begin(), pairs.end(), reinterpret_cast<int2 *>(stage + pair_off));
@@ -932,6 +1141,23 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
 
     size_t batch = npairs;
     if (has_ff(MODE)) {
+        // which blocks of the Jacobians are not zero
+        const bool sparse = std::max(A.ma1, A.ma2) > kFfDense;
+        A.order1 = reinterpret_cast<const FfOrder *>(dev + order_off);
+        A.order2 = A.order1 + (one_set ? 0 : nm1);
+        uint2 *w = static_cast<uint2 *>(
+            workspace(WS_PLAN2, sizeof(uint2) * (nm1 + nm2) * A.rep, stream));
+        KF_REQUIRE(w, KF_ERR_NOMEM, "workspace allocation failed");
+        A.blocks1 = w;
+        A.blocks2 = one_set ? w : w + nm1 * A.rep;
+        const unsigned nrun = (A.rep + kBlkRun - 1) / kBlkRun;
+        for (int set = 0; sparse && set < (one_set ? 1 : 2); ++set) {
+            hipLaunchKernelGGL(ff_blocks_kernel, dim3(set ? nm2 : nm1, nrun), dim3(NT), 0, stream,
+                               set ? A.dx2 : A.dx1, set ? A.n2 : A.n1,
+                               set ? A.order2 : A.order1, set ? A.ma2 : A.ma1, A.rep,
+                               w + (set ? nm1 * A.rep : 0));
+            KF_HIP_TRY(hipGetLastError());
+        }
         // slot layout and the largest matched count over the pairs
         int maxm = 1;
         for (const int2 &p : pairs) {

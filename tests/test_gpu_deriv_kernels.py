@@ -276,6 +276,39 @@ def test_feature_runs(lk, nm, ma, rep):
     assert rel_err(got, oracle.hessian(X[:m], dX[:m], X, dX, Q[:m], Q, N[:m], N, 2.1)) < TOL
 
 
+# Jacobians that are zero in whole blocks, as a descriptor's are for atoms a feature does not
+# depend on: molecules of one to 32 atoms in every bucket, labels that start at multiples of 4
+# rows and ones that cannot (too many of them), last force columns alone in their block, small
+# values that decide whether a block counts, and a feature with a value that is not finite
+@pytest.mark.parametrize("ma,nlab", [(1, 1), (5, 2), (10, 3), (16, 3), (21, 3), (22, 5), (24, 9),
+                                     (32, 4)])
+def test_zero_blocks(lk, ma, nlab):
+    nm, rep = 6, 70
+    X, dX, Q, N = rand_set(nm, ma, rep, nlab, 50 + ma, max(1, ma - 3))
+    rng = np.random.default_rng(ma)
+    lab = rng.integers(0, nlab + 1, (rep, 2))  # a feature's labels (0: none)
+    for m in range(nm):
+        on = (lab[:, :1] == Q[m]) | (lab[:, 1:] == Q[m])  # (rep, atom)
+        keep = on[None] | np.eye(ma, dtype=bool)[:, None]  # and the centre itself
+        dX[m] *= np.repeat(keep, 3, axis=2) * np.where(rng.random((ma, rep, 1)) < 0.3, 1e-9, 1.0)
+        dX[m, N[m]:] = 0.0
+        dX[m, :, :, 3 * N[m]:] = 0.0
+    a = lk.kernel_gaussian_hessian_symm(X, dX, Q, N, 1.7)
+    assert rel_err(a, oracle.hessian_symm(X, dX, Q, N, 1.7)) < TOL
+    for _ in range(10):
+        np.testing.assert_array_equal(lk.kernel_gaussian_hessian_symm(X, dX, Q, N, 1.7), a)
+    got = lk.kernel_gaussian_full(X[:2], dX[:2], X[1:], dX[1:], Q[:2], Q[1:], N[:2], N[1:], 1.7)
+    assert rel_err(got, oracle.full(X[:2], dX[:2], X[1:], dX[1:], Q[:2], Q[1:], N[:2], N[1:],
+                                    1.7)) < TOL
+    dX[2, 0, 7, 3 * N[2] - 1] = np.inf
+    got = lk.kernel_gaussian_hessian_symm(X, dX, Q, N, 1.7)
+    col = int(3 * N[:3].sum()) - 1
+    assert not np.isfinite(got[col, col])
+    far = np.ones(len(got), bool)
+    far[3 * N[:2].sum(): 3 * N[:3].sum()] = False
+    np.testing.assert_array_equal(got[np.ix_(far, far)], a[np.ix_(far, far)])
+
+
 @pytest.mark.parametrize("nm,ma,rep", [(1, 2, 5), (70, 2, 300), (3, 30, 97), (40, 5, 17)])
 def test_unused_columns_found_anywhere(lk, nm, ma, rep):
     """A column used by a single entry -- of the last live atom, in the Jacobian only, or of a
