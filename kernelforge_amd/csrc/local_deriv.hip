@@ -20,8 +20,9 @@
 //    Jacobian forms).  Writes EE / EF / FE, and e_m, v_m, u_m to a per-pair slot.
 //  * deriv_ff_kernel (FP64 MFMA 16x16x4): per feature f, T_f = C J_b[:,f,:] and
 //    FF += J_a[:,f,:]^T T_f, both on MFMA with operands streamed from HBM into
-//    registers (T_f's accumulators are the B operands of the second product), then
-//    the rank-1 sum as a second MFMA pass over the slot; writes FF.
+//    registers (T_f's accumulators are the B operands of the second product; blocks that
+//    ff_blocks_kernel found zero left out), then the rank-1 sum as a second MFMA pass over
+//    the slot; writes FF.
 // Every output entry belongs to exactly one molecule pair, so no atomics are used
 // and results are deterministic.
 #include <algorithm>
@@ -1252,7 +1253,7 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
             KF_HIP_TRY(hipGetLastError());
             // Few pairs: each pair's features in several runs (of 32 and more), so that there
             // are about 2,048 work-groups, four per slot of the GPU (512): 703 pairs of mixed
-            // molecules of 5-23 atoms 3.5 ms, 4.5 with one run each
+            // molecules of 5-23 atoms 3.5 ms, 4.5 with one run each (every block taken)
             int runs = std::max(1, std::min((int)(2048 / nb), A.rep / 32));
             const int run = (A.rep + runs - 1) / runs;
             runs = (A.rep + run - 1) / run;  // none of them empty
