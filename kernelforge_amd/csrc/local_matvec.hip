@@ -662,8 +662,10 @@ void mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, 
     close();
     L.q_rows = q0;
     L.t_rows = r2;
-    // runs of features per query row in the back-projection: 2,048 work-groups, at most 16
-    L.parts = std::max(1, std::min({16, 2048 / std::max(1, q0), (rep + 31) / 32}));
+    // runs of features per query row in the back-projection: 2,048 work-groups, at most 16;
+    // a run is held in LDS, 4,096 features (32 KB) at most
+    L.parts = std::max({1, (rep + 4095) / 4096,
+                        std::min({16, 2048 / std::max(1, q0), (rep + 31) / 32})});
 }
 
 MvDev mv_place(const MvLayout &L, char *meta, double *train, double *query, double *acc) {

@@ -243,6 +243,20 @@ def test_matvec_float32_operands(lk):
     np.testing.assert_array_equal(out[0][1], out[1][1])
 
 
+def test_matvec_wide_descriptors(lk):
+    """More features than LDS holds for one query row, and query rows enough for one run."""
+    nm, rep = 1040, 21000
+    rng = np.random.default_rng(4)
+    X1 = np.tile(rng.standard_normal((nm, 1, 300)) * 0.02, 70)
+    dX1 = np.tile(rng.standard_normal((nm, 1, 300, 3)) * 0.2, (70, 1))
+    X2, ad = rng.standard_normal((2, 1, rep)) * 0.02, rng.standard_normal((2, 1, rep)) * 0.02
+    one, two = np.ones(nm, np.int32), np.ones(2, np.int32)
+    args = (X1, dX1, X2, ad, np.ones(2), one[:, None], two[:, None], one, two, 2.0)
+    E, F = lk.kernel_gaussian_local_full_matvec(*args)
+    Eo, Fo = oracle.full_matvec(*args)
+    assert rel_err(E, Eo) < TOL and rel_err(F, Fo) < TOL
+
+
 def test_matvec_conformers_symmetric(lk):
     """Training-set operator on C9H8O4 conformers equals the RFP E+F kernel times alpha."""
     from kernelforge_amd import synthetic
