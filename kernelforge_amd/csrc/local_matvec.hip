@@ -468,6 +468,20 @@ __global__ __launch_bounds__(NT) void backproj_kernel(const MvSeg *__restrict__ 
     }
 }
 
+// erow and the Fat rows of the atoms in idx are zero: atoms whose label the training side
+// lacks, which the products leave out (0 times what they hold would make NaN of a value that
+// is not finite).
+__global__ __launch_bounds__(64) void zero_rows_kernel(const int *__restrict__ idx, int ld,
+                                                       int parts, int natoms,
+                                                       double *__restrict__ erow,
+                                                       double *__restrict__ Fat) {
+    const int src = idx[blockIdx.x];
+    if (threadIdx.x == 0) erow[src] = 0.0;
+    if (!Fat) return;
+    for (int t = threadIdx.x; t < parts * ld; t += 64)
+        Fat[((size_t)(t / ld) * natoms + src) * ld + t % ld] = 0.0;
+}
+
 // E[a] = sum_i erow[a*ma+i]; F[offs[a] + c] = sum over the parts and the atoms of
 // Fat[part][a*ma+i, c] (fixed order).  Atom counts come from the force offsets.  The
 // (part, atom) rows are dealt over the groups of nc threads: one molecule of 21 atoms in 16
@@ -520,13 +534,14 @@ struct MvLayout {
     int nm1 = 0, ma1 = 0, rep = 0, nf = 0, nfp = 0, parts = 1;
     int q_rows = 0, t_rows = 0;             // packed rows, padding included
     std::vector<int> offs, src1, src2, inv;  // force offsets, packed rows' sources, columns
+    std::vector<int> src0;                   // query atoms without a partner
     std::vector<MvSeg> segs;
     std::vector<MvRound> rounds;
     size_t T_len = 0, G_len = 0, e_len = 0;  // per round, the largest
     // one device block of ints: segments first (8-byte aligned), then the vectors
     size_t meta_bytes() const {
         return sizeof(MvSeg) * segs.size() +
-               sizeof(int) * (offs.size() + src1.size() + src2.size() + inv.size());
+               sizeof(int) * (offs.size() + src1.size() + src2.size() + inv.size() + src0.size());
     }
     void write_meta(char *p) const {
         auto put = [&](const void *v, size_t n) { std::copy((const char *)v, (const char *)v + n, p); p += n; };
@@ -535,6 +550,7 @@ struct MvLayout {
         put(src1.data(), sizeof(int) * src1.size());
         put(src2.data(), sizeof(int) * src2.size());
         put(inv.data(), sizeof(int) * inv.size());
+        put(src0.data(), sizeof(int) * src0.size());
     }
     size_t train_doubles() const { return (size_t)2 * t_rows * nfp + 3 * (size_t)t_rows; }
     size_t query_doubles() const {
@@ -548,7 +564,7 @@ struct MvLayout {
 // device addresses of a layout's pieces
 struct MvDev {
     const MvSeg *segs;
-    const int *offs, *src1, *src2, *inv;
+    const int *offs, *src1, *src2, *inv, *src0;
     double *P2, *n2, *rdot, *aE;
     double *Xq, *nq, *T, *G, *ep, *wp;
     double *erow, *Fat;
@@ -631,6 +647,10 @@ void mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, 
             b2 = m2[0];
             R2 = m2[nm2] - b2;
         }
+        if (R2 == 0) {
+            L.src0.insert(L.src0.end(), p1.src.begin() + m1[0], p1.src.begin() + m1[nm1]);
+            continue;
+        }
         if (R1 == 0) continue;
         const int R2p = round_up16(R2);
         L.src2.insert(L.src2.end(), p2.src.begin() + b2, p2.src.begin() + b2 + R2);
@@ -664,8 +684,9 @@ void mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, 
     L.t_rows = r2;
     // runs of features per query row in the back-projection: 2,048 work-groups, at most 16;
     // a run is held in LDS, 4,096 features (32 KB) at most
-    L.parts = std::max({1, (rep + 4095) / 4096,
-                        std::min({16, 2048 / std::max(1, q0), (rep + 31) / 32})});
+    L.parts = q0 == 0 ? 1
+                      : std::max({1, (rep + 4095) / 4096,
+                                  std::min({16, 2048 / q0, (rep + 31) / 32})});
 }
 
 MvDev mv_place(const MvLayout &L, char *meta, double *train, double *query, double *acc) {
@@ -675,6 +696,7 @@ MvDev mv_place(const MvLayout &L, char *meta, double *train, double *query, doub
     D.src1 = D.offs + L.offs.size();
     D.src2 = D.src1 + L.src1.size();
     D.inv = D.src2 + L.src2.size();
+    D.src0 = D.inv + L.inv.size();
     D.P2 = train;
     D.n2 = D.P2 + (size_t)2 * L.t_rows * L.nfp;
     D.rdot = D.n2 + L.t_rows;
@@ -697,6 +719,14 @@ int mv_pack_train(const MvLayout &L, const MvDev &D, const T *X2, const T *ad, c
     hipLaunchKernelGGL(pack_rows_kernel<T>, dim3((L.t_rows + 3) / 4), dim3(NT), 0, stream, X2, ad,
                        D.src2, L.t_rows, ma2, L.rep, D.inv, L.nf, L.nfp, D.segs,
                        (int)L.segs.size(), aE, D.P2, D.n2, D.rdot, D.aE);
+    KF_HIP_TRY(hipGetLastError());
+    return KF_OK;
+}
+
+int mv_zero_unmatched(const MvLayout &L, const MvDev &D, bool forces, hipStream_t stream) {
+    if (L.src0.empty()) return KF_OK;
+    hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)L.src0.size()), dim3(64), 0, stream, D.src0,
+                       3 * L.ma1, L.parts, L.nm1 * L.ma1, D.erow, forces ? D.Fat : (double *)nullptr);
     KF_HIP_TRY(hipGetLastError());
     return KF_OK;
 }
@@ -826,6 +856,7 @@ int matvec_impl(const T *X1, const T *dX1, const T *X2, const T *ad, const T *aE
     ScopedTimer timer(TM_MATVEC, stream);
     if ((rc = mv_pack_train(L, D, X2, ad, (mode & 4) ? aE : (const T *)nullptr, ma2, stream)))
         return rc;
+    if ((rc = mv_zero_unmatched(L, D, mode & 2, stream))) return rc;
     return mv_run(L, D, X1, dX1, sigma, E, F, mode, stream);
 }
 
@@ -890,6 +921,8 @@ int plan_create(const int *Q1, const int *N1, int nm1, int ma1, const double *X2
     KF_HIP_TRY(hipMemcpyAsync(P->meta, meta.data(), meta.size(), hipMemcpyHostToDevice, stream));
     P->dev = mv_place(L, P->meta, P->train, P->query, P->acc);
     if ((rc = mv_pack_train(L, P->dev, X2, ad, aE, ma2, stream))) return rc;
+    // (executions do not write these rows)
+    if ((rc = mv_zero_unmatched(L, P->dev, true, stream))) return rc;
     // the host vector above is released on return: wait for the copy that reads it
     KF_HIP_TRY(hipStreamSynchronize(stream));
     return KF_OK;

@@ -219,6 +219,60 @@ def test_matvec_variants(lk, case):
     assert rel_err(Ej, oracle.jacobian_t_matvec(X1, X2, ad, Q1, Q2, N1, N2, s)) < TOL
 
 
+def plan_matvec(X1, dX1, X2, ad, aE, Q1, Q2, N1, N2, s):
+    """(E, F) of a matvec plan on host arrays."""
+    import ctypes
+
+    from kernelforge_amd import capi
+
+    L, DA = capi.lib(), capi.DeviceArray
+    dq1, dn1, dq2, dn2 = (DA.from_numpy(a) for a in (Q1, N1, Q2, N2))
+    dx1, ddx1, dx2, dad, dae = (DA.from_numpy(a) for a in (X1, dX1, X2, ad, aE))
+    E, F = DA(len(X1)), DA(3 * int(np.clip(N1, 0, Q1.shape[1]).sum()))
+    h = ctypes.c_void_p()
+    capi.check(L.kf_matvec_plan_create(dq1.ptr, dn1.ptr, *Q1.shape, dx2.ptr, dad.ptr, dae.ptr,
+                                       dq2.ptr, dn2.ptr, *Q2.shape, X1.shape[2], s,
+                                       ctypes.byref(h), None), "plan")
+    try:
+        for _ in range(2):
+            capi.check(L.kf_matvec_plan_execute(h, dx1.ptr, ddx1.ptr, E.ptr, F.ptr, None), "plan")
+        capi.synchronize()
+        return E.numpy(), F.numpy()
+    finally:
+        L.kf_matvec_plan_destroy(h)
+
+
+def test_matvec_ignores_unmatched_atoms(lk):
+    """Query atoms whose label the training side lacks contribute nothing, whatever their
+    descriptors and Jacobians hold: all results are bit for bit those of finite ones."""
+    X1, dX1, Q1, N1 = rand_set(4, 5, 24, 2, 41, 5)
+    X2, _, Q2, N2 = rand_set(6, 4, 24, 2, 42, 1)
+    Q1[0, 2] = Q1[2, :] = 9
+    rng = np.random.default_rng(3)
+    ad, aE, s = rng.standard_normal(X2.shape), rng.standard_normal(6), 1.4
+    ad[np.arange(4)[None] >= N2[:, None]] = 0.0
+    Xb, dXb = X1.copy(), dX1.copy()
+    Xb[0, 2], Xb[2, 1, 3] = np.nan, np.inf
+    dXb[0, 2, 5], dXb[2] = np.inf, np.nan
+
+    def results(X, dX):
+        E, F = lk.kernel_gaussian_local_full_matvec(X, dX, X2, ad, aE, Q1, Q2, N1, N2, s)
+        return [E, F, lk.kernel_gaussian_local_hessian_matvec(X, dX, X2, ad, Q1, Q2, N1, N2, s),
+                lk.kernel_gaussian_local_jacobian_t_matvec(X, X2, ad, Q1, Q2, N1, N2, s),
+                *plan_matvec(X, dX, X2, ad, aE, Q1, Q2, N1, N2, s)]
+
+    want = results(X1, dX1)
+    Eo, Fo = oracle.full_matvec(X1, dX1, X2, ad, aE, Q1, Q2, N1, N2, s)
+    assert rel_err(want[0], Eo) < TOL and rel_err(want[1], Fo) < TOL
+    assert want[0][2] == 0.0 and not want[1][30:45].any()
+    for got, w in zip(results(Xb, dXb), want):
+        np.testing.assert_array_equal(got, w)
+    # no atom of the query set has a partner
+    Q1[:] = 9
+    for got in results(Xb, dXb):
+        assert not got.any()
+
+
 def test_matvec_float32_operands(lk):
     """float32 operands give what the same numbers held in FP64 give."""
     from kernelforge_amd import capi
