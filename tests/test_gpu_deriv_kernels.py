@@ -273,6 +273,28 @@ def test_matvec_ignores_unmatched_atoms(lk):
         assert not got.any()
 
 
+def test_matvec_far_and_non_finite_query_rows(lk):
+    """A query row so far away that its squared norm overflows has no neighbours: exactly as
+    if its label were absent.  An infinity in a column that the training side does not use
+    still shows as NaN."""
+    X1, dX1, Q1, N1 = rand_set(3, 4, 20, 2, 51, 4)
+    X2, _, Q2, N2 = rand_set(5, 4, 20, 2, 52, 4)
+    rng = np.random.default_rng(4)
+    ad, aE, s = rng.standard_normal(X2.shape), rng.standard_normal(5), 1.4
+    X2[..., 15:] = ad[..., 15:] = 0.0
+    Qa = Q1.copy()
+    Qa[1, 0] = Qa[2, 3] = 9
+    want = lk.kernel_gaussian_local_full_matvec(X1, dX1, X2, ad, aE, Qa, Q2, N1, N2, s)
+    X1[1, 0, 2], X1[2, 3, 17] = 1e160, -1e160
+    got = lk.kernel_gaussian_local_full_matvec(X1, dX1, X2, ad, aE, Q1, Q2, N1, N2, s)
+    for g, w in zip(got, want):
+        assert rel_err(g, w) < TOL
+    X1[1, 0, 2], X1[2, 3, 17] = 0.1, np.inf
+    E, F = lk.kernel_gaussian_local_full_matvec(X1, dX1, X2, ad, aE, Q1, Q2, N1, N2, s)
+    assert np.isnan(E[2]) and np.isnan(F[24:]).all()
+    assert np.isfinite(E[:2]).all() and np.isfinite(F[:24]).all()
+
+
 def test_matvec_float32_operands(lk):
     """float32 operands give what the same numbers held in FP64 give."""
     from kernelforge_amd import capi
