@@ -22,7 +22,7 @@ __global__ __launch_bounds__(256) void fill_int_kernel(int *p, int n, int v) {
 }
 
 // flag[f] = 1 when column f is non-zero in X or dX for some atom of the set.  A work-group
-// takes the columns of one atom (row0 + step * blockIdx.x of the set) that no earlier one
+// takes the columns of one atom (row step * (first + blockIdx.x) of the set) that no earlier one
 // has flagged: it reads the flags once, lists the others in LDS and streams their runs of
 // the Jacobian.  Launched first on a few atoms spread over the set, which find nearly every
 // used column, then on all: the second launch then reads little but the unused columns.
@@ -33,12 +33,12 @@ __global__ __launch_bounds__(256) void fill_int_kernel(int *p, int n, int v) {
 __global__ __launch_bounds__(256) void active_cols_kernel(const double *__restrict__ X,
                                                           const double *__restrict__ dX,
                                                           const int *__restrict__ N, int ma,
-                                                          int rep, int step,
+                                                          int rep, int step, size_t first,
                                                           int *__restrict__ flag) {
     extern __shared__ int lds[];  // unseen columns, then a flag for each
     __shared__ int count;
     const int tid = threadIdx.x;
-    const size_t row = (size_t)blockIdx.x * step;
+    const size_t row = (first + blockIdx.x) * step;
     const int a = (int)(row / ma), i = (int)(row - (size_t)a * ma);
     if (i >= clamp_n(N[a], ma)) return;
     int *list = lds, *seen = lds + rep;
@@ -84,15 +84,15 @@ int flag_columns(const double *X, const double *dX, const int *N, int nm, int ma
     if (rows == 0) return KF_OK;
     const size_t lds = 2 * sizeof(int) * rep;
     const int probe = (int)(rows / 64);  // an atom in so many, in the first launch
-    if (dX && probe > 1) {
-        hipLaunchKernelGGL(active_cols_kernel, dim3((unsigned)((rows + probe - 1) / probe)),
-                           dim3(256), lds, stream, X, dX, N, ma, rep, probe, flag);
-        KF_HIP_TRY(hipGetLastError());
-    }
-    hipLaunchKernelGGL(active_cols_kernel, dim3((unsigned)rows), dim3(256), lds, stream, X, dX, N,
-                       ma, rep, 1, flag);
-    KF_HIP_TRY(hipGetLastError());
-    return KF_OK;
+    auto scan = [&](int step) {
+        return for_groups((rows + step - 1) / step, [&](size_t first, unsigned n) {
+            hipLaunchKernelGGL(active_cols_kernel, dim3(n), dim3(256), lds, stream, X, dX, N, ma,
+                               rep, step, first, flag);
+        });
+    };
+    int rc = KF_OK;
+    if (dX && probe > 1) rc = scan(probe);
+    return rc ? rc : scan(1);
 }
 
 // Y[r][g][c] = X[r][cols[g]][c]: row r of rep runs of L doubles -> nf runs.  One
@@ -120,15 +120,15 @@ int gather_set(const double *X, const double *dX, int nm, int ma, int rep, const
     *Xc = buf;
     *dXc = dX ? buf + nx : nullptr;
     if (rows == 0) return KF_OK;
-    hipLaunchKernelGGL(gather_cols_kernel, dim3((unsigned)rows), dim3(256), 0, stream, X, rep, 1,
-                       cols, nf, buf);
-    KF_HIP_TRY(hipGetLastError());
-    if (dX) {
-        hipLaunchKernelGGL(gather_cols_kernel, dim3((unsigned)rows), dim3(256), 0, stream, dX, rep,
-                           (int)L, cols, nf, buf + nx);
-        KF_HIP_TRY(hipGetLastError());
-    }
-    return KF_OK;
+    auto gather = [&](const double *from, size_t run, double *to) {
+        return for_groups(rows, [&](size_t first, unsigned n) {
+            hipLaunchKernelGGL(gather_cols_kernel, dim3(n), dim3(256), 0, stream,
+                               from + first * rep * run, rep, (int)run, cols, nf,
+                               to + first * nf * run);
+        });
+    };
+    const int rc = gather(X, 1, buf);
+    return rc || !dX ? rc : gather(dX, L, buf + nx);
 }
 
 }  // namespace

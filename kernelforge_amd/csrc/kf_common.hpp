@@ -139,6 +139,18 @@ __host__ __device__ inline size_t rfp_upper(size_t n, size_t i, size_t j) {
 
 __host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
+// Launches over any number of work-groups of up to 512 threads: launch(first, count) for
+// one run of them after another.  A grid of 2^32 threads or more is cut off without an error.
+template <class Launch>
+int for_groups(size_t groups, Launch launch) {
+    constexpr size_t kMost = size_t(1) << 22;
+    for (size_t first = 0; first < groups; first += kMost) {
+        launch(first, (unsigned)(groups - first < kMost ? groups - first : kMost));
+        KF_HIP_TRY(hipGetLastError());
+    }
+    return KF_OK;
+}
+
 // Row of result register v held by `lane` in a 16x16x4 MFMA (column = lane & 15).
 // Both take A[i][k] from lane i + 16k and B[k][j] from lane j + 16k, but they place
 // the 16x16 result differently: the FP64 form interleaves the four registers across

@@ -1153,11 +1153,15 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
         A.blocks2 = one_set ? w : w + nm1 * A.rep;
         const unsigned nrun = (A.rep + kBlkRun - 1) / kBlkRun;
         for (int set = 0; sparse && set < (one_set ? 1 : 2); ++set) {
-            hipLaunchKernelGGL(ff_blocks_kernel, dim3(set ? nm2 : nm1, nrun), dim3(NT), 0, stream,
-                               set ? A.dx2 : A.dx1, set ? A.n2 : A.n1,
-                               set ? A.order2 : A.order1, set ? A.ma2 : A.ma1, A.rep,
-                               w + (set ? nm1 * A.rep : 0));
-            KF_HIP_TRY(hipGetLastError());
+            const int ma = set ? A.ma2 : A.ma1;
+            const int rc = for_groups(set ? nm2 : nm1, [&](size_t first, unsigned n) {
+                hipLaunchKernelGGL(ff_blocks_kernel, dim3(n, nrun), dim3(NT), 0, stream,
+                                   (set ? A.dx2 : A.dx1) + first * ma * A.rep * 3 * ma,
+                                   (set ? A.n2 : A.n1) + first,
+                                   (set ? A.order2 : A.order1) + first, ma, A.rep,
+                                   w + ((set ? nm1 : 0) + first) * A.rep);
+            });
+            if (rc) return rc;
         }
         // slot layout and the largest matched count over the pairs
         int maxm = 1;

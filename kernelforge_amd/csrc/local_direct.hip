@@ -323,11 +323,12 @@ __global__ __launch_bounds__(NT) void pair_sums_kernel(const DirectSeg *__restri
                                                        const double *__restrict__ Ex,
                                                        const int *__restrict__ mol1,
                                                        const int *__restrict__ mol2, int nseg,
-                                                       int nm1, int nm2,
+                                                       int nm1, int nm2, size_t first,
                                                        double *__restrict__ out) {
     constexpr bool SYMM = MODE != DIRECT_RECT;
     const int nbk = (nm2 + 31) / 32, sub = threadIdx.x & 7;
-    const int a = blockIdx.x / nbk, b = (blockIdx.x % nbk) * 32 + (threadIdx.x >> 3);
+    const size_t blk = first + blockIdx.x;
+    const int a = (int)(blk / nbk), b = (int)(blk % nbk) * 32 + (threadIdx.x >> 3);
     if (b >= nm2 || (SYMM && b < a)) return;
     double s = 0.0;
     for (int l = 0; l < nseg; ++l) {
@@ -430,16 +431,15 @@ int local_direct(int mode, const LocalPlan &p1, const double *X1, const LocalPla
         }
         KF_HIP_TRY(hipGetLastError());
     }
-    const unsigned grid = (unsigned)nm1 * (unsigned)ceil_div(nm2, 32);
     auto sums = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, stream, dseg, Ex, mol1, mol2, L, nm1, nm2,
-                           out);
+        return for_groups((size_t)nm1 * ceil_div(nm2, 32), [&](size_t first, unsigned n) {
+            hipLaunchKernelGGL(kern, dim3(n), dim3(NT), 0, stream, dseg, Ex, mol1, mol2, L, nm1,
+                               nm2, first, out);
+        });
     };
-    if (mode == DIRECT_SYMM_RFP) sums(pair_sums_kernel<DIRECT_SYMM_RFP>);
-    else if (mode == DIRECT_SYMM_DENSE) sums(pair_sums_kernel<DIRECT_SYMM_DENSE>);
-    else sums(pair_sums_kernel<DIRECT_RECT>);
-    KF_HIP_TRY(hipGetLastError());
-    return KF_OK;
+    if (mode == DIRECT_SYMM_RFP) return sums(pair_sums_kernel<DIRECT_SYMM_RFP>);
+    if (mode == DIRECT_SYMM_DENSE) return sums(pair_sums_kernel<DIRECT_SYMM_DENSE>);
+    return sums(pair_sums_kernel<DIRECT_RECT>);
 }
 
 }  // namespace kf

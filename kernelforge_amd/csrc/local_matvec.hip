@@ -140,7 +140,7 @@ template <typename T>
 __global__ __launch_bounds__(NT) void pack_rows_kernel(const T *__restrict__ src,
                                                        const T *__restrict__ src2,
                                                        const int *__restrict__ idx, int rows,
-                                                       int ma, int rep,
+                                                       size_t first, int ma, int rep,
                                                        const int *__restrict__ inv, int nf, int nfp,
                                                        const MvSeg *__restrict__ segs, int nseg,
                                                        const T *__restrict__ aE,
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(NT) void pack_rows_kernel(const T *__restrict__ src
                                                        double *__restrict__ dot,
                                                        double *__restrict__ aEr) {
     const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int r = (int)(first + blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (r >= rows) return;
     const int at = idx[r];
     double *d = dst + (size_t)r * nfp, *da = nullptr;
@@ -494,10 +494,10 @@ __global__ __launch_bounds__(64) void zero_rows_kernel(const int *__restrict__ i
 constexpr int kReduceThreads = 512;
 __global__ __launch_bounds__(kReduceThreads) void reduce_mol_kernel(
     const double *__restrict__ erow, const double *__restrict__ Fat, int parts,
-    const int *__restrict__ offs, int natoms, int ma, double *__restrict__ E,
+    const int *__restrict__ offs, int natoms, int ma, size_t first, double *__restrict__ E,
     double *__restrict__ F) {
     __shared__ double red[kReduceThreads];
-    const int a = blockIdx.x, tid = threadIdx.x;
+    const int a = (int)(first + blockIdx.x), tid = threadIdx.x;
     const int nc = offs[a + 1] - offs[a], na = nc / 3, ld = 3 * ma;
     if (E && tid < 64) {
         double s = 0.0;
@@ -722,19 +722,20 @@ template <typename T>
 int mv_pack_train(const MvLayout &L, const MvDev &D, const T *X2, const T *ad, const T *aE,
                   int ma2, hipStream_t stream) {
     if (L.t_rows == 0) return KF_OK;
-    hipLaunchKernelGGL(pack_rows_kernel<T>, dim3((L.t_rows + 3) / 4), dim3(NT), 0, stream, X2, ad,
-                       D.src2, L.t_rows, ma2, L.rep, D.inv, L.nf, L.nfp, D.segs,
-                       (int)L.segs.size(), aE, D.P2, D.n2, D.rdot, D.aE);
-    KF_HIP_TRY(hipGetLastError());
-    return KF_OK;
+    return for_groups((L.t_rows + 3) / 4, [&](size_t first, unsigned n) {
+        hipLaunchKernelGGL(pack_rows_kernel<T>, dim3(n), dim3(NT), 0, stream, X2, ad, D.src2,
+                           L.t_rows, first, ma2, L.rep, D.inv, L.nf, L.nfp, D.segs,
+                           (int)L.segs.size(), aE, D.P2, D.n2, D.rdot, D.aE);
+    });
 }
 
 int mv_zero_unmatched(const MvLayout &L, const MvDev &D, bool forces, hipStream_t stream) {
     if (L.src0.empty()) return KF_OK;
-    hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)L.src0.size()), dim3(64), 0, stream, D.src0,
-                       3 * L.ma1, L.parts, L.nm1 * L.ma1, D.erow, forces ? D.Fat : (double *)nullptr);
-    KF_HIP_TRY(hipGetLastError());
-    return KF_OK;
+    return for_groups(L.src0.size(), [&](size_t first, unsigned n) {
+        hipLaunchKernelGGL(zero_rows_kernel, dim3(n), dim3(64), 0, stream, D.src0 + first,
+                           3 * L.ma1, L.parts, L.nm1 * L.ma1, D.erow,
+                           forces ? D.Fat : (double *)nullptr);
+    });
 }
 
 // mode bits: 1 E, 2 F
@@ -743,13 +744,13 @@ int mv_run(const MvLayout &L, const MvDev &D, const T *X1, const T *dX1, double 
            double *E, double *F, int mode, hipStream_t stream) {
     const double cexp = -1.0 / (2.0 * sigma * sigma), inv_s2 = 1.0 / (sigma * sigma);
     const int natoms = L.nm1 * L.ma1;
-    if (L.q_rows > 0) {
-        hipLaunchKernelGGL(pack_rows_kernel<T>, dim3((L.q_rows + 3) / 4), dim3(NT), 0, stream, X1,
-                           (const T *)nullptr, D.src1, L.q_rows, L.ma1, L.rep, D.inv, L.nf,
+    int rc = for_groups((L.q_rows + 3) / 4, [&](size_t first, unsigned n) {
+        hipLaunchKernelGGL(pack_rows_kernel<T>, dim3(n), dim3(NT), 0, stream, X1,
+                           (const T *)nullptr, D.src1, L.q_rows, first, L.ma1, L.rep, D.inv, L.nf,
                            L.nfp, D.segs, (int)L.segs.size(), (const T *)nullptr, D.Xq, D.nq,
                            D.zq, (double *)nullptr);
-        KF_HIP_TRY(hipGetLastError());
-    }
+    });
+    if (rc) return rc;
     const bool forces = mode & 2;
     for (const MvRound &R : L.rounds) {
         const MvSeg *segs = D.segs + R.seg0;
@@ -779,11 +780,11 @@ int mv_run(const MvLayout &L, const MvDev &D, const T *X1, const T *dX1, double 
                            forces ? D.Fat : (double *)nullptr);
         KF_HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL(reduce_mol_kernel, dim3(L.nm1), dim3(kReduceThreads), 0, stream, D.erow, D.Fat,
-                       L.parts, D.offs, natoms, L.ma1, (mode & 1) ? E : (double *)nullptr,
-                       forces ? F : (double *)nullptr);
-    KF_HIP_TRY(hipGetLastError());
-    return KF_OK;
+    return for_groups(L.nm1, [&](size_t first, unsigned n) {
+        hipLaunchKernelGGL(reduce_mol_kernel, dim3(n), dim3(kReduceThreads), 0, stream, D.erow,
+                           D.Fat, L.parts, D.offs, natoms, L.ma1, first,
+                           (mode & 1) ? E : (double *)nullptr, forces ? F : (double *)nullptr);
+    });
 }
 
 // Labels and counts of both sets and the training side's used columns on the host, with one

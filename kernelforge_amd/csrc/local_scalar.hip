@@ -261,10 +261,10 @@ __device__ __forceinline__ unsigned long long wave_or64(unsigned long long m) {
 // work-group per (label, block), a wave per tile.
 __global__ __launch_bounds__(256) void tile_mask_kernel(const unsigned long long *__restrict__ rowmask,
                                                         const int *__restrict__ mol_row, int nm,
-                                                        int mb, int nblk,
+                                                        int mb, int nblk, size_t first,
                                                         const int *__restrict__ tbase,
                                                         ulonglong2 *__restrict__ tmask) {
-    const int la = blockIdx.x, l = la / nblk, A = la - l * nblk;
+    const int la = (int)(first + blockIdx.x), l = la / nblk, A = la - l * nblk;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int *mr = mol_row + (size_t)l * (nm + 1);
     const int r0 = mr[A * mb], r1 = mr[min(A * mb + mb, nm)];
@@ -1008,8 +1008,11 @@ int molecule_windows(const double *X, const int *N, int nm, int ma, int rep, int
     auto *dm = static_cast<unsigned long long *>(workspace(ws, bytes, stream));
     auto *hm = static_cast<unsigned long long *>(host_staging(ws, bytes));
     KF_REQUIRE(dm && hm, KF_ERR_NOMEM, "workspace allocation failed (%zu B)", bytes);
-    hipLaunchKernelGGL(mol_winmask_kernel, dim3(nm), dim3(256), 0, stream, X, N, ma, rep, dm);
-    KF_HIP_TRY(hipGetLastError());
+    const int rc = for_groups(nm, [&](size_t first, unsigned n) {
+        hipLaunchKernelGGL(mol_winmask_kernel, dim3(n), dim3(256), 0, stream,
+                           X + first * ma * rep, N + first, ma, rep, dm + 2 * first);
+    });
+    if (rc) return rc;
     KF_HIP_TRY(hipMemcpyAsync(hm, dm, bytes, hipMemcpyDeviceToHost, stream));
     KF_HIP_TRY(hipStreamSynchronize(stream));
     std::copy(hm, hm + 2 * (size_t)nm, out.begin());
@@ -1172,9 +1175,11 @@ int upload_and_pack(const LocalPlan &p, const std::vector<int> &perm, const doub
                                static_cast<double *>(d.Xp), d.n2, d.rowmask);
         KF_HIP_TRY(hipGetLastError());
         if (masked && nla > 0) {
-            hipLaunchKernelGGL(tile_mask_kernel, dim3((unsigned)nla), dim3(256), 0, stream,
-                               d.rowmask, d.mol_row, p.nm, mb, d.nblk, d.tbase, d.tmask);
-            KF_HIP_TRY(hipGetLastError());
+            const int rc = for_groups(nla, [&](size_t first, unsigned n) {
+                hipLaunchKernelGGL(tile_mask_kernel, dim3(n), dim3(256), 0, stream, d.rowmask,
+                                   d.mol_row, p.nm, mb, d.nblk, first, d.tbase, d.tmask);
+            });
+            if (rc) return rc;
         }
     }
     return KF_OK;
