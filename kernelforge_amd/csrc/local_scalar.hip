@@ -62,7 +62,8 @@ enum Mode { SYMM_RFP = 0, SYMM_DENSE = 1, RECT = 2 };
 // end, so a slot's cache lines only ever live in one XCD's L2 -- a slot handed between
 // XCDs could be overwritten later by the other L2's write-back of the previous owner's
 // lines.  Fewer work-groups than slots are resident on an XCD (the host checks), so the
-// probe ends; the flags are cleared by a small kernel before every launch.  Only the owner
+// probe ends; the flags are cleared by a small kernel before every launch.  An owner waits
+// until its stores have reached the L2 before it frees the slot.  Only the owner
 // thread of an entry touches it between two barriers, as in LDS; launches on one device do
 // not overlap (the entry points order them).
 constexpr int kXcc = 8, kSlotsPerXcc = 128, kSlots = kXcc * kSlotsPerXcc;
@@ -933,7 +934,11 @@ __global__ __launch_bounds__(NT, NS ? 2 : 3) void local_scalar_f64_kernel(
             out[ib * nm1 + ia] = val;
         }
     }
-    __syncthreads();  // every read of the slot is done
+    // The slot's next owner, on another CU, must not be overtaken by a store still on its way to
+    // the L2: a barrier does not wait for those, and a wave whose rows the block does not reach
+    // (oa0 >= na) has read nothing back since it added to rows that another wave wrote out.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // every read of the slot is done, and every store has arrived
     if (threadIdx.x == 0) atomicExch(&g_slot_busy[s_slot], 0);
 }
 

@@ -94,6 +94,21 @@ def test_rect_block_sizes(lk, nm1, nm2, rep):
                    oracle.kernel_rect(x1, x2, q1, q2, n1, n2, s)) < 1e-12
 
 
+def test_short_blocks_repeat_exactly(lk):
+    """Many output blocks of fewer than 64 molecules that end soon after another, so that
+    accumulators pass from one work-group to the next all the time."""
+    x1, q1, n1 = random_set(300, 12, 16, 3, 61, nmin=12)
+    x2, q2, n2 = random_set(6000, 12, 16, 3, 62, nmin=12)
+    first = lk.kernel_gaussian(x1, x2, q1, q2, n1, n2, 1.5)
+    assert rel_err(first[::29], oracle.kernel_rect(x1[::29], x2, q1[::29], q2, n1[::29], n2,
+                                                   1.5)) < 1e-12
+    a = lk.kernel_gaussian_symm_rfp(x2[:1500], q2[:1500], n2[:1500], 1.5)
+    for _ in range(30):
+        np.testing.assert_array_equal(lk.kernel_gaussian(x1, x2, q1, q2, n1, n2, 1.5), first)
+        np.testing.assert_array_equal(
+            lk.kernel_gaussian_symm_rfp(x2[:1500], q2[:1500], n2[:1500], 1.5), a)
+
+
 def windowed_set(nm, ma, rep, nlab, seed, ngroups=7):
     """Random rows whose columns fall into groups (spans not aligned to the kernel's
     16-column windows) that each molecule uses or leaves at zero, single atoms dropping
