@@ -78,6 +78,11 @@ int kf_stream_synchronize(void *stream);
  *   0 fchl19, 1 local symmetric kernel, 2 local rectangular kernel,
  *   3 RFP potrf, 4 RFP potrs, 5 E+F kernels, 6 matvecs. */
 int kf_timer_enable(int on);
+
+/* For tests: the nth device workspace request of the calling thread from now on is refused,
+ * as when the device's memory is full (0: none).  Returns how many requests were left until
+ * the last one so asked for, 0 once it has been refused. */
+int kf_workspace_refuse(int nth);
 int kf_timer_reset(void);
 int kf_timer_read(int id, double *total_ms, int *count);
 

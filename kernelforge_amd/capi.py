@@ -38,6 +38,7 @@ SIGNATURES = {
     "kf_memset_zero": [_vp, ctypes.c_size_t, _vp],
     "kf_stream_synchronize": [_vp],
     "kf_timer_enable": [_c_int],
+    "kf_workspace_refuse": [_c_int],
     "kf_timer_reset": [],
     "kf_timer_read": [_c_int, ctypes.POINTER(_c_double), ctypes.POINTER(_c_int)],
     "kf_fchl19_f64": [_vp, _vp, _vp, _c_int, _c_int, _vp, _c_int, _vp, _c_int, _vp, _c_int,

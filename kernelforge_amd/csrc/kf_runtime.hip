@@ -30,10 +30,14 @@ Slot g_ws[kMaxDevices][WS_NSLOTS];
 Slot g_host[WS_NSLOTS];
 }  // namespace
 
+// Requests of this thread until one is refused (0: none), for tests of what a call does then.
+static thread_local int t_refuse = 0;
+
 // Grow-only: a slot is reallocated (after draining the stream) only when a call
 // needs more than it holds.  Sizes are rounded up to 2 MiB so that slowly
 // growing requests do not reallocate every call.
 void *workspace(int slot, size_t bytes, hipStream_t stream) {
+    if (t_refuse > 0 && --t_refuse == 0) return nullptr;
     if (bytes == 0) bytes = 256;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
@@ -200,6 +204,12 @@ void ScopedTimer::stop() {
 }
 
 }  // namespace kf
+
+extern "C" int kf_workspace_refuse(int nth) {
+    const int left = kf::t_refuse;
+    kf::t_refuse = nth > 0 ? nth : 0;
+    return left;
+}
 
 extern "C" int kf_timer_enable(int on) {
     std::lock_guard<std::mutex> lock(kf::g_tm_mutex);

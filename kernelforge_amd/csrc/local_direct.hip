@@ -35,12 +35,28 @@ constexpr int kLdsTiles = 384;
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef double v2d __attribute__((ext_vector_type(2)));
 
-// One label: its packed rows of both sets and where its exponentials go.
+// One label: its packed rows of both sets and where its exponentials go: R1 rows of R2, or,
+// in the symmetric forms, row tile after row tile from the diagonal tile on.
 struct DirectSeg {
     int r1, R1, r2, R2;
-    int it, pad;      // first tile
-    size_t eoff, ld;  // exponentials: R1 rows of ld (R2)
+    int it, pad;  // first tile
+    size_t eoff;
 };
+
+// Exponentials of the row tiles before row c0, a multiple of te, of a symmetric label with R
+// rows: a tile has te rows from its first column on.
+__host__ __device__ inline size_t upper_rows(int c0, int te, int R) {
+    return (size_t)c0 * R - ((size_t)c0 * (c0 - te) >> 1);
+}
+
+// Row i of a label's exponentials, indexed by column (symmetric: from its tile's first row on;
+// te a power of 2).
+template <bool SYMM>
+__device__ inline double *exp_row(const DirectSeg &S, int te, int i, double *Ex) {
+    if (!SYMM) return Ex + S.eoff + (size_t)i * S.R2;
+    const int c0 = i & -te;
+    return Ex + S.eoff + upper_rows(c0, te, S.R2) + (size_t)(i - c0) * (S.R2 - c0) - c0;
+}
 
 // Consecutive tiles (which share operands) on one XCD: work-groups are dealt round-robin
 // over eight of them.
@@ -49,10 +65,10 @@ __device__ inline int xcd_tile() {
     return (G % 8 == 0) ? (g % 8) * (G / 8) + g / 8 : g;
 }
 
-template <class At>
-__device__ inline int seg_of(const DirectSeg *segs, int nseg, int x, At at) {
+// Label of a tile: the last one whose first tile is not beyond it.
+__device__ inline int seg_of(const DirectSeg *segs, int nseg, int tile) {
     int s = 0;
-    while (s + 1 < nseg && at(segs[s + 1]) <= x) ++s;
+    while (s + 1 < nseg && segs[s + 1].it <= tile) ++s;
     return s;
 }
 
@@ -89,6 +105,7 @@ __device__ inline bool tile_at(const DirectSeg &S, int te, int loc, int &rt, int
 
 // Exponentials of a 16 x 16 fragment: s its Gram entries, rows from row0 with squared norms
 // in `nr` (lane r holds row r's), this lane's column with squared norm nc.
+template <bool SYMM, int T>
 __device__ inline void put_exps(const DirectSeg &S, const double (&s)[4], int row0, int col,
                                 double nr, double nc, double cy, const double *etab, int lane,
                                 double *Ex) {
@@ -96,7 +113,7 @@ __device__ inline void put_exps(const DirectSeg &S, const double (&s)[4], int ro
     for (int v = 0; v < 4; ++v) {
         const int rr = mfma16_row_f64(lane, v);
         const double e = exp_scaled(fma(s[v], -2.0 * cy, cy * __shfl(nr, rr, 64) + cy * nc), etab);
-        if (row0 + rr < S.R1 && col < S.R2) Ex[S.eoff + (row0 + rr) * S.ld + col] = e;
+        if (row0 + rr < S.R1 && col < S.R2) exp_row<SYMM>(S, T, row0 + rr, Ex)[col] = e;
     }
 }
 
@@ -117,7 +134,7 @@ __global__ __launch_bounds__(NT, 3) void exp_tiles_kernel(const DirectSeg *__res
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
     if (tid < 64) etab[tid] = kExp2Tab64[tid];
     const int tile = xcd_tile();
-    const DirectSeg S = segs[seg_of(segs, nseg, tile, [](const DirectSeg &t) { return t.it; })];
+    const DirectSeg S = segs[seg_of(segs, nseg, tile)];
     int rt, ct;
     if (!tile_at<SYMM>(S, TE, tile - S.it, rt, ct)) return;
     const double *pa[F], *pb[F];
@@ -201,7 +218,7 @@ __global__ __launch_bounds__(NT, 3) void exp_tiles_kernel(const DirectSeg *__res
 #pragma unroll
         for (int v = 0; v < 4; ++v) s[v] += red[w][(m * F + n) * 4 + v][lane];
     }
-    put_exps(S, s, rt * TE + 16 * m, ct * TE + 16 * n + r, nr, nc, cy, etab, lane, Ex);
+    put_exps<SYMM, TE>(S, s, rt * TE + 16 * m, ct * TE + 16 * n + r, nr, nc, cy, etab, lane, Ex);
 }
 
 // 64 x 64 tiles, 16 columns of both operands at a time through LDS (double-buffered, one
@@ -222,7 +239,7 @@ __global__ __launch_bounds__(NT, 4) void exp_tiles_lds_kernel(
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
     if (tid < 64) etab[tid] = kExp2Tab64[tid];
     const int tile = xcd_tile();
-    const DirectSeg S = segs[seg_of(segs, nseg, tile, [](const DirectSeg &t) { return t.it; })];
+    const DirectSeg S = segs[seg_of(segs, nseg, tile)];
     int rt, ct;
     if (!tile_at<SYMM>(S, TL, tile - S.it, rt, ct)) return;
     const int row = tid >> 2, part = tid & 3;
@@ -311,19 +328,19 @@ __global__ __launch_bounds__(NT, 4) void exp_tiles_lds_kernel(
         for (int n = 0; n < 2; ++n) {
             const int rl = 32 * wr + 16 * m, cl = 32 * wc + 16 * n;
             const double s[4] = {c[m][n][0], c[m][n][1], c[m][n][2], c[m][n][3]};
-            put_exps(S, s, rt * TL + rl, ct * TL + cl + r, nrm[0][rl + r], nrm[1][cl + r], cy, etab,
-                     lane, Ex);
+            put_exps<SYMM, TL>(S, s, rt * TL + rl, ct * TL + cl + r, nrm[0][rl + r],
+                               nrm[1][cl + r], cy, etab, lane, Ex);
         }
 }
 
-// K[a, b] = sum over the labels and the label's rows of a and b of the exponentials.  Eight
-// lanes share a molecule pair, each taking every eighth row of a.
+// K[a, b] = sum over the labels and the label's rows of a and b of the exponentials (in
+// tiles of te rows).  Eight lanes share a molecule pair, each taking every eighth row of a.
 template <int MODE>
 __global__ __launch_bounds__(NT) void pair_sums_kernel(const DirectSeg *__restrict__ segs,
-                                                       const double *__restrict__ Ex,
+                                                       double *__restrict__ Ex,
                                                        const int *__restrict__ mol1,
                                                        const int *__restrict__ mol2, int nseg,
-                                                       int nm1, int nm2, size_t first,
+                                                       int nm1, int nm2, int te, size_t first,
                                                        double *__restrict__ out) {
     constexpr bool SYMM = MODE != DIRECT_RECT;
     const int nbk = (nm2 + 31) / 32, sub = threadIdx.x & 7;
@@ -336,16 +353,13 @@ __global__ __launch_bounds__(NT) void pair_sums_kernel(const DirectSeg *__restri
         const int *ma = mol1 + (size_t)l * (nm1 + 1) + a, *mb = mol2 + (size_t)l * (nm2 + 1) + b;
         const int i0 = ma[0] - S.r1, i1 = ma[1] - S.r1, j0 = mb[0] - S.r2, j1 = mb[1] - S.r2;
         for (int i = i0 + sub; i < i1; i += 8) {
-            const double *e = Ex + S.eoff;
             if (SYMM && a == b) {  // only tiles of the upper triangle were formed
-                for (int j = j0; j < j1; ++j) s += e[(size_t)min(i, j) * S.ld + max(i, j)];
+                for (int j = j0; j < j1; ++j) s += exp_row<SYMM>(S, te, min(i, j), Ex)[max(i, j)];
             } else {
+                const double *p = exp_row<SYMM>(S, te, i, Ex);
                 int j = j0;
-                for (; j + 4 <= j1; j += 4) {
-                    const double *p = e + (size_t)i * S.ld + j;
-                    s += (p[0] + p[1]) + (p[2] + p[3]);
-                }
-                for (; j < j1; ++j) s += e[(size_t)i * S.ld + j];
+                for (; j + 4 <= j1; j += 4) s += (p[j] + p[j + 1]) + (p[j + 2] + p[j + 3]);
+                for (; j < j1; ++j) s += p[j];
             }
         }
     }
@@ -387,20 +401,21 @@ int local_direct(int mode, const LocalPlan &p1, const double *X1, const LocalPla
     const int small = count(TE);
     const bool lds = tiles >= kLdsTiles && 2.8 * tiles < small;
     tiles = lds ? count(TL) : small;
+    const int te = lds ? TL : TE;
     size_t elen = 0;
     for (int l = 0; l < L; ++l) {
         const int *a = &p1.mol_row[(size_t)l * (nm1 + 1)], *b = &p2.mol_row[(size_t)l * (nm2 + 1)];
         const int R1 = a[nm1] - a[0], R2 = b[nm2] - b[0];
-        segs[l] = {a[0], R1, b[0], R2, segs[l].it, 0, elen, (size_t)R2};
-        elen += (size_t)R1 * R2;
+        segs[l] = {a[0], R1, b[0], R2, segs[l].it, 0, elen};
+        elen += symm ? upper_rows(ceil_div(R1, te) * te, te, R1) : (size_t)R1 * R2;
     }
     // one upload: segments, then the rows' sources and the molecules' row ranges
     const size_t n1 = p1.src.size(), m1 = p1.mol_row.size();
     const size_t n2 = symm ? 0 : p2.src.size(), m2 = symm ? 0 : p2.mol_row.size();
     const size_t bytes = sizeof(DirectSeg) * L + sizeof(int) * (n1 + m1 + n2 + m2);
+    double *Ex = static_cast<double *>(workspace(WS_PACK, sizeof(double) * elen, stream));
     char *dev = static_cast<char *>(workspace(WS_PLAN, bytes, stream));
     char *stage = static_cast<char *>(host_staging(WS_PLAN, bytes));
-    double *Ex = static_cast<double *>(workspace(WS_PACK, sizeof(double) * elen, stream));
     KF_REQUIRE(dev && stage && Ex, KF_ERR_NOMEM, "workspace allocation failed (%zu B)",
                sizeof(double) * elen);
     std::copy(segs.begin(), segs.end(), reinterpret_cast<DirectSeg *>(stage));
@@ -434,7 +449,7 @@ int local_direct(int mode, const LocalPlan &p1, const double *X1, const LocalPla
     auto sums = [&](auto kern) {
         return for_groups((size_t)nm1 * ceil_div(nm2, 32), [&](size_t first, unsigned n) {
             hipLaunchKernelGGL(kern, dim3(n), dim3(NT), 0, stream, dseg, Ex, mol1, mol2, L, nm1,
-                               nm2, first, out);
+                               nm2, te, first, out);
         });
     };
     if (mode == DIRECT_SYMM_RFP) return sums(pair_sums_kernel<DIRECT_SYMM_RFP>);

@@ -1252,7 +1252,8 @@ int upload_block_order(int nb1, int nb2, bool symm, hipStream_t stream, const in
 // Up to this many label-matched atom pairs the packing-free form (local_direct.hip) is
 // faster: 800 molecules (2.2e7 pairs) 826 us a call against 873, 333 against 2,000 (4.5e7)
 // 1,496 against 1,835; beyond, skipping the zero windows pays: 1,200 molecules (4.9e7) 1,618
-// against 1,500, 1,500 against 1,500 (1.5e8) 6.3 ms against 3.9.
+// against 1,500, 1,500 against 1,500 (1.5e8) 6.3 ms against 3.9.  It needs 8 bytes a pair
+// (320 MB at the limit); where that is refused, the blocked form takes the call.
 constexpr long long kDirectPairs = 40000000;
 
 // Molecules per block of the symmetric kernel for `pairs` matched atom pairs.  Small blocks
@@ -1334,8 +1335,9 @@ int symm_impl(int precision, const double *X, const int *Q, const int *N, int nm
     const long long pairs = matched_pairs(cnt, cnt, true);
     if (ns == 0 && pairs <= kDirectPairs) {
         build_plan(hQ.data(), hN.data(), nm, ma, labels, p);
-        return local_direct(MODE == SYMM_RFP ? DIRECT_SYMM_RFP : DIRECT_SYMM_DENSE, p, X, p, X,
-                            rep, cy, static_cast<double *>(out), TM_LOCAL_SYMM, stream);
+        rc = local_direct(MODE == SYMM_RFP ? DIRECT_SYMM_RFP : DIRECT_SYMM_DENSE, p, X, p, X, rep,
+                          cy, static_cast<double *>(out), TM_LOCAL_SYMM, stream);
+        if (rc != KF_ERR_NOMEM) return rc;
     }
     std::vector<int> perm, Qp, Np;
     if (windows_masked(rep, ns)) {
@@ -1419,8 +1421,9 @@ extern "C" int kf_local_kernel(int precision, const double *X1, const double *X2
     if (ns == 0 && pairs <= kDirectPairs) {
         build_plan(q1.data(), n1.data(), nm1, max_atoms1, labels, p1);
         build_plan(q2.data(), n2.data(), nm2, max_atoms2, labels, p2);
-        return local_direct(DIRECT_RECT, p1, X1, p2, X2, rep, cy, static_cast<double *>(K),
-                            TM_LOCAL_RECT, stream);
+        rc = local_direct(DIRECT_RECT, p1, X1, p2, X2, rep, cy, static_cast<double *>(K),
+                          TM_LOCAL_RECT, stream);
+        if (rc != KF_ERR_NOMEM) return rc;
     }
     std::vector<int> perm1, perm2;
     if (windows_masked(rep, ns)) {

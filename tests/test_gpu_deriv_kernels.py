@@ -421,3 +421,26 @@ def test_unused_columns_found_anywhere(lk, nm, ma, rep):
 
 def rng_mask(shape, seed):
     return (np.random.default_rng(seed).random(shape) < 0.5).astype(np.float64)
+
+
+def test_refused_scratch(lk):
+    """Each device workspace request of a Hessian kernel refused in turn: an error, or the
+    result without what the scratch was for (features in several runs)."""
+    from kernelforge_amd import capi
+
+    X, dX, Q, N = rand_set(5, 12, 130, 3, 77, 5)
+    want = lk.kernel_gaussian_hessian_symm(X, dX, Q, N, 1.7)
+    assert rel_err(want, oracle.hessian_symm(X, dX, Q, N, 1.7)) < TOL
+    done = []
+    for nth in range(1, 9):
+        capi.lib().kf_workspace_refuse(nth)
+        try:
+            got = lk.kernel_gaussian_hessian_symm(X, dX, Q, N, 1.7)
+        except (MemoryError, RuntimeError):
+            got = None
+        left = capi.lib().kf_workspace_refuse(0)
+        if got is not None:
+            assert rel_err(got, want) < TOL
+            done.append(left)
+    assert done[:1] == [0]  # the last request is one that it can do without
+    assert rel_err(lk.kernel_gaussian_hessian_symm(X, dX, Q, N, 1.7), want) < TOL

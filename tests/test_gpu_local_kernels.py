@@ -109,6 +109,35 @@ def test_short_blocks_repeat_exactly(lk):
             lk.kernel_gaussian_symm_rfp(x2[:1500], q2[:1500], n2[:1500], 1.5), a)
 
 
+class Blocked:
+    """The module with the packing-free form's scratch refused, so that its calls take the
+    blocked form."""
+
+    def __init__(self, lk):
+        self.lk = lk
+
+    def __getattr__(self, name):
+        def call(*args, **kw):
+            from kernelforge_amd import capi
+
+            capi.lib().kf_workspace_refuse(1)
+            try:
+                return getattr(self.lk, name)(*args, **kw)
+            finally:
+                assert capi.lib().kf_workspace_refuse(0) == 0  # refused, and gone on without it
+
+        return call
+
+
+@pytest.mark.parametrize("nm,ma,rep", [(1, 3, 7), (33, 4, 16), (130, 9, 720)])
+def test_refused_scratch_takes_the_blocked_form(lk, nm, ma, rep):
+    test_symm_and_rfp_random(Blocked(lk), nm, ma, rep, 3)
+
+
+def test_refused_scratch_takes_the_blocked_form_rect(lk):
+    test_rect_random(Blocked(lk), 33, 65)
+
+
 def windowed_set(nm, ma, rep, nlab, seed, ngroups=7):
     """Random rows whose columns fall into groups (spans not aligned to the kernel's
     16-column windows) that each molecule uses or leaves at zero, single atoms dropping
