@@ -94,6 +94,17 @@ def test_rect_block_sizes(lk, nm1, nm2, rep):
                    oracle.kernel_rect(x1, x2, q1, q2, n1, n2, s)) < 1e-12
 
 
+@pytest.mark.parametrize("nlab", [255, 257, 700])
+def test_direct_many_labels(lk, nlab):
+    """More labels than a work-group has threads, few of them in any one molecule, and
+    molecules without atoms."""
+    x, q, n = random_set(90, 6, 20, nlab, nlab, nmin=0)
+    q[:, 0] = np.arange(90) % 3 * (nlab - 1) // 2  # the first, a middle and the last label
+    assert rel_err(lk.kernel_gaussian_symm(x, q, n, 1.3), oracle.kernel_symm(x, q, n, 1.3)) < 1e-12
+    assert rel_err(lk.kernel_gaussian(x[:41], x, q[:41], q, n[:41], n, 1.3),
+                   oracle.kernel_rect(x[:41], x, q[:41], q, n[:41], n, 1.3)) < 1e-12
+
+
 def test_short_blocks_repeat_exactly(lk):
     """Many output blocks of fewer than 64 molecules that end soon after another, so that
     accumulators pass from one work-group to the next all the time."""
