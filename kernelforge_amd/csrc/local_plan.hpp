@@ -77,35 +77,59 @@ inline void build_plan(const int *Q, const int *N, int nm, int ma, const std::ve
     }
 }
 
-// Atoms (i < N[a]) of each of the given (sorted) labels.
-inline std::vector<long long> label_counts(const int *Q, const int *N, int nm, int ma,
-                                           const std::vector<int> &labels) {
-    constexpr int kDirect = 256;
-    long long direct[kDirect] = {};
-    std::vector<long long> out(labels.size(), 0);
+// Packed rows of every label before each `step` molecules: at[l * (n + 1) + k] is the first
+// one of molecule k * step, counted from any start.
+struct RowTable {
+    const int *at;
+    int n, step, nm, max_atoms, nlabels;
+    // rows of label l in molecules a0 .. a1 - 1, multiples of step or the end
+    int rows(int l, int a0, int a1) const {
+        const int *r = at + (size_t)l * (n + 1);
+        return r[std::min((a1 + step - 1) / step, n)] - r[a0 / step];
+    }
+};
+inline RowTable row_table(const LocalPlan &p) {
+    return {p.mol_row.data(), p.nm, 1, p.nm, p.max_atoms, p.nlabels};
+}
+
+// The same by groups of eight molecules, without a plan; `at` holds it.
+inline RowTable count_rows(const int *Q, const int *N, int nm, int ma,
+                           const std::vector<int> &labels, std::vector<int> &at) {
+    constexpr int kStep = 8, kDirect = 256;
+    const int n = (nm + kStep - 1) / kStep, L = (int)labels.size();
+    at.assign((size_t)L * (n + 1), 0);
+    int direct[kDirect];
+    std::fill(direct, direct + kDirect, -1);
+    for (int l = 0; l < L; ++l)
+        if (labels[l] >= 0 && labels[l] < kDirect) direct[labels[l]] = l;
     for (int a = 0; a < nm; ++a) {
         const int na = clamp_atoms(N[a], ma);
         const int *q = Q + (size_t)a * ma;
+        int *to = at.data() + a / kStep + 1;
         for (int i = 0; i < na; ++i) {
+            int l;
             if (q[i] >= 0 && q[i] < kDirect) {
-                ++direct[q[i]];
+                l = direct[q[i]];
             } else {
                 const auto it = std::lower_bound(labels.begin(), labels.end(), q[i]);
-                if (it != labels.end() && *it == q[i]) ++out[it - labels.begin()];
+                l = it != labels.end() && *it == q[i] ? int(it - labels.begin()) : -1;
             }
+            if (l >= 0) ++to[(size_t)l * (n + 1)];
         }
     }
-    for (size_t l = 0; l < labels.size(); ++l)
-        if (labels[l] >= 0 && labels[l] < kDirect) out[l] = direct[labels[l]];
-    return out;
+    for (int l = 0; l < L; ++l)
+        for (int k = 0; k < n; ++k) at[(size_t)l * (n + 1) + k + 1] += at[(size_t)l * (n + 1) + k];
+    return {at.data(), n, kStep, nm, ma, L};
 }
 
 // Label-matched atom pairs of two sets; half of them (rounded up per label) for the
 // symmetric kernels, where both are one set.
-inline long long matched_pairs(const std::vector<long long> &c1, const std::vector<long long> &c2,
-                               bool symm) {
+inline long long matched_pairs(const RowTable &t1, const RowTable &t2, bool symm) {
     long long n = 0;
-    for (size_t l = 0; l < c1.size(); ++l) n += symm ? (c1[l] * c2[l] + 1) / 2 : c1[l] * c2[l];
+    for (int l = 0; l < t1.nlabels; ++l) {
+        const long long p = (long long)t1.rows(l, 0, t1.nm) * t2.rows(l, 0, t2.nm);
+        n += symm ? (p + 1) / 2 : p;
+    }
     return n;
 }
 

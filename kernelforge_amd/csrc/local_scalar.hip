@@ -42,7 +42,7 @@ namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-constexpr int MB = 64;       // most molecules per output block (block_size)
+constexpr int MB = 64;       // most molecules per output block (choose_blocks)
 constexpr int TS = 64;       // sub-tile edge (packed rows)
 constexpr int KA = 32;       // row-operand chunk staged in LDS (descriptor columns)
 constexpr int KS = 16;       // column-operand sub-chunk held in registers
@@ -1249,25 +1249,93 @@ int upload_block_order(int nb1, int nb2, bool symm, hipStream_t stream, const in
     return KF_OK;
 }
 
-// Up to this many label-matched atom pairs the packing-free form (local_direct.hip) is
-// faster: 800 molecules (2.2e7 pairs) 826 us a call against 873, 333 against 2,000 (4.5e7)
-// 1,496 against 1,835; beyond, skipping the zero windows pays: 1,200 molecules (4.9e7) 1,618
-// against 1,500, 1,500 against 1,500 (1.5e8) 6.3 ms against 3.9.  It needs 8 bytes a pair
-// (320 MB at the limit); where that is refused, the blocked form takes the call.
+// Most label-matched atom pairs of the packing-free form (local_direct.hip): its scratch, 8
+// bytes a pair, is 320 MB there.  Beyond, or where that is refused, the blocked form takes a
+// call.
 constexpr long long kDirectPairs = 40000000;
 
-// Molecules per block of the symmetric kernel for `pairs` matched atom pairs.  Small blocks
-// give more work-groups and a shorter longest one, large ones fuller tiles (1,600 molecules,
-// 8.7e7 pairs: blocks of 24 2.0 ms, 32 2.0, 64 3.6; 3,200, 3.5e8: 6.9, 6.4 and 7.6; 6,400,
-// 1.4e9: 25.8, 24.4 and 22.3).
-int symm_block(long long pairs) { return pairs < 140000000 ? 24 : pairs < 1100000000 ? 32 : MB; }
+// Columns that a tile pair is taken to multiply where zero windows are left out.  The host
+// cannot know before it has read the windows back, which a small call has no time for; FCHL19
+// descriptors of C/H/N/O/S molecules share 335 of 720 columns (five elements) and, in windows
+// that the element pairs do not align with, some more of 1,288 (seven in the list) or 2,016
+// (nine).
+double shared_columns(int rep) { return windows_masked(rep, 0) ? std::min(rep, 500) : rep; }
 
-// The rectangular kernel's, by the same measure (333 against 10,000 molecules: 16 x 32
-// 5.0 ms, 32 x 64 5.7, 64 x 64 7.1; 1,500 against 12,000: 22.1, 19.8 and 21.3 ms).
-void rect_blocks(long long pairs, int &mb1, int &mb2) {
-    const bool small = pairs < 460000000;
-    mb1 = small ? 16 : 32;
-    mb2 = small ? 32 : 64;
+// The times of both forms, in microseconds, by what they multiply; the host chooses by them.
+// Fitted to 90 calls with each block size and in both forms (one to 100 atoms a molecule, one
+// to 500 labels, 64 to 2,048 columns, 8e5 to 1.7e9 pairs).  What is chosen is on average 1%
+// slower than the best of the four, at most 28% (500 molecules with the columns of nine
+// elements), and never more than 2% slower than blocks of 64.
+//
+// Blocked form, `mb1` and `mb2` molecules a block.  Small blocks give more work-groups and a
+// shorter longest one, large ones fuller 64-row tiles and fewer of them: with 14 atoms a
+// molecule 24 is best to 1,600 molecules (2.35 ms; 2.46 at 32, 3.72 at 64), 32 at 3,200 (7.1;
+// 7.3 at 24, 8.4 at 64), 64 at 6,400 (23.6; 25.6 at 32); 15,000 molecules of one atom 15.2,
+// 9.7 and 5.4 ms; 6,000 of 14 atoms and 50 labels 18.0, 11.3 and 4.4.  Rectangles: 333 against
+// 10,000 of 14 atoms 6.6 ms at 16 x 32, 7.5 at 32 x 64, 9.3 at 64 x 64; 5,000 against 30,000
+// of one atom 16.4, 7.0 and 5.9.
+double blocked_time(const RowTable &p1, int mb1, const RowTable &p2, int mb2, bool symm, int rep) {
+    const double half = symm ? 0.5 : 1.0;
+    auto count = [](const RowTable &p, int l, int mb, double &tiles, double &frags) {
+        tiles = frags = 0.0;
+        for (int a = 0; a < p.nm; a += mb) {
+            const int n = p.rows(l, a, std::min(a + mb, p.nm));
+            tiles += (n + TS - 1) / TS;
+            frags += (n + 15) / 16;
+        }
+    };
+    double tiles = 0.0, frags = 0.0;
+    for (int l = 0; l < p1.nlabels; ++l) {
+        double t1, f1, t2, f2;
+        count(p1, l, mb1, t1, f1);
+        if (symm) t2 = t1, f2 = f1;
+        else count(p2, l, mb2, t2, f2);
+        tiles += half * t1 * t2;
+        frags += half * f1 * f2;
+    }
+    const double blocks = half * std::ceil((double)p1.nm / mb1) * std::ceil((double)p2.nm / mb2);
+    const double cols = shared_columns(rep);
+    // the host orders the molecules by their windows
+    const double atoms = (double)p1.nm * p1.max_atoms + (symm ? 0.0 : (double)p2.nm * p2.max_atoms);
+    return 300.0 + 1e-3 * atoms + blocks * (0.024 + 0.0015 * p1.nlabels) + tiles * (0.0064 + 2.2e-5 * cols) +
+           frags * 8.5e-6 * cols + tiles / blocks * (10.7 + 0.039 * cols);
+}
+
+// Packing-free form: every column is multiplied, and the sums take a step for every molecule
+// pair and label of the row molecule.  800 molecules of 14 atoms and 720 columns 0.87 ms (1.11
+// blocked), 1,090 1.46 (1.28), 9,000 of one atom 3.6 (2.2); 800 with the columns of nine
+// elements 1.98 (1.32).
+double direct_time(const RowTable &p1, const RowTable &p2, long long pairs, bool symm, int rep) {
+    double own = 0.0;  // molecules that have a label, over the labels (atoms spread at random)
+    for (int l = 0; l < p1.nlabels; ++l)
+        own += p1.nm * (1.0 - std::exp(-(double)p1.rows(l, 0, p1.nm) / p1.nm));
+    const double half = symm ? 0.5 : 1.0;
+    return 170.0 + 4.2e-8 * pairs * rep +
+           half * p2.nm * (2.5e-5 * own + 2.1e-5 * p1.nm * ((p1.nlabels + 255) / 256));
+}
+
+// Blocks of a call's blocked form (of fewer than 2^24 work-groups, except the largest).
+void choose_blocks(const RowTable &p1, const RowTable &p2, bool symm, int rep, int &mb1,
+                   int &mb2, double *time = nullptr) {
+    static const int symm_sizes[3][2] = {{MB, MB}, {32, 32}, {24, 24}},
+                     rect_sizes[3][2] = {{MB, MB}, {32, MB}, {16, 32}};
+    double best = 0.0;
+    for (int k = 0; k < 3; ++k) {
+        const int *m = symm ? symm_sizes[k] : rect_sizes[k];
+        if (k > 0 && std::ceil((double)p1.nm / m[0]) * std::ceil((double)p2.nm / m[1]) > 1.6e7)
+            break;
+        const double t = blocked_time(p1, m[0], p2, m[1], symm, rep);
+        if (k == 0 || t < best) best = t, mb1 = m[0], mb2 = m[1];
+    }
+    if (time) *time = best;
+}
+
+// Whether the packing-free form takes a call of `pairs` matched pairs (at most kDirectPairs).
+bool direct_is_faster(const RowTable &p1, const RowTable &p2, long long pairs, bool symm, int rep) {
+    int mb1, mb2;
+    double blocked;
+    choose_blocks(p1, p2, symm, rep, mb1, mb2, &blocked);
+    return direct_time(p1, p2, pairs, symm, rep) <= blocked;
 }
 
 // Launch of the scalar kernel in its FP64 form (ns = 0) or int8-split form (ns slices).
@@ -1331,13 +1399,16 @@ int symm_impl(int precision, const double *X, const int *Q, const int *N, int nm
         KF_HIP_TRY(hipMemsetAsync(out, 0, n * sizeof(double), stream));
         return KF_OK;
     }
-    const std::vector<long long> cnt = label_counts(hQ.data(), hN.data(), nm, ma, labels);
-    const long long pairs = matched_pairs(cnt, cnt, true);
-    if (ns == 0 && pairs <= kDirectPairs) {
-        build_plan(hQ.data(), hN.data(), nm, ma, labels, p);
-        rc = local_direct(MODE == SYMM_RFP ? DIRECT_SYMM_RFP : DIRECT_SYMM_DENSE, p, X, p, X, rep,
-                          cy, static_cast<double *>(out), TM_LOCAL_SYMM, stream);
-        if (rc != KF_ERR_NOMEM) return rc;
+    if (ns == 0) {
+        std::vector<int> at;
+        const RowTable t = count_rows(hQ.data(), hN.data(), nm, ma, labels, at);
+        const long long pairs = matched_pairs(t, t, true);
+        if (pairs <= kDirectPairs && direct_is_faster(t, t, pairs, true, rep)) {
+            build_plan(hQ.data(), hN.data(), nm, ma, labels, p);
+            rc = local_direct(MODE == SYMM_RFP ? DIRECT_SYMM_RFP : DIRECT_SYMM_DENSE, p, X, p, X,
+                              rep, cy, static_cast<double *>(out), TM_LOCAL_SYMM, stream);
+            if (rc != KF_ERR_NOMEM) return rc;
+        }
     }
     std::vector<int> perm, Qp, Np;
     if (windows_masked(rep, ns)) {
@@ -1350,7 +1421,8 @@ int symm_impl(int precision, const double *X, const int *Q, const int *N, int nm
         build_plan(hQ.data(), hN.data(), nm, ma, labels, p);
     }
     DevicePacked d;
-    const int mb = ns ? MB : symm_block(pairs);
+    int mb = MB, mb2 = MB;
+    if (ns == 0) choose_blocks(row_table(p), row_table(p), true, rep, mb, mb2);
     if ((rc = upload_and_pack(p, perm, X, rep, ns, mb, WS_PACK, WS_PLAN, stream, d))) return rc;
     const int nblk = d.nblk;
     const int2 *order = nullptr;
@@ -1415,15 +1487,18 @@ extern "C" int kf_local_kernel(int precision, const double *X1, const double *X2
                                 static_cast<float *>(K), stream);
     }
     const double cy = -kExpScale / (2.0 * sigma * sigma);  // squared distance -> exp_scaled's y
-    const long long pairs =
-        matched_pairs(label_counts(q1.data(), n1.data(), nm1, max_atoms1, labels),
-                      label_counts(q2.data(), n2.data(), nm2, max_atoms2, labels), false);
-    if (ns == 0 && pairs <= kDirectPairs) {
-        build_plan(q1.data(), n1.data(), nm1, max_atoms1, labels, p1);
-        build_plan(q2.data(), n2.data(), nm2, max_atoms2, labels, p2);
-        rc = local_direct(DIRECT_RECT, p1, X1, p2, X2, rep, cy, static_cast<double *>(K),
-                          TM_LOCAL_RECT, stream);
-        if (rc != KF_ERR_NOMEM) return rc;
+    if (ns == 0) {
+        std::vector<int> at1, at2;
+        const RowTable t1 = count_rows(q1.data(), n1.data(), nm1, max_atoms1, labels, at1),
+                       t2 = count_rows(q2.data(), n2.data(), nm2, max_atoms2, labels, at2);
+        const long long pairs = matched_pairs(t1, t2, false);
+        if (pairs <= kDirectPairs && direct_is_faster(t1, t2, pairs, false, rep)) {
+            build_plan(q1.data(), n1.data(), nm1, max_atoms1, labels, p1);
+            build_plan(q2.data(), n2.data(), nm2, max_atoms2, labels, p2);
+            rc = local_direct(DIRECT_RECT, p1, X1, p2, X2, rep, cy, static_cast<double *>(K),
+                              TM_LOCAL_RECT, stream);
+            if (rc != KF_ERR_NOMEM) return rc;
+        }
     }
     std::vector<int> perm1, perm2;
     if (windows_masked(rep, ns)) {
@@ -1444,7 +1519,7 @@ extern "C" int kf_local_kernel(int precision, const double *X1, const double *X2
     }
     DevicePacked d1, d2;
     int mb1 = MB, mb2 = MB;
-    if (ns == 0) rect_blocks(pairs, mb1, mb2);
+    if (ns == 0) choose_blocks(row_table(p1), row_table(p2), false, rep, mb1, mb2);
     if ((rc = upload_and_pack(p1, perm1, X1, rep, ns, mb1, WS_PACK, WS_PLAN, stream, d1))) return rc;
     if ((rc = upload_and_pack(p2, perm2, X2, rep, ns, mb2, WS_PACK2, WS_PLAN2, stream, d2))) return rc;
     const int nblk1 = d1.nblk, nblk2 = d2.nblk;

@@ -171,6 +171,38 @@ def windowed_set(nm, ma, rep, nlab, seed, ngroups=7):
     return x, q, n
 
 
+def ragged_set(nm, ma, rep, seed):
+    """windowed_set with molecules without atoms, two common labels and a third one that only
+    the first nine molecules have (no row in any other block)."""
+    x, q, n = windowed_set(nm, ma, rep, 2, seed)
+    n = np.random.default_rng(seed).integers(0, ma + 1, nm).astype(np.int32)
+    n[:9] = ma
+    q[:9, 0] = 2
+    return x, q, n
+
+
+# the blocked form's blocks: 24, 32 and 64 molecules, and 24 where no window is masked
+@pytest.mark.parametrize("nm,ma,rep", [(150, 9, 720), (700, 4, 33), (900, 2, 40), (130, 7, 2100)])
+def test_blocked_symm_blocks(lk, nm, ma, rep):
+    x, q, n = ragged_set(nm, ma, rep, nm)
+    s = 0.35 * np.sqrt(rep)
+    b = Blocked(lk)
+    assert rel_err(b.kernel_gaussian_symm(x, q, n, s), oracle.kernel_symm(x, q, n, s)) < 1e-12
+    assert rel_err(b.kernel_gaussian_symm_rfp(x, q, n, s),
+                   oracle.kernel_symm_rfp(x, q, n, s)) < 1e-12
+
+
+# 16 x 32, 32 x 64 and 64 x 64 molecules, and 16 x 32 where no window is masked
+@pytest.mark.parametrize("nm1,ma1,nm2,ma2,rep", [(60, 9, 200, 8, 720), (300, 3, 2000, 4, 40),
+                                                 (300, 2, 900, 2, 40), (40, 7, 90, 5, 2100)])
+def test_blocked_rect_blocks(lk, nm1, ma1, nm2, ma2, rep):
+    x1, q1, n1 = ragged_set(nm1, ma1, rep, nm1)
+    x2, q2, n2 = ragged_set(nm2, ma2, rep, nm2 + 1)
+    s = 0.35 * np.sqrt(rep)
+    assert rel_err(Blocked(lk).kernel_gaussian(x1, x2, q1, q2, n1, n2, s),
+                   oracle.kernel_rect(x1, x2, q1, q2, n1, n2, s)) < 1e-12
+
+
 @pytest.mark.parametrize("nm,ma,rep,nlab", [(300, 7, 720, 3), (200, 5, 1500, 2), (150, 4, 2100, 2),
                                             (129, 6, 40, 2)])
 def test_symm_zero_windows(lk, nm, ma, rep, nlab):
