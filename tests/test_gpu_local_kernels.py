@@ -224,6 +224,39 @@ def test_rect_zero_windows(lk, nm1, nm2, rep):
     assert rel_err(K, oracle.kernel_rect(x1, x2, q1, q2, n1, n2, sigma)) < 1e-12
 
 
+# the sets above and below through the blocked form, which their sizes alone would not reach
+def test_blocked_zero_windows(lk):
+    b = Blocked(lk)
+    for case in ((300, 7, 720, 3), (200, 5, 1500, 2), (150, 4, 2100, 2), (129, 6, 40, 2)):
+        test_symm_zero_windows(b, *case)
+    for case in ((250, 190, 720), (70, 130, 1100)):
+        test_rect_zero_windows(b, *case)
+
+
+def test_blocked_random_sets(lk):
+    b = Blocked(lk)
+    for case in ((1, 3, 7, 2), (13, 5, 9, 3), (70, 6, 33, 4), (130, 9, 720, 5)):
+        test_symm_and_rfp_random(b, *case)
+    for case in ((1, 1), (5, 40), (100, 7)):
+        test_rect_random(b, *case)
+
+
+@pytest.mark.parametrize("sigma", [4.0, 1.0, 0.5, 0.25])
+def test_blocked_exp_range(lk, sigma):
+    test_exp_range_exact_distances(Blocked(lk), sigma)
+
+
+def test_blocked_config0(lk, config0):
+    test_config0_descriptors(Blocked(lk), config0)
+
+
+def test_blocked_clamps_counts(lk):
+    x, q, n = random_set(9, 4, 8, 2, 3)
+    n[0], n[1] = 99, -3
+    assert rel_err(Blocked(lk).kernel_gaussian_symm(x, q, n, 1.0),
+                   oracle.kernel_symm(x, q, n, 1.0)) < 1e-12
+
+
 def test_config0_descriptors(lk, config0):
     _, _, _, C, Q, N = config0
     X = oracle.fchl19_batch(C, Q, N)
