@@ -207,7 +207,8 @@ __device__ inline void load4(const double *p, double (&v)[4]) {
 // and per 16 training rows the row sums of e aE + c inner (ep) and of B (wp).
 template <int MF, int NFT, int KW>
 __global__ __launch_bounds__(NT, 2) void coef_kernel(
-    const MvSeg *__restrict__ segs, int nseg, int items, const double *__restrict__ Xq, int qrows,
+    const MvSeg *__restrict__ segs, int nseg, int items, const double *__restrict__ Xq, int row0,
+    int qrows,
     const double *__restrict__ nq, const double *__restrict__ zq, const double *__restrict__ P2,
     const double *__restrict__ n2, const double *__restrict__ rdot,
     const double *__restrict__ aE, int nfp, double cexp,
@@ -217,12 +218,12 @@ __global__ __launch_bounds__(NT, 2) void coef_kernel(
     const int item = KW == 1 ? xcd_tile() * 4 + wv : xcd_tile();
     if (item >= items) return;
     const MvSeg S = segs[find_seg(segs, nseg, item, [](const MvSeg &t) { return t.it1; })];
-    const int mt = (S.R1 + 16 * MF - 1) / (16 * MF);
+    const int mt = (S.R1 + 16 * MF - 1) / (16 * MF), q0 = S.q0 - row0;
     const int loc = item - S.it1, m0 = (loc % mt) * 16 * MF, n0 = (loc / mt) * 16 * NFT;
     const double *pa[MF], *pb[NFT], *pd[NFT];
 #pragma unroll
     for (int m = 0; m < MF; ++m)
-        pa[m] = Xq + (size_t)min(S.q0 + m0 + 16 * m + r, qrows - 1) * nfp + 2 * g;
+        pa[m] = Xq + (size_t)min(q0 + m0 + 16 * m + r, qrows - 1) * nfp + 2 * g;
 #pragma unroll
     for (int n = 0; n < NFT; ++n) {
         pb[n] = P2 + (size_t)(2 * S.r2 + min(n0 + 16 * n + r, S.R2p - 1)) * nfp + 2 * g;
@@ -294,7 +295,7 @@ __global__ __launch_bounds__(NT, 2) void coef_kernel(
                         pv += red[w][(m * NFT + n) * 8 + 4 + v][lane];
                     }
                 }
-                const int qr = min(S.q0 + row, qrows - 1);
+                const int qr = min(q0 + row, qrows - 1);
                 const double q = nq[qr];
                 const double d2 = fmax(q + nt - 2.0 * sv, 0.0);
                 const double e = live ? exp(cexp * d2) : 0.0, c = e * inv_s2;
@@ -537,7 +538,8 @@ struct MvRound {
 
 struct MvLayout {
     int nm1 = 0, ma1 = 0, rep = 0, nf = 0, nfp = 0, parts = 1;
-    int q_rows = 0, t_rows = 0;             // packed rows, padding included
+    int q_rows = 0, t_rows = 0;             // packed rows, padding included: of the longest
+                                            // round, of the training set
     std::vector<int> offs, src1, src2, inv;  // force offsets, packed rows' sources, columns
     std::vector<int> src0;                   // query atoms without a partner
     std::vector<MvSeg> segs;
@@ -577,12 +579,15 @@ struct MvDev {
 
 int round_up16(int n) { return (n + 15) & ~15; }
 
-// T of one round stays within this many doubles (1 GiB), whatever the query set's size.
+// The packed query rows of one round with their parts of T and G stay within this many doubles
+// (1 GiB), whatever the query set's size.
 constexpr size_t kTBudget = (size_t(1) << 30) / sizeof(double);
 
-void mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, int ma1,
+// The layout of all labels of the query set, or of its `only`th (with `parts` runs of features
+// then); returns how many there are.
+int mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, int ma1,
                const std::vector<int> &q2, const std::vector<int> &n2, int nm2, int ma2, int rep,
-               const int *flag, bool forces, MvLayout &L) {
+               const int *flag, bool forces, MvLayout &L, int only = -1, int parts = 0) {
     L.nm1 = nm1;
     L.ma1 = ma1;
     L.rep = rep;
@@ -638,12 +643,13 @@ void mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, 
         L.T_len = std::max(L.T_len, forces ? T + (T & 1) : 0);
         L.G_len = std::max(L.G_len, forces ? G : 0);
         L.e_len = std::max(L.e_len, E);
+        L.q_rows = std::max(L.q_rows, R.rows);
         L.rounds.push_back(R);
         T = G = E = 0;
         R = MvRound{};
     };
     size_t held = 0;
-    for (int l = 0; l < p1.nlabels; ++l) {
+    for (int l = only < 0 ? 0 : only; l < (only < 0 ? p1.nlabels : only + 1); ++l) {
         const int *m1 = &p1.mol_row[(size_t)l * (nm1 + 1)];
         const int R1 = m1[nm1] - m1[0];
         int R2 = 0, b2 = 0;
@@ -660,12 +666,12 @@ void mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, 
         const int R2p = round_up16(R2);
         L.src2.insert(L.src2.end(), p2.src.begin() + b2, p2.src.begin() + b2 + R2);
         L.src2.insert(L.src2.end(), R2p - R2, -1);
-        const int qb = std::max<int>(64, (int)std::min<size_t>(
-                                             (size_t)round_up16(R1),
-                                             kTBudget / std::max(1, 2 * R2p) / 64 * 64));
+        const size_t per_row = 2 * ((size_t)R2p + L.nfp);
+        const int qb = std::max<int>(
+            64, (int)std::min<size_t>((size_t)round_up16(R1), kTBudget / per_row / 64 * 64));
         for (int x = 0; x < R1; x += qb) {
             const int n = std::min(qb, R1 - x), np = round_up16(n);
-            const size_t need = (size_t)n * 2 * R2p;
+            const size_t need = n * per_row;
             if (R.nseg > 0 && held + need > kTBudget) {
                 close();
                 held = 0;
@@ -685,13 +691,14 @@ void mv_layout(const std::vector<int> &q1, const std::vector<int> &n1, int nm1, 
         r2 += R2p;
     }
     close();
-    L.q_rows = q0;
     L.t_rows = r2;
     // runs of features per query row in the back-projection: 2,048 work-groups, at most 16;
     // a run is held in LDS, 4,096 features (32 KB) at most
-    L.parts = q0 == 0 ? 1
-                      : std::max({1, (rep + 4095) / 4096,
-                                  std::min({16, 2048 / q0, (rep + 31) / 32})});
+    const int least = (rep + 4095) / 4096;
+    L.parts = parts > 0 ? std::max(parts, least)
+              : q0 == 0 ? 1
+                        : std::max(least, std::min({16, 2048 / q0, (rep + 31) / 32}));
+    return p1.nlabels;
 }
 
 MvDev mv_place(const MvLayout &L, char *meta, double *train, double *query, double *acc) {
@@ -738,26 +745,26 @@ int mv_zero_unmatched(const MvLayout &L, const MvDev &D, bool forces, hipStream_
     });
 }
 
-// mode bits: 1 E, 2 F
+// The per-atom energies (mode bit 1) and back-projections (bit 2) of the layout's labels.
 template <typename T>
-int mv_run(const MvLayout &L, const MvDev &D, const T *X1, const T *dX1, double sigma,
-           double *E, double *F, int mode, hipStream_t stream) {
+int mv_run(const MvLayout &L, const MvDev &D, const T *X1, const T *dX1, double sigma, int mode,
+           hipStream_t stream) {
     const double cexp = -1.0 / (2.0 * sigma * sigma), inv_s2 = 1.0 / (sigma * sigma);
     const int natoms = L.nm1 * L.ma1;
-    int rc = for_groups((L.q_rows + 3) / 4, [&](size_t first, unsigned n) {
-        hipLaunchKernelGGL(pack_rows_kernel<T>, dim3(n), dim3(NT), 0, stream, X1,
-                           (const T *)nullptr, D.src1, L.q_rows, first, L.ma1, L.rep, D.inv, L.nf,
-                           L.nfp, D.segs, (int)L.segs.size(), (const T *)nullptr, D.Xq, D.nq,
-                           D.zq, (double *)nullptr);
-    });
-    if (rc) return rc;
     const bool forces = mode & 2;
     for (const MvRound &R : L.rounds) {
         const MvSeg *segs = D.segs + R.seg0;
+        const int rc = for_groups((R.rows + 3) / 4, [&](size_t first, unsigned n) {
+            hipLaunchKernelGGL(pack_rows_kernel<T>, dim3(n), dim3(NT), 0, stream, X1,
+                               (const T *)nullptr, D.src1 + R.row0, R.rows, first, L.ma1, L.rep,
+                               D.inv, L.nf, L.nfp, segs, R.nseg, (const T *)nullptr, D.Xq, D.nq,
+                               D.zq, (double *)nullptr);
+        });
+        if (rc) return rc;
         if (R.items1 > 0) {
             auto coef = [&](auto kern, int per) {
                 hipLaunchKernelGGL(kern, dim3((R.items1 + per - 1) / per), dim3(NT), 0, stream,
-                                   segs, R.nseg, R.items1, D.Xq, L.q_rows, D.nq, D.zq, D.P2,
+                                   segs, R.nseg, R.items1, D.Xq, R.row0, R.rows, D.nq, D.zq, D.P2,
                                    D.n2, D.rdot, D.aE, L.nfp, cexp, inv_s2,
                                    forces ? D.T : (double *)nullptr, D.ep, D.wp);
             };
@@ -780,10 +787,17 @@ int mv_run(const MvLayout &L, const MvDev &D, const T *X1, const T *dX1, double 
                            forces ? D.Fat : (double *)nullptr);
         KF_HIP_TRY(hipGetLastError());
     }
+    return KF_OK;
+}
+
+// E and F from the per-atom sums of mv_run
+int mv_reduce(const MvLayout &L, const MvDev &D, double *E, double *F, int mode,
+              hipStream_t stream) {
     return for_groups(L.nm1, [&](size_t first, unsigned n) {
         hipLaunchKernelGGL(reduce_mol_kernel, dim3(n), dim3(kReduceThreads), 0, stream, D.erow,
-                           D.Fat, L.parts, D.offs, natoms, L.ma1, first,
-                           (mode & 1) ? E : (double *)nullptr, forces ? F : (double *)nullptr);
+                           D.Fat, L.parts, D.offs, L.nm1 * L.ma1, L.ma1, first,
+                           (mode & 1) ? E : (double *)nullptr,
+                           (mode & 2) ? F : (double *)nullptr);
     });
 }
 
@@ -844,27 +858,37 @@ int matvec_impl(const T *X1, const T *dX1, const T *X2, const T *ad, const T *aE
     if ((rc = mv_read(Q1, N1, nm1, ma1, X2, ad, Q2, N2, nm2, ma2, rep, q1, n1, q2, n2, flag,
                       stream)))
         return rc;
-    MvLayout L;
-    mv_layout(q1, n1, nm1, ma1, q2, n2, nm2, ma2, rep, flag.data(), mode & 2, L);
-    char *meta = static_cast<char *>(workspace(WS_PLAN, L.meta_bytes(), stream));
-    char *stage = static_cast<char *>(host_staging(WS_PLAN, L.meta_bytes()));
-    const size_t qb = sizeof(double) * L.query_doubles();
-    // (not in WS_PACK or WS_PACK2: the matrix-free solver keeps its operands there)
-    const size_t tpad = (L.train_doubles() + 31) & ~size_t(31);
-    double *train = static_cast<double *>(workspace(WS_AUX2, sizeof(double) * tpad + qb, stream));
-    double *query = train + tpad;
-    double *acc = static_cast<double *>(
-        workspace(WS_AUX3, sizeof(double) * L.acc_doubles(mode & 2), stream));
-    KF_REQUIRE(meta && stage && train && acc, KF_ERR_NOMEM,
-               "workspace allocation failed (%zu B)", sizeof(double) * tpad + qb);
-    L.write_meta(stage);
-    KF_HIP_TRY(hipMemcpyAsync(meta, stage, L.meta_bytes(), hipMemcpyHostToDevice, stream));
-    const MvDev D = mv_place(L, meta, train, query, acc);
-    ScopedTimer timer(TM_MATVEC, stream);
-    if ((rc = mv_pack_train(L, D, X2, ad, (mode & 4) ? aE : (const T *)nullptr, ma2, stream)))
-        return rc;
-    if ((rc = mv_zero_unmatched(L, D, mode & 2, stream))) return rc;
-    return mv_run(L, D, X1, dX1, sigma, E, F, mode, stream);
+    // All labels in one layout; where its scratch is refused, one label after another, each
+    // with the scratch of its own rows alone (and one run of features).
+    int nlabels = 1;
+    for (int only = -1; only < nlabels; ++only) {
+        MvLayout L;
+        nlabels = mv_layout(q1, n1, nm1, ma1, q2, n2, nm2, ma2, rep, flag.data(), mode & 2, L,
+                            only, only < 0 ? 0 : 1);
+        if (only >= nlabels) break;  // no atoms at all
+        if (only > 0) KF_HIP_TRY(hipStreamSynchronize(stream));  // the staging is still read
+        char *meta = static_cast<char *>(workspace(WS_PLAN, L.meta_bytes(), stream));
+        char *stage = static_cast<char *>(host_staging(WS_PLAN, L.meta_bytes()));
+        const size_t qb = sizeof(double) * L.query_doubles();
+        // (not in WS_PACK or WS_PACK2: the matrix-free solver keeps its operands there)
+        const size_t tpad = (L.train_doubles() + 31) & ~size_t(31);
+        double *train = static_cast<double *>(workspace(WS_AUX2, sizeof(double) * tpad + qb, stream));
+        double *acc = static_cast<double *>(
+            workspace(WS_AUX3, sizeof(double) * L.acc_doubles(mode & 2), stream));
+        if (only < 0 && nlabels > 0 && !(meta && stage && train && acc)) continue;
+        KF_REQUIRE(meta && stage && train && acc, KF_ERR_NOMEM,
+                   "workspace allocation failed (%zu B)", sizeof(double) * tpad + qb);
+        L.write_meta(stage);
+        KF_HIP_TRY(hipMemcpyAsync(meta, stage, L.meta_bytes(), hipMemcpyHostToDevice, stream));
+        const MvDev D = mv_place(L, meta, train, train + tpad, acc);
+        ScopedTimer timer(TM_MATVEC, stream);
+        if ((rc = mv_pack_train(L, D, X2, ad, (mode & 4) ? aE : (const T *)nullptr, ma2, stream)) ||
+            (rc = mv_zero_unmatched(L, D, mode & 2, stream)) ||
+            (rc = mv_run(L, D, X1, dX1, sigma, mode, stream)))
+            return rc;
+        if (only < 0 || only + 1 == nlabels) return mv_reduce(L, D, E, F, mode, stream);
+    }
+    return KF_OK;
 }
 
 }  // namespace
@@ -942,7 +966,8 @@ int plan_execute(const kf_matvec_plan *P, const double *X1, const double *dX1, d
     KF_HIP_TRY(hipGetDevice(&dev));
     KF_REQUIRE(dev == P->device, KF_ERR_ARG, "plan was created on device %d, current is %d",
                P->device, dev);
-    return mv_run(P->layout, P->dev, X1, dX1, P->sigma, E, F, 1 | 2, stream);
+    const int rc = mv_run(P->layout, P->dev, X1, dX1, P->sigma, 1 | 2, stream);
+    return rc ? rc : mv_reduce(P->layout, P->dev, E, F, 1 | 2, stream);
 }
 
 }  // namespace

@@ -444,3 +444,35 @@ def test_refused_scratch(lk):
             done.append(left)
     assert done[:1] == [0]  # the last request is one that it can do without
     assert rel_err(lk.kernel_gaussian_hessian_symm(X, dX, Q, N, 1.7), want) < TOL
+
+
+@pytest.mark.parametrize("nlab2", [3, 2, 1])
+def test_matvec_refused_scratch(lk, nlab2):
+    """Each workspace request of the matvecs refused in turn: the product goes label by label,
+    labels without a partner among them, or the call says that memory is out."""
+    from kernelforge_amd import capi
+
+    X1, dX1, Q1, N1 = rand_set(9, 6, 70, 3, 91, 2)
+    X2, _, Q2, N2 = rand_set(12, 5, 70, nlab2, 92, 1)
+    rng = np.random.default_rng(9)
+    ad, aE, s = rng.standard_normal(X2.shape), rng.standard_normal(12), 1.5
+    ad[np.arange(5)[None] >= N2[:, None]] = 0.0
+    calls = {
+        "full": lambda: lk.kernel_gaussian_local_full_matvec(X1, dX1, X2, ad, aE, Q1, Q2, N1, N2, s),
+        "forces": lambda: (lk.kernel_gaussian_local_hessian_matvec(X1, dX1, X2, ad, Q1, Q2, N1,
+                                                                   N2, s),),
+        "energies": lambda: (lk.kernel_gaussian_local_jacobian_t_matvec(X1, X2, ad, Q1, Q2, N1,
+                                                                        N2, s),)}
+    for name, call in calls.items():
+        want, went_on = call(), 0
+        for nth in range(1, 6):
+            capi.lib().kf_workspace_refuse(nth)
+            try:
+                got = call()
+            except (MemoryError, RuntimeError):
+                got = None
+            left = capi.lib().kf_workspace_refuse(0)
+            if got is not None:
+                assert all(rel_err(g, w) < TOL for g, w in zip(got, want)), (name, nth)
+                went_on += left == 0
+        assert went_on == 3, name  # the plan, the operands and the per-atom sums
