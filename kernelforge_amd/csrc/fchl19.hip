@@ -51,6 +51,14 @@ __device__ inline int pair_channel(int nelem, int p, int q) {
     return p * nelem - p * (p - 1) / 2 + (q - p);
 }
 
+// The x-th pair j < k of n, counted j by j.
+__device__ inline void triangle_at(int n, int x, int &j, int &k) {
+    j = (int)((2 * n - 1 - sqrtf((float)((2 * n - 1) * (2 * n - 1) - 8 * x))) * 0.5f);
+    while (j > 0 && x < j * (2 * n - j - 1) / 2) --j;
+    while (x >= (j + 1) * (2 * n - j - 2) / 2) ++j;
+    k = j + 1 + x - j * (2 * n - j - 1) / 2;
+}
+
 __device__ inline double cut_fn(double r, double cut) {
     const double inv = cut > 0.0 ? 1.0 / cut : 0.0;
     return 0.5 * (cospi(r * inv) + 1.0);
@@ -114,6 +122,13 @@ __device__ inline void wave_sync() {
 // 2.30 ms (5.40 with a read-modify-write of an LDS accumulator per record and slot, 3.33 with
 // a wave per centre, 2.65 with one radial term per thread); without the exponential sums 1.5,
 // without the pair geometry 1.7, without both 1.0, of which the stores 0.4.
+//
+// LONG: molecules whose batches are of so few items (10 for one element and a centre at a time)
+// that most of a work-group would be idle, or whose centres have more pairs than fit at once.
+// Several lanes share an item and add up what they have at its end, and a chunk's pairs are
+// found from their places instead of going through all pairs again.  1,000 molecules of one
+// element: 60 atoms 4.8 ms (24.5 without, 12.0 with an accumulator in LDS), 128 atoms 51 (380,
+// 104); of five elements 5.0 and 69 ms.
 // ---------------------------------------------------------------------------
 constexpr int kRepThreads = 256;
 constexpr int kLB = 2;  // radial terms per thread
@@ -142,7 +157,22 @@ __host__ inline size_t rep_lds_bytes(int ma, int nelem, int nchan, int na) {
     return sizeof(double) * (size_t)g.ints + sizeof(int) * (size_t)g.total_ints;
 }
 
-template <typename O>
+// Centres of an n-atom molecule taken at a time.
+__host__ __device__ inline int rep_batch(const RepLds &g, int n) {
+    const int npair = (n - 1) * (n - 2) / 2;
+    const int by_nbr = g.nbrs / n, by_pair = npair > 0 ? g.pairs / npair : n;
+    const int b = by_nbr < by_pair ? by_nbr : by_pair;
+    return b > 1 ? b : 1;
+}
+// Lanes that share one of a batch's (channel, centre, radial terms) items, as a power of 2: at
+// most 64, up to four lanes of work per thread, and 32 and more of the centre's pairs each.
+__host__ __device__ inline int rep_share_log(int items, int npair) {
+    int lg = 0;
+    while (lg < 6 && (2 << lg) * items <= 4 * kRepThreads && 64 << lg <= npair) ++lg;
+    return lg;
+}
+
+template <typename O, bool LONG>
 __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
     const double *__restrict__ coords, const int *__restrict__ Q, const int *__restrict__ N,
     FchlParams P, O *__restrict__ X, int *__restrict__ err) {
@@ -214,7 +244,9 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
     __syncthreads();
 
     const int npair = (n - 1) * (n - 2) / 2;
-    const int batch = max(1, min(g.nbrs / n, npair > 0 ? g.pairs / npair : n));
+    const int batch = rep_batch(g, n);
+    const int nlb = (P.nb3 + kLB - 1) / kLB;
+    const int lg = LONG ? rep_share_log(nchan * nlb * batch, npair) : 0, share = 1 << lg;
     const double ysc = -P.eta3 * kExpScale;
     for (int i0 = row0; i0 < cen1; i0 += batch) {
         const int B = min(batch, cen1 - i0);
@@ -261,20 +293,38 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
             // place is its channel's first one plus its index in the channel
             const float inv_np = 1.0f / (float)max(npair, 1);
             const int n1 = n - 1;
-            for (int t = tid; t < B * npair; t += kRepThreads) {
-                const int b = (int)(((float)t + 0.5f) * inv_np), x = t - b * npair, i = i0 + b;
-                int ja = (int)((2 * n1 - 1 - sqrtf((float)((2 * n1 - 1) * (2 * n1 - 1) - 8 * x))) * 0.5f);
-                while (ja > 0 && x < ja * (2 * n1 - ja - 1) / 2) --ja;
-                while (x >= (ja + 1) * (2 * n1 - ja - 2) / 2) ++ja;
-                const int ka = ja + 1 + x - ja * (2 * n1 - ja - 1) / 2;
+            const bool chunked = LONG && npair > g.pairs;
+            for (int t = tid; t < (chunked ? qn : B * npair); t += kRepThreads) {
+                const int b = chunked ? 0 : (int)(((float)t + 0.5f) * inv_np), i = i0 + b;
                 const int pi = place[i], ei = el[i];
+                int at, ja, ka;
+                if (chunked) {  // the other way: from the place, channel by channel
+                    const int *cs = cst + ei * (nchan + 1), x = q0 + t;
+                    int c = 0;
+                    for (int h = nchan; h - c > 1;) {
+                        const int mid = (c + h) >> 1;
+                        if (cs[mid] <= x) c = mid;
+                        else h = mid;
+                    }
+                    const int p = chan[c] >> 16, q = chan[c] & 0xffff, y = x - cs[c];
+                    const int np = est[p + 1] - est[p] - (p == ei), nq = est[q + 1] - est[q] - (q == ei);
+                    int jl, kl;
+                    if (p == q) triangle_at(np, y, jl, kl);
+                    else jl = y / nq, kl = y - jl * nq;
+                    at = t;
+                    ja = est[p] + jl - (p > ei);
+                    ka = est[q] + kl - (q > ei);
+                } else {
+                    triangle_at(n1, t - b * npair, ja, ka);
+                }
                 const int j = ord[ja + (ja >= pi)], k = ord[ka + (ka >= pi)];
-                const int p = el[j], q = el[k];
-                const int jl = ja - est[p] + (p > ei), kl = ka - est[q] + (q > ei);
-                const int np = est[p + 1] - est[p] - (p == ei), nq = est[q + 1] - est[q] - (q == ei);
-                const int at = cst[ei * (nchan + 1) + pair_channel(nelem, p, q)] +
-                               (p == q ? jl * (2 * np - jl - 1) / 2 + kl - jl - 1 : jl * nq + kl) - q0;
-                if (B == 1 && (at < 0 || at >= qn)) continue;  // another chunk's
+                if (!chunked) {
+                    const int p = el[j], q = el[k];
+                    const int jl = ja - est[p] + (p > ei), kl = ka - est[q] + (q > ei);
+                    const int np = est[p + 1] - est[p] - (p == ei), nq = est[q + 1] - est[q] - (q == ei);
+                    at = cst[ei * (nchan + 1) + pair_channel(nelem, p, q)] +
+                         (p == q ? jl * (2 * np - jl - 1) / 2 + kl - jl - 1 : jl * nq + kl);
+                }
                 const int xj = b * n + j, xk = b * n + k;
                 const double rij = rr[xj], rik = rr[xk];
                 double fa = 0.0, ci = 0.0, rb = 0.0;
@@ -308,16 +358,16 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
                 }
             }
             __syncthreads();
-            // (channel, centre, kLB radial terms)
-            const int nlb = (P.nb3 + kLB - 1) / kLB;
+            // (channel, centre, kLB radial terms), `share` lanes each
             for (;;) {
                 // the waves draw 64 items at a time: channels differ in length
                 int t0 = 0;
                 if ((tid & 63) == 0) t0 = atomicAdd(&next, 64);
                 const int t = __shfl(t0, 0, 64) + (tid & 63);
-                if (t - (tid & 63) >= nchan * B * nlb) break;
-                if (t >= nchan * B * nlb) continue;
-                const int cb = t / nlb, l0 = (t - cb * nlb) * kLB, c = cb / B, b = cb - c * B,
+                if (t - (tid & 63) >= nchan * B * nlb << lg) break;
+                if (t >= nchan * B * nlb << lg) continue;
+                const int it = t >> lg, part = t & (share - 1);
+                const int cb = it / nlb, l0 = (it - cb * nlb) * kLB, c = cb / B, b = cb - c * B,
                           i = i0 + b;
                 const int *cs = cst + el[i] * (nchan + 1);
                 const int lo = max(cs[c], q0) - q0, hi = min(cs[c + 1], q0 + qn) - q0;
@@ -333,7 +383,7 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
 #pragma unroll
                     for (int u = 0; u < kLB; ++u) v0[u] = v1[u] = 0.0;
                     const double *a0 = amp + ta * g.pairs, *a1 = a0 + g.pairs;
-                    for (int x = b * qn + lo; x < b * qn + hi; ++x) {
+                    for (int x = b * qn + lo + part; x < b * qn + hi; x += share) {
                         const double rb = rbar[x], c0 = a0[x], c1 = a1[x];
 #pragma unroll
                         for (int u = 0; u < kLB; ++u) {
@@ -343,6 +393,14 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
                             v1[u] = fma(e, c1, v1[u]);
                         }
                     }
+                    for (int o = 1; o < share; o <<= 1) {
+#pragma unroll
+                        for (int u = 0; u < kLB; ++u) {
+                            v0[u] += __shfl_xor(v0[u], o, 64);
+                            v1[u] += __shfl_xor(v1[u], o, 64);
+                        }
+                    }
+                    if (part) continue;
 #pragma unroll
                     for (int u = 0; u < kLB; ++u) {
                         if (u >= ln) break;
@@ -541,10 +599,8 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
     // ---------------- pair records: (j, k) and (k, j) of every neighbour pair ----------------
     const int n1 = n - 1, ntri = n1 * (n1 - 1) / 2;
     for (int t = tid; t < ntri; t += kGradThreads) {
-        int ja = (int)((2 * n1 - 1 - sqrtf((float)((2 * n1 - 1) * (2 * n1 - 1) - 8 * t))) * 0.5f);
-        while (ja > 0 && t < ja * (2 * n1 - ja - 1) / 2) --ja;
-        while (t >= (ja + 1) * (2 * n1 - ja - 2) / 2) ++ja;
-        const int ka = ja + 1 + t - ja * (2 * n1 - ja - 1) / 2;
+        int ja, ka;
+        triangle_at(n1, t, ja, ka);
         const int j = ja + (ja >= i), k = ka + (ka >= i);  // neighbour index -> atom (not i)
         double *rj = rec + (size_t)(j * ma + k) * 6, *rk = rec + (size_t)(k * ma + j) * 6;
         const double rij = u4[4 * j + 3], rik = u4[4 * k + 3];
@@ -759,6 +815,12 @@ bool fchl19_fits(int ma, int nelem, int nchan, int nb2, int nb3, int na, bool gr
     return ma <= kMaxAtoms && (grad ? grad_lds_bytes(ma, nb2, nb3, na)
                                     : rep_lds_bytes(ma, nelem, nchan, na)) <= 160 * 1024;
 }
+bool fchl19_long(int ma, int nelem, int nchan, int nb3, int na) {
+    const RepLds g = rep_lds(ma, nelem, nchan, na);
+    const int npair = (ma - 1) * (ma - 2) / 2;  // (ma <= kMaxAtoms)
+    return npair > g.pairs ||
+           rep_share_log(nchan * ((nb3 + kLB - 1) / kLB) * rep_batch(g, ma), npair) > 0;
+}
 bool fchl19_one_chunk(int ma, int nelem, int nchan, int na) {
     return (long)(ma - 1) * (ma - 2) / 2 <= rep_lds(ma, nelem, nchan, na).pairs;
 }
@@ -808,8 +870,12 @@ int fchl19_impl(const double *coords, const int *Q, const int *N, int nm, int ma
         // up to a work-group per two rows while there are fewer molecules than the GPU takes
         // work-groups
         const int splits = std::max(1, std::min((ma + 1) / 2, 1024 / nm));
-        hipLaunchKernelGGL(fchl19_rep_kernel<O>, dim3(nm, splits), dim3(kRepThreads), lds, stream,
-                           coords, Q, N, P, X, err);
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(nm, splits), dim3(kRepThreads), lds, stream, coords, Q,
+                               N, P, X, err);
+        };
+        if (fchl19_long(ma, P.nelem, P.nchan, P.nb3, P.na)) launch(fchl19_rep_kernel<O, true>);
+        else launch(fchl19_rep_kernel<O, false>);
     } else {
         KF_REQUIRE(P.nelem * P.nb2 > 0, KF_ERR_BASIS, "empty two-body basis");
         // Several work-groups per centre while the batch has fewer centres than the GPU takes

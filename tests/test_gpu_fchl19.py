@@ -170,3 +170,23 @@ def test_representation_kernel_edges(fr, ma, nm, kw):
                                   [rng.choice(el, n).astype(np.int32) for n in Ns])
     X = fr.generate_fchl_acsf_batch(C, Q, N, **kw)
     assert row_rel_err(X, oracle.fchl19_batch(C, Q, N, **kw), lead=2) < 1e-12
+
+
+# molecules whose items are shared by 2 to 64 lanes: of few elements and radial terms, at the
+# sizes where the number of lanes changes, and centres whose pairs take several chunks, with
+# channels that end inside one and absent elements; a chunk's pairs with no sharing (16 elements)
+@pytest.mark.parametrize("ma,nm,kw", [
+    (13, 3, dict(elements=[8], nRs3=3)), (22, 600, dict(elements=[8])),
+    (31, 40, dict(elements=[1, 8])), (47, 3, dict(elements=[6], nRs3=1)),
+    (66, 2, dict(elements=[1, 6, 7], nFourier=3)), (101, 1, dict(elements=[1, 6])),
+    (128, 2, {}), (128, 1, dict(elements=[1], nRs3=7)), (50, 1, dict(elements=list(range(1, 17))))])
+def test_representation_long_molecules(fr, ma, nm, kw):
+    test_representation_kernel_edges(fr, ma, nm, kw)
+    if len(kw.get("elements", [])) > 1:  # one of the elements absent
+        from kernelforge_amd import synthetic
+
+        rng = np.random.default_rng(ma)
+        z = rng.choice(kw["elements"][1:], ma).astype(np.int32)
+        C, Q, N = synthetic.pad_batch([synthetic._place_atoms(rng, ma)], [z])
+        assert row_rel_err(fr.generate_fchl_acsf_batch(C, Q, N, **kw),
+                           oracle.fchl19_batch(C, Q, N, **kw), lead=2) < 1e-12
