@@ -435,7 +435,7 @@ __global__ __launch_bounds__(kRepThreads, 4) void fchl19_rep_kernel(
 // (Non-temporal stores are no faster here and cost a following reader the cached rows: the
 // back-projection of one molecule's matvec 1.8 ms instead of 1.1.)
 // ---------------------------------------------------------------------------
-constexpr int kGradThreads = 256;
+constexpr int kGradThreads = 256;  // NTG: 64 for small molecules (fchl19_impl)
 constexpr int kTwoW = 8;  // two-body scalars per neighbour
 
 // LDS of one work-group, in doubles from the start (ints at the end).
@@ -470,24 +470,24 @@ __host__ inline size_t grad_lds_bytes(int ma, int nb2, int nb3, int na) {
 }
 
 // n doubles of `src` (LDS; zeros when null) to dst, 16 bytes a lane where dst allows it.
-template <typename O>
+template <int NTG, typename O>
 __device__ inline void stream_out(O *dst, const double *src, int n) {
     constexpr int V = 16 / sizeof(O);
     typedef O vec __attribute__((ext_vector_type(V)));
     if (((reinterpret_cast<size_t>(dst) & 15) | (n % V)) == 0) {
-        for (int t = threadIdx.x; t < n / V; t += kGradThreads) {
+        for (int t = threadIdx.x; t < n / V; t += NTG) {
             vec v;
 #pragma unroll
             for (int u = 0; u < V; ++u) v[u] = src ? O(src[t * V + u]) : O(0);
             reinterpret_cast<vec *>(dst)[t] = v;
         }
     } else {
-        for (int t = threadIdx.x; t < n; t += kGradThreads) dst[t] = src ? O(src[t]) : O(0);
+        for (int t = threadIdx.x; t < n; t += NTG) dst[t] = src ? O(src[t]) : O(0);
     }
 }
 
-template <typename O>
-__global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
+template <typename O, int NTG>
+__global__ __launch_bounds__(NTG) void fchl19_grad_kernel(
     const double *__restrict__ coords, const int *__restrict__ Q, const int *__restrict__ N,
     FchlParams P, int splits, O *__restrict__ X, O *__restrict__ dX,
     int *__restrict__ err) {
@@ -525,37 +525,36 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
             nr = min(lrun, P.nb3 - l0) * P.na;
         }
     };
-    auto zero_unit = [&](int unit) {
-        int f0, nr;
-        unit_rows(unit, f0, nr);
-        for (int t = tid; t < nr; t += kGradThreads) Xi[f0 + t] = O(0);
-        stream_out<O>(dXi + (size_t)f0 * ld, nullptr, nr * ld);
+    auto zero_rows = [&](int f0, int nr) {
+        for (int t = tid; t < nr; t += NTG) Xi[f0 + t] = O(0);
+        stream_out<NTG, O>(dXi + (size_t)f0 * ld, nullptr, nr * ld);
     };
 
     bool bad = false;
     if (i < n) {
         const double *Cm = coords + (size_t)m * ma * 3;
-        for (int t = tid; t < 3 * n; t += kGradThreads) R[t] = Cm[t];
-        for (int t = tid; t < n; t += kGradThreads) {
+        for (int t = tid; t < 3 * n; t += NTG) R[t] = Cm[t];
+        for (int t = tid; t < n; t += NTG) {
             const int e = elem_index(P, Q[(size_t)m * ma + t]);
             el[t] = e;
             bad |= e < 0;
         }
-        for (int t = tid; t < 64; t += kGradThreads) tab[t] = kExp2Tab64[t];
-        for (int t = tid; t < g.tile_rows * ld; t += kGradThreads) tile[t] = 0.0;
+        for (int t = tid; t < 64; t += NTG) tab[t] = kExp2Tab64[t];
+        for (int t = tid; t < g.tile_rows * ld; t += NTG) tile[t] = 0.0;
     }
     // a molecule with an unknown element is reported through *err; its rows are zeroed
     if (__syncthreads_or(bad)) {
         if (tid == 0) *err = 1;
         bad = true;
     }
-    if (i >= n || bad) {  // padding centre: zero row and Jacobian rows
-        for (int unit = split; unit < nunits; unit += splits) zero_unit(unit);
+    if (i >= n || bad || n == 1) {  // padding centre or nothing near it: zero rows
+        const int f0 = (int)((long)P.rs * split / splits), f1 = (int)((long)P.rs * (split + 1) / splits);
+        zero_rows(f0, f1 - f0);
         return;
     }
 
     // ---------------- per neighbour ----------------
-    for (int j = tid; j < n; j += kGradThreads) {
+    for (int j = tid; j < n; j += NTG) {
         const double r = dist(R, i, j);
         // (an atom at infinity adds nothing: its vector must not make NaN of a zero factor)
         const bool far = r > 1e150;
@@ -585,12 +584,12 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
             ord[rank] = j;
         }
     }
-    for (int e = tid; e <= P.nelem; e += kGradThreads) {
+    for (int e = tid; e <= P.nelem; e += NTG) {
         int c = 0;
         for (int t = 0; t < n; ++t) c += (int)(t != i) & (el[t] < e);
         est[e] = c;
     }
-    for (int t = tid; t < n * n; t += kGradThreads) {  // no triplet (j, j)
+    for (int t = tid; t < n * n; t += NTG) {  // no triplet (j, j)
         if (t / n == t % n)
             for (int c = 0; c < 6; ++c) rec[(size_t)(t / n * ma + t % n) * 6 + c] = 0.0;
     }
@@ -598,7 +597,7 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
 
     // ---------------- pair records: (j, k) and (k, j) of every neighbour pair ----------------
     const int n1 = n - 1, ntri = n1 * (n1 - 1) / 2;
-    for (int t = tid; t < ntri; t += kGradThreads) {
+    for (int t = tid; t < ntri; t += NTG) {
         int ja, ka;
         triangle_at(n1, t, ja, ka);
         const int j = ja + (ja >= i), k = ka + (ka >= i);  // neighbour index -> atom (not i)
@@ -655,24 +654,36 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
 
     // ---------------- feature blocks ----------------
     const double ysc = -P.eta3 * kExpScale;
-    for (int unit = split; unit < nunits; unit += splits) {
-        int f0, nr;
-        unit_rows(unit, f0, nr);
-        const bool is2 = unit < P.nelem * nu2;
-        // species p (and q) of the block: neighbours ord[pb..pe) and ord[qb..qe)
-        int p = 0, q = 0;
-        if (is2) {
+    // species p (and q) of a block: neighbours ord[pb..pe) and ord[qb..qe); false where there
+    // are none
+    auto species = [&](int unit, int &p, int &q) {
+        const bool two_body = unit < P.nelem * nu2;
+        p = 0;
+        if (two_body) {
             p = q = unit / nu2;
         } else {
             int c = (unit - P.nelem * nu2) / nu3;
             while (c >= P.nelem - p) c -= P.nelem - p, ++p;
             q = p + c;
         }
-        const int pb = est[p], np = est[p + 1] - pb, qb = est[q], nq = est[q + 1] - qb;
-        if (np == 0 || nq == 0 || (!is2 && p == q && np < 2)) {
-            zero_unit(unit);
+        const int np = est[p + 1] - est[p], nq = est[q + 1] - est[q];
+        return np > 0 && nq > 0 && (two_body || p != q || np > 1);
+    };
+    for (int unit = split; unit < nunits; unit += splits) {
+        int f0, nr, p, q;
+        unit_rows(unit, f0, nr);
+        const bool is2 = unit < P.nelem * nu2;
+        if (!species(unit, p, q)) {
+            if constexpr (NTG < kGradThreads)  // with the empty blocks that follow as one run
+                for (int e0, en; splits == 1 && unit + 1 < nunits && !species(unit + 1, p, q);
+                     ++unit) {
+                    unit_rows(unit + 1, e0, en);
+                    nr = e0 + en - f0;
+                }
+            zero_rows(f0, nr);
             continue;
         }
+        const int pb = est[p], np = est[p + 1] - pb, qb = est[q], nq = est[q + 1] - qb;
         const int nact = p == q ? np : np + nq;
         const int nl = is2 ? nr : nr / P.na;
         // neighbour of item a: the block's first, then the others (their columns are zero)
@@ -684,7 +695,7 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
             if (p != q && a >= qb) a += nq;  // p < q, so its range lies behind p's
             return ord[a];
         };
-        for (int item = tid; item < n1 * nl; item += kGradThreads) {
+        for (int item = tid; item < n1 * nl; item += NTG) {
             const int a = item / nl, l = item - a * nl, j = atom_of(a);
             if (a >= nact) {
                 for (int row = is2 ? l : l * P.na, e = is2 ? row + 1 : row + P.na; row < e; ++row)
@@ -748,7 +759,7 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
         __syncthreads();
         // centre column and value of each row; in a channel of two elements every pair is
         // seen from both, so the values are summed over the first element's atoms only
-        for (int t = tid; t < 4 * nr; t += kGradThreads) {
+        for (int t = tid; t < 4 * nr; t += NTG) {
             const int row = t >> 2, d = t & 3;
             double s = 0.0;
             if (d < 3) {
@@ -760,7 +771,7 @@ __global__ __launch_bounds__(kGradThreads) void fchl19_grad_kernel(
             }
         }
         __syncthreads();
-        stream_out<O>(dXi + (size_t)f0 * ld, tile, nr * ld);
+        stream_out<NTG, O>(dXi + (size_t)f0 * ld, tile, nr * ld);
         __syncthreads();
     }
 }
@@ -882,8 +893,16 @@ int fchl19_impl(const double *coords, const int *Q, const int *N, int nm, int ma
         // work-groups (256 CUs, three each): one molecule of 21 atoms takes 20 us with 8 per centre (181 us before, one per centre)
         const long centres = (long)nm * ma;
         const int splits = centres >= 768 ? 1 : (int)std::min<long>(8, 768 / centres);
-        hipLaunchKernelGGL(fchl19_grad_kernel<O>, dim3(ma * splits, nm), dim3(kGradThreads), lds,
-                           stream, coords, Q, N, P, splits, X, dX, err);
+        auto launch = [&](auto kern, int threads) {
+            hipLaunchKernelGGL(kern, dim3(ma * splits, nm), dim3(threads), lds, stream, coords, Q,
+                               N, P, splits, X, dX, err);
+        };
+        // A small molecule's centre is a chain of short steps: one wave each keeps four times as
+        // many in flight.  20,000 molecules of 2 atoms of one element 0.17 ms (0.45 with four
+        // waves), 5,000 of 5 atoms of five elements 0.49 (1.14), 500 of 10 atoms 0.31 (0.41);
+        // 500 of 14 atoms 0.80 (0.71), and 50 of 8 atoms, which do not fill the GPU, 103 us (87).
+        if (ma <= 10 && centres >= 1024) launch(fchl19_grad_kernel<O, 64>, 64);
+        else launch(fchl19_grad_kernel<O, kGradThreads>, kGradThreads);
     }
     KF_HIP_TRY(hipGetLastError());
     KF_HIP_TRY(hipStreamSynchronize(stream));

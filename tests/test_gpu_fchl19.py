@@ -190,3 +190,13 @@ def test_representation_long_molecules(fr, ma, nm, kw):
         C, Q, N = synthetic.pad_batch([synthetic._place_atoms(rng, ma)], [z])
         assert row_rel_err(fr.generate_fchl_acsf_batch(C, Q, N, **kw),
                            oracle.fchl19_batch(C, Q, N, **kw), lead=2) < 1e-12
+
+
+# small molecules in batches that fill the GPU, a wave per centre: none, one and some
+# neighbours, blocks of absent elements on end, alone and at the end of a row
+@pytest.mark.parametrize("ma,nm,kw", [
+    (1, 1100, {}), (2, 700, dict(elements=[1, 8])), (2, 600, {}), (3, 400, dict(nRs2=3, nRs3=1)),
+    (4, 300, dict(nRs2=41, nRs3=37)), (7, 160, dict(nFourier=3)), (10, 110, {})])
+def test_jacobian_small_molecules(fr, ma, nm, kw):
+    test_jacobian_kernel_edges(fr, ma, nm, kw)
+    test_float32_results(fr, ma, nm, True, {k: v for k, v in kw.items() if k.startswith("nRs")})
