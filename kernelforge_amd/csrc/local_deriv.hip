@@ -88,8 +88,8 @@ struct DerivArgs {
     double *slot;  // per-pair scratch: e[maxm] | V[maxm][ldv] | U[maxm][ldu]
     size_t slot_len;
     int maxm, ldv, ldu;
-    const FfOrder *order1, *order2;               // a row per molecule (Hessian forms)
-    const uint2 *blocks1, *blocks2;               // ff_blocks_kernel: a word per (molecule, feature)
+    const FfOrder *order1, *order2;  // a row per molecule (Hessian forms over kFfDense atoms)
+    const uint2 *blocks1, *blocks2;  // ff_blocks_kernel: a word per (molecule, feature), as well
 };
 
 __device__ inline int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
@@ -1121,11 +1121,13 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
     const bool one_set = is_symm(MODE) || MODE == M_DIAG_BLOCKS;
     const size_t order_off = pair_off + sizeof(int2) * npairs, nm1 = s1.n.size(),
                  nm2 = one_set ? 0 : s2.n.size();
-    const size_t bytes = order_off + (has_ff(MODE) ? sizeof(FfOrder) * (nm1 + nm2) : 0);
+    // (up to kFfDense atoms no block is left out, and the atoms keep their own order)
+    const bool sparse = has_ff(MODE) && std::max(A.ma1, A.ma2) > kFfDense;
+    const size_t bytes = order_off + (sparse ? sizeof(FfOrder) * (nm1 + nm2) : 0);
     char *dev = static_cast<char *>(workspace(WS_PLAN, bytes, stream));
     char *stage = static_cast<char *>(host_staging(WS_PLAN, bytes));
     KF_REQUIRE(dev && stage, KF_ERR_NOMEM, "workspace allocation failed (%zu B)", bytes);
-    if (has_ff(MODE)) {
+    if (sparse) {
         FfOrder *o = reinterpret_cast<FfOrder *>(stage + order_off);
         for (size_t m = 0; m < nm1; ++m)
             o[m] = ff_order(s1.q.data() + m * A.ma1, (s1.offs[m + 1] - s1.offs[m]) / 3);
@@ -1142,26 +1144,26 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
 
     size_t batch = npairs;
     if (has_ff(MODE)) {
-        // which blocks of the Jacobians are not zero
-        const bool sparse = std::max(A.ma1, A.ma2) > kFfDense;
-        A.order1 = reinterpret_cast<const FfOrder *>(dev + order_off);
-        A.order2 = A.order1 + (one_set ? 0 : nm1);
-        uint2 *w = static_cast<uint2 *>(
-            workspace(WS_PLAN2, sizeof(uint2) * (nm1 + nm2) * A.rep, stream));
-        KF_REQUIRE(w, KF_ERR_NOMEM, "workspace allocation failed");
-        A.blocks1 = w;
-        A.blocks2 = one_set ? w : w + nm1 * A.rep;
-        const unsigned nrun = (A.rep + kBlkRun - 1) / kBlkRun;
-        for (int set = 0; sparse && set < (one_set ? 1 : 2); ++set) {
-            const int ma = set ? A.ma2 : A.ma1;
-            const int rc = for_groups(set ? nm2 : nm1, [&](size_t first, unsigned n) {
-                hipLaunchKernelGGL(ff_blocks_kernel, dim3(n, nrun), dim3(NT), 0, stream,
-                                   (set ? A.dx2 : A.dx1) + first * ma * A.rep * 3 * ma,
-                                   (set ? A.n2 : A.n1) + first,
-                                   (set ? A.order2 : A.order1) + first, ma, A.rep,
-                                   w + ((set ? nm1 : 0) + first) * A.rep);
-            });
-            if (rc) return rc;
+        if (sparse) {  // which blocks of the Jacobians are not zero
+            A.order1 = reinterpret_cast<const FfOrder *>(dev + order_off);
+            A.order2 = A.order1 + (one_set ? 0 : nm1);
+            uint2 *w = static_cast<uint2 *>(
+                workspace(WS_PLAN2, sizeof(uint2) * (nm1 + nm2) * A.rep, stream));
+            KF_REQUIRE(w, KF_ERR_NOMEM, "workspace allocation failed");
+            A.blocks1 = w;
+            A.blocks2 = one_set ? w : w + nm1 * A.rep;
+            const unsigned nrun = (A.rep + kBlkRun - 1) / kBlkRun;
+            for (int set = 0; set < (one_set ? 1 : 2); ++set) {
+                const int ma = set ? A.ma2 : A.ma1;
+                const int rc = for_groups(set ? nm2 : nm1, [&](size_t first, unsigned n) {
+                    hipLaunchKernelGGL(ff_blocks_kernel, dim3(n, nrun), dim3(NT), 0, stream,
+                                       (set ? A.dx2 : A.dx1) + first * ma * A.rep * 3 * ma,
+                                       (set ? A.n2 : A.n1) + first,
+                                       (set ? A.order2 : A.order1) + first, ma, A.rep,
+                                       w + ((set ? nm1 : 0) + first) * A.rep);
+                });
+                if (rc) return rc;
+            }
         }
         // slot layout and the largest matched count over the pairs
         int maxm = 1;
@@ -1258,7 +1260,9 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
             // Few pairs: each pair's features in several runs (of 32 and more), so that there
             // are about 2,048 work-groups, four per slot of the GPU (512): 703 pairs of mixed
             // molecules of 5-23 atoms 3.5 ms, 4.5 with one run each (every block taken)
+            // (not two runs of a few atoms: 465 pairs of 3 atoms, 64 features, 165 us, 135 with one)
             int runs = std::max(1, std::min((int)(2048 / nb), A.rep / 32));
+            if (!sparse && A.rep < 128) runs = 1;
             const int run = (A.rep + runs - 1) / runs;
             runs = (A.rep + run - 1) / run;  // none of them empty
             double *parts = nullptr;
