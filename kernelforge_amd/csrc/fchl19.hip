@@ -33,7 +33,7 @@ constexpr double kEps = 1e-12;
 constexpr double kSqrt2Pi = 2.5066282746310005;
 
 struct FchlParams {
-    int nelem, nb2, nb3, na, nharm, nchan, rs, three_off, max_atoms, grad_path;
+    int nelem, nb2, nb3, na, nharm, nchan, rs, three_off, max_atoms;
     int elements[kMaxElem];
     double Rs2[kMaxRs], logRs2[kMaxRs], Rs3[kMaxRs];
     double angw[kMaxHarm];
@@ -96,12 +96,6 @@ __device__ inline bool two_body(const FchlParams &P, double r, TwoBody &t, bool 
         t.df = cut_dfn(r, P.rcut);
     }
     return true;
-}
-
-__device__ inline void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // ---------------------------------------------------------------------------
@@ -798,7 +792,6 @@ int build_params(FchlParams &P, int max_atoms, const int *elements, int nelem, c
     P.three_off = nelem * nRs2;
     P.rs = P.three_off + P.nchan * nRs3 * nabasis;
     P.max_atoms = max_atoms;
-    P.grad_path = grad ? 1 : 0;
     for (int e = 0; e < kMaxElem; ++e) P.elements[e] = e < nelem ? elements[e] : 0;
     for (int k = 0; k < kMaxRs; ++k) {
         P.Rs2[k] = k < nRs2 ? Rs2[k] : 1.0;

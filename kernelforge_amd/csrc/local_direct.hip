@@ -4,18 +4,17 @@
 // windows they use and gives each work-group a block of molecule pairs, whose labels and
 // tiles it walks one after another.  For a few hundred thousand molecule pairs that leaves
 // most of the GPU waiting on the longest chain, and the packing and ordering cost as much
-// as the products.  This form has no packing: rows are read where they are, in 32 x 32
-// tiles of one label's Gram matrix (a work-group's four waves share the descriptor columns
-// of a tile while there are few tiles, a wave has a tile of its own beyond that), straight
-// from global memory into registers (32-byte loads with the summation index of a step
-// permuted the same way in both operands, as in local_matvec.hip).  The tile's rows pass
-// through the registers whole, so their squared norms come from the same loads.  The
-// exponentials go to memory (8 bytes per matched atom pair), and a second kernel sums
-// those of each molecule pair in a fixed order.
-// Measured for the symmetric kernel (whole call): 50 molecules 84 us against 1,001 of the
-// blocked form with its 64 x 64 blocks (268 with the smallest blocks), 400 molecules 301
-// against 2,499 (446), 800 molecules 826 against 3,129 (873); one molecule against 1,000
-// 129 against 474 us.
+// as the products.  This form has no packing: rows are read where they are, tile by tile of
+// one label's Gram matrix.  While there are few tiles they are 32 x 32, and a work-group's
+// four waves share a tile's descriptor columns, straight from global memory into registers
+// (two 16-byte loads of a row at a time, with the summation index of a step permuted the same
+// way in both operands, as in local_matvec.hip); beyond, they are 64 x 64 and both operands
+// go through LDS.  A tile's rows pass through the registers whole in either, so their squared
+// norms come from the same loads.  The exponentials go to memory (8 bytes per matched atom
+// pair), and a second kernel sums those of each molecule pair in a fixed order.
+// Measured for whole calls on molecules of 5-23 atoms, 720 columns: 50 molecules 77 us, 400
+// 323 (719 of the blocked form with its smallest blocks, 2,657 with 64 x 64), 800 867 (1,108,
+// 3,244); one molecule against 5,000 446 us (1,244 with 64 x 64).
 #include <algorithm>
 #include <cmath>
 
@@ -27,11 +26,11 @@ namespace {
 
 constexpr int NT = 256;
 constexpr int TE = 32;  // tile edge (rows of one label)
-// Row tiles of a band: its rows (2.9 MB of 720 columns in 32-row tiles) stay in an XCD's L2
-// while the column tiles pass, so the columns are fetched once per band instead of once per
-// row tile.
+// Row tiles of a band: while the column tiles pass, its rows are read again and again, so the
+// columns are fetched once per band instead of once per row tile.  Of 720 columns it is 2.9 MB
+// in 32-row tiles, which stay in an XCD's 4 MB of L2, and 5.9 MB in 64-row ones, which do in part.
 constexpr int BT = 16;
-constexpr int kLdsTiles = 384;
+constexpr int kLdsTiles = 384;  // 64 x 64 tiles from which on they are taken (local_direct)
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef double v2d __attribute__((ext_vector_type(2)));
 
@@ -125,8 +124,7 @@ __device__ inline void put_exps(const DirectSeg &S, const double (&s)[4], int ro
 // descriptors straight into registers: no barrier until the end, the shortest chain.
 template <bool SYMM, bool VEC>
 __global__ __launch_bounds__(NT, 3) void exp_tiles_kernel(const DirectSeg *__restrict__ segs,
-                                                          int nseg, int tiles,
-                                                          const double *__restrict__ X1,
+                                                          int nseg, const double *__restrict__ X1,
                                                           const int *__restrict__ src1,
                                                           const double *__restrict__ X2,
                                                           const int *__restrict__ src2, int rep,
@@ -229,12 +227,13 @@ __global__ __launch_bounds__(NT, 3) void exp_tiles_kernel(const DirectSeg *__res
 // barrier a step), each wave a 32 x 32 quarter.  A row's 16 columns are four threads' loads
 // of 64 contiguous bytes: with a lane per row instead (operands straight into registers)
 // every lane is a cache access of its own, and the accesses, one a cycle, bound the kernel
-// (92% of its cycles; 920 us at 800 molecules against 675 here).  LDS holds fragments in lane order, 16-byte units with
-// the row XORed by 4 (column pair) so that neither the stores nor the reads conflict.
+// (92% of its cycles; 920 us at 800 molecules against 675 here).  LDS holds fragments in lane
+// order, 16-byte units with the row XORed by 4 (column pair) so that neither the stores nor the
+// reads conflict.
 constexpr int TL = 64;
 template <bool SYMM, bool VEC>
 __global__ __launch_bounds__(NT, 4) void exp_tiles_lds_kernel(
-    const DirectSeg *__restrict__ segs, int nseg, int tiles, const double *__restrict__ X1,
+    const DirectSeg *__restrict__ segs, int nseg, const double *__restrict__ X1,
     const int *__restrict__ src1, const double *__restrict__ X2, const int *__restrict__ src2,
     int rep, double cy, double *__restrict__ Ex) {
     // [buffer][operand][row group][8-column half][lane]
@@ -464,8 +463,8 @@ int local_direct(int mode, const LocalPlan &p1, const double *X1, const LocalPla
     const bool vec = rep % 2 == 0 && ((reinterpret_cast<size_t>(X1) | reinterpret_cast<size_t>(X2)) & 15) == 0;
     if (tiles > 0) {
         auto launch = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3(tiles), dim3(NT), 0, stream, dseg, L, tiles, X1, src1, X2,
-                               src2, rep, cy, Ex);
+            hipLaunchKernelGGL(kern, dim3(tiles), dim3(NT), 0, stream, dseg, L, X1, src1, X2, src2,
+                               rep, cy, Ex);
         };
         if (symm) {
             if (lds) vec ? launch(exp_tiles_lds_kernel<true, true>) : launch(exp_tiles_lds_kernel<true, false>);

@@ -29,9 +29,9 @@
 // training rows can be read.
 //
 // Measured (whole calls on 21-atom C/H/O conformers, with the descriptors): one molecule
-// against 200 in a plan 84 us (2,110 before: one wave per atom for the back-projection,
+// against 200 in a plan 81 us (2,110 before: one wave per atom for the back-projection,
 // 64-row tiles without splits for the products); 100 against 1,000, float32 in and out,
-// 2.6 ms (8.6), of which the two products 0.56 ms each at 36 TFLOP/s.
+// 1.7 ms (8.5), of which the two products 0.5 ms each at 36 TFLOP/s.
 #include <algorithm>
 #include <new>
 #include <cmath>
@@ -1046,7 +1046,7 @@ extern "C" int kf_local_full_matvec(const double *X1, const double *dX1, const d
                        max_atoms2, rep, sigma, E, F, 1 | 2 | 4, as_stream(stream));
 }
 
-// 100 float32 molecules of 21 atoms against 1,000, descriptors and Jacobians included: 1.71 ms
+// 100 float32 molecules of 21 atoms against 1,000, descriptors and Jacobians included: 1.7 ms
 // (2.60 ms with FP64 copies of the operands made first; the Jacobians of the 100 molecules
 // are 0.38 GB, written and read once, where they were 0.76 GB, copied and read).
 extern "C" int kf_local_full_matvec_f32(const float *X1, const float *dX1, const float *X2,
