@@ -934,20 +934,25 @@ inline size_t ff_lds_bytes(int ma1, int ma2) {
 
 // Shape buckets by m = max(atoms of a, atoms of b): NK k-steps of 4 atoms, NP 16-column
 // force blocks (3 m columns).
-template <int MODE>
-__global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0,
-                                                         double *__restrict__ parts) {
+// SMALL: a set of up to kFfDense atoms per molecule, whose kernel holds no larger bucket: those
+// set the registers of all (256; 100 without them), and with two work-groups on a CU a pair of
+// a few atoms is a chain of waits.  E+F kernels of 800 molecules of 5 atoms of one element
+// 23.5 ms (31.9 in the kernel of all sizes), 1,500 of 3 atoms 68 (91), 400 of 10 atoms 28 (41).
+template <int MODE, bool SMALL>
+__global__ __launch_bounds__(NT, SMALL ? 4 : 2) void deriv_ff_kernel(DerivArgs A, int pair0,
+                                                                     double *__restrict__ parts) {
+    constexpr int MM = SMALL ? kFfDense * kFfDense : MAXM;
     __shared__ FfPair L;
     extern __shared__ double Jbuf[];  // two staged J_a features of the largest bucket
-    __shared__ int qa[MAXA], qb_[MAXA], ia[MAXA], ib[MAXA], ist[MAXA + 1], mi[MAXM], mj[MAXM];
-    __shared__ double mc[MAXM];
+    __shared__ int qa[MAXA], qb_[MAXA], ia[MAXA], ib[MAXA], ist[MAXA + 1], mi[MM], mj[MM];
+    __shared__ double mc[MM];
     __shared__ int s_np;
     const int tid = threadIdx.x;
     const int t = pair0 + pair_slot();
     const int a = A.pairs[t].x, b = A.pairs[t].y;
     const int na = clampi(A.n1[a], 0, A.ma1), nb = clampi(A.n2[b], 0, A.ma2);
     const int mx = na > nb ? na : nb;
-    const bool sparse = mx > kFfDense;
+    const bool sparse = !SMALL && mx > kFfDense;
     // a molecule without atoms still gets its zero EE / FE / EF entries written
     const double *slot = A.slot + (size_t)(t - pair0) * A.slot_len;
     if (tid < na) qa[tid] = A.q1[(size_t)a * A.ma1 + tid];
@@ -1017,12 +1022,17 @@ __global__ __launch_bounds__(NT, 2) void deriv_ff_kernel(DerivArgs A, int pair0,
     double *part = gridDim.y > 1 ? parts + ((size_t)(t - pair0) * gridDim.y + blockIdx.y) *
                                                A.ldv * A.ldu
                                  : nullptr;
-    if (mx <= 5) ff_pair<MODE, 2, 1>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
-    else if (mx <= 10) ff_pair<MODE, 3, 2>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
-    else if (mx <= 16) ff_pair<MODE, 4, 3>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
-    else if (mx <= 21) ff_pair<MODE, 6, 4>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
-    else if (mx <= 24) ff_pair<MODE, 6, 5>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
-    else ff_pair<MODE, 8, 6>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+    if constexpr (SMALL) {
+        if (mx <= 5) ff_pair<MODE, 2, 1>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+        else ff_pair<MODE, 3, 2>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+    } else {
+        if (mx <= 5) ff_pair<MODE, 2, 1>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+        else if (mx <= 10) ff_pair<MODE, 3, 2>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+        else if (mx <= 16) ff_pair<MODE, 4, 3>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+        else if (mx <= 21) ff_pair<MODE, 6, 4>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+        else if (mx <= 24) ff_pair<MODE, 6, 5>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+        else ff_pair<MODE, 8, 6>(A, a, b, na, nb, L, Jbuf, np, mc, slot, f0, fe, part);
+    }
 }
 
 // FF of a pair from the parts of its runs of features, in order.
@@ -1271,8 +1281,12 @@ int deriv_launch(DerivArgs A, const std::vector<int2> &pairs, const SideMeta &s1
                 parts = static_cast<double *>(workspace(WS_AUX0, bytes, stream));
                 if (!parts) runs = 1;  // (up to 150 MB that the one-run form does without)
             }
-            hipLaunchKernelGGL(deriv_ff_kernel<MODE>, dim3(nb, runs), dim3(NT),
-                               ff_lds_bytes(A.ma1, A.ma2), stream, A, (int)p0, parts);
+            auto ff = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(nb, runs), dim3(NT), ff_lds_bytes(A.ma1, A.ma2),
+                                   stream, A, (int)p0, parts);
+            };
+            if (sparse) ff(deriv_ff_kernel<MODE, false>);
+            else ff(deriv_ff_kernel<MODE, true>);
             KF_HIP_TRY(hipGetLastError());
             if (runs > 1) {
                 hipLaunchKernelGGL(ff_sum_kernel<MODE>, dim3(nb), dim3(NT), 0, stream, A, (int)p0,
