@@ -1399,7 +1399,10 @@ int symm_impl(int precision, const double *X, const int *Q, const int *N, int nm
         KF_HIP_TRY(hipMemsetAsync(out, 0, n * sizeof(double), stream));
         return KF_OK;
     }
-    if (ns == 0) {
+    // (L labels over n atoms have at least n^2 / (2 L) matched pairs: a large set is not counted)
+    double atoms = 0.0;
+    for (int a = 0; a < nm; ++a) atoms += clamp_atoms(hN[a], ma);
+    if (ns == 0 && atoms * atoms <= 2.0 * labels.size() * kDirectPairs) {
         std::vector<int> at;
         const RowTable t = count_rows(hQ.data(), hN.data(), nm, ma, labels, at);
         const long long pairs = matched_pairs(t, t, true);
