@@ -134,8 +134,8 @@ __global__ __launch_bounds__(NT) void train_cols_kernel(const T *__restrict__ X2
 // Packed row r < rows takes source row src[r] (-1: a zero row) on the columns with
 // inv[f] >= 0 (its place in the packed row of nfp columns, the rest zero).  For a training
 // set (src2) row r goes to the stacked block of its segment, X2 rows first, then AD rows,
-// with |x|^2, x . ad and the molecule's alpha_E; for a query set to row r with |x|^2 and, in
-// dot, 0 times the columns left out: 0, or NaN where one of them is not finite.
+// with |x|^2, x . ad and the molecule's alpha_E; for a query set to row r with |x|^2, NaN where
+// a column left out is not finite.
 template <typename T>
 __global__ __launch_bounds__(NT) void pack_rows_kernel(const T *__restrict__ src,
                                                        const T *__restrict__ src2,
@@ -179,8 +179,8 @@ __global__ __launch_bounds__(NT) void pack_rows_kernel(const T *__restrict__ src
     nn = wave_sum(nn);
     dd = wave_sum(dd);
     if (lane == 0) {
-        n2[r] = nn;
-        dot[r] = dd;
+        n2[r] = src2 ? nn : nn + dd;
+        if (dot) dot[r] = dd;
         if (aEr) aEr[r] = (aE && at >= 0) ? (double)aE[at / ma] : 0.0;
     }
 }
@@ -209,9 +209,8 @@ template <int MF, int NFT, int KW>
 __global__ __launch_bounds__(NT, 2) void coef_kernel(
     const MvSeg *__restrict__ segs, int nseg, int items, const double *__restrict__ Xq, int row0,
     int qrows,
-    const double *__restrict__ nq, const double *__restrict__ zq, const double *__restrict__ P2,
-    const double *__restrict__ n2, const double *__restrict__ rdot,
-    const double *__restrict__ aE, int nfp, double cexp,
+    const double *__restrict__ nq, const double *__restrict__ P2, const double *__restrict__ n2,
+    const double *__restrict__ rdot, const double *__restrict__ aE, int nfp, double cexp,
     double inv_s2, double *__restrict__ T, double *__restrict__ ep, double *__restrict__ wp) {
     __shared__ double red[KW > 1 ? KW : 1][KW > 1 ? MF * NFT * 8 : 1][64];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -295,13 +294,12 @@ __global__ __launch_bounds__(NT, 2) void coef_kernel(
                         pv += red[w][(m * NFT + n) * 8 + 4 + v][lane];
                     }
                 }
-                const int qr = min(q0 + row, qrows - 1);
-                const double q = nq[qr];
+                const double q = nq[min(q0 + row, qrows - 1)];
                 const double d2 = fmax(q + nt - 2.0 * sv, 0.0);
                 const double e = live ? exp(cexp * d2) : 0.0, c = e * inv_s2;
-                // + zq: a query row with an infinity or a NaN in a column that the training
-                // side lacks still gives NaN
-                const double inner = pv - rd + zq[qr];
+                // a query row with an infinity or a NaN in a column that the training side
+                // lacks still gives NaN; an infinite norm alone is a row far away
+                const double inner = q != q ? q : pv - rd;
                 double bco = c * inv_s2 * inner + c * ae;
                 double es = e * ae + c * inner;
                 if (!live) bco = es = 0.0;
@@ -561,7 +559,7 @@ struct MvLayout {
     }
     size_t train_doubles() const { return (size_t)2 * t_rows * nfp + 3 * (size_t)t_rows; }
     size_t query_doubles() const {
-        return (size_t)q_rows * nfp + 2 * (size_t)q_rows + T_len + G_len + 2 * e_len;
+        return (size_t)q_rows * nfp + q_rows + T_len + G_len + 2 * e_len;
     }
     size_t acc_doubles(bool forces) const {
         const size_t natom = (size_t)nm1 * ma1;
@@ -573,7 +571,7 @@ struct MvDev {
     const MvSeg *segs;
     const int *offs, *src1, *src2, *inv, *src0;
     double *P2, *n2, *rdot, *aE;
-    double *Xq, *nq, *zq, *T, *G, *ep, *wp;
+    double *Xq, *nq, *T, *G, *ep, *wp;
     double *erow, *Fat;
 };
 
@@ -715,8 +713,7 @@ MvDev mv_place(const MvLayout &L, char *meta, double *train, double *query, doub
     D.aE = D.rdot + L.t_rows;
     D.Xq = query;
     D.nq = D.Xq + (size_t)L.q_rows * L.nfp;
-    D.zq = D.nq + L.q_rows;
-    D.T = D.zq + L.q_rows;
+    D.T = D.nq + L.q_rows;
     D.G = D.T + L.T_len;
     D.ep = D.G + L.G_len;
     D.wp = D.ep + L.e_len;
@@ -758,14 +755,14 @@ int mv_run(const MvLayout &L, const MvDev &D, const T *X1, const T *dX1, double 
             hipLaunchKernelGGL(pack_rows_kernel<T>, dim3(n), dim3(NT), 0, stream, X1,
                                (const T *)nullptr, D.src1 + R.row0, R.rows, first, L.ma1, L.rep,
                                D.inv, L.nf, L.nfp, segs, R.nseg, (const T *)nullptr, D.Xq, D.nq,
-                               D.zq, (double *)nullptr);
+                               (double *)nullptr, (double *)nullptr);
         });
         if (rc) return rc;
         if (R.items1 > 0) {
             auto coef = [&](auto kern, int per) {
                 hipLaunchKernelGGL(kern, dim3((R.items1 + per - 1) / per), dim3(NT), 0, stream,
-                                   segs, R.nseg, R.items1, D.Xq, R.row0, R.rows, D.nq, D.zq, D.P2,
-                                   D.n2, D.rdot, D.aE, L.nfp, cexp, inv_s2,
+                                   segs, R.nseg, R.items1, D.Xq, R.row0, R.rows, D.nq, D.P2, D.n2,
+                                   D.rdot, D.aE, L.nfp, cexp, inv_s2,
                                    forces ? D.T : (double *)nullptr, D.ep, D.wp);
             };
             if (!R.wide) coef(coef_kernel<1, 1, 4>, 1);
