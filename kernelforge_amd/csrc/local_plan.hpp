@@ -98,23 +98,27 @@ inline RowTable count_rows(const int *Q, const int *N, int nm, int ma,
     constexpr int kStep = 8, kDirect = 256;
     const int n = (nm + kStep - 1) / kStep, L = (int)labels.size();
     at.assign((size_t)L * (n + 1), 0);
-    int direct[kDirect];
-    std::fill(direct, direct + kDirect, -1);
-    for (int l = 0; l < L; ++l)
-        if (labels[l] >= 0 && labels[l] < kDirect) direct[labels[l]] = l;
-    for (int a = 0; a < nm; ++a) {
-        const int na = clamp_atoms(N[a], ma);
-        const int *q = Q + (size_t)a * ma;
-        int *to = at.data() + a / kStep + 1;
-        for (int i = 0; i < na; ++i) {
-            int l;
-            if (q[i] >= 0 && q[i] < kDirect) {
-                l = direct[q[i]];
-            } else {
-                const auto it = std::lower_bound(labels.begin(), labels.end(), q[i]);
-                l = it != labels.end() && *it == q[i] ? int(it - labels.begin()) : -1;
+    // labels in [0, 256) are counted in a table that each group reads and empties, any others
+    // searched for one by one (long long: no alias of Q)
+    long long count[kDirect] = {};
+    for (int k = 0; k < n; ++k) {
+        for (int a = k * kStep, end = std::min(a + kStep, nm); a < end; ++a) {
+            const int na = clamp_atoms(N[a], ma);
+            const int *q = Q + (size_t)a * ma;
+            for (int i = 0; i < na; ++i) {
+                if (q[i] >= 0 && q[i] < kDirect) {
+                    ++count[q[i]];
+                } else {
+                    const auto it = std::lower_bound(labels.begin(), labels.end(), q[i]);
+                    if (it != labels.end() && *it == q[i])
+                        ++at[(size_t)(it - labels.begin()) * (n + 1) + k + 1];
+                }
             }
-            if (l >= 0) ++to[(size_t)l * (n + 1)];
+        }
+        for (int l = 0; l < L; ++l) {
+            if (labels[l] < 0 || labels[l] >= kDirect) continue;
+            at[(size_t)l * (n + 1) + k + 1] = (int)count[labels[l]];
+            count[labels[l]] = 0;
         }
     }
     for (int l = 0; l < L; ++l)

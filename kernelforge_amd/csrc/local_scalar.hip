@@ -1262,8 +1262,8 @@ constexpr long long kDirectPairs = 40000000;
 double shared_columns(int rep) { return windows_masked(rep, 0) ? std::min(rep, 500) : rep; }
 
 // The times of both forms, in microseconds, by what they multiply; the host chooses by them.
-// Fitted to 90 calls with each block size and in both forms (one to 100 atoms a molecule, one
-// to 500 labels, 64 to 2,048 columns, 8e5 to 1.7e9 pairs).  What is chosen is on average 1%
+// Fitted to calls on 101 sets with each block size and in both forms (one to 100 atoms a molecule,
+// one to 500 labels, 64 to 2,048 columns, 8e5 to 1.7e9 pairs).  What is chosen is on average 1%
 // slower than the best of the four, at most 28% (500 molecules with the columns of nine
 // elements), and never more than 2% slower than blocks of 64.
 //
