@@ -445,7 +445,7 @@ __global__ __launch_bounds__(NT, 2) void deriv_vproj_kernel(DerivArgs A, const P
     const int rep = A.rep, x = gp->x, n = gp->n;
     const int nx = clampi(Nx[x], 0, max_), ncx = 3 * nx;
     const int lda = 3 * max_;
-    if (tid < MAXA) qx[tid] = tid < nx ? Qx[(size_t)x * max_ + tid] : -1;
+    if (tid < MAXA) qx[tid] = tid < nx ? Qx[(size_t)x * max_ + tid] : 0;
     if (tid < PG) {
         gy[tid] = tid < n ? gp->y[tid] : 0;
         gslot[tid] = tid < n ? gp->slot[tid] : 0;
@@ -454,7 +454,7 @@ __global__ __launch_bounds__(NT, 2) void deriv_vproj_kernel(DerivArgs A, const P
     __syncthreads();
     {
         const int k = tid >> 5, j = tid & 31;  // 8 x 32 = NT
-        qy[k][j] = (k < n && j < ny[k]) ? Qy[(size_t)gy[k] * may + j] : -2;
+        qy[k][j] = j < ny[k] ? Qy[(size_t)gy[k] * may + j] : 0;
     }
     __syncthreads();
     {
@@ -501,9 +501,10 @@ __global__ __launch_bounds__(NT, 2) void deriv_vproj_kernel(DerivArgs A, const P
         __syncthreads();  // the previous label's columns and atoms consumed
         const int l = qx[i0];
         {
-            // columns: every (k, j) with q_y[k][j] == l, k-major
+            // columns: every (k, j) with q_y[k][j] == l, k-major (j < ny[k]: a label may have any
+            // value, so none can stand for the places past the atoms; ny is 0 past the partners)
             const int k = tid >> 5, j = tid & 31;
-            const bool v = qy[k][j] == l;
+            const bool v = (j < ny[k]) & (qy[k][j] == l);
             const unsigned long long bal = __ballot(v);
             const int pre = __popcll(bal & ((1ull << lane) - 1));
             if (lane == 0) wbase[wv + 1] = __popcll(bal);

@@ -137,6 +137,25 @@ def test_zero_atoms_and_no_shared_labels(lk):
     assert lk.kernel_gaussian_jacobian_t(X, dX, X, Q, Q, N0, N, 1.0).shape == (0, 4)
 
 
+@pytest.mark.parametrize("ma1,ma2", [(5, 9), (30, 6), (9, 30)])
+def test_any_label_value(lk, ma1, ma2):
+    # labels are compared and nothing else: negative ones are labels too, also where molecules
+    # have places past their atoms and a group of partners is not full; the two sets' molecules
+    # may differ in size by any amount
+    X1, dX1, Q1, N1 = rand_set(3, ma1, 20, 3, 5, 1)
+    X2, dX2, Q2, N2 = rand_set(5, ma2, 20, 3, 6, 1)
+    N1[0], N2[-1] = ma1, 2
+    s = 1.6
+    for lab in (np.array([0, -2, -1, 7]), np.array([0, 0, -(2**31), 2**31 - 1])):
+        q1, q2 = lab[Q1].astype(np.int32), lab[Q2].astype(np.int32)
+        got = lk.kernel_gaussian_full(X1, dX1, X2, dX2, q1, q2, N1, N2, s)
+        assert rel_err(got, oracle.full(X1, dX1, X2, dX2, Q1, Q2, N1, N2, s)) < TOL
+        got = lk.kernel_gaussian_hessian(X1, dX1, X2, dX2, q1, q2, N1, N2, s)
+        assert rel_err(got, oracle.hessian(X1, dX1, X2, dX2, Q1, Q2, N1, N2, s)) < TOL
+        got = lk.kernel_gaussian_hessian_symm(X2, dX2, q2, N2, s)
+        assert rel_err(got, oracle.hessian_symm(X2, dX2, Q2, N2, s)) < TOL
+
+
 def test_errors(lk):
     X, dX, Q, N = rand_set(3, 2, 6, 2, 4)
     with pytest.raises(ValueError):
